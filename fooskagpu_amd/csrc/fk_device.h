@@ -89,6 +89,26 @@ __device__ __forceinline__ T clamp_avf(const Mat<T> &m, T a) {
   return fmin(fmax(m.avfMin / 100, a), (T)1.0 - m.avfMin / 100);
 }
 
+// Correctly rounded FP64 quotients x / d for several x: the reciprocal of d
+// to full precision once (hardware estimate, two Newton steps), then each
+// quotient by Markstein's correction of x (1 / d) with the exact residual
+// x - d q: four instructions instead of the twelve of a division.  The bits
+// of x / d while d, x and the quotient stay clear of the ends of the exponent
+// range (|x| > 2^-960; no operand here comes near); div_fixup gives IEEE's
+// results for zeros, infinities and NaN.
+struct Divisor {
+  double d, y;
+  __device__ __forceinline__ explicit Divisor(double v) : d(v) {
+    y = __builtin_amdgcn_rcp(v);
+    y = fma(fma(-v, y, 1.0), y, y);
+    y = fma(fma(-v, y, 1.0), y, y);
+  }
+  __device__ __forceinline__ double operator()(double x) const {
+    const double q = x * y;
+    return __builtin_amdgcn_div_fixup(fma(fma(-d, q, x), y, q), d, x);
+  }
+};
+
 // ---------------- conserved -> primitive (double) ----------------
 // Copies the N doubles of one AoS record into registers with 16-byte loads
 // when N is even (records of 10 doubles start 16-byte aligned): half the
@@ -127,20 +147,22 @@ __device__ __forceinline__ void store_rec(double *__restrict__ p, const double (
 template <int NEQ>
 __device__ __forceinline__ void cons2prim(const Mat<double> &m, const double *U, double *s) {
   if constexpr (NEQ == 5) {
+    const Divisor rho(U[0]);
     s[0] = U[0];
-    s[1] = U[1] / s[0];
-    s[2] = U[2] / s[0];
-    s[3] = U[3] / s[0];
-    s[4] = U[4] / s[0] - 0.5 * (s[1] * s[1] + s[2] * s[2] + s[3] * s[3]);
+    s[1] = rho(U[1]);
+    s[2] = rho(U[2]);
+    s[3] = rho(U[3]);
+    s[4] = rho(U[4]) - 0.5 * (s[1] * s[1] + s[2] * s[2] + s[3] * s[3]);
     s[4] = p1_of(m, s[0], s[4]);
   } else {
     s[0] = clamp_avf(m, U[0]);
     s[1] = U[1] / s[0];
     s[2] = U[2] / (1 - s[0]);
     double rm = s[0] * s[1] + (1 - s[0]) * s[2];
-    s[3] = U[3] / rm;
-    s[4] = U[4] / rm;
-    s[5] = U[5] / rm;
+    const Divisor dm(rm);
+    s[3] = dm(U[3]);
+    s[4] = dm(U[4]);
+    s[5] = dm(U[5]);
     double eL = U[6] / (s[0] * s[1]);
     double eG = U[7] / ((1 - s[0]) * s[2]);
     s[6] = p_of(m, 0, s[1], eL);

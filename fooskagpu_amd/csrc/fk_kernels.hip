@@ -232,7 +232,8 @@ __global__ void __launch_bounds__(kBlock, (sizeof(T) == 8 ? 2 : 1))
     mx[v] = (T)-1e12;
   }
   const T V = (T)vol[c];
-  const T iV = (T)1 / V;  // FP32: one division per cell
+  const T iV = sizeof(T) == 4 ? (T)1 / V : (T)0;  // FP32: one division per cell
+  const fk::Divisor dV((double)V);                // FP64: the shared divisor of the gradient terms
   // The NS slot links are loaded before the face loop and rotated through
   // registers, so each iteration's neighbour gather does not wait on its link
   // load (rolled loop: 6.19 against 6.49 ms mixed, 12.8 against 12.9 ms FP64
@@ -263,13 +264,11 @@ __global__ void __launch_bounds__(kBlock, (sizeof(T) == 8 ? 2 : 1))
     // in the limiter saved another 0.1 ms but moved the bubble collapse's
     // loss of positivity earlier (48^3 mesh: step 33 instead of after 50;
     // the scheme is not positivity preserving there), so those stay as the
-    // reference writes them.
+    // reference writes them.  FP64: the signed normal.
     T nav[3];
-    if constexpr (sizeof(T) == 4) {
-      const T sa = (own ? ga.w : -ga.w) * iV;
+    const T sa = sizeof(T) == 4 ? (own ? ga.w : -ga.w) * iV : (T)(own ? 1 : -1);
 #pragma unroll
-      for (int d = 0; d < 3; ++d) nav[d] = n[d] * sa;
-    }
+    for (int d = 0; d < 3; ++d) nav[d] = n[d] * sa;
     T Wn[NEQ];
     if (nb >= 0) {
       if constexpr (FROMW) {
@@ -296,59 +295,75 @@ __global__ void __launch_bounds__(kBlock, (sizeof(T) == 8 ? 2 : 1))
 #pragma unroll
     for (int v = 0; v < NEQ; ++v) {
       const T o = Wn[v];
-      if (!(mx[v] >= o)) mx[v] = o;
-      if (!(mn[v] <= o)) mn[v] = o;
+      mx[v] = fmax(mx[v], o);
+      mn[v] = fmin(mn[v], o);
       const T avg = (W[v] + Wn[v]) / 2;
       if constexpr (sizeof(T) == 8) {
-        // owner +, neighbour -: (-a) b = -(a b) exactly, so selecting the
-        // sign of the term equals evaluating -avg n A / V (no branch)
+        // ((avg n) A) / V with the sign of the side on n: rounding is
+        // symmetric, so these are the bits of +-(avg n A / V)
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          const T t = avg * n[d] * ga.w / V;
-          g[v][d] += own ? t : -t;
-        }
+        for (int d = 0; d < 3; ++d) g[v][d] += dV(avg * nav[d] * ga.w);
       } else {
 #pragma unroll
         for (int d = 0; d < 3; ++d) g[v][d] = fmaf(avg, nav[d], g[v][d]);
       }
     }
   }
-  // limiter: theta = min over faces of clamp(phi, 0, 1)
+  // Limiter, theta = min over faces of clamp(phi_f, 0, 1), and MUSCL face
+  // states, variable by variable.  phi_f = (mx - W) / (2 d_f) where
+  // d_f = wu_f - W > 0, (mn - W) / (2 d_f) where d_f < 0, 1 where d_f = 0.  A
+  // rounded quotient is monotonic in its divisor, so the smallest clamped
+  // phi_f of either sign is that of the largest |d_f| of that sign: two
+  // divisions per variable instead of one per face, the same bits (a negative
+  // numerator clamps to 0 at every face; a NaN d_f counts as phi = 1, as
+  // before).  Slots past the last face have r = 0, so d = 0 there.  With the
+  // products r g shared by wu and the extrapolation, mixed pass G executes
+  // 1467 instead of 2136 VALU instructions per cell, FP64 (with the gradient's
+  // shared divisor) 2796 instead of 4869: FP64 237 -> 187 us at 1.05M
+  // tetrahedra, 13.4 -> 10.1 us (single-phase) at 12k, mixed 285 -> 272 us at
+  // 3.1M (it is then bound by the bytes it moves) and 64 -> 51 us at 373k
+  // hexahedra.
   T th[NEQ];
-#pragma unroll
-  for (int v = 0; v < NEQ; ++v) th[v] = (T)1e9;
-  // slots past the last face have r = 0: phi = 1 there, which leaves theta
-  // (at most 1 after the first face) unchanged
+  T r[NS][3];
 #pragma unroll
   for (int j = 0; j < NS; ++j) {
-    const V4<T> r = ld4<T>(rvec, c * NS + j);
+    const V4<T> q = ld4<T>(rvec, c * NS + j);
+    r[j][0] = q.x;
+    r[j][1] = q.y;
+    r[j][2] = q.z;
+  }
 #pragma unroll
-    for (int v = 0; v < NEQ; ++v) {
-      const T wu = W[v] + r.x * g[v][0] + r.y * g[v][1] + r.z * g[v][2];
-      T phi;
-      if (wu - W[v] != 0)
-        phi = (wu > W[v]) ? (mx[v] - W[v]) / (2 * (wu - W[v])) : (mn[v] - W[v]) / (2 * (wu - W[v]));
-      else
-        phi = 1;
-      const T tt = fmax((T)0, fmin(phi, (T)1));
-      if (!(th[v] <= tt)) th[v] = tt;
+  for (int v = 0; v < NEQ; ++v) {
+    T dmx = 0, dmn = 0;
+    T ext[NS];
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+      const T px = r[j][0] * g[v][0], py = r[j][1] * g[v][1], pz = r[j][2] * g[v][2];
+      const T d = (W[v] + px + py + pz) - W[v];
+      dmx = fmax(dmx, d);
+      dmn = fmin(dmn, d);
+      ext[j] = px + py + pz;
+    }
+    const T hi = dmx > 0 ? (mx[v] - W[v]) / (2 * dmx) : (T)1;
+    const T lo = dmn < 0 ? (mn[v] - W[v]) / (2 * dmn) : (T)1;
+    th[v] = fmin(fmax((T)0, fmin(hi, (T)1)), fmax((T)0, fmin(lo, (T)1)));
+    // through LDS the records leave whole whatever the order they are
+    // written in; stored directly, each record is written at once below
+    if constexpr (SOUT) {
+#pragma unroll
+      for (int j = 0; j < NS; ++j) reinterpret_cast<T *>(sOut)[threadIdx.x * SPT + j * NEQ + v] = W[v] + th[v] * ext[j];
     }
   }
-  // MUSCL face states
+  if constexpr (!SOUT) {
 #pragma unroll
-  for (int j = 0; j < NS; ++j) {
-    V4<T> r = ld4<T>(rvec, c * NS + j);
-    // r g is also formed by the limiter loop; the empty asm keeps the
-    // compiler from holding those 4 NEQ products in registers until here (it
-    // recomputes them instead): mixed 127 instead of 166 VGPRs, 4 waves per
-    // SIMD, 5.34 against 5.50 ms with the LDS store path (without it, when
-    // the stores bounded the kernel, holding them had measured faster).
-    asm volatile("" : "+v"(r.x), "+v"(r.y), "+v"(r.z));
-    T *out = SOUT ? reinterpret_cast<T *>(sOut) + threadIdx.x * SPT + j * NEQ : face + (c * NS + j) * NEQ;
+    for (int j = 0; j < NS; ++j) {
+      // the empty asm keeps the compiler from holding the 3 NS NEQ products
+      // r g of the loop above in registers until here (it recomputes them)
+      V4<T> q = ld4<T>(rvec, c * NS + j);
+      asm volatile("" : "+v"(q.x), "+v"(q.y), "+v"(q.z));
+      T *out = face + (c * NS + j) * NEQ;
 #pragma unroll
-    for (int v = 0; v < NEQ; ++v) {
-      const T ext = r.x * g[v][0] + r.y * g[v][1] + r.z * g[v][2];
-      out[v] = W[v] + th[v] * ext;
+      for (int v = 0; v < NEQ; ++v) out[v] = W[v] + th[v] * (q.x * g[v][0] + q.y * g[v][1] + q.z * g[v][2]);
     }
   }
   if constexpr (SOUT) {

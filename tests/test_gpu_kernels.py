@@ -1,0 +1,47 @@
+"""Kernel variants at the sizes and values where they can go wrong: edges of
+workgroups, remainders, one-sided and empty slopes, against the FP64 oracle."""
+import numpy as np
+import pytest
+
+from fooskagpu_amd import GpuSolver, Mesh, _lib, cases
+from oracle.pyoracle import Oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def rough_state(neq, n, kind, seed=0):
+    """Positive states without smoothness ("random"), all alike ("uniform":
+    every slope 0) or with one cell raised ("spike": slopes of one sign)."""
+    rng = np.random.default_rng(seed)
+    f = {"random": rng.uniform(0.5, 1.5, (n, neq)), "uniform": np.ones((n, neq)), "spike": np.ones((n, neq))}[kind]
+    if kind == "spike":
+        f[n // 2] = 1.4
+    if neq == 5:
+        return f * [1.0, 0.3, -0.2, 0.1, 2.5]
+    a = 0.5 * f[:, :1]
+    return np.concatenate([a, a * 900 * f[:, 1:2], (1 - a) * 20 * f[:, 2:3], 300 * (f[:, 3:6] - 0.7),
+                           a * 900 * 1.5e6 * f[:, 6:7], (1 - a) * 20 * 2.4e6 * f[:, 7:8], 8e8 * f[:, 8:9],
+                           0.01 * f[:, 9:]], 1)
+
+
+@pytest.mark.parametrize("kind", ["random", "uniform", "spike"])
+@pytest.mark.parametrize("elements", ["tets", "mixed"])
+@pytest.mark.parametrize("model", [_lib.MODEL_SINGLE, _lib.MODEL_TWO_PHASE])
+def test_limiter_and_gradients_are_the_oracles_bits(gpu, model, elements, kind):
+    """Gradients (shared-divisor quotients), limiter (two quotients per
+    variable) and face states: the oracle's operations with the same rounding,
+    so equal bits."""
+    p = dict(cases.BASE) if model == _lib.MODEL_SINGLE else cases._two_phase_params()
+    m = Mesh.box(3, 5, 5, jitter=0.1, seed=5) if elements == "tets" else Mesh.mixed_box(7, 3, 3, jitter=0.1, seed=5)
+    U = rough_state(5 if model == _lib.MODEL_SINGLE else 10, m.n_cells, kind)
+    o = Oracle(p, m, U)
+    o.compute_face_values()
+    with GpuSolver(p, m, U) as g:
+        g.set_debug(True)
+        g.compute_face_values()
+        live = g.download("slots") >= 0
+        for name in ("grad", "theta", "face"):
+            a, b = g.download(name), o.get(name)
+            if name == "face":
+                a, b = a[live], b[live]
+            assert np.array_equal(a, b), (name, np.abs(a - b).max())
