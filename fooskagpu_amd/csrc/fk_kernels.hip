@@ -1008,11 +1008,17 @@ __global__ void __launch_bounds__(kBlock) relax_chem(fk_params P, double *__rest
                                                      unsigned long long *__restrict__ counts, float *__restrict__ W) {
   const int64_t n = (int64_t)counts[5];
   unsigned long long nit = 0;
-  for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < n; e += (int64_t)gridDim.x * kBlock) {
+  // 8 lanes per cell (fk::chem_dev8) up to kChemGroup cells, then one lane
+  const int per = n <= fk::kChemGroup ? 8 : 1;
+  const int64_t nt = (int64_t)gridDim.x * kBlock / per;
+  const bool lead = per == 1 || (threadIdx.x & 7) == 0;
+  for (int64_t e = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / per; e < n; e += nt) {
     const int64_t c = list[e];
     double u[10];
     fk::load_rec<10>(U + c * 10, u);
-    nit += chem_dev(P, u);
+    const int it = per == 8 ? fk::chem_dev8(P, u) : chem_dev(P, u);
+    if (!lead) continue;
+    nit += it;
     U[c * 10 + 0] = u[0];
     U[c * 10 + 1] = u[1];
     U[c * 10 + 2] = u[2];

@@ -535,14 +535,17 @@ __global__ void __launch_bounds__(256) relax_list_k(fk_params P, double *__restr
                                                     int64_t cap, uint32_t *__restrict__ fall) {
   // chunks of 64 entries: the chemical ones from the list's front, then the
   // thermal ones from its back
+  // (up to kPolishGroup of them 4 lanes to an entry, fk::chem_polish4)
   const int64_t nfr = (int64_t)counts[5], nbk = (int64_t)counts[6];
-  const int64_t cf = (nfr + 63) / 64, nchunk = cf + (nbk + 63) / 64;
+  const int per = nfr <= fk::kPolishGroup ? 4 : 1, epw = 64 / per;
+  const int64_t cf = (nfr + epw - 1) / epw, nchunk = cf + (nbk + 63) / 64;
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
   unsigned long long nit = 0, nwarm = 0;
   for (int64_t ch = (int64_t)blockIdx.x * 4 + wv; ch < nchunk; ch += (int64_t)gridDim.x * 4) {
     const bool front = ch < cf;  // wave-uniform
-    const int64_t e = (front ? ch : ch - cf) * 64 + l;
+    const int64_t e = front ? ch * epw + l / per : (ch - cf) * 64 + l;
     const bool live = e < (front ? nfr : nbk);
+    const bool lead = !front || per == 1 || (l & 3) == 0;
     const uint32_t ent = live ? list[front ? e : cap - 1 - e] : 0u;
     const int64_t c = (int64_t)(ent >> 1);
     const int chem = (int)(ent & 1u);
@@ -556,10 +559,10 @@ __global__ void __launch_bounds__(256) relax_list_k(fk_params P, double *__restr
     }
     if (!live) continue;
     if (chem && !WARM) fk::chem_cold(P, u, T0, p0);
-    nwarm += (WARM && chem) ? 1 : 0;
+    nwarm += (WARM && chem && lead) ? 1 : 0;
     int it;
     if (chem) {
-      it = fk::chem_polish(P, u, T0, p0, P.polishTol, 30);
+      it = per == 4 ? fk::chem_polish4(P, u, T0, p0, P.polishTol, 30) : fk::chem_polish(P, u, T0, p0, P.polishTol, 30);
     } else {  // thermal cells: the cell state
       fk::ThermProb t;
       fk::therm_setup(P, u, t);
@@ -567,6 +570,7 @@ __global__ void __launch_bounds__(256) relax_list_k(fk_params P, double *__restr
       fk::therm_cold(P, u, t, rk, ek);
       it = fk::therm_polish(P, u, rk, ek, P.polishTol, 30);
     }
+    if (!lead) continue;
     // a failed polish leaves U as it was: the cell goes to the fallback list
     // (relax_fallback_k runs the reference solve from the cell state)
     const bool failed = it < 0;
@@ -610,12 +614,20 @@ __global__ void __launch_bounds__(256) relax_fallback_k(fk_params P, double *__r
                                                         float *__restrict__ W) {
   const int64_t n = (int64_t)counts[7];
   unsigned long long nit = 0, nfb = 0;
-  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
+  // 8 lanes per cell (fk::chem_dev8, thermal cells on each of them alike) up
+  // to kChemGroup cells, then one lane
+  const int per = n <= fk::kChemGroup ? 8 : 1;
+  const int64_t nt = (int64_t)gridDim.x * 256 / per;
+  const bool lead = per == 1 || (threadIdx.x & 7) == 0;
+  for (int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) / per; e < n; e += nt) {
     const uint32_t ent = fall[e];
     const int64_t c = (int64_t)(ent >> 1);
     double u[10];
     for (int v = 0; v < 10; ++v) u[v] = U[c * 10 + v];
-    const int it = (ent & 1u) ? fk::chem_dev(P, u) : fk::therm_dev(P, u);
+    int it;
+    if (ent & 1u) it = per == 8 ? fk::chem_dev8(P, u) : fk::chem_dev(P, u);
+    else it = fk::therm_dev(P, u);
+    if (!lead) continue;
     nit += 30 + (unsigned long long)it;
     ++nfb;
     for (int v = 0; v < 10; ++v) U[c * 10 + v] = u[v];

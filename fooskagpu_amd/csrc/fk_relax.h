@@ -584,6 +584,32 @@ FK_HD inline int plain_cell(const fk_params &P, double *u, int *iters, int *tsat
 // alpha_L outside (0, 1) -- no two-phase equilibrium at this (rho, e) -- or a
 // phase outside its EOS domain); the caller then falls back to the
 // reference solve.
+FK_HD inline bool chem_commit(const fk_params &P, double *U, double a0, double rho, double rE, double lp, double T) {
+  const double pf = fkmath::exp(lp);
+  const double rl = (pf + P.pInf[0]) / ((P.Cp[0] / P.gamma[0]) * (P.gamma[0] - 1) * T);
+  const double rg = (pf + P.pInf[1]) / ((P.Cp[1] / P.gamma[1]) * (P.gamma[1] - 1) * T);
+  const double aL = (rho - rg) / (rl - rg);
+  if (!(aL > 0 && aL < 1)) return false;
+  const int pm = (1 - a0 > a0) ? 1 : 0, k = 1 - pm;
+  double x[6];
+  x[k] = k == 0 ? aL : 1 - aL;
+  x[k + 2] = k == 0 ? rl : rg;
+  x[k + 4] = ((pf + P.gamma[k] * P.pInf[k]) / (P.gamma[k] - 1) + P.eta[k] * x[k + 2]) / x[k + 2];
+  const double s1 = x[k], s2 = x[k] * x[k + 2], s3 = x[k] * x[k + 2] * x[k + 4];
+  x[pm] = 1 - s1;
+  x[pm + 2] = (rho - s2) / x[pm];
+  x[pm + 4] = (rE - s3) / (x[pm] * x[pm + 2]);
+  if (!(x[pm + 2] > 0)) return false;
+  if (!eos_domain(P, 0, x[2], x[4]) || !eos_domain(P, 1, x[3], x[5])) return false;
+  U[0] = clampd(P, x[0]);
+  U[1] = x[0] * x[2];
+  U[2] = x[1] * x[3];
+  U[6] = x[0] * x[2] * x[4];
+  U[7] = x[1] * x[3] * x[5];
+  U[9] = x[1] * x[3];
+  return true;
+}
+
 FK_HD inline int chem_polish(const fk_params &P, double *U, double T0, double p0, double tol, int itmax) {
   constexpr double kLn10 = 2.302585092994045684;
   const double a0 = clampd(P, U[0]);
@@ -631,31 +657,7 @@ FK_HD inline int chem_polish(const fk_params &P, double *U, double T0, double p0
     lp -= dl;
     T -= dT;
     if (!(T > 0)) return -1;
-    if (fabs(dl) <= tol && fabs(dT) <= tol * T) {
-      const double pf = fkmath::exp(lp);
-      const double rl = (pf + P.pInf[0]) / ((P.Cp[0] / P.gamma[0]) * (P.gamma[0] - 1) * T);
-      const double rg = (pf + P.pInf[1]) / ((P.Cp[1] / P.gamma[1]) * (P.gamma[1] - 1) * T);
-      const double aL = (rho - rg) / (rl - rg);
-      if (!(aL > 0 && aL < 1)) return -1;
-      const int pm = (1 - a0 > a0) ? 1 : 0, k = 1 - pm;
-      double x[6];
-      x[k] = k == 0 ? aL : 1 - aL;
-      x[k + 2] = k == 0 ? rl : rg;
-      x[k + 4] = ((pf + P.gamma[k] * P.pInf[k]) / (P.gamma[k] - 1) + P.eta[k] * x[k + 2]) / x[k + 2];
-      const double s1 = x[k], s2 = x[k] * x[k + 2], s3 = x[k] * x[k + 2] * x[k + 4];
-      x[pm] = 1 - s1;
-      x[pm + 2] = (rho - s2) / x[pm];
-      x[pm + 4] = (rE - s3) / (x[pm] * x[pm + 2]);
-      if (!(x[pm + 2] > 0)) return -1;
-      if (!eos_domain(P, 0, x[2], x[4]) || !eos_domain(P, 1, x[3], x[5])) return -1;
-      U[0] = clampd(P, x[0]);
-      U[1] = x[0] * x[2];
-      U[2] = x[1] * x[3];
-      U[6] = x[0] * x[2] * x[4];
-      U[7] = x[1] * x[3] * x[5];
-      U[9] = x[1] * x[3];
-      return it;
-    }
+    if (fabs(dl) <= tol && fabs(dT) <= tol * T) return chem_commit(P, U, a0, rho, rE, lp, T) ? it : -1;
   }
   return -1;
 }
@@ -672,6 +674,219 @@ FK_HD inline void chem_cold(const fk_params &P, const double *U, double &T0, dou
 }
 
 #if defined(__HIPCC__)
+// ---------------- one cell on several lanes ----------------
+// The listed cells of a step are usually few (tens to thousands), and a
+// reference chemical solve or a polish is one long chain of FP64 operations
+// and logarithms: one cell per lane, a few waves run at the issue rate of one
+// SIMD while the chip idles.  These variants give a cell to a group of lanes
+// that evaluate different residuals (or logarithms) at the same time; every
+// lane of a group holds the same iterate, and each quantity is formed by the
+// same operations as in the one-lane form, so the results are the same bits.
+
+// Up to this many listed cells the groups are used: below, the chip has idle
+// SIMDs and the chain sets the time; above, the redundant work of a group's
+// lanes does.  Reference chemical solve (us, one lane / 8 lanes): 510 cells
+// 356 / 126, 25k 395 / 214, 50k 398 / 313, 119k 531 / 664; its use as fallback
+// of 530 polishes 327 / 84.  Polish (one lane / 4 lanes): network start 510
+// cells 37 / 23, 9.5k 63 / 48, 50k 119 / 103; cell state 9.5k 68 / 49, 25k
+// 85 / 86, 50k 105 / 162.
+constexpr int64_t kChemGroup = 65536, kPolishGroup = 16384;
+
+
+// value of lane L of the quad on every lane of it
+template <int L>
+__device__ __forceinline__ double quad_bcast(double v) {
+  constexpr int ctrl = L | (L << 2) | (L << 4) | (L << 6);  // quad_perm [L, L, L, L]
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+// value of lane l ^ 4
+__device__ __forceinline__ double swap4(double v) {
+  constexpr int pat = (4 << 10) | 0x1f;  // ds_swizzle bit mode: xor 4
+  const int lo = __builtin_amdgcn_ds_swizzle(__double2loint(v), pat);
+  const int hi = __builtin_amdgcn_ds_swizzle(__double2hiint(v), pat);
+  return __hiloint2double(hi, lo);
+}
+
+// chem_dev on 8 lanes: lane bits 0-1 select the residual evaluation of an
+// iteration (the iterate, or unknown 1, 2, 3 perturbed), bit 2 the phase whose
+// pressure, temperature and Gibbs energy the lane forms.  The unknowns are
+// those of the secondary phase, y = (alpha, rho, e); the primary phase follows
+// from the balances.  As in chem_dev an unknown keeps the rounding of adding
+// and removing its perturbation in the evaluations after its own.
+__device__ inline int chem_dev8(const fk_params &P, double *U) {
+  const int l = threadIdx.x & 63, ev = l & 3, ph = (l >> 2) & 1;
+  const double urf = P.chemUrf;
+  const double a0 = clampd(P, U[0]), a1 = 1 - a0;
+  const double r0 = U[1] / a0, r1 = U[2] / a1;
+  const double e0 = U[6] / (a0 * r0), e1 = U[7] / (a1 * r1);
+  const double rhoMix = a0 * r0 + a1 * r1;
+  const double u = U[3] / rhoMix, v = U[4] / rhoMix, w = U[5] / rhoMix;
+  const double rE = U[8] - 0.5 * rhoMix * (u * u + v * v + w * w);
+  const bool k0 = a1 > a0;  // the secondary phase is phase 0
+  const bool mine = (ph == 0) == k0;
+  double y0 = k0 ? a0 : a1, y1 = k0 ? r0 : r1, y2 = k0 ? e0 : e1;
+  double b0 = y0, b1 = y1, b2 = y2;  // best iterate
+  const double g = P.gamma[ph], pi = P.pInf[ph], cp = P.Cp[ph], eta = P.eta[ph], cv = cp / g;
+  int abortFlag = 0, itr = 0;
+  float minRes = 1e9f;
+  bool conv = false;
+  while (!conv) {
+    itr++;
+    const double s0 = fabs(y0) < 1e-9 ? 1e-10 : 1.e-5 * y0;
+    const double s1 = fabs(y1) < 1e-9 ? 1e-10 : 1.e-5 * y1;
+    const double s2 = fabs(y2) < 1e-9 ? 1e-10 : 1.e-5 * y2;
+    const double p0 = y0 + s0, p1 = y1 + s1, p2 = y2 + s2;
+    const double d0 = p0 - s0, d1 = p1 - s1, d2 = p2 - s2;
+    const double a = ev == 0 ? y0 : (ev == 1 ? p0 : d0);
+    const double b = ev <= 1 ? y1 : (ev == 2 ? p1 : d1);
+    const double c = ev <= 2 ? y2 : p2;
+    const double zb0 = 1 - a;
+    const double zb1 = (rhoMix - a * b) / zb0;
+    const double zb2 = (rE - a * b * c) / (zb0 * zb1);
+    const double rho = mine ? b : zb1, en = mine ? c : zb2;
+    const double pr = (g - 1) * rho * en - g * pi - (g - 1) * eta * rho;
+    const double te = (pr + pi) / (cv * (g - 1) * rho);
+    const double lp = P.satConst[0] * fkmath::log10(pr) + P.satConst[1];
+    const double et = ph == 0 ? 0.0 : lp;
+    const double h = cp * te + eta;
+    const double gi = h - te * (cv * (g * fkmath::log10(te) - (g - 1) * fkmath::log10(pr + pi)) + et);
+    const double po = swap4(pr), to = swap4(te), go = swap4(gi);
+    const double f0 = ph == 0 ? pr - po : po - pr, f1 = ph == 0 ? te - to : to - te, f2 = ph == 0 ? gi - go : go - gi;
+    const double r[3] = {quad_bcast<0>(f0), quad_bcast<0>(f1), quad_bcast<0>(f2)};
+    const double se = ev <= 1 ? s0 : (ev == 2 ? s1 : s2);
+    const double c0 = (f0 - r[0]) / se, c1 = (f1 - r[1]) / se, c2 = (f2 - r[2]) / se;
+    const double J[3][3] = {{quad_bcast<1>(c0), quad_bcast<2>(c0), quad_bcast<3>(c0)},
+                            {quad_bcast<1>(c1), quad_bcast<2>(c1), quad_bcast<3>(c1)},
+                            {quad_bcast<1>(c2), quad_bcast<2>(c2), quad_bcast<3>(c2)}};
+    for (int i = 0; i < 3; ++i)
+      for (int j = 0; j < 3; ++j)
+        if (__builtin_isnan(J[i][j])) abortFlag = 1;
+    const double det = J[0][0] * (J[1][1] * J[2][2] - J[1][2] * J[2][1]) - J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
+                       J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0]);
+    if (det == 0) abortFlag = 1;
+    const double id = 1.0 / det;
+    double I[3][3];
+    I[0][0] = id * (J[1][1] * J[2][2] - J[1][2] * J[2][1]);
+    I[0][1] = -id * (J[0][1] * J[2][2] - J[0][2] * J[2][1]);
+    I[0][2] = id * (J[0][1] * J[1][2] - J[0][2] * J[1][1]);
+    I[1][0] = -id * (J[1][0] * J[2][2] - J[1][2] * J[2][0]);
+    I[1][1] = id * (J[0][0] * J[2][2] - J[0][2] * J[2][0]);
+    I[1][2] = -id * (J[0][0] * J[1][2] - J[0][2] * J[1][0]);
+    I[2][0] = id * (J[1][0] * J[2][1] - J[1][1] * J[2][0]);
+    I[2][1] = -id * (J[0][0] * J[2][1] - J[0][1] * J[2][0]);
+    I[2][2] = id * (J[0][0] * J[1][1] - J[0][1] * J[1][0]);
+    // the primary phase of the last evaluation, as chem_dev leaves it
+    const double za = quad_bcast<3>(zb0), zr = quad_bcast<3>(zb1);
+    y0 = d0;
+    y1 = d1;
+    y2 = d2;
+    if (abortFlag == 0 && y0 > 0.0 && y0 < 1.0 && za > 0.0 && za < 1.0 && y1 > 0.0 && zr > 0.0) {
+      const float chk = (float)sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
+      if (chk < minRes) {
+        minRes = chk;
+        b0 = y0;
+        b1 = y1;
+        b2 = y2;
+      }
+    }
+    int abortLocal = abortFlag;
+    double x[3] = {y0, 0.0, y1};  // alpha and rho at chk_update's places
+    double dx = 0;
+    for (int j = 0; j < 3; j++) dx += I[0][j] * r[j];
+    x[0] = x[0] - urf * dx;
+    chk_update(P, x[0] + urf * dx, x, dx, 0, (float)urf, &abortLocal, rhoMix);
+    dx = 0;
+    for (int j = 0; j < 3; j++) dx += I[1][j] * r[j];
+    x[2] = x[2] - urf * dx;
+    chk_update(P, x[2] + urf * dx, x, dx, 2, (float)urf, &abortLocal, rhoMix);
+    dx = 0;
+    for (int j = 0; j < 3; j++) dx += I[2][j] * r[j];
+    y0 = x[0];
+    y1 = x[2];
+    y2 = y2 - urf * dx;
+    if (!(fabs(r[0]) > 1.e-1) && !(fabs(r[1]) > 1.e-1) && !(fabs(r[2]) > 1.e-1)) conv = true;
+    if (abortLocal == 1 || itr > P.chemItrMax) {
+      y0 = b0;
+      y1 = b1;
+      y2 = b2;
+      conv = true;
+    }
+  }
+  const double z0 = 1 - y0;
+  const double z1 = (rhoMix - y0 * y1) / z0;
+  const double z2 = (rE - y0 * y1 * y2) / (z0 * z1);
+  const double x0 = k0 ? y0 : z0, x1 = k0 ? z0 : y0, x2 = k0 ? y1 : z1, x3 = k0 ? z1 : y1;
+  const double x4 = k0 ? y2 : z2, x5 = k0 ? z2 : y2;
+  U[0] = clampd(P, x0);
+  U[1] = x0 * x2;
+  U[2] = x1 * x3;
+  U[6] = x0 * x2 * x4;
+  U[7] = x1 * x3 * x5;
+  U[9] = x1 * x3;
+  return itr;
+}
+
+// chem_polish on 4 lanes: each takes one of an iteration's logarithms (T,
+// p + pinf_L, p + pinf_G, p), and a pair the quantities of one phase.
+__device__ inline int chem_polish4(const fk_params &P, double *U, double T0, double p0, double tol, int itmax) {
+  constexpr double kLn10 = 2.302585092994045684;
+  const int l = threadIdx.x & 3, q = l >> 1;
+  const double a0 = clampd(P, U[0]);
+  const double rho = a0 * (U[1] / a0) + (1 - a0) * (U[2] / (1 - a0));
+  const double u = U[3] / rho, v = U[4] / rho, w = U[5] / rho;
+  const double rE = U[8] - 0.5 * rho * (u * u + v * v + w * w);
+  if (!(T0 > 0) || !__builtin_isfinite(T0) || !__builtin_isfinite(p0)) return -1;
+  const double gm = P.gamma[q], pi = P.pInf[q], cp = P.Cp[q], eta = P.eta[q], cv = cp / gm;
+  const double pia = P.pInf[l == 1 ? 0 : 1];
+  double lp = fkmath::log(fmax(p0, 1.0)), T = T0;
+  for (int it = 1; it <= itmax; ++it) {
+    const double p = fkmath::exp(lp);
+    const double lg = fkmath::log10(l == 0 ? T : (l == 3 ? p : p + pia));
+    const double lT = quad_bcast<0>(lg), lP = quad_bcast<3>(lg), l0 = quad_bcast<1>(lg), l1 = quad_bcast<2>(lg);
+    const double r = (p + pi) / (cv * (gm - 1) * T);
+    const double drp = r / (p + pi);
+    const double drT = -r / T;
+    const double E = (p + gm * pi) / (gm - 1) + eta * r;
+    const double dEp = 1 / (gm - 1) + eta * drp;
+    const double dET = eta * drT;
+    const double et = q == 0 ? 0.0 : P.satConst[0] * lP + P.satConst[1];
+    const double s = cv * (gm * lT - (gm - 1) * (q == 0 ? l0 : l1)) + et;
+    const double g = cp * T + eta - T * s;
+    const double gT = cp - s - cp / kLn10;
+    const double dsp = -cv * (gm - 1) / ((p + pi) * kLn10) + (q == 0 ? 0.0 : P.satConst[0] / (p * kLn10));
+    const double gp = -T * dsp;
+    const double rL = quad_bcast<0>(r), rG = quad_bcast<2>(r);
+    const double dEpL = quad_bcast<0>(dEp), dEpG = quad_bcast<2>(dEp), dETL = quad_bcast<0>(dET), dETG = quad_bcast<2>(dET);
+    const double EL = quad_bcast<0>(E), EG = quad_bcast<2>(E);
+    const double drpL = quad_bcast<0>(drp), drpG = quad_bcast<2>(drp), drTL = quad_bcast<0>(drT), drTG = quad_bcast<2>(drT);
+    const double D = rL - rG;
+    const double al = (rho - rG) / D;
+    const double dap = (-drpG - al * (drpL - drpG)) / D, daT = (-drTG - al * (drTL - drTG)) / D;
+    const double dE = EL - EG;
+    const double R1 = EG + al * dE - rE, R2 = quad_bcast<0>(g) - quad_bcast<2>(g);
+    const double J00 = p * (dEpG + dap * dE + al * (dEpL - dEpG));
+    const double J01 = dETG + daT * dE + al * (dETL - dETG);
+    const double J10 = p * (quad_bcast<0>(gp) - quad_bcast<2>(gp));
+    const double J11 = quad_bcast<0>(gT) - quad_bcast<2>(gT);
+    const double det = J00 * J11 - J01 * J10;
+    if (!(fabs(det) > 0) || !__builtin_isfinite(det)) return -1;
+    double dl = (J11 * R1 - J01 * R2) / det, dT = (J00 * R2 - J10 * R1) / det;
+    if (!__builtin_isfinite(dl) || !__builtin_isfinite(dT)) return -1;
+    const double lim = fmax(fabs(dl), fabs(dT) / (0.2 * T));
+    if (lim > 1) {
+      dl /= lim;
+      dT /= lim;
+    }
+    lp -= dl;
+    T -= dT;
+    if (!(T > 0)) return -1;
+    if (fabs(dl) <= tol && fabs(dT) <= tol * T) return chem_commit(P, U, a0, rho, rE, lp, T) ? it : -1;
+  }
+  return -1;
+}
+
 // Append of cell c to the surrogate relaxation's work list, wave-aggregated:
 // chemical cells from the front (their count in cnt[5]), thermal cells from
 // the back (count in cnt[6], k-th entry at list[cap - 1 - k]); entries are

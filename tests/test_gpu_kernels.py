@@ -45,3 +45,20 @@ def test_limiter_and_gradients_are_the_oracles_bits(gpu, model, elements, kind):
             if name == "face":
                 a, b = a[live], b[live]
             assert np.array_equal(a, b), (name, np.abs(a - b).max())
+
+
+@pytest.mark.parametrize("mode", [_lib.RELAX_PLAIN, _lib.RELAX_COLD])
+def test_relaxation_of_a_cell_does_not_depend_on_the_list_length(gpu, mode):
+    """The listed cells are solved by groups of lanes in short lists and one
+    lane each in long ones (thresholds 65,536 and 16,384): the first cells of
+    a long list against the same cells alone, bit for bit, and the counts."""
+    from fooskagpu_amd import surrogate
+    p = dict(cases._two_phase_params(), relaxFlag=1)
+    big, small = Mesh.box(38, 38, 38), Mesh.box(11, 11, 11)
+    U = surrogate.uniform_states(big.n_cells, p, seed=9)
+    with GpuSolver(p, big, U) as a, GpuSolver(p, small, U[:small.n_cells]) as b:
+        sa, sb = a.relaxation(mode), b.relaxation(mode)
+        Ua, Ub = a.download_state(), b.download_state()
+    print(f"[lists] chemical cells {sa['n_chem']} / {sb['n_chem']}, fallbacks {sa['n_fallback']} / {sb['n_fallback']}")
+    assert sa["n_chem"] > 65536 > 16384 > sb["n_chem"] > 0
+    assert np.array_equal(Ua[:small.n_cells], Ub, equal_nan=True)
