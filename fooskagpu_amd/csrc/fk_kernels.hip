@@ -445,7 +445,7 @@ __global__ void __launch_bounds__(kBlock, (sizeof(T) == 8 ? 2 : 1))
 // just formed, so the state is not read back by a separate kernel: 1 runs
 // stage 1 of the surrogate relaxation (fk::screen_cell), 2 the plain
 // per-cell relaxation (fk::plain_cell).  Cells left for a second kernel go to
-// rlist (1: fk::list_push, lengths in rcnt[5], rcnt[6]; 2: chemical cells,
+// rlist (1: fk::list_push, both lengths in rcnt[5]; 2: chemical cells,
 // length in rcnt[5]); each wave stores its counts in rpart[wave]
 // ([n_chem, iterations], and Tsat iterations for 2); Wout gets the primitive
 // records of the cells relaxed here.
@@ -977,7 +977,6 @@ __global__ void __launch_bounds__(kBlock) relax_therm(fk_params P, int64_t nc, d
                                                       unsigned long long *__restrict__ counts,
                                                       unsigned long long *__restrict__ part, float *__restrict__ W) {
   const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  const int l = threadIdx.x & 63;
   int chem = 0, it = 0, ts = 0;
   if (c < nc) {
     double u[10];
@@ -990,15 +989,7 @@ __global__ void __launch_bounds__(kBlock) relax_therm(fk_params P, int64_t nc, d
       if (W) fk::store_prims<10>(fk::make_mat<double>(P), u, W + c * 10);  // chemical cells: relax_chem
     }
   }
-  const unsigned long long mask = __ballot(chem);
-  const int npush = __popcll(mask);
-  if (npush) {
-    const int leader = __ffsll((long long)mask) - 1;
-    unsigned long long base = 0;
-    if (l == leader) base = atomicAdd(&counts[5], (unsigned long long)npush);
-    base = __shfl(base, leader, 64);
-    if (chem) list[base + __popcll(mask & ((1ull << l) - 1ull))] = (uint32_t)c;
-  }
+  fk::list_push_block(chem != 0, true, (uint32_t)c, list, nc, counts);
   unsigned long long v[3] = {(unsigned long long)chem, (unsigned long long)it, (unsigned long long)ts};
   fk::block_partials<3>(v, part);  // [n_chem, newton iterations, tsat iterations]
 }
@@ -1006,7 +997,7 @@ __global__ void __launch_bounds__(kBlock) relax_therm(fk_params P, int64_t nc, d
 __global__ void __launch_bounds__(kBlock) relax_chem(fk_params P, double *__restrict__ U,
                                                      const uint32_t *__restrict__ list,
                                                      unsigned long long *__restrict__ counts, float *__restrict__ W) {
-  const int64_t n = (int64_t)counts[5];
+  const int64_t n = fk::list_front(counts[5]);
   unsigned long long nit = 0;
   // 8 lanes per cell (fk::chem_dev8) up to kChemGroup cells, then one lane
   const int per = n <= fk::kChemGroup ? 8 : 1;
@@ -1027,8 +1018,7 @@ __global__ void __launch_bounds__(kBlock) relax_chem(fk_params P, double *__rest
     U[c * 10 + 9] = u[9];
     if (W) fk::store_prims<10>(fk::make_mat<double>(P), u, W + c * 10);
   }
-  for (int off = 32; off > 0; off >>= 1) nit += __shfl_down(nit, off, 64);
-  if ((threadIdx.x & 63) == 0 && nit) atomicAdd(&counts[1], nit);
+  fk::block_add(nit, &counts[1]);
 }
 
 // sum_c U_i V_c per block (consCalc.cu:3-34); i = 0 integrates 1 - alpha.

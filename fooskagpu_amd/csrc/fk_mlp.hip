@@ -450,15 +450,14 @@ __global__ void __launch_bounds__(256) mlp_label_k(fk_params P, int64_t n, const
 // (cell << 1) | chem for stage 2.  The last RK stage's fused pass F runs the
 // same stage 1 on the state it produces (fk_kernels.hip).
 // counts: [n_chem, newton iterations, -, fallbacks, warm-started, list
-// length from the front (chemical), list length from the back (thermal),
-// fallback list length].
+// lengths (chemical from the front in the low half, thermal from the back in
+// the high half), -, fallback list length].
 
 __global__ void __launch_bounds__(256) relax_screen_k(fk_params P, int64_t nc, double *__restrict__ U,
                                                       uint32_t *__restrict__ list,
                                                       unsigned long long *__restrict__ counts,
                                                       unsigned long long *__restrict__ part, float *__restrict__ W) {
   const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int l = threadIdx.x & 63;
   int chem = 0, it = 0, push = 0;
   if (c < nc) {
     double u[10];
@@ -473,7 +472,7 @@ __global__ void __launch_bounds__(256) relax_screen_k(fk_params P, int64_t nc, d
     // relax_list_k)
     if (W && !push) fk::store_prims<10>(fk::make_mat<double>(P), u, W + c * 10);
   }
-  fk::list_push(push, chem, c, list, nc, counts);
+  fk::list_push_block(push != 0, chem != 0, (uint32_t)((c << 1) | chem), list, nc, counts);
   unsigned long long v[2] = {(unsigned long long)chem, (unsigned long long)it};
   fk::block_partials<2>(v, part);  // [n_chem, newton iterations]
 }
@@ -491,7 +490,7 @@ __global__ void __launch_bounds__(256) relax_infer_k(fk_params P, const double *
   __shared__ __attribute__((aligned(16))) uint16_t wb[8192];
   __shared__ FwdLds lds[4];
   __shared__ SmallW sw;
-  const int64_t nfr = (int64_t)counts[5];
+  const int64_t nfr = fk::list_front(counts[5]);
   const int64_t cf = (nfr + 63) / 64;
   if ((int64_t)blockIdx.x * 4 >= cf) return;  // whole block idle: skip the weight load
   load_small(w, sw);
@@ -536,7 +535,7 @@ __global__ void __launch_bounds__(256) relax_list_k(fk_params P, double *__restr
   // chunks of 64 entries: the chemical ones from the list's front, then the
   // thermal ones from its back
   // (up to kPolishGroup of them 4 lanes to an entry, fk::chem_polish4)
-  const int64_t nfr = (int64_t)counts[5], nbk = (int64_t)counts[6];
+  const int64_t nfr = fk::list_front(counts[5]), nbk = fk::list_back(counts[5]);
   const int per = nfr <= fk::kPolishGroup ? 4 : 1, epw = 64 / per;
   const int64_t cf = (nfr + epw - 1) / epw, nchunk = cf + (nbk + 63) / 64;
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -592,14 +591,8 @@ __global__ void __launch_bounds__(256) relax_list_k(fk_params P, double *__restr
     U[c * 10 + 9] = u[9];
     if (W) fk::store_prims<10>(fk::make_mat<double>(P), u, W + c * 10);
   }
-  for (int off = 32; off > 0; off >>= 1) {
-    nit += __shfl_down(nit, off, 64);
-    nwarm += __shfl_down(nwarm, off, 64);
-  }
-  if (l == 0) {
-    atomicAdd(&counts[1], nit);
-    atomicAdd(&counts[4], nwarm);
-  }
+  fk::block_add(nit, &counts[1]);
+  fk::block_add(nwarm, &counts[4]);
 }
 
 // Fallback of the surrogate relaxation: the reference solve (thermRlx /

@@ -686,11 +686,11 @@ FK_HD inline void chem_cold(const fk_params &P, const double *U, double &T0, dou
 // Up to this many listed cells the groups are used: below, the chip has idle
 // SIMDs and the chain sets the time; above, the redundant work of a group's
 // lanes does.  Reference chemical solve (us, one lane / 8 lanes): 510 cells
-// 356 / 126, 25k 395 / 214, 50k 398 / 313, 119k 531 / 664; its use as fallback
+// 370 / 124, 25k 390 / 205, 50k 400 / 283, 119k 533 / 611; its use as fallback
 // of 530 polishes 327 / 84.  Polish (one lane / 4 lanes): network start 510
-// cells 37 / 23, 9.5k 63 / 48, 50k 119 / 103; cell state 9.5k 68 / 49, 25k
-// 85 / 86, 50k 105 / 162.
-constexpr int64_t kChemGroup = 65536, kPolishGroup = 16384;
+// cells 34 / 22, 25k 57 / 48, 50k 63 / 53, 119k 73 / 80; cell state 510 cells
+// 45 / 35, 25k 76 / 60, 50k 72 / 69, 119k 88 / 129.
+constexpr int64_t kChemGroup = 65536, kPolishGroup = 49152;
 
 
 // value of lane L of the quad on every lane of it
@@ -887,29 +887,59 @@ __device__ inline int chem_polish4(const fk_params &P, double *U, double T0, dou
   return -1;
 }
 
-// Append of cell c to the surrogate relaxation's work list, wave-aggregated:
-// chemical cells from the front (their count in cnt[5]), thermal cells from
-// the back (count in cnt[6], k-th entry at list[cap - 1 - k]); entries are
-// (c << 1) | chem.  Stage 2 then runs the network on the waves of chemical
-// entries only.  The list order does not affect results: every cell is
-// solved independently.
+// Work list of the relaxation: chemical cells from the front, thermal cells
+// (surrogate only) from the back, k-th entry at list[cap - 1 - k].  Both
+// lengths share one 64-bit counter cnt[5], front in the low half, back in the
+// high half: an append is one atomic.  Appends to one counter retire at about
+// 12 ns each whoever makes them, so that far from equilibrium, where most
+// waves append, they set the time of the kernel: with two atomics per wave
+// stage 1 took 200 us on 511k cells (16k atomics), with one per workgroup 36;
+// stage 2, whose waves added even zero counts, 107 -> 16 us after a step of
+// 3.1M cells with few listed cells (block_add).
+// The list order does not affect results: every cell is solved independently.
+__device__ __forceinline__ int64_t list_front(unsigned long long n) { return (int64_t)(n & 0xffffffffull); }
+__device__ __forceinline__ int64_t list_back(unsigned long long n) { return (int64_t)(n >> 32); }
+
+// Place of this lane's entry given the counter's value before its wave's
+// appends; mf, mb: the wave's lanes that append to the front and to the back.
+__device__ __forceinline__ int64_t list_place(unsigned long long base, unsigned long long mf, unsigned long long mb,
+                                              bool front, int64_t cap) {
+  const unsigned long long below = (1ull << (threadIdx.x & 63)) - 1ull;
+  return front ? list_front(base) + __popcll(mf & below) : cap - 1 - (list_back(base) + __popcll(mb & below));
+}
+
+// Append by the wave (kernels whose waves end on their own): entries are
+// (c << 1) | chem.
 __device__ inline void list_push(bool push, int chem, int64_t c, uint32_t *__restrict__ list, int64_t cap,
                                  unsigned long long *__restrict__ cnt) {
-  const int l = threadIdx.x & 63;
-#pragma unroll
-  for (int side = 0; side < 2; ++side) {
-    const bool mine = push && (side == 0) == (chem != 0);
-    const unsigned long long m = __ballot(mine);
-    if (!m) continue;
-    const int leader = __ffsll((long long)m) - 1;
-    unsigned long long b = 0;
-    if (l == leader) b = atomicAdd(&cnt[5 + side], (unsigned long long)__popcll(m));
-    b = __shfl(b, leader, 64);
-    if (mine) {
-      const int64_t k = (int64_t)(b + (unsigned long long)__popcll(m & ((1ull << l) - 1ull)));
-      list[side == 0 ? k : cap - 1 - k] = (uint32_t)((c << 1) | chem);
-    }
+  const unsigned long long mf = __ballot(push && chem), mb = __ballot(push && !chem);
+  if (!(mf | mb)) return;
+  const int leader = __ffsll((long long)(mf | mb)) - 1;
+  unsigned long long b = 0;
+  if ((int)(threadIdx.x & 63) == leader)
+    b = atomicAdd(&cnt[5], (unsigned long long)__popcll(mf) | ((unsigned long long)__popcll(mb) << 32));
+  b = __shfl(b, leader, 64);
+  if (push) list[list_place(b, mf, mb, chem != 0, cap)] = (uint32_t)((c << 1) | chem);
+}
+
+// Append by a 256-thread workgroup (every thread calls).
+__device__ inline void list_push_block(bool push, bool front, uint32_t entry, uint32_t *__restrict__ list, int64_t cap,
+                                       unsigned long long *__restrict__ cnt) {
+  __shared__ unsigned long long sh[4];
+  __shared__ unsigned long long base;
+  const unsigned long long mf = __ballot(push && front), mb = __ballot(push && !front);
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) sh[w] = (unsigned long long)__popcll(mf) | ((unsigned long long)__popcll(mb) << 32);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned long long n = sh[0] + sh[1] + sh[2] + sh[3];
+    base = n ? atomicAdd(&cnt[5], n) : 0;
   }
+  __syncthreads();
+  if (!push) return;
+  unsigned long long b = base;
+  for (int k = 0; k < w; ++k) b += sh[k];
+  list[list_place(b, mf, mb, front, cap)] = entry;
 }
 #endif
 
@@ -964,6 +994,19 @@ __device__ inline void block_partials(unsigned long long (&v)[K], unsigned long 
     const int k = threadIdx.x;
     part[(int64_t)blockIdx.x * K + k] = sh[0][k] + sh[1][k] + sh[2][k] + sh[3][k];
   }
+}
+
+// cnt += the 256-thread workgroup's sum of v, one atomic if it is not zero.
+__device__ inline void block_add(unsigned long long v, unsigned long long *cnt) {
+  __shared__ unsigned long long sh[4];
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned long long t = sh[0] + sh[1] + sh[2] + sh[3];
+    if (t) atomicAdd(cnt, t);
+  }
+  __syncthreads();
 }
 
 // counts[k] += sum over blocks of part[b][k], k < K.  Each 256-thread block

@@ -50,7 +50,7 @@ def test_limiter_and_gradients_are_the_oracles_bits(gpu, model, elements, kind):
 @pytest.mark.parametrize("mode", [_lib.RELAX_PLAIN, _lib.RELAX_COLD])
 def test_relaxation_of_a_cell_does_not_depend_on_the_list_length(gpu, mode):
     """The listed cells are solved by groups of lanes in short lists and one
-    lane each in long ones (thresholds 65,536 and 16,384): the first cells of
+    lane each in long ones (thresholds 65,536 and 49,152): the first cells of
     a long list against the same cells alone, bit for bit, and the counts."""
     from fooskagpu_amd import surrogate
     p = dict(cases._two_phase_params(), relaxFlag=1)
@@ -60,5 +60,5 @@ def test_relaxation_of_a_cell_does_not_depend_on_the_list_length(gpu, mode):
         sa, sb = a.relaxation(mode), b.relaxation(mode)
         Ua, Ub = a.download_state(), b.download_state()
     print(f"[lists] chemical cells {sa['n_chem']} / {sb['n_chem']}, fallbacks {sa['n_fallback']} / {sb['n_fallback']}")
-    assert sa["n_chem"] > 65536 > 16384 > sb["n_chem"] > 0
+    assert sa["n_chem"] > 65536 > 49152 > sb["n_chem"] > 0
     assert np.array_equal(Ua[:small.n_cells], Ub, equal_nan=True)
