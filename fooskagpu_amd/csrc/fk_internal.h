@@ -36,6 +36,13 @@ struct Timer {
   std::vector<hipEvent_t> pool;
 };
 
+// Events of the large host copies (fk_xfer.h), made by the first one of a
+// context.
+constexpr int kXferThreads = 8;
+struct Xfer {
+  hipEvent_t ev[2 * kXferThreads] = {};
+};
+
 // Surrogate (MLP 3-64-64-64-3) state of a context.
 struct Mlp {
   float *w = nullptr;      // FP32 master parameters [kMlpParams]
@@ -52,7 +59,12 @@ struct Mlp {
   int64_t n_data = 0, cap_data = 0;
   // emission of solver states during plain relaxations
   int64_t emit_stride = 0, emit_phase = 0;
+  // device copies of a label or inference call's inputs and outputs, kept
+  // between calls up to kWorkKeep bytes
+  char *work = nullptr;
+  size_t work_cap = 0;
 };
+constexpr size_t kWorkKeep = (size_t)256 << 20;
 
 }  // namespace fkx
 
@@ -108,6 +120,7 @@ struct fk_ctx {
   bool w_valid = false;
   fkx::Timer tm;
   fkx::Mlp mlp;
+  fkx::Xfer xfer;
   // host geometry kept to rebuild the precision-dependent arrays
   std::vector<double> h_geo, h_r, h_ls;
 };

@@ -40,6 +40,7 @@
 #include "fk_device.h"
 #include "fk_relax.h"
 #include "fk_internal.h"
+#include "fk_xfer.h"
 
 using namespace fkx;
 
@@ -1592,6 +1593,7 @@ int fk_create(int device, const fk_params *p, fk_ctx **out) {
     delete c;
     return fail(FK_EDEVICE, std::string("hipStreamCreate: ") + hipGetErrorString(e));
   }
+  g_xfer.attach();
   *out = c;
   return FK_OK;
 }
@@ -1607,6 +1609,8 @@ int fk_destroy(fk_ctx *c) {
   for (auto e : c->tm.pool) (void)hipEventDestroy(e);
   free_all(c);
   fk_mlp_free(c);
+  xfer_free(c);
+  g_xfer.detach();
   (void)hipStreamDestroy(c->stream);
   delete c;
   return FK_OK;
@@ -1757,7 +1761,8 @@ int fk_upload_state(fk_ctx *c, const double *U) {
   if (!c->have_mesh) return fail(FK_ESTATE, "upload the mesh first");
   HIPCHK(hipSetDevice(c->device));
   c->ia = c->iu0 = 0;
-  HIPCHK(hipMemcpy(c->U[0], U, (size_t)c->nc * c->neq * 8, hipMemcpyHostToDevice));
+  int rc = copy_up(c, c->U[0], U, (size_t)c->nc * c->neq * 8);
+  if (rc) return rc;
   c->have_state = true;
   c->w_valid = false;
   c->rhs_valid = false;
@@ -1769,9 +1774,7 @@ int fk_download_state(fk_ctx *c, double *U) {
   if (rc) return rc;
   if (!U) return fail(FK_EINVAL, "null argument");
   HIPCHK(hipSetDevice(c->device));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  HIPCHK(hipMemcpy(U, c->U[c->ia], (size_t)c->nc * c->neq * 8, hipMemcpyDeviceToHost));
-  return FK_OK;
+  return copy_down(c, U, c->U[c->ia], (size_t)c->nc * c->neq * 8);
 }
 
 int fk_init_rk(fk_ctx *c) {

@@ -30,6 +30,7 @@
 #include "fk_device.h"
 #include "fk_internal.h"
 #include "fk_relax.h"
+#include "fk_xfer.h"
 
 using namespace fkx;
 
@@ -715,6 +716,26 @@ int pack(fk_ctx *c) {
   return FK_OK;
 }
 
+// Device scratch of one label or inference call (m.work); work_done gives a
+// large one back.
+int work_take(fk_ctx *c, size_t bytes) {
+  Mlp &m = c->mlp;
+  if (bytes <= m.work_cap) return FK_OK;
+  if (m.work) (void)hipFree(m.work);
+  m.work = nullptr;
+  m.work_cap = 0;
+  HIPCHK(hipMalloc(&m.work, bytes));
+  m.work_cap = bytes;
+  return FK_OK;
+}
+void work_done(fk_ctx *c) {
+  Mlp &m = c->mlp;
+  if (m.work_cap <= kWorkKeep) return;
+  (void)hipFree(m.work);
+  m.work = nullptr;
+  m.work_cap = 0;
+}
+
 int ensure_data(fk_ctx *c, int64_t cap) {
   Mlp &m = c->mlp;
   if (cap <= m.cap_data) return FK_OK;
@@ -813,7 +834,7 @@ int fk_relax_emit_impl(fk_ctx *c, bool *done) {
 
 void fk_mlp_free(fk_ctx *c) {
   Mlp &m = c->mlp;
-  void *ptrs[] = {m.w, m.m, m.v, m.wb, m.grad, m.part, m.dx, m.dy};
+  void *ptrs[] = {m.w, m.m, m.v, m.wb, m.grad, m.part, m.dx, m.dy, m.work};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   m = Mlp{};
@@ -853,21 +874,20 @@ int fk_mlp_label(fk_ctx *c, const double *U, int64_t n, float *x, float *y) {
   if (c->p.model != FK_MODEL_TWO_PHASE) return fail(FK_EINVAL, "labels need the two-phase model");
   if (n == 0) return FK_OK;
   HIPCHK(hipSetDevice(c->device));
-  double *dU = nullptr;
-  float *dx = nullptr, *dy = nullptr;
-  HIPCHK(hipMalloc(&dU, (size_t)n * 80));
-  HIPCHK(hipMalloc(&dx, (size_t)n * 12));
-  HIPCHK(hipMalloc(&dy, (size_t)n * 12));
-  HIPCHK(hipMemcpy(dU, U, (size_t)n * 80, hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(mlp_label_k, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, c->p, n, dU, dx, dy);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(c->stream));
-  HIPCHK(hipMemcpy(x, dx, (size_t)n * 12, hipMemcpyDeviceToHost));
-  HIPCHK(hipMemcpy(y, dy, (size_t)n * 12, hipMemcpyDeviceToHost));
-  (void)hipFree(dU);
-  (void)hipFree(dx);
-  (void)hipFree(dy);
-  return FK_OK;
+  int rc = work_take(c, (size_t)n * 104);
+  if (rc) return rc;
+  double *dU = reinterpret_cast<double *>(c->mlp.work);
+  float *dx = reinterpret_cast<float *>(dU + n * 10), *dy = dx + n * 3;
+  rc = copy_up(c, dU, U, (size_t)n * 80);
+  if (!rc) {
+    hipLaunchKernelGGL(mlp_label_k, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, c->p, n, dU, dx, dy);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) rc = fail(FK_EDEVICE, std::string("mlp_label: ") + hipGetErrorString(e));
+  }
+  if (!rc) rc = copy_down(c, x, dx, (size_t)n * 12);
+  if (!rc) rc = copy_down(c, y, dy, (size_t)n * 12);
+  work_done(c);
+  return rc;
 }
 
 int fk_mlp_data(fk_ctx *c, const float *x, const float *y, int64_t n, int append) {
@@ -1012,19 +1032,21 @@ int fk_mlp_infer(fk_ctx *c, const float *x, int64_t n, float *y) {
   if (!c->mlp.w) return fail(FK_ESTATE, "no MLP weights");
   if (n == 0) return FK_OK;
   HIPCHK(hipSetDevice(c->device));
-  float *dx = nullptr, *dy = nullptr;
-  HIPCHK(hipMalloc(&dx, (size_t)n * 12));
-  HIPCHK(hipMalloc(&dy, (size_t)n * 12));
-  HIPCHK(hipMemcpy(dx, x, (size_t)n * 12, hipMemcpyHostToDevice));
-  const int64_t nchunk = (n + 63) / 64;
-  const unsigned grid = (unsigned)std::min<int64_t>((nchunk + 3) / 4, 4096);
-  hipLaunchKernelGGL(mlp_infer_k, dim3(grid), dim3(256), 0, c->stream, n, dx, dy, c->mlp.w, c->mlp.wb, norm_of(c->mlp));
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(c->stream));
-  HIPCHK(hipMemcpy(y, dy, (size_t)n * 12, hipMemcpyDeviceToHost));
-  (void)hipFree(dx);
-  (void)hipFree(dy);
-  return FK_OK;
+  int rc = work_take(c, (size_t)n * 24);
+  if (rc) return rc;
+  float *dx = reinterpret_cast<float *>(c->mlp.work), *dy = dx + n * 3;
+  rc = copy_up(c, dx, x, (size_t)n * 12);
+  if (!rc) {
+    const int64_t nchunk = (n + 63) / 64;
+    const unsigned grid = (unsigned)std::min<int64_t>((nchunk + 3) / 4, 4096);
+    hipLaunchKernelGGL(mlp_infer_k, dim3(grid), dim3(256), 0, c->stream, n, dx, dy, c->mlp.w, c->mlp.wb,
+                       norm_of(c->mlp));
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) rc = fail(FK_EDEVICE, std::string("mlp_infer: ") + hipGetErrorString(e));
+  }
+  if (!rc) rc = copy_down(c, y, dy, (size_t)n * 12);
+  work_done(c);
+  return rc;
 }
 
 }  // extern "C"

@@ -62,3 +62,40 @@ def test_relaxation_of_a_cell_does_not_depend_on_the_list_length(gpu, mode):
     print(f"[lists] chemical cells {sa['n_chem']} / {sb['n_chem']}, fallbacks {sa['n_fallback']} / {sb['n_fallback']}")
     assert sa["n_chem"] > 65536 > 49152 > sb["n_chem"] > 0
     assert np.array_equal(Ua[:small.n_cells], Ub, equal_nan=True)
+
+
+@pytest.mark.parametrize("n", [9, 25, 34, 50])
+def test_states_pass_through_the_copies_unchanged(gpu, n):
+    """Uploads and downloads below, between and above the sizes where they go
+    through page-locked slots (5 MB down, 48 MB up; slots of 1, 2 and 4 MB,
+    last slot partly filled): bytes are bytes."""
+    m = Mesh.box(n, n, n, rcm=False)
+    U = np.random.default_rng(n).uniform(0.1, 1, (m.n_cells, 10))
+    with GpuSolver(cases._two_phase_params(), m, U) as g:
+        print(f"[copies] {U.nbytes} bytes", flush=True)
+        assert np.array_equal(g.download_state(), U)
+        g.upload_state(2 * U)
+        assert np.array_equal(g.download_state(), 2 * U)
+
+
+def test_copies_of_several_threads(gpu):
+    """The page-locked slots are lent to one copy at a time: contexts that
+    copy from several threads at once all get their own bytes."""
+    import threading
+    m = Mesh.box(26, 26, 26, rcm=False)
+    wrong = []
+
+    def work(k):
+        U = np.full((m.n_cells, 10), float(k + 1))
+        with GpuSolver(cases._two_phase_params(), m, U) as g:
+            for _ in range(4):
+                g.upload_state(U)
+                if not np.array_equal(g.download_state(), U):
+                    wrong.append(k)
+
+    th = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not wrong
