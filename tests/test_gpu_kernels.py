@@ -99,3 +99,35 @@ def test_copies_of_several_threads(gpu):
     for t in th:
         t.join()
     assert not wrong
+
+
+@pytest.mark.parametrize("batch", [1, 31, 33, 1057])
+def test_training_step_is_adam_on_the_gradient(gpu, batch):
+    """One training step on device-drawn samples (splitmix64 of the seed)
+    against Adam in NumPy on fk_mlp_grad's gradient of the same samples, at
+    batches that leave blocks of 32 samples and runs of 32 partials part
+    full.  The step's arithmetic is FP32 with the operations of the formula:
+    a few ulp (the device's square root and division, 1 ulp each) of the
+    update lr = 2e-3, far below 1e-6."""
+    from fooskagpu_amd import surrogate
+    rng = np.random.default_rng(batch)
+    n, seed = 777, 12345
+    x = rng.normal(size=(n, 3)).astype(np.float32)
+    y = rng.normal(size=(n, 3)).astype(np.float32)
+    z = np.uint64(seed) + np.arange(1, batch + 1, dtype=np.uint64) * np.uint64(0x9E3779B97F4A7C15)
+    z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+    z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+    idx = ((z ^ (z >> np.uint64(31))) % np.uint64(n)).astype(np.int64)
+    w0, norm = surrogate.init_weights(2), surrogate.fit_norm(x, y)
+    with GpuSolver(cases._two_phase_params()) as g:
+        sg = surrogate.Surrogate(g)
+        sg.set_data(x, y)
+        sg.set_weights(w0, norm)
+        grad, loss = sg.grad(idx)
+        l0, l1 = sg.train(1, batch=batch, lr=2e-3, seed=seed)
+        w1 = sg.weights()[0]
+    gr = grad.astype(np.float64)
+    want = w0 - 2e-3 * gr / (np.sqrt(gr * gr) + 1e-8)  # first step: m / (1 - b1) = g, v / (1 - b2) = g^2
+    print(f"[train] batch {batch}: loss {loss:.5f} {l0:.5f}, max |dw| {np.abs(w1 - want).max():.2e}")
+    assert l0 == l1 == loss
+    assert np.abs(w1 - want).max() < 1e-6
