@@ -89,6 +89,16 @@ __device__ __forceinline__ T clamp_avf(const Mat<T> &m, T a) {
   return fmin(fmax(m.avfMin / 100, a), (T)1.0 - m.avfMin / 100);
 }
 
+// FP32 quotient a / b as mantissa times hardware reciprocal (about 1 ulp): the
+// form the build's flags give a division, unless the compiler moves it out of
+// a condition and so loses the licence for it.  Written out where two kernels
+// have to give the same bits.
+__device__ __forceinline__ float quot(float a, float b) {
+  const float q = __builtin_amdgcn_frexp_mantf(a) * __builtin_amdgcn_rcpf(__builtin_amdgcn_frexp_mantf(b));
+  return ldexpf(q, __builtin_amdgcn_frexp_expf(a) - __builtin_amdgcn_frexp_expf(b));
+}
+__device__ __forceinline__ double quot(double a, double b) { return a / b; }
+
 // Correctly rounded FP64 quotients x / d for several x: the reciprocal of d
 // to full precision once (hardware estimate, two Newton steps), then each
 // quotient by Markstein's correction of x (1 / d) with the exact residual

@@ -108,10 +108,10 @@ struct fk_ctx {
   bool rhs_valid = false;
   bool rhs_f32 = false;      // c->rhs holds FP32 values (mixed dt stage, pass F MODE 1)
   bool fuse_update = true;   // RK update inside pass F (else residual + rk_update)
-  bool stage_f = true;       // pass F stages the workgroup's face states in LDS (tetrahedral meshes)
+  int stage_f = 1;           // pass F: 0 one lane per cell, 2 with LDS staging, 1 by size (or four lanes per cell)
   bool prims_w = true;       // mixed: producers of U also write wprim, pass G reads it
   bool fuse_relax = true;    // per-cell relaxation pass inside the last fused pass F
-  bool stage_g = true;       // mixed pass G writes its face records through LDS (4 slots per cell)
+  int stage_g = 1;           // pass G: 0 direct stores, 2 face records through LDS, 1 by size (or four lanes per cell)
   int64_t pf_waves = 0;      // waves of the last pass F launch (its per-wave relaxation counts)
   // FP32 primitive records [C][NEQ] of U[ia] (mixed precision), valid while
   // w_valid: set by the kernels that write them with a new state, cleared by

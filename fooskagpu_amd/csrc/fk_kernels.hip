@@ -126,6 +126,45 @@ __device__ __forceinline__ int link_of(T w) {
   else return (int)w;
 }
 
+// Gradient row of the viscous pass: velocity gradient, and with the heat flux
+// the temperature gradient.
+template <int NEQ, typename T, bool HEAT>
+__device__ __forceinline__ void store_grad(const fk_params &P, const T (&W)[NEQ], const T (&g)[NEQ][3], T *G) {
+  constexpr int iu = Model<NEQ>::iu;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) G[i * 3 + d] = g[iu + i][d];
+  if constexpr (HEAT) {
+    const T gm = (T)P.gamma[0];
+    // FP32 path: W[4] is the deviation from pRef, absolute p = W[4] + pRef
+    const T pi = sizeof(T) == 4 ? (T)(P.pInf[0] + P.pRef) : (T)P.pInf[0];
+    const T R = (T)P.Cp[0] * (gm - 1) / gm;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) G[9 + d] = (g[4][d] - ((W[4] + pi) / W[0]) * g[0][d]) / (W[0] * R);
+  }
+}
+
+// RK stage irk of one cell from its residual (update.cu:19-103), in the
+// operation order of rk_update.
+template <int NEQ>
+__device__ __forceinline__ void rk_stage(const fk_params &P, int irk, double dt, double Vc, const double *uc,
+                                         const double *__restrict__ U0, const double *r, double (&un)[NEQ]) {
+  constexpr int iz = NEQ == 5 ? 3 : 5;
+  double u0[NEQ];
+  if (P.rkSteps != 1) fk::load_rec<NEQ>(U0, u0);
+#pragma unroll
+  for (int v = 0; v < NEQ; ++v) {
+    const int neglect = (v == iz && P.neglectZ == 1);
+    double u;
+    if (P.rkSteps == 1) u = (1 - neglect) * (uc[v] + dt * (1.0 / Vc) * r[v]);
+    else if (irk == 0) u = (1 - neglect) * (u0[v] + dt * (1.0 / Vc) * r[v]);
+    else if (irk == 1) u = (1 - neglect) * ((3.0 / 4.0) * u0[v] + (1.0 / 4.0) * uc[v] + (1.0 / 4.0) * dt * (1.0 / Vc) * r[v]);
+    else u = (1 - neglect) * ((1.0 / 3.0) * u0[v] + (2.0 / 3.0) * uc[v] + (2.0 / 3.0) * dt * (1.0 / Vc) * r[v]);
+    un[v] = u;
+  }
+}
+
 // Pass G: first-order states, Green-Gauss gradient, neighbour min/max,
 // limiter and MUSCL face states (computePrimVec.cu:38-80,
 // computeGrad.cu:51-91, computeFaceValues.cu:29-113).  Every cell converts
@@ -345,8 +384,8 @@ __global__ void __launch_bounds__(kBlock, (sizeof(T) == 8 ? 2 : 1))
       dmn = fmin(dmn, d);
       ext[j] = px + py + pz;
     }
-    const T hi = dmx > 0 ? (mx[v] - W[v]) / (2 * dmx) : (T)1;
-    const T lo = dmn < 0 ? (mn[v] - W[v]) / (2 * dmn) : (T)1;
+    const T hi = dmx > 0 ? fk::quot(mx[v] - W[v], 2 * dmx) : (T)1;
+    const T lo = dmn < 0 ? fk::quot(mn[v] - W[v], 2 * dmn) : (T)1;
     th[v] = fmin(fmax((T)0, fmin(hi, (T)1)), fmax((T)0, fmin(lo, (T)1)));
     // through LDS the records leave whole whatever the order they are
     // written in; stored directly, each record is written at once below
@@ -388,24 +427,11 @@ __global__ void __launch_bounds__(kBlock, (sizeof(T) == 8 ? 2 : 1))
     }
   }
   if constexpr (VISC) {
-    constexpr int iu = Model<NEQ>::iu;
     constexpr int NG = ngrad<NEQ, HEAT>();
     // SOUT: the gradient rows go through the same LDS (after the face copy
     // has read it), stride NG, and out as the block's contiguous range
     if constexpr (SOUT) __syncthreads();
-    T *G = SOUT ? reinterpret_cast<T *>(sOut) + threadIdx.x * NG : gvel + c * NG;
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int d = 0; d < 3; ++d) G[i * 3 + d] = g[iu + i][d];
-    if constexpr (HEAT) {
-      const T gm = (T)P.gamma[0];
-      // FP32 path: W[4] is the deviation from pRef, absolute p = W[4] + pRef
-      const T pi = sizeof(T) == 4 ? (T)(P.pInf[0] + P.pRef) : (T)P.pInf[0];
-      const T R = (T)P.Cp[0] * (gm - 1) / gm;
-#pragma unroll
-      for (int d = 0; d < 3; ++d) G[9 + d] = (g[4][d] - ((W[4] + pi) / W[0]) * g[0][d]) / (W[0] * R);
-    }
+    store_grad<NEQ, T, HEAT>(P, W, g, SOUT ? reinterpret_cast<T *>(sOut) + threadIdx.x * NG : gvel + c * NG);
     if constexpr (SOUT) {
       __syncthreads();
       const int64_t ncell = (nc - c0) < GB ? (nc - c0) : GB;
@@ -421,6 +447,139 @@ __global__ void __launch_bounds__(kBlock, (sizeof(T) == 8 ? 2 : 1))
       dtheta[c * NEQ + v] = (double)th[v];
 #pragma unroll
       for (int d = 0; d < 3; ++d) dgrad[(c * NEQ + v) * 3 + d] = (double)g[v][d];
+    }
+  }
+}
+
+// Side terms of a cell (fluxSource / computeCenterPress, two-phase).
+template <typename T>
+struct CellSide {
+  T avf = 0, pLiq = 0, pGas = 0;
+  double pCd = 0;
+};
+template <int NEQ, typename T>
+__device__ __forceinline__ CellSide<T> cell_side(const fk::Mat<double> &md, const double *Uc) {
+  CellSide<T> cs;
+  if constexpr (NEQ == 10) {
+    const double a = fk::clamp_avf(md, Uc[0]);
+    const double rl = Uc[1] / a, rg = Uc[2] / (1 - a);
+    const double el = Uc[6] / (a * rl), eg = Uc[7] / ((1 - a) * rg);
+    const double pl = fk::p_of(md, 0, rl, el), pg = fk::p_of(md, 1, rg, eg);
+    cs.pCd = a * pl + (1 - a) * pg;
+    cs.avf = (T)a;
+    cs.pLiq = (T)pl;
+    cs.pGas = (T)pg;
+  }
+  return cs;
+}
+
+// Terms of one face for one of its cells: adds the inviscid and
+// non-conservative terms to rhs, the viscous ones to rv, and (SIG) raises sig
+// to the face's signal speed.  L, R: face states (owner, neighbour or ghost);
+// Gc, Gn: velocity gradients of this cell and the neighbour; wls: WALE width
+// of the slot; Wc1: first-order state of this cell.
+template <int NEQ, typename T, bool VISC, bool HEAT, bool SIG>
+__device__ __forceinline__ void face_terms(const fk_params &P, const fk::Mat<T> &mt, const CellSide<T> &cs, int nb,
+                                           bool own, const T (&n)[3], T A, const T (&L)[NEQ], const T (&R)[NEQ],
+                                           const T *Gc, const T *Gn, const T *wls, const T (&Wc1)[NEQ],
+                                           double (&rhs)[NEQ], double (&rv)[5], T &sig) {
+  constexpr int iu = Model<NEQ>::iu;
+  fk::FaceRes<T, NEQ> fr;
+  fk::riemann<NEQ, T>(mt, L, R, n, nb == -5, fr);
+  if constexpr (NEQ == 5) {
+#pragma unroll
+    for (int v = 0; v < 5; ++v) rhs[v] += (double)(own ? -fr.f[v] * A : fr.f[v] * A);
+  } else {
+    const T sign = own ? (T)-1.0 : (T)1.0;
+    const T *u = fr.unc;
+    const T nc0 = cs.avf * u[0] * n[0] + cs.avf * u[1] * n[1] + cs.avf * u[2] * n[2];
+    const T nc1 = cs.avf * cs.pLiq * u[0] * n[0] + cs.avf * cs.pLiq * u[1] * n[1] + cs.avf * cs.pLiq * u[2] * n[2];
+    const T nc2 = (1 - cs.avf) * cs.pGas * u[0] * n[0] + (1 - cs.avf) * cs.pGas * u[1] * n[1] + (1 - cs.avf) * cs.pGas * u[2] * n[2];
+    T Pc;
+    if constexpr (sizeof(T) == 8) Pc = fr.pF - (T)cs.pCd;
+    else Pc = (T)((double)fr.pF - cs.pCd);
+    rhs[0] += (double)(sign * (fr.f[0] - nc0) * A);
+    rhs[1] += (double)(sign * (fr.f[1]) * A);
+    rhs[2] += (double)(sign * (fr.f[2]) * A);
+    rhs[3] += (double)(sign * (fr.f[3] + Pc * n[0]) * A);
+    rhs[4] += (double)(sign * (fr.f[4] + Pc * n[1]) * A);
+    rhs[5] += (double)(sign * (fr.f[5] + Pc * n[2]) * A);
+    rhs[6] += (double)(sign * (fr.f[6] + nc1) * A);
+    rhs[7] += (double)(sign * (fr.f[7] + nc2) * A);
+    rhs[8] += (double)(sign * (fr.f[8]) * A);
+    rhs[9] += (double)(sign * (fr.f[9]) * A);
+  }
+  if constexpr (SIG) {
+    const T cl = fk::signal<NEQ, T>(mt, L, n);
+    const T cr = nb >= 0 ? fk::signal<NEQ, T>(mt, R, n) : (T)0.0;
+    const T cm = fmax(cl, cr);
+    if (!(sig >= cm)) sig = cm;
+  }
+  if constexpr (VISC) {
+    if (nb < 0) Gn = Gc;
+    const T *G0 = own ? Gc : Gn;  // owner's gradient first, as (g_o + g_n)/2
+    const T *G1 = own ? Gn : Gc;
+    T gm[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) gm[i][d] = (G0[i * 3 + d] + G1[i * 3 + d]) / 2;
+    T eddy = 0;
+    if (P.turbulence == 1) eddy = fk::wale<T>(gm, *wls);
+    const T ux = gm[0][0], uy = gm[0][1], uz = gm[0][2], vx = gm[1][0], vy = gm[1][1], vz = gm[1][2];
+    const T wx = gm[2][0], wy = gm[2][1], wz = gm[2][2];
+    T st[3][3];
+    st[0][0] = (2 * ux - (T)(2.0 / 3.0) * (ux + vy + wz));
+    st[1][1] = (2 * vy - (T)(2.0 / 3.0) * (ux + vy + wz));
+    st[2][2] = (2 * wz - (T)(2.0 / 3.0) * (ux + vy + wz));
+    st[0][1] = st[1][0] = (uy + vx);
+    st[0][2] = st[2][0] = (uz + wx);
+    st[1][2] = st[2][1] = (vz + wy);
+    // side-1 state: reconstructed neighbour, or the first-order ghost on boundaries
+    T R1[NEQ];
+    if (nb >= 0) {
+#pragma unroll
+      for (int v = 0; v < NEQ; ++v) R1[v] = R[v];
+    } else {
+#pragma unroll
+      for (int v = 0; v < NEQ; ++v) R1[v] = Wc1[v];
+      fk::ghost<NEQ, T>(mt, -nb, n, R1);
+    }
+    T mu;
+    if constexpr (NEQ == 5) {
+      const T rhoF = (L[0] + R1[0]) / 2;
+      mu = mt.mu[0] + rhoF * eddy;
+    } else {
+      const T a1 = L[0], r1 = a1 * L[1] + (1 - a1) * L[2];
+      const T a2 = R1[0], r2 = a2 * R1[1] + (1 - a2) * R1[2];
+      const T rhoF = (r1 + r2) / 2, avfF = (a1 + a2) / 2;
+      mu = avfF * mt.mu[0] + (1 - avfF) * mt.mu[1] + rhoF * eddy;
+    }
+    T fm[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) fm[i] = (mu * st[i][0]) * n[0] + (mu * st[i][1]) * n[1] + (mu * st[i][2]) * n[2];
+    T vf[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) vf[i] = (L[iu + i] + R1[iu + i]) / 2;
+    T fe[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      T stv = 0;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) stv += st[i][d] * vf[d];
+      fe[i] = (mu * stv) * n[i];
+    }
+    const T en = fe[0] + fe[1] + fe[2];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) rv[i] += (double)(own ? fm[i] * A : -(fm[i]) * A);
+    rv[3] += (double)(own ? en * A : -(en) * A);
+    if constexpr (HEAT) {
+      const T k = mt.cp[0] * mu / mt.Pr0;
+      T gf[3];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) gf[d] = (G0[9 + d] + G1[9 + d]) / 2;
+      const T q = k * (gf[0] * n[0] + gf[1] * n[1] + gf[2] * n[2]);
+      rv[4] += (double)(own ? q * A : -(q) * A);
     }
   }
 }
@@ -575,19 +734,7 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
       }
     }
   }
-  // side terms of this cell (fluxSource / computeCenterPress, two-phase)
-  T avf = 0, pLiq = 0, pGas = 0;
-  double pCd = 0;
-  if constexpr (NEQ == 10) {
-    const double a = fk::clamp_avf(md, Uc[0]);
-    const double rl = Uc[1] / a, rg = Uc[2] / (1 - a);
-    const double el = Uc[6] / (a * rl), eg = Uc[7] / ((1 - a) * rg);
-    const double pl = fk::p_of(md, 0, rl, el), pg = fk::p_of(md, 1, rg, eg);
-    pCd = a * pl + (1 - a) * pg;
-    avf = (T)a;
-    pLiq = (T)pl;
-    pGas = (T)pg;
-  }
+  const CellSide<T> cs = cell_side<NEQ, T>(md, Uc);
   double rhs[NEQ];
 #pragma unroll
   for (int v = 0; v < NEQ; ++v) rhs[v] = 0.0;
@@ -641,105 +788,8 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
       for (int v = 0; v < NEQ; ++v) L[v] = R[v] = Fs[v];
       fk::ghost<NEQ, T>(mt, -nb, n, R);
     }
-    fk::FaceRes<T, NEQ> fr;
-    fk::riemann<NEQ, T>(mt, L, R, n, nb == -5, fr);
-    if constexpr (NEQ == 5) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v) rhs[v] += (double)(own ? -fr.f[v] * A : fr.f[v] * A);
-    } else {
-      const T sign = own ? (T)-1.0 : (T)1.0;
-      const T *u = fr.unc;
-      const T nc0 = avf * u[0] * n[0] + avf * u[1] * n[1] + avf * u[2] * n[2];
-      const T nc1 = avf * pLiq * u[0] * n[0] + avf * pLiq * u[1] * n[1] + avf * pLiq * u[2] * n[2];
-      const T nc2 = (1 - avf) * pGas * u[0] * n[0] + (1 - avf) * pGas * u[1] * n[1] + (1 - avf) * pGas * u[2] * n[2];
-      T Pc;
-      if constexpr (sizeof(T) == 8) Pc = fr.pF - (T)pCd;
-      else Pc = (T)((double)fr.pF - pCd);
-      rhs[0] += (double)(sign * (fr.f[0] - nc0) * A);
-      rhs[1] += (double)(sign * (fr.f[1]) * A);
-      rhs[2] += (double)(sign * (fr.f[2]) * A);
-      rhs[3] += (double)(sign * (fr.f[3] + Pc * n[0]) * A);
-      rhs[4] += (double)(sign * (fr.f[4] + Pc * n[1]) * A);
-      rhs[5] += (double)(sign * (fr.f[5] + Pc * n[2]) * A);
-      rhs[6] += (double)(sign * (fr.f[6] + nc1) * A);
-      rhs[7] += (double)(sign * (fr.f[7] + nc2) * A);
-      rhs[8] += (double)(sign * (fr.f[8]) * A);
-      rhs[9] += (double)(sign * (fr.f[9]) * A);
-    }
-    if constexpr (MODE == 1) {
-      const T cl = fk::signal<NEQ, T>(mt, L, n);
-      const T cr = nb >= 0 ? fk::signal<NEQ, T>(mt, R, n) : (T)0.0;
-      const T cm = fmax(cl, cr);
-      if (!(sig >= cm)) sig = cm;
-    }
-    if constexpr (VISC) {
-      const T *Gc = grad_ptr(c);
-      const T *Gn = nb >= 0 ? grad_ptr(nb) : Gc;
-      const T *G0 = own ? Gc : Gn;  // owner's gradient first, as (g_o + g_n)/2
-      const T *G1 = own ? Gn : Gc;
-      T gm[3][3];
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) gm[i][d] = (G0[i * 3 + d] + G1[i * 3 + d]) / 2;
-      T eddy = 0;
-      if (P.turbulence == 1) eddy = fk::wale<T>(gm, wls[s]);
-      const T ux = gm[0][0], uy = gm[0][1], uz = gm[0][2], vx = gm[1][0], vy = gm[1][1], vz = gm[1][2];
-      const T wx = gm[2][0], wy = gm[2][1], wz = gm[2][2];
-      T st[3][3];
-      st[0][0] = (2 * ux - (T)(2.0 / 3.0) * (ux + vy + wz));
-      st[1][1] = (2 * vy - (T)(2.0 / 3.0) * (ux + vy + wz));
-      st[2][2] = (2 * wz - (T)(2.0 / 3.0) * (ux + vy + wz));
-      st[0][1] = st[1][0] = (uy + vx);
-      st[0][2] = st[2][0] = (uz + wx);
-      st[1][2] = st[2][1] = (vz + wy);
-      // side-1 state: reconstructed neighbour, or the first-order ghost on boundaries
-      T R1[NEQ];
-      if (nb >= 0) {
-#pragma unroll
-        for (int v = 0; v < NEQ; ++v) R1[v] = R[v];
-      } else {
-#pragma unroll
-        for (int v = 0; v < NEQ; ++v) R1[v] = Wc1[v];
-        fk::ghost<NEQ, T>(mt, -nb, n, R1);
-      }
-      T mu;
-      if constexpr (NEQ == 5) {
-        const T rhoF = (L[0] + R1[0]) / 2;
-        mu = mt.mu[0] + rhoF * eddy;
-      } else {
-        const T a1 = L[0], r1 = a1 * L[1] + (1 - a1) * L[2];
-        const T a2 = R1[0], r2 = a2 * R1[1] + (1 - a2) * R1[2];
-        const T rhoF = (r1 + r2) / 2, avfF = (a1 + a2) / 2;
-        mu = avfF * mt.mu[0] + (1 - avfF) * mt.mu[1] + rhoF * eddy;
-      }
-      T fm[3];
-#pragma unroll
-      for (int i = 0; i < 3; ++i) fm[i] = (mu * st[i][0]) * n[0] + (mu * st[i][1]) * n[1] + (mu * st[i][2]) * n[2];
-      T vf[3];
-#pragma unroll
-      for (int i = 0; i < 3; ++i) vf[i] = (L[iu + i] + R1[iu + i]) / 2;
-      T fe[3];
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        T stv = 0;
-#pragma unroll
-        for (int d = 0; d < 3; ++d) stv += st[i][d] * vf[d];
-        fe[i] = (mu * stv) * n[i];
-      }
-      const T en = fe[0] + fe[1] + fe[2];
-#pragma unroll
-      for (int i = 0; i < 3; ++i) rv[i] += (double)(own ? fm[i] * A : -(fm[i]) * A);
-      rv[3] += (double)(own ? en * A : -(en) * A);
-      if constexpr (HEAT) {
-        const T k = mt.cp[0] * mu / mt.Pr0;
-        T gf[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) gf[d] = (G0[9 + d] + G1[9 + d]) / 2;
-        const T q = k * (gf[0] * n[0] + gf[1] * n[1] + gf[2] * n[2]);
-        rv[4] += (double)(own ? q * A : -(q) * A);
-      }
-    }
+    face_terms<NEQ, T, VISC, HEAT, MODE == 1>(P, mt, cs, nb, own, n, A, L, R, VISC ? grad_ptr(c) : nullptr,
+                                              VISC && nb >= 0 ? grad_ptr(nb) : nullptr, VISC ? wls + s : nullptr, Wc1, rhs, rv, sig);
   }
   if constexpr (VISC) {
 #pragma unroll
@@ -783,17 +833,11 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
                      "+s"(mw.eta[1]), "+s"(mw.avfMin));
         fk::store_prims<NEQ>(mw, un, Wout + c * NEQ);
       }
-      // chemical cells to the list of relax_chem, wave-aggregated; counts
-      // summed bit by bit from ballots (no atomics on the counters)
+      // chemical cells to the list of relax_chem; counts summed bit by bit
+      // from ballots (no atomics on the counters)
       const int l = threadIdx.x & 63;
       const unsigned long long mp = __ballot(chem);
-      if (mp) {
-        const int leader = __ffsll((long long)mp) - 1;
-        unsigned long long b = 0;
-        if (l == leader) b = atomicAdd(&rcnt[5], (unsigned long long)__popcll(mp));
-        b = __shfl(b, leader, 64);
-        if (chem) rlist[b + __popcll(mp & ((1ull << l) - 1ull))] = (uint32_t)c;
-      }
+      fk::list_push_plain(chem != 0, c, rlist, rcnt);
       unsigned long long nit = 0, nts = 0;
       for (int k = 0; __ballot((it >> k) != 0); ++k) nit += (unsigned long long)__popcll(__ballot((it >> k) & 1)) << k;
       for (int k = 0; __ballot((ts >> k) != 0); ++k) nts += (unsigned long long)__popcll(__ballot((ts >> k) & 1)) << k;
@@ -836,6 +880,326 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
       asm volatile("" : "+s"(mw.g[0]), "+s"(mw.g[1]), "+s"(mw.pi[0]), "+s"(mw.pi[1]), "+s"(mw.eta[0]), "+s"(mw.eta[1]),
                    "+s"(mw.avfMin));
       fk::store_prims<NEQ>(mw, un, Wout + c * NEQ);
+    }
+  }
+}
+
+// ---- four lanes per cell ----
+//
+// One thread per cell leaves a small mesh with less than a wave per SIMD, each
+// a chain of four to six faces (neighbour gather, conversion, some 300 to 1000
+// dependent instructions each).  pass_g_q and pass_f_q give a cell to the four
+// lanes of a quad: lane q takes the slots q and, with 6 slots per cell, q + 4;
+// then the quad adds the faces' terms in slot order.  Every term is formed by
+// the operations of pass_g / pass_f and added in the same order, so the
+// results are the same bits.  Own-cell work is repeated on the four lanes, so
+// that the kernels lose once the chip is full (quad_cells_g, quad_cells_f).
+// Sod 12k cells: pass G 10 -> 7 us, pass F 10 -> 6; bubble 83k: pass F 29 -> 21,
+// with the plain relaxation 64 -> 53.
+
+__device__ __forceinline__ double quad_bcast(double v, int l) {
+  return l == 0 ? fk::quad_bcast<0>(v) : (l == 1 ? fk::quad_bcast<1>(v) : (l == 2 ? fk::quad_bcast<2>(v) : fk::quad_bcast<3>(v)));
+}
+__device__ __forceinline__ float quad_bcast(float v, int l) {
+  const int i = __float_as_int(v);
+  const int r = l == 0   ? __builtin_amdgcn_mov_dpp(i, 0x00, 0xf, 0xf, true)
+                : l == 1 ? __builtin_amdgcn_mov_dpp(i, 0x55, 0xf, 0xf, true)
+                : l == 2 ? __builtin_amdgcn_mov_dpp(i, 0xaa, 0xf, 0xf, true)
+                         : __builtin_amdgcn_mov_dpp(i, 0xff, 0xf, 0xf, true);
+  return __int_as_float(r);
+}
+// values of lanes l ^ 1 and l ^ 2 of the quad
+template <int X>
+__device__ __forceinline__ float quad_xor(float v) {
+  constexpr int ctrl = X == 1 ? 0xb1 : 0x4e;  // quad_perm [1, 0, 3, 2], [2, 3, 0, 1]
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ctrl, 0xf, 0xf, true));
+}
+template <int X>
+__device__ __forceinline__ double quad_xor(double v) {
+  constexpr int ctrl = X == 1 ? 0xb1 : 0x4e;
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true),
+                          __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true));
+}
+template <typename T>
+__device__ __forceinline__ T quad_max(T v) {
+  v = fmax(v, quad_xor<1>(v));
+  return fmax(v, quad_xor<2>(v));
+}
+template <typename T>
+__device__ __forceinline__ T quad_min(T v) {
+  v = fmin(v, quad_xor<1>(v));
+  return fmin(v, quad_xor<2>(v));
+}
+// lanes of round r (slots 4 r + lane) that hold a slot
+template <int NS>
+constexpr int quad_lanes(int r) {
+  return NS - 4 * r < 4 ? NS - 4 * r : 4;
+}
+
+// First-order state of a cell as pass G takes it (primitive record, FP32
+// primitives of U, or cons2prim of U).
+template <int NEQ, typename T, bool FROMW>
+__device__ __forceinline__ void first_order(const fk::Mat<double> &md, const double *__restrict__ U,
+                                            const float *__restrict__ Wp, int64_t c, T (&W)[NEQ]) {
+  if constexpr (FROMW) {
+#pragma unroll
+    for (int v = 0; v < NEQ; ++v) W[v] = (T)Wp[c * NEQ + v];
+  } else if constexpr (sizeof(T) == 4) {
+    float Wf[NEQ];
+    double Uc[NEQ];
+    fk::load_rec<NEQ>(U + c * NEQ, Uc);
+    fk::prims_f32<NEQ>(md, Uc, Wf);
+#pragma unroll
+    for (int v = 0; v < NEQ; ++v) W[v] = Wf[v];
+  } else {
+    double Uc[NEQ], Wd[NEQ];
+    fk::load_rec<NEQ>(U + c * NEQ, Uc);
+    fk::cons2prim<NEQ>(md, Uc, Wd);
+#pragma unroll
+    for (int v = 0; v < NEQ; ++v) W[v] = (T)Wd[v];
+  }
+}
+
+template <int NEQ, typename T, bool VISC, bool HEAT, bool FROMW, int NS>
+__global__ void __launch_bounds__(64, 2) pass_g_q(fk_params P, int64_t nc, const double *__restrict__ U,
+                                               const float *__restrict__ Wp, const int32_t *__restrict__ link,
+                                               const void *__restrict__ geo, const void *__restrict__ rvec,
+                                               const double *__restrict__ vol, T *__restrict__ face,
+                                               T *__restrict__ gvel, double *__restrict__ dgrad,
+                                               double *__restrict__ dtheta, unsigned long long *__restrict__ health,
+                                               int step) {
+  constexpr int R = (NS + 3) / 4;
+  const int64_t c = xcd_block() * 16 + (threadIdx.x >> 2);
+  const int q = threadIdx.x & 3;
+  if (c >= nc) return;  // whole quads
+  const fk::Mat<double> md = fk::make_mat<double>(P);
+  const fk::Mat<T> mt = fk::make_mat<T>(P);
+  V4<T> rv[R], ga[R];
+  int lk[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const bool in = q < quad_lanes<NS>(r);
+    const int64_t s = c * NS + (in ? 4 * r + q : 0);
+    rv[r] = ld4<T>(rvec, s);
+    ga[r] = ld4<T>(geo, s);
+    lk[r] = in ? link[s] : kNoFace;
+  }
+  T W[NEQ], Wn[R][NEQ];
+  first_order<NEQ, T, FROMW>(md, U, Wp, c, W);
+  const T V = (T)vol[c];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int nb = link_nb<NS>(lk[r]);
+    first_order<NEQ, T, FROMW>(md, U, Wp, nb >= 0 ? nb : c, Wn[r]);
+    if (nb < 0 && lk[r] != kNoFace) {
+      const T n[3] = {ga[r].x, ga[r].y, ga[r].z};
+#pragma unroll
+      for (int v = 0; v < NEQ; ++v) Wn[r][v] = W[v];
+      fk::ghost<NEQ, T>(mt, -nb, n, Wn[r]);
+    }
+  }
+  {  // health of the state, as in pass_g
+    T sum = 0;
+#pragma unroll
+    for (int v = 0; v < NEQ; ++v) sum += W[v];
+    const bool ok = (NEQ == 10 ? (W[1] > 0 && W[2] > 0) : W[0] > 0) && fabs(sum) < (T)INFINITY;
+    if (!ok && q == 0) atomicMin(health, ((unsigned long long)(unsigned)step << 32) | (unsigned long long)c);
+  }
+  const T iV = sizeof(T) == 4 ? (T)1 / V : (T)0;
+  const fk::Divisor dV((double)V);
+  T g[NEQ][3];
+#pragma unroll
+  for (int v = 0; v < NEQ; ++v) g[v][0] = g[v][1] = g[v][2] = 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const bool real = lk[r] != kNoFace;
+    const bool own = link_own(lk[r]);
+    const T sa = sizeof(T) == 4 ? (own ? ga[r].w : -ga[r].w) * iV : (T)(own ? 1 : -1);
+    const T nav[3] = {ga[r].x * sa, ga[r].y * sa, ga[r].z * sa};
+#pragma unroll
+    for (int v = 0; v < NEQ; ++v) {
+      // one variable after the other: interleaved, their terms spill (FP64)
+      __builtin_amdgcn_sched_barrier(0);
+      const T avg = (W[v] + Wn[r][v]) / 2;
+      if constexpr (sizeof(T) == 8) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const T t = real ? dV(avg * nav[d] * ga[r].w) : 0;
+#pragma unroll
+          for (int j = 0; j < quad_lanes<NS>(r); ++j) g[v][d] += quad_bcast(t, j);
+        }
+      } else {
+        // FMAs in slot order: the operands cross the quad (zero past the last face)
+        const T am = real ? avg : 0;
+#pragma unroll
+        for (int j = 0; j < quad_lanes<NS>(r); ++j) {
+          const T aj = quad_bcast(am, j);
+#pragma unroll
+          for (int d = 0; d < 3; ++d) g[v][d] = fmaf(aj, quad_bcast(nav[d], j), g[v][d]);
+        }
+      }
+    }
+  }
+  T th[NEQ];
+#pragma unroll
+  for (int v = 0; v < NEQ; ++v) {
+    __builtin_amdgcn_sched_barrier(0);
+    T ext[R];
+    T mx = (T)-1e12, mn = (T)1e12;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (lk[r] != kNoFace) {
+        mx = fmax(mx, Wn[r][v]);
+        mn = fmin(mn, Wn[r][v]);
+      }
+    mx = quad_max(mx);
+    mn = quad_min(mn);
+    T t = 1;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const T px = rv[r].x * g[v][0], py = rv[r].y * g[v][1], pz = rv[r].z * g[v][2];
+      const T d = (W[v] + px + py + pz) - W[v];
+      ext[r] = px + py + pz;
+      const T num = d > 0 ? mx - W[v] : mn - W[v];
+      const T phi = (d != 0 && lk[r] != kNoFace) ? fk::quot(num, 2 * d) : (T)1;
+      t = fmin(t, fmax((T)0, fmin(phi, (T)1)));
+    }
+    th[v] = quad_min(t);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (q < quad_lanes<NS>(r)) face[(c * NS + 4 * r + q) * NEQ + v] = W[v] + th[v] * ext[r];
+  }
+  if (q != 0) return;
+  if constexpr (VISC) store_grad<NEQ, T, HEAT>(P, W, g, gvel + c * ngrad<NEQ, HEAT>());
+  if (dgrad) {
+#pragma unroll
+    for (int v = 0; v < NEQ; ++v) {
+      dtheta[c * NEQ + v] = (double)th[v];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) dgrad[(c * NEQ + v) * 3 + d] = (double)g[v][d];
+    }
+  }
+}
+
+template <int NEQ, typename T, bool VISC, bool HEAT, int MODE, int NS, bool WOUT = false, int RLX = 0>
+__global__ void __launch_bounds__(64, 2) pass_f_q(fk_params P, int64_t nc, const double *__restrict__ U,
+                                               const double *__restrict__ U0, double *__restrict__ Unew,
+                                               const int32_t *__restrict__ link, const void *__restrict__ geo,
+                                               const T *__restrict__ wls, const double *__restrict__ vol,
+                                               const double *__restrict__ volcfl, const T *__restrict__ face,
+                                               const T *__restrict__ gvel, double *__restrict__ rhs_out,
+                                               double *__restrict__ dtc, int irk, double dt_val,
+                                               const double *__restrict__ dt_ptr, float *__restrict__ Wout,
+                                               uint32_t *__restrict__ rlist, unsigned long long *__restrict__ rcnt,
+                                               unsigned long long *__restrict__ rpart) {
+  static_assert(!RLX || (MODE == 0 && NEQ == 10), "fused relaxation: two-phase RK stage only");
+  constexpr int R = (NS + 3) / 4, NG = ngrad<NEQ, HEAT>(), iu = Model<NEQ>::iu;
+  const int64_t blk = xcd_block();
+  const int64_t c = blk * 16 + (threadIdx.x >> 2);
+  const int q = threadIdx.x & 3;
+  if (c >= nc) {
+    if constexpr (RLX != 0)  // a wave without cells still stores its relaxation counts
+      if (threadIdx.x == 0)
+        for (int k = 0; k < RLX + 1; ++k) rpart[blk * (RLX + 1) + k] = 0;
+    return;
+  }
+  const fk::Mat<double> md = fk::make_mat<double>(P);
+  const fk::Mat<T> mt = fk::make_mat<T>(P);
+  double Uc[NEQ];
+  fk::load_rec<NEQ>(U + c * NEQ, Uc);
+  const CellSide<T> cs = cell_side<NEQ, T>(md, Uc);
+  T Wc1[NEQ];  // first-order state of this cell (viscous boundary ghost)
+  if constexpr (VISC) {
+    double t[NEQ];
+    fk::cons2prim<NEQ>(md, Uc, t);
+    if constexpr (NEQ == 5 && sizeof(T) == 4) t[4] -= md.pr;
+#pragma unroll
+    for (int v = 0; v < NEQ; ++v) Wc1[v] = (T)t[v];
+  }
+  double rhs[NEQ], rv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int v = 0; v < NEQ; ++v) rhs[v] = 0.0;
+  T sig = (T)-1e9;
+#pragma unroll 1
+  for (int r = 0; r < R; ++r) {
+    const bool in = NS == 4 || 4 * r + q < NS;
+    const int64_t s = c * NS + (in ? 4 * r + q : 0);
+    const V4<T> ga = ld4<T>(geo, s);
+    const int lk = in ? link[s] : kNoFace;
+    double fr[NEQ], fv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int v = 0; v < NEQ; ++v) fr[v] = 0.0;
+    if (lk != kNoFace) {
+      const int nb = link_nb<NS>(lk);
+      const bool own = link_own(lk);
+      const T n[3] = {ga.x, ga.y, ga.z};
+      T A1[NEQ], A2[NEQ], L[NEQ], Rt[NEQ];
+      const T *Fs = face + s * NEQ, *Fn = nb >= 0 ? face + (int64_t)(lk >> 1) * NEQ : Fs;
+#pragma unroll
+      for (int v = 0; v < NEQ; ++v) {
+        A1[v] = Fs[v];
+        A2[v] = Fn[v];
+      }
+#pragma unroll
+      for (int v = 0; v < NEQ; ++v) {
+        L[v] = own ? A1[v] : A2[v];
+        Rt[v] = own ? A2[v] : A1[v];
+      }
+      if (nb < 0) fk::ghost<NEQ, T>(mt, -nb, n, Rt);
+      face_terms<NEQ, T, VISC, HEAT, MODE == 1>(P, mt, cs, nb, own, n, ga.w, L, Rt, VISC ? gvel + c * NG : nullptr,
+                                                VISC && nb >= 0 ? gvel + (int64_t)nb * NG : nullptr,
+                                                VISC ? wls + s : nullptr, Wc1, fr, fv, sig);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {  // lanes without a slot add 0
+#pragma unroll
+      for (int v = 0; v < NEQ; ++v) rhs[v] += quad_bcast(fr[v], j);
+      if constexpr (VISC) {
+#pragma unroll
+        for (int i = 0; i < (HEAT ? 5 : 4); ++i) rv[i] += quad_bcast(fv[i], j);
+      }
+    }
+  }
+  if constexpr (VISC) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) rhs[iu + i] += rv[i];
+    rhs[NEQ == 5 ? 4 : 8] += rv[3];
+    if constexpr (HEAT) rhs[4] += rv[4];
+  }
+  if constexpr (MODE != 0) {
+    sig = quad_max(sig);
+#pragma unroll
+    for (int v = 0; v < NEQ; ++v)
+      if (q == (v & 3)) {
+        if constexpr (MODE == 1 && sizeof(T) == 4) reinterpret_cast<float *>(rhs_out)[c * NEQ + v] = (float)rhs[v];
+        else rhs_out[c * NEQ + v] = rhs[v];
+      }
+    if (MODE == 1 && q == 0) dtc[c] = volcfl[c] / (double)sig;
+  } else {
+    const double dt = dt_ptr ? *dt_ptr : dt_val;
+    double un[NEQ];
+    rk_stage<NEQ>(P, irk, dt, vol[c], Uc, U0 + c * NEQ, rhs, un);
+    int chem = 0, push = 0, it = 0, ts = 0;
+    if constexpr (RLX == 1) push = fk::screen_cell(P, un, &chem, &it);
+    if constexpr (RLX == 2) push = chem = fk::plain_cell4(P, un, &it, &ts);
+#pragma unroll
+    for (int v = 0; v < NEQ; ++v)
+      if (q == (v & 3)) Unew[c * NEQ + v] = un[v];
+    if constexpr (WOUT || RLX != 0)
+      if (Wout && !push && q == 0) fk::store_prims<NEQ>(md, un, Wout + c * NEQ);
+    if constexpr (RLX != 0) {
+      const bool lead = q == 0;
+      if constexpr (RLX == 1) fk::list_push(push && lead, chem, c, rlist, nc, rcnt);
+      else fk::list_push_plain(chem && lead, c, rlist, rcnt);
+      unsigned long long nch = __popcll(__ballot(chem && lead)), nit = 0, nts = 0;
+      const int iq = lead ? it : 0, tq = lead ? ts : 0;
+      for (int k = 0; __ballot((iq >> k) != 0); ++k) nit += (unsigned long long)__popcll(__ballot((iq >> k) & 1)) << k;
+      for (int k = 0; __ballot((tq >> k) != 0); ++k) nts += (unsigned long long)__popcll(__ballot((tq >> k) & 1)) << k;
+      if (threadIdx.x == 0) {
+        rpart[blk * (RLX + 1)] = nch;
+        rpart[blk * (RLX + 1) + 1] = nit;
+        if constexpr (RLX == 2) rpart[blk * 3 + 2] = nts;
+      }
     }
   }
 }
@@ -885,8 +1249,7 @@ __global__ void __launch_bounds__(kBlock) rk_update_w(fk_params P, int64_t nc, c
   const int64_t c = c0 + threadIdx.x < nc ? c0 + threadIdx.x : nc - 1;
   const double dt = dt_ptr ? *dt_ptr : dt_val;
   const double Vc = vol[c];
-  constexpr int iz = NEQ == 5 ? 3 : 5;
-  double r[NEQ], uc[NEQ], u0[NEQ], un[NEQ];
+  double r[NEQ], uc[NEQ], un[NEQ];
   if constexpr (sizeof(RT) == 8) {
     fk::load_rec<NEQ>(rhs + c * NEQ, r);
   } else {
@@ -894,17 +1257,7 @@ __global__ void __launch_bounds__(kBlock) rk_update_w(fk_params P, int64_t nc, c
     for (int v = 0; v < NEQ; ++v) r[v] = (double)rhs[c * NEQ + v];
   }
   if (P.rkSteps == 1 || irk != 0) fk::load_rec<NEQ>(U + c * NEQ, uc);
-  if (P.rkSteps != 1) fk::load_rec<NEQ>(U0 + c * NEQ, u0);
-#pragma unroll
-  for (int v = 0; v < NEQ; ++v) {
-    const int neglect = (v == iz && P.neglectZ == 1);
-    double u;
-    if (P.rkSteps == 1) u = (1 - neglect) * (uc[v] + dt * (1.0 / Vc) * r[v]);
-    else if (irk == 0) u = (1 - neglect) * (u0[v] + dt * (1.0 / Vc) * r[v]);
-    else if (irk == 1) u = (1 - neglect) * ((3.0 / 4.0) * u0[v] + (1.0 / 4.0) * uc[v] + (1.0 / 4.0) * dt * (1.0 / Vc) * r[v]);
-    else u = (1 - neglect) * ((1.0 / 3.0) * u0[v] + (2.0 / 3.0) * uc[v] + (2.0 / 3.0) * dt * (1.0 / Vc) * r[v]);
-    un[v] = u;
-  }
+  rk_stage<NEQ>(P, irk, dt, Vc, uc, U0 + c * NEQ, r, un);
 #pragma unroll
   for (int v = 0; v < NEQ; ++v) sU[threadIdx.x * SU + v] = un[v];
   fk::store_prims<NEQ>(fk::make_mat<double>(P), un, sWr + threadIdx.x * SWR);
@@ -1145,6 +1498,35 @@ void free_all(fk_ctx *c) {
   c->lcount = nullptr;
 }
 
+// Cells up to which pass G and pass F run four lanes per cell (pass_g_q,
+// pass_f_q) rather than one with the LDS paths.  What the quads win is waves
+// in flight and shorter chains; what they lose is the own-cell work on four
+// lanes and, with records of half the size (FP32), pass F's LDS reuse.  us,
+// quads / one lane, near the lines:
+//   pass G  FP64 single-phase 7 / 10 at 12k cells, 11 / 12 at 55k, 14 / 14 at
+//           73k; FP32 11 / 11 at 48k tetrahedra, 13 / 12 at 27k hexahedra; FP64
+//           two-phase spills and stays with one lane (17 / 14 at 25k)
+//   pass F  FP64 21 / 29 at 83k, 45 / 71 at 236k, 297 / 306 (residual 292 / 325)
+//           at 1.05M, 857 / 846 (832 / 905) at 3.1M: its one-lane kernel runs
+//           2 waves per SIMD; FP32 two-phase 29 / 34 at 162k, 60 / 56 at 280k,
+//           hexahedra 37 / 33 at 85k; single-phase 30 / 39 at 280k, 47 / 46 at 384k
+//   with the relaxation (it is on four lanes alike, but for the plain solve's
+//   residuals) FP64 53 / 65 at 83k, 106 / 125 at 236k, 234 / 214 at 384k,
+//           hexahedral slots 26 / 46 at 7k, 66 / 53 at 55k; FP32 25 / 22 at 48k
+inline int64_t quad_cells_g(const fk_ctx *c) {
+  if (c->neq == 10 && c->p.precision == FK_FP64) return 0;
+  return c->ns == 6 ? 15000 : (c->neq == 5 ? 60000 : 40000);
+}
+inline int64_t quad_cells_f(const fk_ctx *c, int relax) {
+  const bool f64 = c->p.precision == FK_FP64;
+  if (relax) return c->ns == 4 && f64 ? 250000 : 30000;
+  if (f64) return 4000000;
+  return c->ns == 6 ? 60000 : (c->neq == 5 ? 300000 : 200000);
+}
+inline bool quad_g(const fk_ctx *c) { return c->stage_g == 1 && c->nc <= quad_cells_g(c); }
+inline bool quad_f(const fk_ctx *c, int relax) { return c->stage_f == 1 && c->nc <= quad_cells_f(c, relax); }
+inline unsigned grid_quad(int64_t nc) { return (unsigned)((nc + 16 * kXcd - 1) / (16 * kXcd) * kXcd); }
+
 template <typename T, int NS>
 int launch_pass_g_t(fk_ctx *c) {
   const unsigned gr = grid_xcd(c->nc);
@@ -1156,6 +1538,7 @@ int launch_pass_g_t(fk_ctx *c) {
   T *face = (T *)c->face;
   T *gv = (T *)c->gvel;
   const bool fromw = sizeof(T) == 4 && c->prims_w && c->w_valid;
+  const bool quad = quad_g(c);
   // face records through LDS (workgroup sizes: pass_g_block)
   const bool sout = c->stage_g;
   constexpr int gbs = pass_g_block<T, NS, true>();
@@ -1168,6 +1551,15 @@ int launch_pass_g_t(fk_ctx *c) {
                                   c->health, (int)std::min<int64_t>(c->step, INT32_MAX)))
 #define PG2(NEQ, VISC, HEAT, FW)                                                                                     \
   do {                                                                                                               \
+    if constexpr (NEQ == 5 || sizeof(T) == 4) {                                                                      \
+      if (quad) {                                                                                                    \
+        LAUNCH_TIMED(c, "pass_g",                                                                                    \
+                     hipLaunchKernelGGL((pass_g_q<NEQ, T, VISC, HEAT, FW, NS>), dim3(grid_quad(c->nc)), dim3(64), 0, \
+                                        c->stream, c->p, c->nc, U, c->wprim, c->link, c->geo, c->rvec, c->vol, face, \
+                                        gv, dg, dth, c->health, (int)std::min<int64_t>(c->step, INT32_MAX)));        \
+        break;                                                                                                       \
+      }                                                                                                              \
+    }                                                                                                                \
     if constexpr (pass_g_sout_ok<T, NS, NEQ>()) {                                                                    \
       if (sout) {                                                                                                    \
         PG3(NEQ, VISC, HEAT, FW, true);                                                                              \
@@ -1224,10 +1616,36 @@ int launch_pass_f_t(fk_ctx *c, int irk, double dt, const double *dtp, double *Un
   const size_t lds = stage ? (size_t)bs * (NS * c->neq + 12) * sizeof(T) : 0;
   // waves of this launch (per-wave relaxation counts of the fused last stage)
   c->pf_waves = (int64_t)(stage ? (int64_t)gs * (bs / 64) : (int64_t)gr * (kBlock / 64));
+  const bool quad = quad_f(c, relax);
+  if (quad) c->pf_waves = grid_quad(c->nc);
 #define PF_ARGS(W) \
   c->p, c->nc, U, U0, Unew, c->link, c->geo, wl, c->vol, c->volcfl, face, gv, c->rhs, c->dtc, irk, dt, dtp, W
+#define PFQ(NEQ, VISC, HEAT, WO, RX, NAME, W, LIST, CNT, PART)                                                         \
+  LAUNCH_TIMED(c, NAME,                                                                                                \
+               hipLaunchKernelGGL((pass_f_q<NEQ, T, VISC, HEAT, MODE, NS, WO, RX>), dim3(grid_quad(c->nc)), dim3(64), 0, \
+                                  c->stream, PF_ARGS(W), LIST, CNT, PART))
 #define PF(NEQ, VISC, HEAT)                                                                                            \
   do {                                                                                                                 \
+    if (quad) {                                                                                                        \
+      if constexpr (MODE == 0 && NEQ == 10) {                                                                          \
+        if (relax == 1) {                                                                                              \
+          PFQ(NEQ, VISC, HEAT, false, 1, "pass_f_relax", Wr, c->rlist, cnt, c->rpart);                                 \
+          break;                                                                                                       \
+        }                                                                                                              \
+        if (relax == 2) {                                                                                              \
+          PFQ(NEQ, VISC, HEAT, false, 2, "pass_f_relax", Wr, c->rlist, cnt, c->rpart);                                 \
+          break;                                                                                                       \
+        }                                                                                                              \
+      }                                                                                                                \
+      if constexpr (MODE == 0 && sizeof(T) == 4) {                                                                     \
+        if (Wout) {                                                                                                    \
+          PFQ(NEQ, VISC, HEAT, true, 0, nm, Wout, nullptr, nullptr, nullptr);                                          \
+          break;                                                                                                       \
+        }                                                                                                              \
+      }                                                                                                                \
+      PFQ(NEQ, VISC, HEAT, false, 0, nm, nullptr, nullptr, nullptr, nullptr);                                          \
+      break;                                                                                                           \
+    }                                                                                                                  \
     if constexpr (MODE == 0 && NEQ == 10) {                                                                            \
       if (relax == 1) {                                                                                                \
         if (stage)                                                                                                     \
@@ -1281,6 +1699,7 @@ int launch_pass_f_t(fk_ctx *c, int irk, double dt, const double *dtp, double *Un
     else PF(10, false, false);
   }
 #undef PF
+#undef PFQ
 #undef PF_ARGS
   return FK_OK;
 }
@@ -1428,8 +1847,10 @@ int ensure_rlist(fk_ctx *c) {
   HIPCHK(hipMalloc(&c->rlist, (size_t)c->nc * sizeof(uint32_t)));
   HIPCHK(hipMalloc(&c->rfall, (size_t)c->nc * sizeof(uint32_t)));
   // [blocks][4] partials of the relaxation kernels, or [waves][2 or 3] of the
-  // fused pass F (grid_xcd blocks of 4 waves)
-  HIPCHK(hipMalloc(&c->rpart, (size_t)grid_xcd(c->nc) * 12 * sizeof(unsigned long long)));
+  // fused pass F (grid_xcd blocks of 4 waves, or one wave for 16 cells)
+  size_t parts = (size_t)grid_xcd(c->nc) * 12;
+  if (c->nc <= quad_cells_f(c, 1)) parts = std::max(parts, (size_t)grid_quad(c->nc) * 3);
+  HIPCHK(hipMalloc(&c->rpart, parts * sizeof(unsigned long long)));
   c->rlist_cap = c->nc;
   return FK_OK;
 }
@@ -1850,7 +2271,7 @@ int fk_set_tuning(fk_ctx *c, const char *name, int64_t value) {
     return FK_OK;
   }
   if (std::strcmp(name, "stage_f") == 0) {
-    c->stage_f = value != 0;
+    c->stage_f = value == 2 ? 2 : value != 0;
     return FK_OK;
   }
   if (std::strcmp(name, "prims_w") == 0) {
@@ -1863,7 +2284,7 @@ int fk_set_tuning(fk_ctx *c, const char *name, int64_t value) {
     return FK_OK;
   }
   if (std::strcmp(name, "stage_g") == 0) {
-    c->stage_g = value != 0;
+    c->stage_g = value == 2 ? 2 : value != 0;
     return FK_OK;
   }
   return fail(FK_EINVAL, std::string("unknown tuning option ") + name);

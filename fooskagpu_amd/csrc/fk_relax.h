@@ -828,6 +828,131 @@ __device__ inline int chem_dev8(const fk_params &P, double *U) {
   return itr;
 }
 
+// tsat_dev on 4 lanes: the saturation function at T (even lanes) and T + dt
+// (odd lanes) at once.
+__device__ inline double tsat4(const fk_params &P, double Pr, double temp, double urf, int *iters) {
+  const int odd = threadIdx.x & 1;
+  const double Pinf = P.pInf[0], g1 = P.gamma[0], g2 = P.gamma[1], Cp1 = P.Cp[0], Cp2 = P.Cp[1];
+  const double Cv1 = Cp1 / g1, Cv2 = Cp2 / g2;
+  const double lg = fkmath::log10(odd ? Pr + Pinf : Pr);
+  const double lpp = quad_bcast<1>(lg), lp = quad_bcast<0>(lg);
+  const double et2 = P.satConst[0] * lp + P.satConst[1];
+  const double As = (Cp1 - Cp2 + et2 - 0.0) / (Cp2 - Cv2);
+  const double Bs = (P.eta[0] - P.eta[1]) / (Cp2 - Cv2);
+  const double Cs = (Cp2 - Cp1) / (Cp2 - Cv2);
+  const double Ds = (Cp1 - Cv1) / (Cp2 - Cv2);
+  const double dt = 1.e-3;
+  double fun = 1, T = temp;
+  int itr = 0;
+  while (fabs(fun) > 1.e-2 && itr < 50) {
+    const double x = odd ? T + dt : T;
+    const double f = As + Bs / x + Cs * fkmath::log10(x) + Ds * lpp - lp;
+    fun = quad_bcast<0>(f);
+    const double gr = (quad_bcast<1>(f) - fun) / dt;
+    T = T - urf * fun / gr;
+    itr++;
+  }
+  *iters = itr;
+  return T;
+}
+
+// therm_dev on 4 lanes: lane bits 0-1 select the residual evaluation (the
+// iterate, or unknown 1 or 2 perturbed; lane 3 repeats lane 2).  The unknowns
+// are (rho, e) of the secondary phase k.
+__device__ inline int therm_dev4(const fk_params &P, double *U) {
+  const int ev = threadIdx.x & 3;
+  const double urf = P.thermUrf;
+  const double avf0 = clampd(P, U[0]), avf1 = 1 - avf0;
+  const double rho0 = U[1] / avf0, rho1 = U[2] / avf1;
+  const double ar0 = avf0 * rho0, ar1 = avf1 * rho1;
+  double en0 = U[6] / ar0, en1 = U[7] / ar1;
+  const double rhoMix = ar0 + ar1;
+  const double v0 = U[3] / rhoMix, v1 = U[4] / rhoMix, v2 = U[5] / rhoMix;
+  const double Y0 = ar0 / rhoMix, Y1 = ar1 / rhoMix;
+  const bool k0 = avf1 > avf0;  // the secondary phase is phase 0
+  double y0 = k0 ? rho0 : rho1, y1 = k0 ? en0 : en1;
+  double b0 = y0, b1 = y1;  // best iterate
+  const double de = U[8] / rhoMix - Y0 * en0 - Y1 * en1 - 0.5 * (v0 * v0 + v1 * v1 + v2 * v2);
+  en0 += de;
+  en1 += de;
+  float dP = 0.0f, dT = 0.0f;
+  if (P.thermFntRlxFlag == 1) {
+    const double avf[2] = {avf0, avf1}, rho[2] = {rho0, rho1}, enr[2] = {en0, en1};
+    fnt_press_rlx(P, avf, rho, enr, &dP, &dT);
+  }
+  const double ark = k0 ? ar0 : ar1, arm = k0 ? ar1 : ar0, enk = k0 ? en0 : en1, enm = k0 ? en1 : en0;
+  const double iarm = 1 / arm;
+  int abortFlag = 0, itr = 0;
+  float minRes = 1e9f;
+  bool conv = false;
+  while (!conv) {
+    itr++;
+    const double s0 = 1e-4 * y0, s1 = 1e-4 * y1;
+    const double p0 = y0 + s0, p1 = y1 + s1;
+    const double d0 = p0 - s0, d1 = p1 - s1;
+    const double a = ev == 0 ? y0 : (ev == 1 ? p0 : d0), b = ev <= 1 ? y1 : p1;
+    const double zr = (1 / (1 - ark / a)) * arm, ze = enm - iarm * (ark * (b - enk));
+    const double x0 = k0 ? a : zr, x1 = k0 ? zr : a, x2 = k0 ? b : ze, x3 = k0 ? ze : b;
+    const double f0 = eos_p(P, 0, x0, x2) - eos_p(P, 1, x1, x3) - (double)dP;
+    const double f1 = eos_T(P, 0, x0, x2) - eos_T(P, 1, x1, x3) - (double)dT;
+    const double r0 = quad_bcast<0>(f0), r1 = quad_bcast<0>(f1);
+    const double se = ev <= 1 ? s0 : s1;
+    const double c0 = (f0 - r0) / se, c1 = (f1 - r1) / se;
+    const double J00 = quad_bcast<1>(c0), J10 = quad_bcast<1>(c1), J01 = quad_bcast<2>(c0), J11 = quad_bcast<2>(c1);
+    if (__builtin_isnan(J00) || __builtin_isnan(J01) || __builtin_isnan(J10) || __builtin_isnan(J11)) abortFlag = 1;
+    const double det = J00 * J11 - J10 * J01;
+    const double I00 = J11 / det, I11 = J00 / det, I10 = -J10 / det, I01 = -J01 / det;
+    if (det == 0) abortFlag = 1;
+    y0 = d0;
+    y1 = d1;
+    // the primary density of the last evaluation, as therm_dev leaves it
+    if (abortFlag == 0 && y0 > 0.0 && quad_bcast<2>(zr) > 0.0) {
+      const float chk = (float)sqrt(r0 * r0 + r1 * r1);
+      if (chk < minRes) {
+        minRes = chk;
+        b0 = y0;
+        b1 = y1;
+      }
+    }
+    double dx0 = 0;
+    dx0 += I00 * r0;
+    dx0 += I01 * r1;
+    y0 = y0 - urf * dx0;
+    double dx1 = 0;
+    dx1 += I10 * r0;
+    dx1 += I11 * r1;
+    y1 = y1 - urf * dx1;
+    if (!(fabs(r0) > 1.e-2) && !(fabs(r1) > 1.e-2)) conv = true;
+    if (abortFlag == 1 || itr > P.thermItrMax) {
+      y0 = b0;
+      y1 = b1;
+      conv = true;
+    }
+  }
+  const double zr = (1 / (1 - ark / y0)) * arm, ze = enm - iarm * (ark * (y1 - enk));
+  U[0] = clampd(P, ar0 / (k0 ? y0 : zr));
+  U[6] = ar0 * (k0 ? y1 : ze);
+  U[7] = ar1 * (k0 ? ze : y1);
+  return itr;
+}
+
+// plain_cell on 4 lanes.
+__device__ inline int plain_cell4(const fk_params &P, double *u, int *iters, int *tsat_iters) {
+  int chem = 0, ts = 0;
+  if (P.chemFlag == 1) {
+    const double avf = clampd(P, u[0]);
+    const double rho = u[1] / avf;
+    const double enr = u[6] / (avf * rho);
+    const double tL = eos_T(P, 0, rho, enr);
+    const double pL = eos_p(P, 0, rho, enr);
+    const double Ts = tsat4(P, pL, tL, P.satTempUrf, &ts);
+    chem = (tL > Ts && avf > P.chemLimit) ? 1 : 0;
+  }
+  *tsat_iters = ts;
+  *iters = chem ? 0 : therm_dev4(P, u);
+  return chem;
+}
+
 // chem_polish on 4 lanes: each takes one of an iteration's logarithms (T,
 // p + pinf_L, p + pinf_G, p), and a pair the quantities of one phase.
 __device__ inline int chem_polish4(const fk_params &P, double *U, double T0, double p0, double tol, int itmax) {
@@ -920,6 +1045,18 @@ __device__ inline void list_push(bool push, int chem, int64_t c, uint32_t *__res
     b = atomicAdd(&cnt[5], (unsigned long long)__popcll(mf) | ((unsigned long long)__popcll(mb) << 32));
   b = __shfl(b, leader, 64);
   if (push) list[list_place(b, mf, mb, chem != 0, cap)] = (uint32_t)((c << 1) | chem);
+}
+
+// The plain relaxation's list by the wave: chemical cells, entries are cells.
+__device__ inline void list_push_plain(bool push, int64_t c, uint32_t *__restrict__ list,
+                                       unsigned long long *__restrict__ cnt) {
+  const unsigned long long m = __ballot(push);
+  if (!m) return;
+  const int leader = __ffsll((long long)m) - 1;
+  unsigned long long b = 0;
+  if ((int)(threadIdx.x & 63) == leader) b = atomicAdd(&cnt[5], (unsigned long long)__popcll(m));
+  b = __shfl(b, leader, 64);
+  if (push) list[list_place(b, m, 0, true, 0)] = (uint32_t)c;
 }
 
 // Append by a 256-thread workgroup (every thread calls).

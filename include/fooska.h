@@ -211,13 +211,19 @@ int fk_set_debug(fk_ctx *ctx, int on);
  *     reduced, and a streaming kernel applies the update); at 48M cells,
  *     mixed: 7.5 ms against 6.7 + 2.5 ms.  0 = always residual + update
  *     kernel.
- *  "stage_f" (default 1): pass F copies the face states and velocity
- *     gradients of its workgroup's cells to LDS and reads in-workgroup mirror
- *     states from there (4 slots per cell: 256 cells, FP64 128; 6 slots:
- *     two-phase FP32, 128 cells, not in the last stage's relaxation pass).
- *  "stage_g" (default 1): pass G writes its workgroup's face records and
- *     velocity gradients from LDS in 16-byte words (4 slots per cell: 256
- *     cells, FP64 128; 6 slots: two-phase FP32, 128 cells).
+ *  "stage_f" (default 1): pass F by the size of the mesh: four lanes per cell
+ *     on small meshes (FP64 up to 4M cells), else one lane per cell with the
+ *     face states and velocity gradients of its workgroup's cells in LDS, in-
+ *     workgroup mirror states read from there (4 slots per cell: 256 cells,
+ *     FP64 128; 6 slots: two-phase FP32, 128 cells, not in the last stage's
+ *     relaxation pass).  2: one lane with LDS at every size; 0: one lane
+ *     without.
+ *  "stage_g" (default 1): pass G by the size of the mesh: four lanes per cell
+ *     up to 15,000 to 60,000 cells, else one lane per cell with the
+ *     workgroup's face records and velocity gradients written from LDS in
+ *     16-byte words (4 slots per cell: 256 cells, FP64 128; 6 slots: two-phase
+ *     FP32, 128 cells).  2: one lane with LDS at every size; 0: one lane with
+ *     direct stores.
  *  "prims_w" (default 1): mixed precision only; the kernels that produce a
  *     new state (fused pass F, relaxation) also write its FP32 primitive
  *     variables, which the next pass G gathers instead of converting the FP64

@@ -131,3 +131,65 @@ def test_training_step_is_adam_on_the_gradient(gpu, batch):
     print(f"[train] batch {batch}: loss {loss:.5f} {l0:.5f}, max |dw| {np.abs(w1 - want).max():.2e}")
     assert l0 == l1 == loss
     assert np.abs(w1 - want).max() < 1e-6
+
+
+QUAD_CASES = {
+    "sod": lambda: cases.sod(nx=7, ny=3, nz=3),
+    "tgv": lambda: cases.tgv(n=7),
+    "bubble": lambda: cases.bubble(n=9),
+    "shock_bubble": lambda: cases.shock_bubble(n=9, nbub=3),
+    "elements": lambda: _elements(_lib.MODEL_TWO_PHASE),
+    "elements_sp": lambda: _elements(_lib.MODEL_SINGLE),
+}
+
+
+def _elements(model):
+    m = Mesh.mixed_box(7, 3, 4, (0, 0, 0), (1.0, 0.4, 0.4), 0.10, 11, bc=(3, 2, 4, 5, 1, 2))
+    if model == _lib.MODEL_SINGLE:
+        p = dict(cases.BASE, viscFlag=1, turbulence=1, heatFlux=1, dynVisc=[1e-3, 1e-3], inletP=1.1, inletT=0.004)
+        return cases.Case("elements_sp", p, m, m.init_sod(1.4, 0.0, 0.45, (1.0, 0.2, 0, 0, 1.0), (0.125, 0, 0, 0, 0.1)), 3)
+    p = cases._two_phase_params(viscFlag=1, turbulence=1, inletP=1e7, inletT=cases.T_WATER)
+    am = p["avfMin"]
+    regions = [dict(kind=0, alphaL=1 - am, p=1e7, T=cases.T_WATER, u=(3.0, 0, 0)),
+               dict(kind=1, c=(0.5, 0.2, 0.2), r=0.15, alphaL=am, p=2340.0, T=cases.T_WATER)]
+    return cases.Case("elements", p, m, m.init_regions(p, regions), 3)
+
+
+@pytest.mark.parametrize("precision", [_lib.FP64, _lib.MIXED])
+@pytest.mark.parametrize("name", sorted(QUAD_CASES))
+def test_four_lanes_per_cell_give_the_bits_of_one(gpu, name, precision):
+    """Small meshes run pass G and pass F on quads (stage 1); the kernels of
+    one lane per cell, with LDS (2) and without (0), give the same states and
+    counts bit for bit: all stages, both relaxations fused and apart, sizes
+    that leave the last wave part full, every boundary code."""
+    c = QUAD_CASES[name]()
+    print(f"[quads] {name} {c.mesh.n_cells} cells", flush=True)
+    modes = [_lib.RELAX_PLAIN, _lib.RELAX_COLD] if c.neq == 10 else [_lib.RELAX_PLAIN]
+    for mode in modes:
+        for fuse in (1, 0):
+            out = []
+            for stage in (1, 2, 0):
+                with GpuSolver(dict(c.params, precision=precision, relaxMode=mode), c.mesh, c.U) as g:
+                    g.set_tuning("stage_f", stage)
+                    g.set_tuning("stage_g", stage)
+                    g.set_tuning("fuse_update", fuse)
+                    dt = g.run_steps(3)
+                    out.append((g.download_state(), dt, g.relax_totals() if c.neq == 10 else None))
+            for o in out[1:]:
+                assert np.array_equal(o[0], out[0][0]) and o[1:] == out[0][1:]
+
+
+@pytest.mark.parametrize("precision", [_lib.FP64, _lib.MIXED])
+@pytest.mark.parametrize("name", ["tgv", "shock_bubble"])
+def test_workgroups_of_one_lane_per_cell_with_a_remainder(gpu, name, precision):
+    """The LDS kernels at a size that fills many workgroups and leaves the last
+    part full, against direct loads and stores, bit for bit."""
+    c = cases.tgv(n=23) if name == "tgv" else cases.shock_bubble(n=23, nbub=5, order="morton")
+    out = []
+    for stage in (2, 0, 1):
+        with GpuSolver(dict(c.params, precision=precision), c.mesh, c.U) as g:
+            g.set_tuning("stage_f", stage)
+            g.set_tuning("stage_g", stage)
+            g.run_steps(2)
+            out.append(g.download_state())
+    assert all(np.array_equal(o, out[0]) for o in out[1:])
