@@ -89,6 +89,10 @@ struct fk_ctx {
   // state health found by pass G: (step << 32) | cell, the smallest of the
   // cells with a non-positive density or a non-finite primitive; ~0 if none
   unsigned long long *health = nullptr;
+  double *dtw = nullptr;     // minima of Vcfl / signal by wave (pass F on quads), dt_parts of them
+  int dt_parts = 0;
+  double *hres = nullptr;    // page-locked results that kernels write for the host, 64 doubles
+  unsigned long long hseq = 0;  // number of the last result asked for
   double *dgrad = nullptr, *dtheta = nullptr;
   // relaxation counters: [0, 5) of the last relaxation (n_chem, Newton
   // iterations, Tsat iterations, fallbacks, warm-started cells; slot 5 is the
@@ -96,6 +100,7 @@ struct fk_ctx {
   // fk_run_steps
   long long *lcount = nullptr;
   int64_t relax_calls = 0;  // relaxations summed in lcount[8, 13)
+  bool counts_clean = true;  // lcount[0, 8) are zero
   // relaxation work list (chemical cells / surrogate list), one entry per cell
   uint32_t *rlist = nullptr;
   uint32_t *rfall = nullptr;   // surrogate relaxation: cells whose polish failed
@@ -126,8 +131,9 @@ struct fk_ctx {
 };
 
 // defined in fk_mlp.hip
-int fk_relax_mlp_impl(fk_ctx *c, bool warm);
+int fk_relax_mlp_impl(fk_ctx *c, bool warm, bool reduce);  // reduce: add stage 1's partial counts here
 int fk_relax_mlp_begin(fk_ctx *c, bool warm);   // checks, scratch, zeroed counts
+int zero_counts(fk_ctx *c);  // defined in fk_kernels.hip
 int fk_relax_mlp_finish(fk_ctx *c, bool warm);  // stage 2 (work list) after stage 1
 int ensure_rlist(fk_ctx *c);  // defined in fk_kernels.hip
 int ensure_rstart(fk_ctx *c);  // defined in fk_kernels.hip

@@ -28,6 +28,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -641,7 +643,8 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
                                                  const T *__restrict__ face, const T *__restrict__ gvel,
                                                  double *__restrict__ rhs_out, double *__restrict__ dtc, int irk,
                                                  double dt_val, const double *__restrict__ dt_ptr,
-                                                 float *__restrict__ Wout, uint32_t *__restrict__ rlist,
+                                                 float *__restrict__ Wout, double *__restrict__ clock,
+                                                 uint32_t *__restrict__ rlist,
                                                  unsigned long long *__restrict__ rcnt,
                                                  unsigned long long *__restrict__ rpart) {
   static_assert(!RLX || (MODE == 0 && NEQ == 10), "fused relaxation: two-phase RK stage only");
@@ -809,6 +812,7 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
     if constexpr (MODE == 1) dtc[c] = volcfl[c] / (double)sig;
   } else {
     const double dt = dt_ptr ? *dt_ptr : dt_val;
+    if (clock && c == 0) clock[1] += clock[0];  // last stage of a step: the physical time
     const double Vc = vol[c];
     constexpr int iz = NEQ == 5 ? 3 : 5;
     double un[NEQ];
@@ -1090,19 +1094,25 @@ __global__ void __launch_bounds__(64, 2) pass_f_q(fk_params P, int64_t nc, const
                                                const T *__restrict__ gvel, double *__restrict__ rhs_out,
                                                double *__restrict__ dtc, int irk, double dt_val,
                                                const double *__restrict__ dt_ptr, float *__restrict__ Wout,
+                                               double *__restrict__ clock, double *__restrict__ dtmin,
                                                uint32_t *__restrict__ rlist, unsigned long long *__restrict__ rcnt,
                                                unsigned long long *__restrict__ rpart) {
   static_assert(!RLX || (MODE == 0 && NEQ == 10), "fused relaxation: two-phase RK stage only");
   constexpr int R = (NS + 3) / 4, NG = ngrad<NEQ, HEAT>(), iu = Model<NEQ>::iu;
   const int64_t blk = xcd_block();
-  const int64_t c = blk * 16 + (threadIdx.x >> 2);
   const int q = threadIdx.x & 3;
-  if (c >= nc) {
-    if constexpr (RLX != 0)  // a wave without cells still stores its relaxation counts
-      if (threadIdx.x == 0)
+  if (blk * 16 >= nc) {  // a wave without cells still stores its counts and minimum
+    if (threadIdx.x == 0) {
+      if constexpr (RLX != 0)
         for (int k = 0; k < RLX + 1; ++k) rpart[blk * (RLX + 1) + k] = 0;
+      if (MODE == 1 && dtmin) dtmin[blk] = 1e15;
+    }
     return;
   }
+  // quads past the last cell compute it again (and store the same values)
+  const int64_t cq = blk * 16 + (threadIdx.x >> 2);
+  const bool live = cq < nc;
+  const int64_t c = live ? cq : nc - 1;
   const fk::Mat<double> md = fk::make_mat<double>(P);
   const fk::Mat<T> mt = fk::make_mat<T>(P);
   double Uc[NEQ];
@@ -1174,9 +1184,17 @@ __global__ void __launch_bounds__(64, 2) pass_f_q(fk_params P, int64_t nc, const
         if constexpr (MODE == 1 && sizeof(T) == 4) reinterpret_cast<float *>(rhs_out)[c * NEQ + v] = (float)rhs[v];
         else rhs_out[c * NEQ + v] = rhs[v];
       }
-    if (MODE == 1 && q == 0) dtc[c] = volcfl[c] / (double)sig;
+    if constexpr (MODE == 1) {
+      double d = volcfl[c] / (double)sig;
+      if (q == 0) dtc[c] = d;
+      if (dtmin) {  // minimum of the wave's cells for the RK update (dt_of)
+        for (int off = 4; off < 64; off <<= 1) d = fmin(d, __shfl_xor(d, off, 64));
+        if (threadIdx.x == 0) dtmin[blk] = fmin(1e15, d);
+      }
+    }
   } else {
     const double dt = dt_ptr ? *dt_ptr : dt_val;
+    if (clock && c == 0 && q == 0 && live) clock[1] += clock[0];
     double un[NEQ];
     rk_stage<NEQ>(P, irk, dt, vol[c], Uc, U0 + c * NEQ, rhs, un);
     int chem = 0, push = 0, it = 0, ts = 0;
@@ -1188,7 +1206,7 @@ __global__ void __launch_bounds__(64, 2) pass_f_q(fk_params P, int64_t nc, const
     if constexpr (WOUT || RLX != 0)
       if (Wout && !push && q == 0) fk::store_prims<NEQ>(md, un, Wout + c * NEQ);
     if constexpr (RLX != 0) {
-      const bool lead = q == 0;
+      const bool lead = q == 0 && live;
       if constexpr (RLX == 1) fk::list_push(push && lead, chem, c, rlist, nc, rcnt);
       else fk::list_push_plain(chem && lead, c, rlist, rcnt);
       unsigned long long nch = __popcll(__ballot(chem && lead)), nit = 0, nts = 0;
@@ -1204,18 +1222,53 @@ __global__ void __launch_bounds__(64, 2) pass_f_q(fk_params P, int64_t nc, const
   }
 }
 
+// dt of the update kernels.  nmin > 0: from the minima that pass F's waves left
+// (up to kDtParts of them, which every block folds for itself; two kernels and
+// their gaps fewer than min_blocks + dt_final: with the time's own kernel gone too a
+// 12k-cell Sod step takes 34 instead of 39 us);
+// block 0 stores it.  clock: the update ends a step, the physical time
+// advances.
+constexpr int kDtParts = 8192;
+struct DtSource {
+  double val;             // the dt, unless ptr or nmin says otherwise
+  const double *ptr;
+  const double *minima;
+  int nmin;
+  double cfl, maxDt;
+  double *scal;           // [dt, time]
+  int clock;
+};
+__device__ __forceinline__ double dt_of(const DtSource &s) {
+  double dt = s.ptr ? *s.ptr : s.val;
+  if (s.nmin > 0) {
+    __shared__ double sh[kBlock / 64];
+    double m = 1e15;
+    for (int i = threadIdx.x; i < s.nmin; i += kBlock) m = fmin(m, s.minima[i]);
+    for (int off = 1; off < 64; off <<= 1) m = fmin(m, __shfl_xor(m, off, 64));
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
+    __syncthreads();
+    for (int k = 0; k < kBlock / 64; ++k) m = fmin(m, sh[k]);
+    dt = fmin(s.cfl * m, s.maxDt);
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (s.nmin > 0) s.scal[0] = dt;
+    if (s.clock) s.scal[1] += dt;
+  }
+  return dt;
+}
+
 // RK stage from a stored residual (update.cu:19-103); RT: its storage type.
 template <int NEQ, typename RT>
 __global__ void __launch_bounds__(kBlock) rk_update(fk_params P, int64_t nc, const double *__restrict__ U,
                                                     const double *__restrict__ U0, double *__restrict__ Unew,
                                                     const RT *__restrict__ rhs_s, const double *__restrict__ vol,
-                                                    int irk, double dt_val, const double *__restrict__ dt_ptr) {
+                                                    int irk, DtSource ds) {
+  const double dt = dt_of(ds);
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= nc * NEQ) return;
   const double ri = (double)rhs_s[i];
   const int64_t c = i / NEQ;
   const int v = (int)(i - c * NEQ);
-  const double dt = dt_ptr ? *dt_ptr : dt_val;
   const double Vc = vol[c];
   constexpr int iz = NEQ == 5 ? 3 : 5;
   const int neglect = (v == iz && P.neglectZ == 1);
@@ -1234,8 +1287,7 @@ template <int NEQ, typename RT>
 __global__ void __launch_bounds__(kBlock) rk_update_w(fk_params P, int64_t nc, const double *__restrict__ U,
                                                       const double *__restrict__ U0, double *__restrict__ Unew,
                                                       const RT *__restrict__ rhs, const double *__restrict__ vol,
-                                                      int irk, double dt_val, const double *__restrict__ dt_ptr,
-                                                      float *__restrict__ W) {
+                                                      int irk, DtSource ds, float *__restrict__ W) {
   // The new state and its primitive record leave through LDS: a thread's
   // 80-byte (and 40-byte) record stored directly goes out as strided partial
   // lines; from LDS the workgroup stores its contiguous ranges in 16-byte
@@ -1247,7 +1299,7 @@ __global__ void __launch_bounds__(kBlock) rk_update_w(fk_params P, int64_t nc, c
   __shared__ __attribute__((aligned(16))) float sWr[kBlock * SWR];
   const int64_t c0 = (int64_t)blockIdx.x * kBlock;
   const int64_t c = c0 + threadIdx.x < nc ? c0 + threadIdx.x : nc - 1;
-  const double dt = dt_ptr ? *dt_ptr : dt_val;
+  const double dt = dt_of(ds);
   const double Vc = vol[c];
   double r[NEQ], uc[NEQ], un[NEQ];
   if constexpr (sizeof(RT) == 8) {
@@ -1276,6 +1328,15 @@ __global__ void __launch_bounds__(kBlock) rk_update_w(fk_params P, int64_t nc, c
   }
 }
 
+// Results for the host, written to the context's page-locked memory: values,
+// then the call's number behind a system-wide fence, so that the host can take
+// them as soon as the number is there (wait_result).
+constexpr int kHostSeq = 63;
+__device__ __forceinline__ void publish(double *host, unsigned long long seq) {
+  __threadfence_system();
+  if (threadIdx.x == 0) reinterpret_cast<volatile unsigned long long *>(host)[kHostSeq] = seq;
+}
+
 // min over cells of Vcfl/signal: per-block minima, then one block folds them
 // and forms dt = min(cfl * min, maxDt) on the device.
 __global__ void __launch_bounds__(kBlock) min_blocks(int64_t n, const double *__restrict__ x, double *__restrict__ out) {
@@ -1292,7 +1353,8 @@ __global__ void __launch_bounds__(kBlock) min_blocks(int64_t n, const double *__
 }
 
 __global__ void __launch_bounds__(kBlock) dt_final(int nb, const double *__restrict__ part, double cfl, double maxDt,
-                                                   double *__restrict__ scal) {
+                                                   double *__restrict__ scal, double *__restrict__ host,
+                                                   unsigned long long seq) {
   __shared__ double sh[kBlock];
   double m = 1e15;
   for (int i = threadIdx.x; i < nb; i += kBlock) m = fmin(m, part[i]);
@@ -1302,12 +1364,11 @@ __global__ void __launch_bounds__(kBlock) dt_final(int nb, const double *__restr
     if ((int)threadIdx.x < s) sh[threadIdx.x] = fmin(sh[threadIdx.x], sh[threadIdx.x + s]);
     __syncthreads();
   }
-  if (threadIdx.x == 0) scal[0] = fmin(cfl * sh[0], maxDt);
-}
-
-// physical time += dt, once per step
-__global__ void advance_time(double *__restrict__ scal) {
-  if (threadIdx.x == 0) scal[1] += scal[0];
+  if (threadIdx.x == 0) {
+    scal[0] = fmin(cfl * sh[0], maxDt);
+    if (host) host[0] = scal[0];  // fk_compute_time_step
+  }
+  if (host && threadIdx.x < 64) publish(host, seq);
 }
 
 // relaxation (relaxation.cu:77-114), reference Newton solves, in two passes:
@@ -1375,39 +1436,55 @@ __global__ void __launch_bounds__(kBlock) relax_chem(fk_params P, double *__rest
   fk::block_add(nit, &counts[1]);
 }
 
-// sum_c U_i V_c per block (consCalc.cu:3-34); i = 0 integrates 1 - alpha.
+// sum_c U_i V_c per block (consCalc.cu:3-34); i = 0 integrates 1 - alpha.  Each
+// record is read once for all variables (one pass per variable read U NEQ
+// times and reduced NEQ times).
 template <int NEQ>
 __global__ void __launch_bounds__(kBlock) integrate(int64_t nc, const double *__restrict__ U,
                                                     const double *__restrict__ vol, double *__restrict__ part) {
-  __shared__ double sh[kBlock];
-  for (int v = 0; v < NEQ; ++v) {
-    double s = 0;
-    for (int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x; c < nc; c += (int64_t)gridDim.x * kBlock) {
-      double u = U[c * NEQ + v];
-      if (NEQ == 10 && v == 0) u = 1 - u;
-      s += u * vol[c];
-    }
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int st = kBlock / 2; st > 0; st >>= 1) {
-      if ((int)threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x * NEQ + v] = sh[0];
+  __shared__ double sh[NEQ][kBlock];
+  double s[NEQ];
+#pragma unroll
+  for (int v = 0; v < NEQ; ++v) s[v] = 0;
+  for (int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x; c < nc; c += (int64_t)gridDim.x * kBlock) {
+    double u[NEQ];
+    fk::load_rec<NEQ>(U + c * NEQ, u);
+    if (NEQ == 10) u[0] = 1 - u[0];
+    const double V = vol[c];
+#pragma unroll
+    for (int v = 0; v < NEQ; ++v) s[v] += u[v] * V;
+  }
+#pragma unroll
+  for (int v = 0; v < NEQ; ++v) sh[v][threadIdx.x] = s[v];
+  __syncthreads();
+  for (int st = kBlock / 2; st > 0; st >>= 1) {
+    if ((int)threadIdx.x < st)
+#pragma unroll
+      for (int v = 0; v < NEQ; ++v) sh[v][threadIdx.x] += sh[v][threadIdx.x + st];
     __syncthreads();
   }
+  if ((int)threadIdx.x < NEQ) part[blockIdx.x * NEQ + threadIdx.x] = sh[threadIdx.x][0];
 }
 
 // Folds the per-block partials of integrate in block order, one thread per
-// variable: out[v] = ((p[0][v] + p[1][v]) + ...), the order of the host sum
-// of fk_cons_calc, so both give the same bits.
+// variable: out[v] = ((p[0][v] + p[1][v]) + ...).  The partials come through
+// LDS: 34 us when the summing thread waited for each from memory.  seq: out is
+// the context's host memory.
 template <int NEQ>
-__global__ void fold_partials(int nb, const double *__restrict__ part, double *__restrict__ out) {
+__global__ void __launch_bounds__(kBlock) fold_partials(int nb, const double *__restrict__ part,
+                                                        double *__restrict__ out, unsigned long long seq) {
+  __shared__ double sh[kConsBlocks * NEQ];
+  for (int i = threadIdx.x; i < nb * NEQ; i += kBlock) sh[i] = part[i];
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
   const int v = threadIdx.x;
-  if (v >= NEQ) return;
-  double s = 0;
-  for (int b = 0; b < nb; ++b) s += part[b * NEQ + v];
-  out[v] = s;
+  if (v < NEQ) {
+    double s = 0;
+#pragma unroll 16
+    for (int b = 0; b < nb; ++b) s += sh[b * NEQ + v];
+    out[v] = s;
+  }
+  if (seq) publish(out, seq);
 }
 
 __global__ void __launch_bounds__(kBlock) stream_copy(int64_t n16, const uint4 *__restrict__ a, uint4 *__restrict__ b) {
@@ -1419,10 +1496,36 @@ __global__ void zero_ull(unsigned long long *p, int n) {
   if (i < n) p[i] = 0ull;
 }
 
-// relaxation totals: counts[8 + i] += counts[i], i < 5
-__global__ void accum_counts(unsigned long long *p) {
-  int i = threadIdx.x;
-  if (i < 5) p[8 + i] += p[i];
+// End of a relaxation of fk_run_steps: the running totals counts[8 + i] take
+// counts[i] (i < 5) and, with nb > 0, the first K of them also the column sums
+// of the per-wave partials part[nb][K] (up to kCountParts, else
+// reduce_partials has added them before); counts[0, 8) are left zero for the
+// next one.
+constexpr int64_t kCountParts = 8192;
+template <int K>
+__global__ void __launch_bounds__(kBlock) accum_counts(const unsigned long long *__restrict__ part, int nb,
+                                                       unsigned long long *__restrict__ p) {
+  __shared__ unsigned long long sh[kBlock / 64][K];
+  unsigned long long v[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) v[k] = 0;
+  for (int b = threadIdx.x; b < nb; b += kBlock)
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += part[(int64_t)b * K + k];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_down(v[k], off, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][k] = v[k];
+  }
+  __syncthreads();
+  const int i = threadIdx.x;
+  if (i < 5) {
+    unsigned long long t = p[i];
+    if (i < K)
+      for (int w = 0; w < kBlock / 64; ++w) t += sh[w][i];
+    p[8 + i] += t;
+  }
+  if (i < 8) p[i] = 0ull;
 }
 
 // ------------------------------------------------------------------------
@@ -1476,8 +1579,8 @@ int upload_geometry(fk_ctx *c) {
 
 void free_all(fk_ctx *c) {
   void *ptrs[] = {c->link, c->geo, c->rvec, c->wls, c->vol, c->volcfl, c->U[0], c->U[1], c->U[2], c->face,
-                  c->gvel, c->rhs, c->dtc, c->red, c->dscal, c->dgrad, c->dtheta, c->lcount, c->rlist,
-                  c->rfall, c->rstart, c->rpart, c->wprim, c->health};
+                  c->gvel, c->rhs, c->dtc, c->red, c->dtw, c->dscal, c->dgrad, c->dtheta, c->lcount, c->rlist,
+                  c->rfall, c->rstart, c->rpart, c->wprim};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   c->link = nullptr;
@@ -1494,7 +1597,7 @@ void free_all(fk_ctx *c) {
   c->vol = c->volcfl = nullptr;
   c->U[0] = c->U[1] = c->U[2] = nullptr;
   c->face = c->gvel = nullptr;
-  c->rhs = c->dtc = c->red = c->dscal = c->dgrad = c->dtheta = nullptr;
+  c->rhs = c->dtc = c->red = c->dtw = c->dscal = c->dgrad = c->dtheta = nullptr;
   c->lcount = nullptr;
 }
 
@@ -1526,6 +1629,17 @@ inline int64_t quad_cells_f(const fk_ctx *c, int relax) {
 inline bool quad_g(const fk_ctx *c) { return c->stage_g == 1 && c->nc <= quad_cells_g(c); }
 inline bool quad_f(const fk_ctx *c, int relax) { return c->stage_f == 1 && c->nc <= quad_cells_f(c, relax); }
 inline unsigned grid_quad(int64_t nc) { return (unsigned)((nc + 16 * kXcd - 1) / (16 * kXcd) * kXcd); }
+
+// Whether the last pass F also runs the relaxation's per-cell pass (kind 1
+// surrogate, 2 plain).  It saves reading the state back, but runs the solve at
+// pass F's registers, and with 6 FP32 slots without LDS staging.  us a step,
+// fused / apart: FP64 plain 115 / 128 at 7k cells, 181 / 172 at 83k, 881 / 856
+// at 511k, 4732 / 4639 at 3.1M; 6 slots FP32 surrogate 103 / 106 at 27k, 526 /
+// 508 at 373k, 1696 / 1599 at 1.3M; the others 0 to 3 % better fused.
+inline bool fuse_pays(const fk_ctx *c, int kind) {
+  if (c->ns == 6) return c->p.precision == FK_FP64 || c->nc <= 200000;
+  return !(kind == 2 && c->p.precision == FK_FP64) || c->nc <= 60000;
+}
 
 template <typename T, int NS>
 int launch_pass_g_t(fk_ctx *c) {
@@ -1593,8 +1707,8 @@ int launch_pass_g_t(fk_ctx *c) {
 }
 
 template <typename T, int MODE, int NS>
-int launch_pass_f_t(fk_ctx *c, int irk, double dt, const double *dtp, double *Unew, bool write_w = false,
-                    int relax = 0) {
+int launch_pass_f_t(fk_ctx *c, int irk, double dt, const double *dtp, double *Unew, bool write_w, int relax,
+                    double *clock) {
   const unsigned gr = grid_xcd(c->nc);
   const bool visc = c->p.viscFlag == 1;
   const bool heat = visc && c->p.model == FK_MODEL_SINGLE && c->p.heatFlux == 1;
@@ -1618,12 +1732,17 @@ int launch_pass_f_t(fk_ctx *c, int irk, double dt, const double *dtp, double *Un
   c->pf_waves = (int64_t)(stage ? (int64_t)gs * (bs / 64) : (int64_t)gr * (kBlock / 64));
   const bool quad = quad_f(c, relax);
   if (quad) c->pf_waves = grid_quad(c->nc);
+  double *dtmin = nullptr;
+  if (MODE == 1) {
+    c->dt_parts = quad && grid_quad(c->nc) <= kDtParts ? (int)grid_quad(c->nc) : 0;
+    if (c->dt_parts) dtmin = c->dtw;
+  }
 #define PF_ARGS(W) \
-  c->p, c->nc, U, U0, Unew, c->link, c->geo, wl, c->vol, c->volcfl, face, gv, c->rhs, c->dtc, irk, dt, dtp, W
+  c->p, c->nc, U, U0, Unew, c->link, c->geo, wl, c->vol, c->volcfl, face, gv, c->rhs, c->dtc, irk, dt, dtp, W, clock
 #define PFQ(NEQ, VISC, HEAT, WO, RX, NAME, W, LIST, CNT, PART)                                                         \
   LAUNCH_TIMED(c, NAME,                                                                                                \
                hipLaunchKernelGGL((pass_f_q<NEQ, T, VISC, HEAT, MODE, NS, WO, RX>), dim3(grid_quad(c->nc)), dim3(64), 0, \
-                                  c->stream, PF_ARGS(W), LIST, CNT, PART))
+                                  c->stream, PF_ARGS(W), dtmin, LIST, CNT, PART))
 #define PF(NEQ, VISC, HEAT)                                                                                            \
   do {                                                                                                                 \
     if (quad) {                                                                                                        \
@@ -1711,9 +1830,9 @@ int launch_pass_g_ns(fk_ctx *c) {
 }
 template <typename T, int MODE>
 int launch_pass_f_ns(fk_ctx *c, int irk, double dt, const double *dtp, double *Unew, bool write_w = false,
-                     int relax = 0) {
-  return c->ns == 4 ? launch_pass_f_t<T, MODE, 4>(c, irk, dt, dtp, Unew, write_w, relax)
-                    : launch_pass_f_t<T, MODE, 6>(c, irk, dt, dtp, Unew, write_w, relax);
+                     int relax = 0, double *clock = nullptr) {
+  return c->ns == 4 ? launch_pass_f_t<T, MODE, 4>(c, irk, dt, dtp, Unew, write_w, relax, clock)
+                    : launch_pass_f_t<T, MODE, 6>(c, irk, dt, dtp, Unew, write_w, relax, clock);
 }
 
 int do_pass_g(fk_ctx *c) {
@@ -1729,18 +1848,21 @@ int do_pass_f_rhs(fk_ctx *c) {
   return FK_OK;
 }
 
-int do_update(fk_ctx *c, int irk, double dt, const double *dtp, bool want_w);
+int do_update(fk_ctx *c, int irk, const DtSource &ds, bool want_w);
+DtSource dt_source(const fk_ctx *c, double val, const double *ptr, double *clock);
 
 // RK stage irk from pass F: fused (MODE 0) or residual (MODE 2) + rk_update,
 // as c->fuse_update selects; both give the same bits.  want_w: the fused
 // kernel also writes the primitive records of the new state (mixed precision).
 // relax (fused form only): the kernel also runs stage 1 of the surrogate
 // relaxation (fk_relax_mlp_begin before, fk_relax_mlp_finish after).
-int do_pass_f_update(fk_ctx *c, int irk, double dt, const double *dtp, bool want_w, int relax = 0) {
+// clock: the stage ends a step of the adaptive loop, time advances by its dt.
+int do_pass_f_update(fk_ctx *c, int irk, double dt, const double *dtp, bool want_w, int relax = 0,
+                     double *clock = nullptr) {
   if (relax) {
     const int nb = next_buffer(c);
-    int rc = c->p.precision == FK_MIXED ? launch_pass_f_ns<float, 0>(c, irk, dt, dtp, c->U[nb], false, relax)
-                                        : launch_pass_f_ns<double, 0>(c, irk, dt, dtp, c->U[nb], false, relax);
+    int rc = c->p.precision == FK_MIXED ? launch_pass_f_ns<float, 0>(c, irk, dt, dtp, c->U[nb], false, relax, clock)
+                                        : launch_pass_f_ns<double, 0>(c, irk, dt, dtp, c->U[nb], false, relax, clock);
     if (rc) return rc;
     c->ia = nb;
     c->w_valid = false;  // until stage 2 has written the listed cells' records
@@ -1752,14 +1874,14 @@ int do_pass_f_update(fk_ctx *c, int irk, double dt, const double *dtp, bool want
                                         : launch_pass_f_ns<double, 2>(c, 0, 0.0, nullptr, nullptr);
     if (rc) return rc;
     c->rhs_f32 = false;
-    rc = do_update(c, irk, dt, dtp, want_w);
+    rc = do_update(c, irk, dt_source(c, dt, dtp, clock), want_w);
     c->rhs_valid = false;
     return rc;
   }
   const int nb = next_buffer(c);
   const bool w = want_w && c->p.precision == FK_MIXED && c->prims_w;
-  int rc = c->p.precision == FK_MIXED ? launch_pass_f_ns<float, 0>(c, irk, dt, dtp, c->U[nb], w)
-                                      : launch_pass_f_ns<double, 0>(c, irk, dt, dtp, c->U[nb], false);
+  int rc = c->p.precision == FK_MIXED ? launch_pass_f_ns<float, 0>(c, irk, dt, dtp, c->U[nb], w, 0, clock)
+                                      : launch_pass_f_ns<double, 0>(c, irk, dt, dtp, c->U[nb], false, 0, clock);
   if (rc) return rc;
   c->ia = nb;
   c->w_valid = w;
@@ -1767,43 +1889,83 @@ int do_pass_f_update(fk_ctx *c, int irk, double dt, const double *dtp, bool want
   return FK_OK;
 }
 
+// dt as given (val), or from the device (ptr)
+DtSource dt_source(const fk_ctx *c, double val, const double *ptr, double *clock) {
+  return DtSource{val, ptr, nullptr, 0, c->p.cfl, c->p.maxDt, c->dscal, clock != nullptr};
+}
+
 // RK stage from the stored residual (FP32 after the mixed dt stage, c->rhs_f32)
 template <int NEQ, typename RT>
-int launch_update_t(fk_ctx *c, int irk, double dt, const double *dtp, int nb, bool w) {
+int launch_update_t(fk_ctx *c, int irk, const DtSource &ds, int nb, bool w) {
   const RT *r = (const RT *)c->rhs;
   if (w)
     LAUNCH_TIMED(c, "rk_update", hipLaunchKernelGGL((rk_update_w<NEQ, RT>), dim3(grid_for(c->nc)), dim3(kBlock), 0,
                                                     c->stream, c->p, c->nc, c->U[c->ia], c->U[c->iu0], c->U[nb], r,
-                                                    c->vol, irk, dt, dtp, c->wprim));
+                                                    c->vol, irk, ds, c->wprim));
   else
     LAUNCH_TIMED(c, "rk_update", hipLaunchKernelGGL((rk_update<NEQ, RT>), dim3(grid_for(c->nc * NEQ)), dim3(kBlock), 0,
                                                     c->stream, c->p, c->nc, c->U[c->ia], c->U[c->iu0], c->U[nb], r,
-                                                    c->vol, irk, dt, dtp));
+                                                    c->vol, irk, ds));
   return FK_OK;
 }
 
-int do_update(fk_ctx *c, int irk, double dt, const double *dtp, bool want_w) {
+int do_update(fk_ctx *c, int irk, const DtSource &ds, bool want_w) {
   const int nb = next_buffer(c);
   const bool w = want_w && c->p.precision == FK_MIXED && c->prims_w;
   int rc;
   if (c->neq == 5)
-    rc = c->rhs_f32 ? launch_update_t<5, float>(c, irk, dt, dtp, nb, w) : launch_update_t<5, double>(c, irk, dt, dtp, nb, w);
+    rc = c->rhs_f32 ? launch_update_t<5, float>(c, irk, ds, nb, w) : launch_update_t<5, double>(c, irk, ds, nb, w);
   else
-    rc = c->rhs_f32 ? launch_update_t<10, float>(c, irk, dt, dtp, nb, w)
-                    : launch_update_t<10, double>(c, irk, dt, dtp, nb, w);
+    rc = c->rhs_f32 ? launch_update_t<10, float>(c, irk, ds, nb, w) : launch_update_t<10, double>(c, irk, ds, nb, w);
   if (rc) return rc;
   c->ia = nb;
   c->w_valid = w;
   return FK_OK;
 }
 
-int do_dt_device(fk_ctx *c) {
-  const int nb = 1024;
-  LAUNCH_TIMED(c, "dt_reduce",
-               hipLaunchKernelGGL(min_blocks, dim3(nb), dim3(kBlock), 0, c->stream, c->nc, c->dtc, c->red);
-               hipLaunchKernelGGL(dt_final, dim3(1), dim3(kBlock), 0, c->stream, nb, c->red, c->p.cfl, c->p.maxDt,
-                                  c->dscal));
+// Waits for the last published result.  A synchronisation of the stream costs
+// about 20 us on top of the kernels; the result is polled for instead, up to
+// 2 ms, and then left to the synchronisation (which also reports errors).
+int wait_result(fk_ctx *c) {
+  const volatile unsigned long long *seq = reinterpret_cast<const volatile unsigned long long *>(c->hres) + kHostSeq;
+  const auto t0 = std::chrono::steady_clock::now();
+  while (*seq != c->hseq) {
+    if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
+      HIPCHK(hipStreamSynchronize(c->stream));
+      return FK_OK;
+    }
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
   return FK_OK;
+}
+
+// dt of the last pass F MODE 1 into dscal[0] (and host[0])
+int do_dt_device(fk_ctx *c, double *host) {
+  const double *part = c->dtw;
+  int nb = c->dt_parts;
+  if (!nb) {
+    part = c->red;
+    nb = 1024;
+    LAUNCH_TIMED(c, "dt_reduce",
+                 hipLaunchKernelGGL(min_blocks, dim3(nb), dim3(kBlock), 0, c->stream, c->nc, c->dtc, c->red));
+  }
+  LAUNCH_TIMED(c, "dt_final", hipLaunchKernelGGL(dt_final, dim3(1), dim3(kBlock), 0, c->stream, nb, part, c->p.cfl,
+                                                 c->p.maxDt, c->dscal, host, host ? ++c->hseq : 0ull));
+  return FK_OK;
+}
+
+// The dt stage of fk_run_steps after pass F MODE 1: dt and the RK update.
+int do_dt_update(fk_ctx *c, int irk, bool want_w, double *clock) {
+  DtSource ds = dt_source(c, 0.0, c->dscal, clock);
+  if (c->dt_parts) {
+    ds.ptr = nullptr;
+    ds.minima = c->dtw;
+    ds.nmin = c->dt_parts;
+  } else {
+    int rc = do_dt_device(c, nullptr);
+    if (rc) return rc;
+  }
+  return do_update(c, irk, ds, want_w);
 }
 
 // stats of the counters at slots [base, base + 5) of c->lcount
@@ -1821,6 +1983,15 @@ int read_counts(fk_ctx *c, int base, fk_relax_stats *st) {
 }
 
 }  // namespace
+
+// counts[0, 8) zero before a relaxation; the loop's relaxations leave them so
+int zero_counts(fk_ctx *c) {
+  if (!c->counts_clean)
+    LAUNCH_TIMED(c, "zero", hipLaunchKernelGGL(zero_ull, dim3(1), dim3(64), 0, c->stream,
+                                               (unsigned long long *)c->lcount, 8));
+  c->counts_clean = false;
+  return FK_OK;
+}
 
 // work list of the relaxation passes (one uint32 per cell), allocated on first use
 // Network starts (float2 per work-list entry) of the surrogate relaxation.
@@ -1872,13 +2043,30 @@ int relax_preflight(fk_ctx *c, int mode) {
   return mode == FK_RELAX_MLP ? ensure_rstart(c) : FK_OK;
 }
 
+// Totals of a relaxation of the loop: K columns of nb partial counts (added by
+// reduce_partials already when there are more than kCountParts).
+int end_counts(fk_ctx *c, int K, int64_t nb) {
+  unsigned long long *cnt = (unsigned long long *)c->lcount;
+  const int n = nb > kCountParts ? 0 : (int)nb;
+  if (K == 2)
+    LAUNCH_TIMED(c, "relax_totals", hipLaunchKernelGGL(accum_counts<2>, dim3(1), dim3(kBlock), 0, c->stream, c->rpart, n, cnt));
+  else
+    LAUNCH_TIMED(c, "relax_totals", hipLaunchKernelGGL(accum_counts<3>, dim3(1), dim3(kBlock), 0, c->stream, c->rpart, n, cnt));
+  c->counts_clean = true;
+  ++c->relax_calls;
+  return FK_OK;
+}
+
 int do_relax(fk_ctx *c, fk_relax_stats *st, int mode = FK_RELAX_PLAIN) {
   if (c->p.model != FK_MODEL_TWO_PHASE) return fail(FK_EINVAL, "relaxation needs the two-phase model");
   unsigned long long *cnt = (unsigned long long *)c->lcount;
+  const int64_t nb = grid_for(c->nc);
+  int K = 3;
   if (mode == FK_RELAX_MLP || mode == FK_RELAX_COLD) {
     if (c->p.thermFntRlxFlag == 1) return fail(FK_EINVAL, "finite-rate relaxation needs FK_RELAX_PLAIN");
-    int rc = fk_relax_mlp_impl(c, mode == FK_RELAX_MLP);
+    int rc = fk_relax_mlp_impl(c, mode == FK_RELAX_MLP, st || grid_for(c->nc) > kCountParts);
     if (rc) return rc;
+    K = 2;
   } else {
     if (!st) {  // plain relaxation that also emits training pairs, when enabled
       bool done = false;
@@ -1889,14 +2077,14 @@ int do_relax(fk_ctx *c, fk_relax_stats *st, int mode = FK_RELAX_PLAIN) {
       }
     }
     int rc = ensure_rlist(c);
-    if (rc) return rc;
-    LAUNCH_TIMED(c, "zero", hipLaunchKernelGGL(zero_ull, dim3(1), dim3(64), 0, c->stream, cnt, 6));
+    if (rc || (rc = zero_counts(c))) return rc;
     // mixed precision: the relaxation also writes the primitive records of pass G
     float *W = (c->p.precision == FK_MIXED && c->prims_w) ? c->wprim : nullptr;
     LAUNCH_TIMED(c, "relax", hipLaunchKernelGGL(relax_therm, dim3(grid_for(c->nc)), dim3(kBlock), 0, c->stream, c->p,
                                                 c->nc, c->U[c->ia], c->rlist, cnt, c->rpart, W));
-    LAUNCH_TIMED(c, "relax_count", hipLaunchKernelGGL(fk::reduce_partials<3>, dim3(fk::reduce_grid(grid_for(c->nc))),
-                                                      dim3(256), 0, c->stream, c->rpart, (int64_t)grid_for(c->nc), cnt));
+    if (st || nb > kCountParts)
+      LAUNCH_TIMED(c, "relax_count", hipLaunchKernelGGL(fk::reduce_partials<3>, dim3(fk::reduce_grid(nb)), dim3(256), 0,
+                                                        c->stream, c->rpart, nb, cnt));
     const unsigned gch = (unsigned)std::max<int64_t>(1, std::min<int64_t>(grid_for(c->nc), 1024));
     LAUNCH_TIMED(c, "relax_chem", hipLaunchKernelGGL(relax_chem, dim3(gch), dim3(kBlock), 0, c->stream, c->p,
                                                      c->U[c->ia], c->rlist, cnt, W));
@@ -1906,27 +2094,20 @@ int do_relax(fk_ctx *c, fk_relax_stats *st, int mode = FK_RELAX_PLAIN) {
     int rc = read_counts(c, 0, st);
     if (rc) return rc;
     st->n_therm = c->nc - st->n_chem;
-  } else {
-    hipLaunchKernelGGL(accum_counts, dim3(1), dim3(64), 0, c->stream, cnt);
-    HIPCHK(hipGetLastError());
-    ++c->relax_calls;
+    return FK_OK;
   }
-  return FK_OK;
+  return end_counts(c, K, nb);
 }
 
 // After a fused pass F ran stage 1 of the surrogate relaxation: its per-wave
 // counts, stage 2 and the running totals (as do_relax).
 int relax_fused_finish(fk_ctx *c, bool warm) {
-  unsigned long long *cnt = (unsigned long long *)c->lcount;
   const int64_t nw = c->pf_waves;
-  LAUNCH_TIMED(c, "relax_count", hipLaunchKernelGGL(fk::reduce_partials<2>, dim3(fk::reduce_grid(nw)), dim3(256), 0,
-                                                    c->stream, c->rpart, nw, cnt));
+  if (nw > kCountParts)
+    LAUNCH_TIMED(c, "relax_count", hipLaunchKernelGGL(fk::reduce_partials<2>, dim3(fk::reduce_grid(nw)), dim3(256), 0,
+                                                      c->stream, c->rpart, nw, (unsigned long long *)c->lcount));
   int rc = fk_relax_mlp_finish(c, warm);
-  if (rc) return rc;
-  hipLaunchKernelGGL(accum_counts, dim3(1), dim3(64), 0, c->stream, cnt);
-  HIPCHK(hipGetLastError());
-  ++c->relax_calls;
-  return FK_OK;
+  return rc ? rc : end_counts(c, 2, nw);
 }
 
 // The plain relaxation inside the last fused pass F: zeroed counts before it,
@@ -1934,26 +2115,21 @@ int relax_fused_finish(fk_ctx *c, bool warm) {
 // running totals (as do_relax).
 int relax_plain_begin(fk_ctx *c) {
   int rc = ensure_rlist(c);
-  if (rc) return rc;
-  unsigned long long *cnt = (unsigned long long *)c->lcount;
-  LAUNCH_TIMED(c, "zero", hipLaunchKernelGGL(zero_ull, dim3(1), dim3(64), 0, c->stream, cnt, 6));
-  return FK_OK;
+  return rc ? rc : zero_counts(c);
 }
 
 int relax_plain_fused_finish(fk_ctx *c) {
   unsigned long long *cnt = (unsigned long long *)c->lcount;
   const int64_t nw = c->pf_waves;
-  LAUNCH_TIMED(c, "relax_count", hipLaunchKernelGGL(fk::reduce_partials<3>, dim3(fk::reduce_grid(nw)), dim3(256), 0,
-                                                    c->stream, c->rpart, nw, cnt));
+  if (nw > kCountParts)
+    LAUNCH_TIMED(c, "relax_count", hipLaunchKernelGGL(fk::reduce_partials<3>, dim3(fk::reduce_grid(nw)), dim3(256), 0,
+                                                      c->stream, c->rpart, nw, cnt));
   float *W = (c->p.precision == FK_MIXED && c->prims_w) ? c->wprim : nullptr;
   const unsigned gch = (unsigned)std::max<int64_t>(1, std::min<int64_t>(grid_for(c->nc), 1024));
   LAUNCH_TIMED(c, "relax_chem", hipLaunchKernelGGL(relax_chem, dim3(gch), dim3(kBlock), 0, c->stream, c->p,
                                                    c->U[c->ia], c->rlist, cnt, W));
   c->w_valid = W != nullptr;
-  hipLaunchKernelGGL(accum_counts, dim3(1), dim3(64), 0, c->stream, cnt);
-  HIPCHK(hipGetLastError());
-  ++c->relax_calls;
-  return FK_OK;
+  return end_counts(c, 3, nw);
 }
 
 int check_params(const fk_params *p) {
@@ -2014,6 +2190,13 @@ int fk_create(int device, const fk_params *p, fk_ctx **out) {
     delete c;
     return fail(FK_EDEVICE, std::string("hipStreamCreate: ") + hipGetErrorString(e));
   }
+  e = hipHostMalloc(reinterpret_cast<void **>(&c->hres), 64 * sizeof(double), hipHostMallocDefault);
+  if (e != hipSuccess) {
+    (void)hipStreamDestroy(c->stream);
+    delete c;
+    return fail(FK_ENOMEM, std::string("hipHostMalloc: ") + hipGetErrorString(e));
+  }
+  std::memset(c->hres, 0, 64 * sizeof(double));
   g_xfer.attach();
   *out = c;
   return FK_OK;
@@ -2031,6 +2214,7 @@ int fk_destroy(fk_ctx *c) {
   free_all(c);
   fk_mlp_free(c);
   xfer_free(c);
+  (void)hipHostFree(c->hres);
   g_xfer.detach();
   (void)hipStreamDestroy(c->stream);
   delete c;
@@ -2156,19 +2340,22 @@ int fk_upload_mesh(fk_ctx *c, int64_t nElem, int64_t nFcs, const int32_t *fc2el,
   HIPCHK(hipMalloc(&c->rhs, cs * neq * 8));
   HIPCHK(hipMalloc(&c->dtc, cs * 8));
   HIPCHK(hipMalloc(&c->red, 4096 * 8));
+  HIPCHK(hipMalloc(&c->dtw, kDtParts * 8));
   HIPCHK(hipMalloc(&c->dscal, 16 * 8));
   HIPCHK(hipMalloc(&c->lcount, 16 * 8));
-  HIPCHK(hipMalloc(&c->health, sizeof(unsigned long long)));
-  {
-    const unsigned long long none = ~0ull;
-    HIPCHK(hipMemcpy(c->health, &none, sizeof none, hipMemcpyHostToDevice));
-  }
   HIPCHK(hipMalloc(&c->wprim, cs * neq * sizeof(float)));
   HIPCHK(hipMemset(c->lcount, 0, 16 * 8));
   HIPCHK(hipMemcpy(c->link, hlink.data(), (size_t)ns * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->vol, volume, cs * 8, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->volcfl, vcfl.data(), cs * 8, hipMemcpyHostToDevice));
   HIPCHK(hipMemset(c->dscal, 0, 16 * 8));
+  // the health record sits behind dt and time: one copy carries all three
+  c->health = reinterpret_cast<unsigned long long *>(c->dscal + 2);
+  {
+    const unsigned long long none = ~0ull;
+    HIPCHK(hipMemcpy(c->health, &none, sizeof none, hipMemcpyHostToDevice));
+  }
+  c->counts_clean = true;
   c->slot_face.swap(sf);
   int rc = upload_geometry(c);
   if (rc) return rc;
@@ -2226,13 +2413,10 @@ int fk_compute_time_step(fk_ctx *c, double *dt) {
   if (rc) return rc;
   if (!c->rhs_valid) return fail(FK_ESTATE, "fk_compute_rhs must run before fk_compute_time_step");
   HIPCHK(hipSetDevice(c->device));
-  rc = do_dt_device(c);
-  if (rc) return rc;
-  double h[2];
-  HIPCHK(hipMemcpyAsync(h, c->dscal, sizeof h, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  c->dt = h[0];
-  if (dt) *dt = h[0];
+  rc = do_dt_device(c, c->hres);
+  if (rc || (rc = wait_result(c))) return rc;
+  c->dt = c->hres[0];
+  if (dt) *dt = c->dt;
   return FK_OK;
 }
 
@@ -2242,7 +2426,7 @@ int fk_update(fk_ctx *c, int irk, double dt) {
   if (!c->rhs_valid) return fail(FK_ESTATE, "fk_compute_rhs must run before fk_update");
   if (irk < 0 || irk >= c->p.rkSteps) return fail(FK_EINVAL, "bad RK stage");
   HIPCHK(hipSetDevice(c->device));
-  rc = do_update(c, irk, dt, nullptr, true);
+  rc = do_update(c, irk, dt_source(c, dt, nullptr, nullptr), true);
   c->rhs_valid = false;
   return rc;
 }
@@ -2312,20 +2496,20 @@ int fk_cons_calc(fk_ctx *c, double *out) {
   if (rc) return rc;
   if (!out) return fail(FK_EINVAL, "null argument");
   HIPCHK(hipSetDevice(c->device));
-  const int nb = kConsBlocks;
-  if (c->neq == 5)
-    hipLaunchKernelGGL((integrate<5>), dim3(nb), dim3(kBlock), 0, c->stream, c->nc, c->U[c->ia], c->vol, c->red);
-  else
-    hipLaunchKernelGGL((integrate<10>), dim3(nb), dim3(kBlock), 0, c->stream, c->nc, c->U[c->ia], c->vol, c->red);
-  HIPCHK(hipGetLastError());
-  std::vector<double> h((size_t)nb * c->neq);
-  HIPCHK(hipMemcpyAsync(h.data(), c->red, h.size() * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  for (int v = 0; v < c->neq; ++v) {
-    double s = 0;
-    for (int b = 0; b < nb; ++b) s += h[(size_t)(b * c->neq + v)];
-    out[v] = s;
+  // the folded sums go straight to page-locked memory (no copy to wait for)
+  if (c->neq == 5) {
+    hipLaunchKernelGGL((integrate<5>), dim3(kConsBlocks), dim3(kBlock), 0, c->stream, c->nc, c->U[c->ia], c->vol, c->red);
+    hipLaunchKernelGGL((fold_partials<5>), dim3(1), dim3(kBlock), 0, c->stream, kConsBlocks, c->red, c->hres,
+                       ++c->hseq);
+  } else {
+    hipLaunchKernelGGL((integrate<10>), dim3(kConsBlocks), dim3(kBlock), 0, c->stream, c->nc, c->U[c->ia], c->vol, c->red);
+    hipLaunchKernelGGL((fold_partials<10>), dim3(1), dim3(kBlock), 0, c->stream, kConsBlocks, c->red, c->hres,
+                       ++c->hseq);
   }
+  HIPCHK(hipGetLastError());
+  rc = wait_result(c);
+  if (rc) return rc;
+  for (int v = 0; v < c->neq; ++v) out[v] = c->hres[v];
   return FK_OK;
 }
 
@@ -2344,10 +2528,10 @@ int fk_cons_calc_noalloc(fk_ctx *c, double *out) {
   double *sums = ptr + (int64_t)kConsBlocks * c->neq;
   if (c->neq == 5) {
     hipLaunchKernelGGL((integrate<5>), dim3(kConsBlocks), dim3(kBlock), 0, c->stream, c->nc, c->U[c->ia], c->vol, ptr);
-    hipLaunchKernelGGL((fold_partials<5>), dim3(1), dim3(64), 0, c->stream, kConsBlocks, ptr, sums);
+    hipLaunchKernelGGL((fold_partials<5>), dim3(1), dim3(kBlock), 0, c->stream, kConsBlocks, ptr, sums, 0ull);
   } else {
     hipLaunchKernelGGL((integrate<10>), dim3(kConsBlocks), dim3(kBlock), 0, c->stream, c->nc, c->U[c->ia], c->vol, ptr);
-    hipLaunchKernelGGL((fold_partials<10>), dim3(1), dim3(64), 0, c->stream, kConsBlocks, ptr, sums);
+    hipLaunchKernelGGL((fold_partials<10>), dim3(1), dim3(kBlock), 0, c->stream, kConsBlocks, ptr, sums, 0ull);
   }
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(out, sums, (size_t)c->neq * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -2367,10 +2551,10 @@ int fk_run_steps(fk_ctx *c, int nsteps, double *dt_last, double *phys_time) {
     return rc;
   // the device scalars hold dt and the physical time; the health record
   // starts clean for this call
-  double h[2] = {c->dt, c->time};
-  HIPCHK(hipMemcpy(c->dscal, h, sizeof h, hipMemcpyHostToDevice));
+  double h[3] = {c->dt, c->time, 0};
   unsigned long long hh = ~0ull;
-  HIPCHK(hipMemcpy(c->health, &hh, sizeof hh, hipMemcpyHostToDevice));
+  std::memcpy(&h[2], &hh, sizeof hh);
+  HIPCHK(hipMemcpy(c->dscal, h, sizeof h, hipMemcpyHostToDevice));
   for (int s = 0; s < nsteps; ++s) {
     if (p.rkSteps > 1) c->iu0 = c->ia;
     const bool newdt = p.adaptDt == 1 && c->step % p.adaptDtItr == 0;
@@ -2385,25 +2569,23 @@ int fk_run_steps(fk_ctx *c, int nsteps, double *dt_last, double *phys_time) {
     int relaxed_in_f = 0;
     for (int irk = 0; irk < p.rkSteps; ++irk) {
       const bool want_w = irk < p.rkSteps - 1 || !relax_next;
+      double *clock = p.adaptDt == 1 && irk == p.rkSteps - 1 ? c->dscal : nullptr;  // the step's last stage
       if ((rc = do_pass_g(c))) return rc;
       if (irk == 0 && newdt) {
         if ((rc = do_pass_f_rhs(c))) return rc;
-        if ((rc = do_dt_device(c))) return rc;
-        if ((rc = do_update(c, irk, 0.0, c->dscal, want_w))) return rc;
+        if ((rc = do_dt_update(c, irk, want_w, clock))) return rc;
       } else {
-        const int fr = (c->fuse_relax && c->fuse_update && irk == p.rkSteps - 1) ? relax_kind : 0;
+        const int fr =
+            (c->fuse_relax && c->fuse_update && irk == p.rkSteps - 1 && fuse_pays(c, relax_kind)) ? relax_kind : 0;
         if (fr == 1 && (rc = fk_relax_mlp_begin(c, warm))) return rc;
         if (fr == 2 && (rc = relax_plain_begin(c))) return rc;
-        if (p.adaptDt == 1) rc = do_pass_f_update(c, irk, 0.0, c->dscal, want_w, fr);
+        if (p.adaptDt == 1) rc = do_pass_f_update(c, irk, 0.0, c->dscal, want_w, fr, clock);
         else rc = do_pass_f_update(c, irk, p.dt, nullptr, want_w, fr);
         if (rc) return rc;
         relaxed_in_f = fr;
       }
     }
-    if (p.adaptDt == 1)
-      LAUNCH_TIMED(c, "advance_time", hipLaunchKernelGGL(advance_time, dim3(1), dim3(64), 0, c->stream, c->dscal));
-    else
-      c->dt = p.dt;
+    if (p.adaptDt != 1) c->dt = p.dt;
     if (relaxed_in_f == 1) {
       if ((rc = relax_fused_finish(c, warm))) return rc;
     } else if (relaxed_in_f == 2) {
@@ -2413,9 +2595,10 @@ int fk_run_steps(fk_ctx *c, int nsteps, double *dt_last, double *phys_time) {
     }
     c->step++;
   }
-  HIPCHK(hipMemcpyAsync(h, c->dscal, sizeof h, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipMemcpyAsync(&hh, c->health, sizeof hh, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipMemcpyAsync(c->hres, c->dscal, sizeof h, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  std::memcpy(h, c->hres, sizeof h);
+  std::memcpy(&hh, &h[2], sizeof hh);
   if (p.adaptDt == 1) {
     c->dt = h[0];
     c->time = h[1];

@@ -786,12 +786,6 @@ __global__ void __launch_bounds__(256) relax_emit_k(fk_params P, int64_t nc, dou
   }
 }
 
-__global__ void zero_u64_k(unsigned long long *p, int n) {
-  if ((int)threadIdx.x < n) p[threadIdx.x] = 0ull;
-}
-
-
-
 // ---------------- host side ----------------
 
 Norm norm_of(const Mlp &m) {
@@ -881,12 +875,10 @@ int fk_relax_mlp_begin(fk_ctx *c, bool warm) {
     return fail(FK_EINVAL, "surrogate classification needs eta_L <= eta_G and Cp_G >= Cp_L");
   int rc = ensure_rlist(c);
   if (rc) return rc;
-  unsigned long long *cnt = (unsigned long long *)c->lcount;
-  LAUNCH_TIMED(c, "zero", hipLaunchKernelGGL(zero_u64_k, dim3(1), dim3(64), 0, c->stream, cnt, 8));
-  return FK_OK;
+  return zero_counts(c);
 }
 
-int fk_relax_mlp_impl(fk_ctx *c, bool warm) {
+int fk_relax_mlp_impl(fk_ctx *c, bool warm, bool reduce) {
   int rc = fk_relax_mlp_begin(c, warm);
   if (rc) return rc;
   unsigned long long *cnt = (unsigned long long *)c->lcount;
@@ -895,8 +887,9 @@ int fk_relax_mlp_impl(fk_ctx *c, bool warm) {
   float *W = (c->p.precision == FK_MIXED && c->prims_w) ? c->wprim : nullptr;
   LAUNCH_TIMED(c, "relax_screen", hipLaunchKernelGGL(relax_screen_k, dim3(gs), dim3(256), 0, c->stream, c->p, c->nc,
                                                      c->U[c->ia], c->rlist, cnt, c->rpart, W));
-  LAUNCH_TIMED(c, "relax_count", hipLaunchKernelGGL(fk::reduce_partials<2>, dim3(fk::reduce_grid(gs)), dim3(256), 0,
-                                                    c->stream, c->rpart, (int64_t)gs, cnt));
+  if (reduce)
+    LAUNCH_TIMED(c, "relax_count", hipLaunchKernelGGL(fk::reduce_partials<2>, dim3(fk::reduce_grid(gs)), dim3(256), 0,
+                                                      c->stream, c->rpart, (int64_t)gs, cnt));
   return fk_relax_mlp_finish(c, warm);
 }
 
