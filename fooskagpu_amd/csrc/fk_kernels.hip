@@ -1022,8 +1022,6 @@ __global__ void __launch_bounds__(64, 2) pass_g_q(fk_params P, int64_t nc, const
     const T nav[3] = {ga[r].x * sa, ga[r].y * sa, ga[r].z * sa};
 #pragma unroll
     for (int v = 0; v < NEQ; ++v) {
-      // one variable after the other: interleaved, their terms spill (FP64)
-      __builtin_amdgcn_sched_barrier(0);
       const T avg = (W[v] + Wn[r][v]) / 2;
       if constexpr (sizeof(T) == 8) {
 #pragma unroll
@@ -1031,6 +1029,9 @@ __global__ void __launch_bounds__(64, 2) pass_g_q(fk_params P, int64_t nc, const
           const T t = real ? dV(avg * nav[d] * ga[r].w) : 0;
 #pragma unroll
           for (int j = 0; j < quad_lanes<NS>(r); ++j) g[v][d] += quad_bcast(t, j);
+          // the sum formed here: moved to its use, the quad's terms stay in
+          // registers and spill (232 instead of 256 VGPRs and 64 spilled)
+          asm volatile("" : "+v"(g[v][d]));
         }
       } else {
         // FMAs in slot order: the operands cross the quad (zero past the last face)
@@ -1163,7 +1164,10 @@ __global__ void __launch_bounds__(64, 2) pass_f_q(fk_params P, int64_t nc, const
 #pragma unroll
     for (int j = 0; j < 4; ++j) {  // lanes without a slot add 0
 #pragma unroll
-      for (int v = 0; v < NEQ; ++v) rhs[v] += quad_bcast(fr[v], j);
+      for (int v = 0; v < NEQ; ++v) {
+        rhs[v] += quad_bcast(fr[v], j);
+        asm volatile("" : "+v"(rhs[v]));
+      }
       if constexpr (VISC) {
 #pragma unroll
         for (int i = 0; i < (HEAT ? 5 : 4); ++i) rv[i] += quad_bcast(fv[i], j);
@@ -1605,26 +1609,31 @@ void free_all(fk_ctx *c) {
 // pass_f_q) rather than one with the LDS paths.  What the quads win is waves
 // in flight and shorter chains; what they lose is the own-cell work on four
 // lanes and, with records of half the size (FP32), pass F's LDS reuse.  us,
-// quads / one lane, near the lines:
-//   pass G  FP64 single-phase 7 / 10 at 12k cells, 11 / 12 at 55k, 14 / 14 at
-//           73k; FP32 11 / 11 at 48k tetrahedra, 13 / 12 at 27k hexahedra; FP64
-//           two-phase spills and stays with one lane (17 / 14 at 25k)
-//   pass F  FP64 21 / 29 at 83k, 45 / 71 at 236k, 297 / 306 (residual 292 / 325)
+// quads / one lane, on either side of the lines:
+//   pass G  FP64 12 / 13 at 55k cells (single-phase), 16 / 19 at 48k and 23 / 21 at
+//           83k (two-phase); FP32 10 / 11 at 48k, 16 / 13 at 94k; 6 slots FP64
+//           21 / 23 at 27k, 33 / 26 at 55k; FP32 9 / 12 at 8k, 13 / 12 at 27k
+//   pass F  FP64 20 / 29 at 83k, 48 / 72 at 280k, 297 / 306 (residual 292 / 325)
 //           at 1.05M, 857 / 846 (832 / 905) at 3.1M: its one-lane kernel runs
-//           2 waves per SIMD; FP32 two-phase 29 / 34 at 162k, 60 / 56 at 280k,
-//           hexahedra 37 / 33 at 85k; single-phase 30 / 39 at 280k, 47 / 46 at 384k
-//   with the relaxation (it is on four lanes alike, but for the plain solve's
-//   residuals) FP64 53 / 65 at 83k, 106 / 125 at 236k, 234 / 214 at 384k,
-//           hexahedral slots 26 / 46 at 7k, 66 / 53 at 55k; FP32 25 / 22 at 48k
+//           2 waves per SIMD; FP32 53 / 56 at 280k, 100 / 90 at 511k (two-phase),
+//           51 / 59 at 511k, 178 / 160 at 1.6M (single-phase); 6 slots FP32
+//           28 / 29 at 55k, 63 / 60 at 176k
+//   with the relaxation (on the quad only the plain solve's residuals go in
+//           parallel) FP64 64 / 70 at 162k, 106 / 103 at 280k; FP32 22 / 22 at 48k,
+//           34 / 31 at 94k, plain 81 / 85 at 162k; 6 slots FP64 26 / 31 at 27k,
+//           65 / 53 at 55k; FP32 22 / 26 at 27k, 48 / 40 at 85k
 inline int64_t quad_cells_g(const fk_ctx *c) {
-  if (c->neq == 10 && c->p.precision == FK_FP64) return 0;
-  return c->ns == 6 ? 15000 : (c->neq == 5 ? 60000 : 40000);
+  if (c->ns == 6) return c->p.precision == FK_FP64 ? 40000 : 20000;
+  return 60000;
 }
 inline int64_t quad_cells_f(const fk_ctx *c, int relax) {
   const bool f64 = c->p.precision == FK_FP64;
-  if (relax) return c->ns == 4 && f64 ? 250000 : 30000;
+  if (relax) {
+    if (c->ns == 6) return 35000;
+    return f64 ? 220000 : (relax == 2 ? 160000 : 50000);
+  }
   if (f64) return 4000000;
-  return c->ns == 6 ? 60000 : (c->neq == 5 ? 300000 : 200000);
+  return c->ns == 6 ? 120000 : (c->neq == 5 ? 600000 : 350000);
 }
 inline bool quad_g(const fk_ctx *c) { return c->stage_g == 1 && c->nc <= quad_cells_g(c); }
 inline bool quad_f(const fk_ctx *c, int relax) { return c->stage_f == 1 && c->nc <= quad_cells_f(c, relax); }
@@ -1665,7 +1674,7 @@ int launch_pass_g_t(fk_ctx *c) {
                                   c->health, (int)std::min<int64_t>(c->step, INT32_MAX)))
 #define PG2(NEQ, VISC, HEAT, FW)                                                                                     \
   do {                                                                                                               \
-    if constexpr (NEQ == 5 || sizeof(T) == 4) {                                                                      \
+    {                                                                                                                \
       if (quad) {                                                                                                    \
         LAUNCH_TIMED(c, "pass_g",                                                                                    \
                      hipLaunchKernelGGL((pass_g_q<NEQ, T, VISC, HEAT, FW, NS>), dim3(grid_quad(c->nc)), dim3(64), 0, \
@@ -2020,7 +2029,7 @@ int ensure_rlist(fk_ctx *c) {
   // [blocks][4] partials of the relaxation kernels, or [waves][2 or 3] of the
   // fused pass F (grid_xcd blocks of 4 waves, or one wave for 16 cells)
   size_t parts = (size_t)grid_xcd(c->nc) * 12;
-  if (c->nc <= quad_cells_f(c, 1)) parts = std::max(parts, (size_t)grid_quad(c->nc) * 3);
+  if (c->nc <= std::max(quad_cells_f(c, 1), quad_cells_f(c, 2))) parts = std::max(parts, (size_t)grid_quad(c->nc) * 3);
   HIPCHK(hipMalloc(&c->rpart, parts * sizeof(unsigned long long)));
   c->rlist_cap = c->nc;
   return FK_OK;

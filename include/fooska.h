@@ -219,7 +219,7 @@ int fk_set_debug(fk_ctx *ctx, int on);
  *     relaxation pass).  2: one lane with LDS at every size; 0: one lane
  *     without.
  *  "stage_g" (default 1): pass G by the size of the mesh: four lanes per cell
- *     up to 15,000 to 60,000 cells, else one lane per cell with the
+ *     up to 20,000 to 60,000 cells, else one lane per cell with the
  *     workgroup's face records and velocity gradients written from LDS in
  *     16-byte words (4 slots per cell: 256 cells, FP64 128; 6 slots: two-phase
  *     FP32, 128 cells).  2: one lane with LDS at every size; 0: one lane with
