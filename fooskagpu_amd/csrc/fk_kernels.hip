@@ -1226,13 +1226,14 @@ __global__ void __launch_bounds__(64, 2) pass_f_q(fk_params P, int64_t nc, const
   }
 }
 
-// dt of the update kernels.  nmin > 0: from the minima that pass F's waves left
-// (up to kDtParts of them, which every block folds for itself; two kernels and
-// their gaps fewer than min_blocks + dt_final: with the time's own kernel gone too a
-// 12k-cell Sod step takes 34 instead of 39 us);
-// block 0 stores it.  clock: the update ends a step, the physical time
-// advances.
-constexpr int kDtParts = 8192;
+// dt of the update kernels.  nmin > 0: from the minima that pass F's waves left,
+// which every block folds for itself; block 0 stores it.  Up to kDtFold of
+// them: two kernels and their gaps fewer than min_blocks + dt_final (with the
+// time's own kernel gone too a 12k-cell Sod step takes 34 instead of 39 us);
+// 5184 minima, folded by 3240 blocks, made the update 20 us long instead of 7,
+// so up to kDtParts dt_final folds them.  clock: the update ends a step, the
+// physical time advances.
+constexpr int kDtParts = 8192, kDtFold = 1024;
 struct DtSource {
   double val;             // the dt, unless ptr or nmin says otherwise
   const double *ptr;
@@ -1966,7 +1967,7 @@ int do_dt_device(fk_ctx *c, double *host) {
 // The dt stage of fk_run_steps after pass F MODE 1: dt and the RK update.
 int do_dt_update(fk_ctx *c, int irk, bool want_w, double *clock) {
   DtSource ds = dt_source(c, 0.0, c->dscal, clock);
-  if (c->dt_parts) {
+  if (c->dt_parts && c->dt_parts <= kDtFold) {
     ds.ptr = nullptr;
     ds.minima = c->dtw;
     ds.nmin = c->dt_parts;
