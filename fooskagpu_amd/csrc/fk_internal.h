@@ -36,11 +36,11 @@ struct Timer {
   std::vector<hipEvent_t> pool;
 };
 
-// Events of the large host copies (fk_xfer.h), made by the first one of a
-// context.
+// Block counts of the large host copies' kernels (fk_xfer.h), made by the first
+// one of a context.
 constexpr int kXferThreads = 8;
 struct Xfer {
-  hipEvent_t ev[2 * kXferThreads] = {};
+  unsigned *count = nullptr;
 };
 
 // Surrogate (MLP 3-64-64-64-3) state of a context.

@@ -4,13 +4,17 @@
 // One hipMemcpy into a buffer the caller has just allocated runs at 11 GB/s
 // (245 MB in 22.7 ms): one thread clears the buffer's fresh pages and copies
 // out of the runtime's staging memory.  Large copies therefore go through
-// page-locked slots of our own, two to a thread, with the DMA of one slot
-// overlapping the host copy of the other, on up to kXferThreads threads: 6.0
-// ms into fresh pages, and 5.4 instead of 8.3 ms from the host.  Slots of 4 MB:
-// an asynchronous copy costs about 18 us however small (1 MB slots: 8.0 ms).
-// Mid sizes use part of a slot, so that a few threads share the copy.
+// page-locked slots of our own, two to a thread on up to kXferThreads threads,
+// the transfer of one slot overlapping the host copy of the other.  The
+// transfers are kernels that read or write the slots over the link: in 1 MB
+// pieces they run at 52 GB/s where hipMemcpyAsync, at about 18 us a piece,
+// reaches 38 (4 MB pieces: 54 and 51), and the last block of a piece reports
+// it to the waiting thread.  Downloads into fresh memory, us, one hipMemcpy /
+// slots: 6.6 MB 420 / 258, 31 MB 1903 / 820, 84 MB 6536 / 1980, 246 MB 23193 /
+// 5940; uploads: 41 MB 1370 / 1070, 84 MB 2922 / 1940, 246 MB 8331 / 5160.
 #pragma once
 #include <atomic>
+#include <chrono>
 #include <cstring>
 #include <mutex>
 #include <thread>
@@ -20,22 +24,26 @@
 namespace fkx {
 
 // Smaller copies stay one hipMemcpy (starting threads costs about 20 us each).
-// To the host: 3.8 MB 232 against 266 us, 6.6 MB 420 against 310.  From the
-// host, where the pages are there already: 31 MB 1.00 against 1.06 ms, 84 MB
-// 2.92 against 2.08.
-constexpr size_t kXferMinDown = (size_t)5 << 20, kXferMinUp = (size_t)48 << 20;
+// To the host 3.8 MB take 225 us either way; from the host, where the pages
+// are there already, 10 MB 314 and 19 MB 540.
+constexpr size_t kXferMinDown = (size_t)5 << 20, kXferMinUp = (size_t)16 << 20;
 
-// The slots, 64 MB for the process (page-locking them costs about 2 ms, which
-// each new context would otherwise pay in its first copy): allocated by the
-// first large copy, freed with the last context, and lent to one copy at a
-// time.  A copy that finds them lent is one hipMemcpy.
+// The slots, 64 MB for the process with a report word each (page-locking
+// costs about 2 ms, which each new context would otherwise pay in its first
+// copy): allocated by the first large copy, freed with the last context, and
+// lent to one copy at a time.  A copy that finds them lent is one hipMemcpy.
 constexpr size_t kXferSlot = (size_t)4 << 20;
+constexpr int kXferSlots = 2 * kXferThreads;
 struct XferPool {
   std::mutex mu;
   char *pin = nullptr;
   int contexts = 0;
   bool lent = false;
+  std::atomic<unsigned long long> seq{0};
 
+  volatile unsigned long long *report(int slot) {
+    return reinterpret_cast<volatile unsigned long long *>(pin + kXferSlots * kXferSlot) + 8 * slot;
+  }
   void attach() {
     std::lock_guard<std::mutex> lk(mu);
     ++contexts;
@@ -49,12 +57,16 @@ struct XferPool {
   char *borrow() {
     std::lock_guard<std::mutex> lk(mu);
     if (lent) return nullptr;
-    if (!pin && hipHostMalloc(reinterpret_cast<void **>(&pin), 2 * kXferThreads * kXferSlot, hipHostMallocPortable) !=
-                    hipSuccess) {
-      (void)hipGetLastError();
-      pin = nullptr;
+    if (!pin) {
+      void *p = nullptr;
+      if (hipHostMalloc(&p, kXferSlots * (kXferSlot + 64), hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+      }
+      pin = static_cast<char *>(p);
+      std::memset(pin + kXferSlots * kXferSlot, 0, kXferSlots * 64);
     }
-    lent = pin != nullptr;
+    lent = true;
     return pin;
   }
   void give_back() {
@@ -64,79 +76,117 @@ struct XferPool {
 };
 inline XferPool g_xfer;
 
+// n16 16-byte words and `tail` bytes after them from a to b, one of them a
+// slot.  The block that ends last writes seq to *report, host memory, behind a
+// system-wide fence of every block, and leaves *count at zero.
+typedef unsigned int xfer_u4 __attribute__((ext_vector_type(4)));
+constexpr unsigned kXferBlocks = 64;
+static __global__ void __launch_bounds__(256) xfer_copy(const char *__restrict__ a, char *__restrict__ b, size_t n16,
+                                                        int tail, unsigned *__restrict__ count,
+                                                        volatile unsigned long long *__restrict__ report,
+                                                        unsigned long long seq) {
+  const xfer_u4 *src = reinterpret_cast<const xfer_u4 *>(a);
+  xfer_u4 *dst = reinterpret_cast<xfer_u4 *>(b);
+  for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n16; i += (size_t)kXferBlocks * 256) dst[i] = src[i];
+  if (blockIdx.x == 0 && (int)threadIdx.x < tail) b[16 * n16 + threadIdx.x] = a[16 * n16 + threadIdx.x];
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  if (atomicAdd(count, 1u) == kXferBlocks - 1) {
+    *count = 0;
+    __threadfence_system();
+    *report = seq;
+  }
+}
+
 // The slots for a copy of context c, or null: then the copy is one hipMemcpy.
 inline char *xfer_begin(fk_ctx *c) {
-  for (hipEvent_t &e : c->xfer.ev)
-    if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+  if (!c->xfer.count) {
+    unsigned *p = nullptr;
+    if (hipMalloc(&p, kXferSlots * sizeof(unsigned)) != hipSuccess ||
+        hipMemset(p, 0, kXferSlots * sizeof(unsigned)) != hipSuccess) {
       (void)hipGetLastError();
-      e = nullptr;
+      if (p) (void)hipFree(p);
       return nullptr;
     }
+    c->xfer.count = p;
+  }
   return g_xfer.borrow();
 }
 
 inline void xfer_free(fk_ctx *c) {
-  for (hipEvent_t &e : c->xfer.ev)
-    if (e) (void)hipEventDestroy(e);
+  if (c->xfer.count) (void)hipFree(c->xfer.count);
   c->xfer = Xfer{};
 }
 
-// The chunks of one copy, taken by the threads in order.
+// The pieces of one copy, taken by the threads in order.
 struct XferJob {
   fk_ctx *c;
   char *pin, *dev, *host;
-  size_t bytes, slot;
+  size_t bytes, piece;
   bool down;
   std::atomic<size_t> next{0};
   std::atomic<int> err{0};
 
-  size_t take() { return next.fetch_add(slot); }
-  size_t len(size_t at) const { return bytes - at < slot ? bytes - at : slot; }
+  size_t take() { return next.fetch_add(piece); }
+  size_t len(size_t at) const { return bytes - at < piece ? bytes - at : piece; }
   bool bad(hipError_t e) {
     if (e != hipSuccess) err.store((int)e);
     return err.load() != 0;
   }
+  char *slot(int s) { return pin + (size_t)s * kXferSlot; }
+  // starts the transfer of the piece at `at` through slot s; its report in *seq
+  bool start(size_t at, int s, unsigned long long *seq) {
+    const size_t n = len(at);
+    *seq = ++g_xfer.seq;
+    const char *a = down ? dev + at : slot(s);
+    char *b = down ? slot(s) : dev + at;
+    hipLaunchKernelGGL(xfer_copy, dim3(kXferBlocks), dim3(256), 0, c->stream, a, b, n / 16, (int)(n % 16),
+                       c->xfer.count + s, g_xfer.report(s), *seq);
+    return !bad(hipGetLastError());
+  }
+  // waits for a report; after 2 s (or an error elsewhere) for the stream
+  bool wait(int s, unsigned long long seq) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int k = 0; *g_xfer.report(s) != seq; ++k)
+      if ((k & 1023) == 1023 && (err.load() || std::chrono::steady_clock::now() - t0 > std::chrono::seconds(2)))
+        return !bad(hipStreamSynchronize(c->stream));
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return true;
+  }
   void work(int t) {
     if (bad(hipSetDevice(c->device))) return;
-    char *buf[2];
-    hipEvent_t ev[2];
-    for (int s = 0; s < 2; ++s) {
-      buf[s] = pin + (size_t)(2 * t + s) * kXferSlot;
-      ev[s] = c->xfer.ev[2 * t + s];
-    }
+    const int s0 = 2 * t;
+    unsigned long long seq[2] = {0, 0};
     if (down) {
-      auto fetch = [&](size_t at, int s) {
-        return !bad(hipMemcpyAsync(buf[s], dev + at, len(at), hipMemcpyDeviceToHost, c->stream)) &&
-               !bad(hipEventRecord(ev[s], c->stream));
-      };
       size_t at = take();
-      if (at >= bytes || !fetch(at, 0)) return;
+      if (at >= bytes || !start(at, s0, &seq[0])) return;
       for (int s = 0;; s ^= 1) {
         const size_t nx = take();
-        if (nx < bytes && !fetch(nx, s ^ 1)) return;
-        if (bad(hipEventSynchronize(ev[s]))) return;
-        std::memcpy(host + at, buf[s], len(at));
+        if (nx < bytes && !start(nx, s0 + (s ^ 1), &seq[s ^ 1])) return;
+        if (!wait(s0 + s, seq[s])) return;
+        std::memcpy(host + at, slot(s0 + s), len(at));
         if (nx >= bytes) return;
         at = nx;
       }
     }
-    int used = 0;
     for (int s = 0;; s ^= 1) {
       const size_t at = take();
       if (at >= bytes) return;
-      if (used++ >= 2 && bad(hipEventSynchronize(ev[s]))) return;
-      std::memcpy(buf[s], host + at, len(at));
-      if (bad(hipMemcpyAsync(dev + at, buf[s], len(at), hipMemcpyHostToDevice, c->stream))) return;
-      if (bad(hipEventRecord(ev[s], c->stream))) return;
+      if (seq[s] && !wait(s0 + s, seq[s])) return;
+      std::memcpy(slot(s0 + s), host + at, len(at));
+      if (!start(at, s0 + s, &seq[s])) return;
     }
   }
 };
 
 inline int xfer_staged(fk_ctx *c, char *pin, void *dev, void *host, size_t bytes, bool down) {
   XferJob job{c, pin, static_cast<char *>(dev), static_cast<char *>(host), bytes, 0, down};
-  job.slot = bytes >= 16 * kXferSlot ? kXferSlot : (bytes >= 4 * kXferSlot ? kXferSlot / 2 : kXferSlot / 4);
-  const size_t chunks = (bytes + job.slot - 1) / job.slot;
-  const int nt = (int)(chunks / 2 < (size_t)kXferThreads ? chunks / 2 : kXferThreads);
+  // mid sizes in smaller pieces, so that a few threads share them; a thread
+  // for every two
+  job.piece = bytes >= 16 * kXferSlot ? kXferSlot : (bytes >= 4 * kXferSlot ? kXferSlot / 2 : kXferSlot / 4);
+  const size_t pieces = (bytes + job.piece - 1) / job.piece;
+  const int nt = (int)(pieces / 2 < (size_t)kXferThreads ? pieces / 2 : kXferThreads);
   std::thread th[kXferThreads];
   for (int t = 1; t < nt; ++t) {
     try {

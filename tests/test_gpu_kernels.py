@@ -67,8 +67,8 @@ def test_relaxation_of_a_cell_does_not_depend_on_the_list_length(gpu, mode):
 @pytest.mark.parametrize("n", [9, 25, 34, 50])
 def test_states_pass_through_the_copies_unchanged(gpu, n):
     """Uploads and downloads below, between and above the sizes where they go
-    through page-locked slots (5 MB down, 48 MB up; slots of 1, 2 and 4 MB,
-    last slot partly filled): bytes are bytes."""
+    through page-locked slots (5 MB down, 16 MB up; pieces of 1, 2 and 4 MB,
+    the last one part full): bytes are bytes."""
     m = Mesh.box(n, n, n, rcm=False)
     U = np.random.default_rng(n).uniform(0.1, 1, (m.n_cells, 10))
     with GpuSolver(cases._two_phase_params(), m, U) as g:
