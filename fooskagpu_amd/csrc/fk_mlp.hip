@@ -479,7 +479,7 @@ __device__ __forceinline__ void pack_param(int i, float v, uint16_t *__restrict_
 // and 32 partials loaded ahead of the adds: the sum waits for memory, not for
 // its 35 blocks (58 us for 256 partials with one load at a time and 256
 // threads a block, and 9 us for the update and the copies as kernels of their
-// own; @R@ us).
+// own; 8 us).
 template <bool ADAM>
 __global__ void __launch_bounds__(64) mlp_update_k(int nb, const float *__restrict__ part, float *__restrict__ g,
                                                    float *__restrict__ w, float *__restrict__ m,
