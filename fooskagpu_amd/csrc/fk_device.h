@@ -51,6 +51,29 @@ __host__ __device__ inline Mat<T> make_mat(const fk_params &p) {
   return m;
 }
 
+// FP32 quotient a / b as mantissa times hardware reciprocal (about 1 ulp): the
+// form the build's flags give a division, unless the compiler moves it out of
+// a condition and so loses the licence for it.  Written out where two kernels
+// have to give the same bits.
+__device__ __forceinline__ float quot(float a, float b) {
+  const float q = __builtin_amdgcn_frexp_mantf(a) * __builtin_amdgcn_rcpf(__builtin_amdgcn_frexp_mantf(b));
+  return ldexpf(q, __builtin_amdgcn_frexp_expf(a) - __builtin_amdgcn_frexp_expf(b));
+}
+__device__ __forceinline__ double quot(double a, double b) { return a / b; }
+
+// Quotient and square root of the face terms.  FP32: one reciprocal (or root)
+// and a product, with the bits of the forms above where divisor, reciprocal
+// and result are normal numbers, as densities, wave speeds and moduli are
+// (the reciprocal's mantissa does not depend on the exponent); a limiter's
+// differences can lie below that and take quot.  Two instructions for eight
+// and one for six: pass F at size is bound by its instructions (mixed, 3.07M
+// cells: VALU busy 75 to 95 %; the dt stage, which also took the sound speeds
+// of both states twice, 390 -> 355 us, the RK stage 454 -> 442).
+__device__ __forceinline__ float face_quot(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
+__device__ __forceinline__ double face_quot(double a, double b) { return a / b; }
+__device__ __forceinline__ float face_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
+__device__ __forceinline__ double face_sqrt(double x) { return sqrt(x); }
+
 // ---------------- EOS (DP eqos.h:1-23, SP eqos.h:2-23) ----------------
 // two-phase stiffened gas with energy offset eta, phase k
 template <typename T>
@@ -59,11 +82,11 @@ __device__ __forceinline__ T p_of(const Mat<T> &m, int k, T rho, T e) {
 }
 template <typename T>
 __device__ __forceinline__ T e_of(const Mat<T> &m, int k, T p, T rho) {
-  return (p + m.g[k] * m.pi[k] + (m.g[k] - 1) * m.eta[k] * rho) / (rho * (m.g[k] - 1));
+  return face_quot(p + m.g[k] * m.pi[k] + (m.g[k] - 1) * m.eta[k] * rho, rho * (m.g[k] - 1));
 }
 template <typename T>
 __device__ __forceinline__ T c_of(const Mat<T> &m, int k, T rho, T p) {
-  return sqrt((m.g[k] * (p + m.pi[k])) / rho);
+  return face_sqrt(face_quot(m.g[k] * (p + m.pi[k]), rho));
 }
 template <typename T>
 __device__ __forceinline__ T T_of(const Mat<T> &m, int k, T rho, T e) {
@@ -81,23 +104,13 @@ __device__ __forceinline__ T p1_of(const Mat<T> &m, T rho, T e) {
 }
 template <typename T>
 __device__ __forceinline__ T e1_of(const Mat<T> &m, T p, T rho) {
-  return (p + m.g[0] * m.pi[0]) / (rho * (m.g[0] - 1));
+  return face_quot(p + m.g[0] * m.pi[0], rho * (m.g[0] - 1));
 }
 
 template <typename T>
 __device__ __forceinline__ T clamp_avf(const Mat<T> &m, T a) {
   return fmin(fmax(m.avfMin / 100, a), (T)1.0 - m.avfMin / 100);
 }
-
-// FP32 quotient a / b as mantissa times hardware reciprocal (about 1 ulp): the
-// form the build's flags give a division, unless the compiler moves it out of
-// a condition and so loses the licence for it.  Written out where two kernels
-// have to give the same bits.
-__device__ __forceinline__ float quot(float a, float b) {
-  const float q = __builtin_amdgcn_frexp_mantf(a) * __builtin_amdgcn_rcpf(__builtin_amdgcn_frexp_mantf(b));
-  return ldexpf(q, __builtin_amdgcn_frexp_expf(a) - __builtin_amdgcn_frexp_expf(b));
-}
-__device__ __forceinline__ double quot(double a, double b) { return a / b; }
 
 // Correctly rounded FP64 quotients x / d for several x: the reciprocal of d
 // to full precision once (hardware estimate, two Newton steps), then each
@@ -268,9 +281,23 @@ __device__ __forceinline__ void ghost(const Mat<T> &m, int bc, const T n[3], T *
   }
 }
 
+// Sound speeds and mass fractions of the phases of a two-phase face state.
+template <typename T>
+struct Sound {
+  T cL, cG, YL, YG;
+  __device__ __forceinline__ Sound() {}
+  __device__ __forceinline__ Sound(const Mat<T> &m, const T *W, T rho)
+      : cL(c_of(m, 0, W[1], W[6])), cG(c_of(m, 1, W[2], W[7])), YL(face_quot(W[0] * W[1], rho)),
+        YG(face_quot((1 - W[0]) * W[2], rho)) {}
+  __device__ __forceinline__ T wood(const T *W, T rho) const {
+    return face_quot((T)1, face_sqrt(rho * (face_quot(W[0], W[1] * cL * cL) + face_quot(1 - W[0], W[2] * cG * cG))));
+  }
+};
+
 // Per-face result of the Riemann solve, shared by the two sides.
 template <typename T, int NEQ>
 struct FaceRes {
+  Sound<T> sl, sr;  // two-phase: of the two face states
   T f[NEQ];    // F + H per equation (two-phase: eq 0, 6, 7 are F only)
   T unc[3];    // velocity of the non-conservative terms
   T pF;        // upwind face pressure
@@ -299,7 +326,7 @@ __device__ __forceinline__ void riemann(const Mat<T> &m, const T *L, const T *R,
     T cR = c_of(m, 0, R[0], pa_R);
     T S0 = fmin(uL - cL, uR - cR);
     T S2 = fmax(uL + cL, uR + cR);
-    T S1 = (R[4] - L[4] + L[0] * uL * (S0 - uL) - R[0] * uR * (S2 - uR)) / (L[0] * (S0 - uL) - R[0] * (S2 - uR));
+    T S1 = face_quot(R[4] - L[4] + L[0] * uL * (S0 - uL) - R[0] * uR * (S2 - uR), L[0] * (S0 - uL) - R[0] * (S2 - uR));
     S1 = (T)(1 - is_wall) * S1;
     const bool left = S1 >= 0;
     const bool star = S0 < 0 && S2 >= 0;
@@ -312,9 +339,9 @@ __device__ __forceinline__ void riemann(const Mat<T> &m, const T *L, const T *R,
     T H[5] = {0, 0, 0, 0, 0};
     if (star) {
       T c0 = s[0], c1 = s[0] * s[1], c2 = s[0] * s[2], c3 = s[0] * s[3], c4 = s[0] * (e + ke);
-      T v0 = s[0] * (SK - un) / (SK - S1);
+      T v0 = face_quot(s[0] * (SK - un), SK - S1);
       T vg0 = s[1] + (S1 - un) * n[0], vg1 = s[2] + (S1 - un) * n[1], vg2 = s[3] + (S1 - un) * n[2];
-      T v4 = v0 * (e + ke + (S1 - un) * (S1 + ps / (s[0] * (SK - un))));
+      T v4 = v0 * (e + ke + (S1 - un) * (S1 + face_quot(ps, s[0] * (SK - un))));
       H[0] = SK * (v0 - c0);
       H[1] = SK * (v0 * vg0 - c1);
       H[2] = SK * (v0 * vg1 - c2);
@@ -338,33 +365,23 @@ __device__ __forceinline__ void riemann(const Mat<T> &m, const T *L, const T *R,
     T uL = L[3] * n[0] + L[4] * n[1] + L[5] * n[2];
     T uR = R[3] * n[0] + R[4] * n[1] + R[5] * n[2];
     T cL, cR;
+    const T rL = L[0] * L[1] + (1 - L[0]) * L[2];
+    const T rR = R[0] * R[1] + (1 - R[0]) * R[2];
+    Sound<T> sl(m, L, rL), sr(m, R, rR);
     if ((L[8] + R[8]) / 2 > m.chemLimit && m.woods == 1) {
-      T rm = L[0] * L[1] + (1 - L[0]) * L[2];
-      T ca = c_of(m, 0, L[1], L[6]), cb = c_of(m, 1, L[2], L[7]);
-      cL = 1 / sqrt(rm * (L[0] / (L[1] * ca * ca) + (1 - L[0]) / (L[2] * cb * cb)));
-      rm = R[0] * R[1] + (1 - R[0]) * R[2];
-      ca = c_of(m, 0, R[1], R[6]);
-      cb = c_of(m, 1, R[2], R[7]);
-      cR = 1 / sqrt(rm * (R[0] / (R[1] * ca * ca) + (1 - R[0]) / (R[2] * cb * cb)));
+      cL = sl.wood(L, rL);
+      cR = sr.wood(R, rR);
     } else {
-      T d = L[0] * L[1] + (1 - L[0]) * L[2];
-      T YL = L[0] * L[1] / d, YG = (1 - L[0]) * L[2] / d;
-      T ca = c_of(m, 0, L[1], L[6]), cb = c_of(m, 1, L[2], L[7]);
-      cL = sqrt(YL * (ca * ca) + YG * (cb * cb));
-      d = R[0] * R[1] + (1 - R[0]) * R[2];
-      YL = R[0] * R[1] / d;
-      YG = (1 - R[0]) * R[2] / d;
-      ca = c_of(m, 0, R[1], R[6]);
-      cb = c_of(m, 1, R[2], R[7]);
-      cR = sqrt(YL * (ca * ca) + YG * (cb * cb));
+      cL = face_sqrt(sl.YL * (sl.cL * sl.cL) + sl.YG * (sl.cG * sl.cG));
+      cR = face_sqrt(sr.YL * (sr.cL * sr.cL) + sr.YG * (sr.cG * sr.cG));
     }
+    out.sl = sl;
+    out.sr = sr;
     T S0 = fmin(uL - cL, uR - cR);
     T S2 = fmax(uL + cL, uR + cR);
     T pL = L[0] * L[6] + (1 - L[0]) * L[7];
     T pR = R[0] * R[6] + (1 - R[0]) * R[7];
-    T rL = L[0] * L[1] + (1 - L[0]) * L[2];
-    T rR = R[0] * R[1] + (1 - R[0]) * R[2];
-    T S1 = (pR - pL + rL * uL * (S0 - uL) - rR * uR * (S2 - uR)) / (rL * (S0 - uL) - rR * (S2 - uR));
+    T S1 = face_quot(pR - pL + rL * uL * (S0 - uL) - rR * uR * (S2 - uR), rL * (S0 - uL) - rR * (S2 - uR));
     const bool left = S1 >= 0;
     const bool star = S0 < 0 && S2 >= 0;
     const T *s = left ? L : R;
@@ -385,20 +402,20 @@ __device__ __forceinline__ void riemann(const Mat<T> &m, const T *L, const T *R,
       unc0 = s[3] + (S1 - un) * n[0];
       unc1 = s[4] + (S1 - un) * n[1];
       unc2 = s[5] + (S1 - un) * n[2];
-      T rSL = s[1] * (SK - un) / (SK - S1);
-      T rSG = s[2] * (SK - un) / (SK - S1);
+      T rSL = face_quot(s[1] * (SK - un), SK - S1);
+      T rSG = face_quot(s[2] * (SK - un), SK - S1);
       T V1 = a * rSL, V2 = a1 * rSG;
       T rS = V1 + V2;
-      T pSL = (s[6] + m.pi[0]) * ((m.g[0] - 1) * s[1] - (m.g[0] + 1) * rSL) / ((m.g[0] - 1) * rSL - (m.g[0] + 1) * s[1]) - m.pi[0];
-      T pSG = (s[7] + m.pi[1]) * ((m.g[1] - 1) * s[2] - (m.g[1] + 1) * rSG) / ((m.g[1] - 1) * rSG - (m.g[1] + 1) * s[2]) - m.pi[1];
+      T pSL = face_quot((s[6] + m.pi[0]) * ((m.g[0] - 1) * s[1] - (m.g[0] + 1) * rSL), (m.g[0] - 1) * rSL - (m.g[0] + 1) * s[1]) - m.pi[0];
+      T pSG = face_quot((s[7] + m.pi[1]) * ((m.g[1] - 1) * s[2] - (m.g[1] + 1) * rSG), (m.g[1] - 1) * rSG - (m.g[1] + 1) * s[2]) - m.pi[1];
       areL = V1 * e_of(m, 0, pSL, rSL);
       areG = V2 * e_of(m, 1, pSG, rSG);
       T press = s[0] * s[6] + (1 - s[0]) * s[7];
       T rhoK = s[0] * s[1] + (1 - s[0]) * s[2];
       T V8;
-      if (m.hllcToro == 1) V8 = ((SK - un) / (SK - S1)) * (C8 + (S1 - un) * (rhoK * S1 + press / (SK - un)));
-      else V8 = ((SK - un) / (SK - S1)) * (C8 + (S1 - un) * (S1 + press / (rhoK * (SK - un))));
-      T V9 = s[8] * (SK - un) / (SK - S1);
+      if (m.hllcToro == 1) V8 = face_quot(SK - un, SK - S1) * (C8 + (S1 - un) * (rhoK * S1 + face_quot(press, SK - un)));
+      else V8 = face_quot(SK - un, SK - S1) * (C8 + (S1 - un) * (S1 + face_quot(press, rhoK * (SK - un))));
+      T V9 = face_quot(s[8] * (SK - un), SK - S1);
       H1 = SK * (V1 - C1);
       H2 = SK * (V2 - C2);
       H3 = SK * (rS * unc0 - rho * s[3]);
@@ -441,22 +458,16 @@ __device__ __forceinline__ void riemann(const Mat<T> &m, const T *L, const T *R,
 // Maximum signal speed |u.n| + c_mix of a face state
 // (DP computeTimeStep.cu:15-46; single-phase: |u.n| + c).
 template <int NEQ, typename T>
-__device__ __forceinline__ T signal(const Mat<T> &m, const T *W, const T n[3]) {
+__device__ __forceinline__ T signal(const Mat<T> &m, const T *W, const T n[3], const Sound<T> &so) {
   if constexpr (NEQ == 5) {
     T un = W[1] * n[0] + W[2] * n[1] + W[3] * n[2];
     T pa = W[4];
     if constexpr (sizeof(T) == 4) pa = W[4] + m.pr;  // FP32 path: deviation from pRef
     return fabs(un) + c_of(m, 0, W[0], pa);
   } else {
-    T avf = W[0], rL = W[1], rG = W[2];
-    T rm = avf * rL + (1 - avf) * rG;
-    T cL = c_of(m, 0, rL, W[6]), cG = c_of(m, 1, rG, W[7]);
     T cmix;
-    if (W[8] > m.chemLimit && m.woods == 1) cmix = 1 / sqrt(rm * (avf / (rL * cL * cL) + (1 - avf) / (rG * cG * cG)));
-    else {
-      T YL = avf * rL / rm, YG = (1 - avf) * rG / rm;
-      cmix = sqrt(YL * cL * cL + YG * cG * cG);
-    }
+    if (W[8] > m.chemLimit && m.woods == 1) cmix = so.wood(W, W[0] * W[1] + (1 - W[0]) * W[2]);
+    else cmix = face_sqrt(so.YL * so.cL * so.cL + so.YG * so.cG * so.cG);
     T un = W[3] * n[0] + W[4] * n[1] + W[5] * n[2];
     return fabs(un) + cmix;
   }
@@ -490,10 +501,10 @@ __device__ __forceinline__ T wale(const T g[3][3], T Ls) {
       sum1 += sd * sd;
       sum2 += st * st;
     }
-  T num = sum1 * sqrt(sum1);
-  T den = sum1 * sqrt(sqrt(sum1)) + sum2 * sum2 * sqrt(sum2) + (T)1e-12;
+  T num = sum1 * face_sqrt(sum1);
+  T den = sum1 * face_sqrt(face_sqrt(sum1)) + sum2 * sum2 * face_sqrt(sum2) + (T)1e-12;
   if (den < (T)1e-10) num = 0;
-  return Ls * Ls * num / den;
+  return face_quot(Ls * Ls * num, den);
 }
 
 }  // namespace fk

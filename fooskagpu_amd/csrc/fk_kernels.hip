@@ -512,8 +512,8 @@ __device__ __forceinline__ void face_terms(const fk_params &P, const fk::Mat<T> 
     rhs[9] += (double)(sign * (fr.f[9]) * A);
   }
   if constexpr (SIG) {
-    const T cl = fk::signal<NEQ, T>(mt, L, n);
-    const T cr = nb >= 0 ? fk::signal<NEQ, T>(mt, R, n) : (T)0.0;
+    const T cl = fk::signal<NEQ, T>(mt, L, n, fr.sl);
+    const T cr = nb >= 0 ? fk::signal<NEQ, T>(mt, R, n, fr.sr) : (T)0.0;
     const T cm = fmax(cl, cr);
     if (!(sig >= cm)) sig = cm;
   }
