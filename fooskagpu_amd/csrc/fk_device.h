@@ -294,10 +294,20 @@ struct Sound {
   }
 };
 
+// Signal speed |u.n| + c_mix of a face state, un = u.n, so: its sound speeds
+// (DP computeTimeStep.cu:15-46; single-phase: |u.n| + c).
+template <typename T>
+__device__ __forceinline__ T signal(const Mat<T> &m, const T *W, T un, const Sound<T> &so, T rho) {
+  T cmix;
+  if (W[8] > m.chemLimit && m.woods == 1) cmix = so.wood(W, rho);
+  else cmix = face_sqrt(so.YL * so.cL * so.cL + so.YG * so.cG * so.cG);
+  return fabs(un) + cmix;
+}
+
 // Per-face result of the Riemann solve, shared by the two sides.
 template <typename T, int NEQ>
 struct FaceRes {
-  Sound<T> sl, sr;  // two-phase: of the two face states
+  T sigL, sigR;  // SIG: signal speeds of the two face states
   T f[NEQ];    // F + H per equation (two-phase: eq 0, 6, 7 are F only)
   T unc[3];    // velocity of the non-conservative terms
   T pF;        // upwind face pressure
@@ -306,7 +316,7 @@ struct FaceRes {
 // HLLC face flux.  Two-phase: DP computeRHS.cu:78-146 with waveSpeeds.h,
 // starRegion.h, flux.h; single-phase: SP computeRHS.cu:23-98.
 // L, R: face states (R already the ghost on boundary faces).
-template <int NEQ, typename T>
+template <int NEQ, bool SIG, typename T>
 __device__ __forceinline__ void riemann(const Mat<T> &m, const T *L, const T *R, const T n[3], int is_wall,
                                         FaceRes<T, NEQ> &out) {
   if constexpr (NEQ == 5) {
@@ -324,6 +334,10 @@ __device__ __forceinline__ void riemann(const Mat<T> &m, const T *L, const T *R,
     T uR = R[1] * n[0] + R[2] * n[1] + R[3] * n[2];
     T cL = c_of(m, 0, L[0], pa_L);
     T cR = c_of(m, 0, R[0], pa_R);
+    if constexpr (SIG) {
+      out.sigL = fabs(uL) + cL;
+      out.sigR = fabs(uR) + cR;
+    }
     T S0 = fmin(uL - cL, uR - cR);
     T S2 = fmax(uL + cL, uR + cR);
     T S1 = face_quot(R[4] - L[4] + L[0] * uL * (S0 - uL) - R[0] * uR * (S2 - uR), L[0] * (S0 - uL) - R[0] * (S2 - uR));
@@ -375,8 +389,11 @@ __device__ __forceinline__ void riemann(const Mat<T> &m, const T *L, const T *R,
       cL = face_sqrt(sl.YL * (sl.cL * sl.cL) + sl.YG * (sl.cG * sl.cG));
       cR = face_sqrt(sr.YL * (sr.cL * sr.cL) + sr.YG * (sr.cG * sr.cG));
     }
-    out.sl = sl;
-    out.sr = sr;
+    if constexpr (SIG) {  // formed here, before the star region: the sound speeds end here
+      out.sigL = signal(m, L, uL, sl, rL);
+      out.sigR = signal(m, R, uR, sr, rR);
+      asm volatile("" : "+v"(out.sigL), "+v"(out.sigR));
+    }
     T S0 = fmin(uL - cL, uR - cR);
     T S2 = fmax(uL + cL, uR + cR);
     T pL = L[0] * L[6] + (1 - L[0]) * L[7];
@@ -452,24 +469,6 @@ __device__ __forceinline__ void riemann(const Mat<T> &m, const T *L, const T *R,
     out.unc[1] = unc1;
     out.unc[2] = unc2;
     out.pF = press;
-  }
-}
-
-// Maximum signal speed |u.n| + c_mix of a face state
-// (DP computeTimeStep.cu:15-46; single-phase: |u.n| + c).
-template <int NEQ, typename T>
-__device__ __forceinline__ T signal(const Mat<T> &m, const T *W, const T n[3], const Sound<T> &so) {
-  if constexpr (NEQ == 5) {
-    T un = W[1] * n[0] + W[2] * n[1] + W[3] * n[2];
-    T pa = W[4];
-    if constexpr (sizeof(T) == 4) pa = W[4] + m.pr;  // FP32 path: deviation from pRef
-    return fabs(un) + c_of(m, 0, W[0], pa);
-  } else {
-    T cmix;
-    if (W[8] > m.chemLimit && m.woods == 1) cmix = so.wood(W, W[0] * W[1] + (1 - W[0]) * W[2]);
-    else cmix = face_sqrt(so.YL * so.cL * so.cL + so.YG * so.cG * so.cG);
-    T un = W[3] * n[0] + W[4] * n[1] + W[5] * n[2];
-    return fabs(un) + cmix;
   }
 }
 

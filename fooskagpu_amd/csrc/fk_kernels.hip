@@ -148,13 +148,11 @@ __device__ __forceinline__ void store_grad(const fk_params &P, const T (&W)[NEQ]
 }
 
 // RK stage irk of one cell from its residual (update.cu:19-103), in the
-// operation order of rk_update.
+// operation order of rk_update; u0 is not read with rkSteps 1.
 template <int NEQ>
 __device__ __forceinline__ void rk_stage(const fk_params &P, int irk, double dt, double Vc, const double *uc,
-                                         const double *__restrict__ U0, const double *r, double (&un)[NEQ]) {
+                                         const double *u0, const double *r, double (&un)[NEQ]) {
   constexpr int iz = NEQ == 5 ? 3 : 5;
-  double u0[NEQ];
-  if (P.rkSteps != 1) fk::load_rec<NEQ>(U0, u0);
 #pragma unroll
   for (int v = 0; v < NEQ; ++v) {
     const int neglect = (v == iz && P.neglectZ == 1);
@@ -479,15 +477,17 @@ __device__ __forceinline__ CellSide<T> cell_side(const fk::Mat<double> &md, cons
 // non-conservative terms to rhs, the viscous ones to rv, and (SIG) raises sig
 // to the face's signal speed.  L, R: face states (owner, neighbour or ghost);
 // Gc, Gn: velocity gradients of this cell and the neighbour; wls: WALE width
-// of the slot; Wc1: first-order state of this cell.
+// of the slot; Uc: this cell's conserved state in memory, read for the
+// first-order viscous ghost of a boundary face (formed there only: kept across
+// the faces it takes 20 registers of the FP64 kernels).
 template <int NEQ, typename T, bool VISC, bool HEAT, bool SIG>
 __device__ __forceinline__ void face_terms(const fk_params &P, const fk::Mat<T> &mt, const CellSide<T> &cs, int nb,
                                            bool own, const T (&n)[3], T A, const T (&L)[NEQ], const T (&R)[NEQ],
-                                           const T *Gc, const T *Gn, const T *wls, const T (&Wc1)[NEQ],
-                                           double (&rhs)[NEQ], double (&rv)[5], T &sig) {
+                                           const T *Gc, const T *Gn, const T *wls, const fk::Mat<double> &md,
+                                           const double *Uc, double (&rhs)[NEQ], double (&rv)[5], T &sig) {
   constexpr int iu = Model<NEQ>::iu;
   fk::FaceRes<T, NEQ> fr;
-  fk::riemann<NEQ, T>(mt, L, R, n, nb == -5, fr);
+  fk::riemann<NEQ, SIG, T>(mt, L, R, n, nb == -5, fr);
   if constexpr (NEQ == 5) {
 #pragma unroll
     for (int v = 0; v < 5; ++v) rhs[v] += (double)(own ? -fr.f[v] * A : fr.f[v] * A);
@@ -512,9 +512,7 @@ __device__ __forceinline__ void face_terms(const fk_params &P, const fk::Mat<T> 
     rhs[9] += (double)(sign * (fr.f[9]) * A);
   }
   if constexpr (SIG) {
-    const T cl = fk::signal<NEQ, T>(mt, L, n, fr.sl);
-    const T cr = nb >= 0 ? fk::signal<NEQ, T>(mt, R, n, fr.sr) : (T)0.0;
-    const T cm = fmax(cl, cr);
+    const T cm = fmax(fr.sigL, nb >= 0 ? fr.sigR : (T)0.0);
     if (!(sig >= cm)) sig = cm;
   }
   if constexpr (VISC) {
@@ -543,8 +541,12 @@ __device__ __forceinline__ void face_terms(const fk_params &P, const fk::Mat<T> 
 #pragma unroll
       for (int v = 0; v < NEQ; ++v) R1[v] = R[v];
     } else {
+      double u[NEQ], w[NEQ];
+      fk::load_rec<NEQ>(Uc, u);
+      fk::cons2prim<NEQ>(md, u, w);
+      if constexpr (NEQ == 5 && sizeof(T) == 4) w[4] -= md.pr;  // FP32 path: pressure as deviation from pRef
 #pragma unroll
-      for (int v = 0; v < NEQ; ++v) R1[v] = Wc1[v];
+      for (int v = 0; v < NEQ; ++v) R1[v] = (T)w[v];
       fk::ghost<NEQ, T>(mt, -nb, n, R1);
     }
     T mu;
@@ -745,14 +747,6 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
   // viscous contributions are summed apart (rv) and added to the inviscid sums
   // after the face loop: the canonical order shared with the oracle
   double rv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  T Wc1[NEQ];  // first-order state of this cell (viscous boundary ghost)
-  if constexpr (VISC) {
-    double t[NEQ];
-    fk::cons2prim<NEQ>(md, Uc, t);
-    if constexpr (NEQ == 5 && sizeof(T) == 4) t[4] -= md.pr;  // FP32 path: pressure as deviation from pRef
-#pragma unroll
-    for (int v = 0; v < NEQ; ++v) Wc1[v] = (T)t[v];
-  }
   // slot links loaded up front and rotated, as in pass G (mixed 6.85 against
   // 7.12 ms for the fused pass, FP64 14.4 against 14.8 ms)
   int mq[NS];
@@ -792,7 +786,7 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
       fk::ghost<NEQ, T>(mt, -nb, n, R);
     }
     face_terms<NEQ, T, VISC, HEAT, MODE == 1>(P, mt, cs, nb, own, n, A, L, R, VISC ? grad_ptr(c) : nullptr,
-                                              VISC && nb >= 0 ? grad_ptr(nb) : nullptr, VISC ? wls + s : nullptr, Wc1, rhs, rv, sig);
+                                              VISC && nb >= 0 ? grad_ptr(nb) : nullptr, VISC ? wls + s : nullptr, md, U + c * NEQ, rhs, rv, sig);
   }
   if constexpr (VISC) {
 #pragma unroll
@@ -1086,8 +1080,14 @@ __global__ void __launch_bounds__(64, 2) pass_g_q(fk_params P, int64_t nc, const
   }
 }
 
+// FP64 with 4 slots is held to 168 VGPRs, three waves per SIMD: at two the
+// kernel waited for its gathers with the vector units 70 % busy.  They fit
+// since the boundary ghost is formed at its face and U is read again for the
+// stage (with both held across the faces three waves spilled, 338 us).  1.05M
+// cells: RK stage 288 -> 257 us, dt stage 269 -> 246.  FP64 with 6 slots takes
+// 208 to 214.
 template <int NEQ, typename T, bool VISC, bool HEAT, int MODE, int NS, bool WOUT = false, int RLX = 0>
-__global__ void __launch_bounds__(64, 2) pass_f_q(fk_params P, int64_t nc, const double *__restrict__ U,
+__global__ void __launch_bounds__(64, (NS == 4 || sizeof(T) == 4 ? 3 : 2)) pass_f_q(fk_params P, int64_t nc, const double *__restrict__ U,
                                                const double *__restrict__ U0, double *__restrict__ Unew,
                                                const int32_t *__restrict__ link, const void *__restrict__ geo,
                                                const T *__restrict__ wls, const double *__restrict__ vol,
@@ -1119,18 +1119,19 @@ __global__ void __launch_bounds__(64, 2) pass_f_q(fk_params P, int64_t nc, const
   double Uc[NEQ];
   fk::load_rec<NEQ>(U + c * NEQ, Uc);
   const CellSide<T> cs = cell_side<NEQ, T>(md, Uc);
-  T Wc1[NEQ];  // first-order state of this cell (viscous boundary ghost)
-  if constexpr (VISC) {
-    double t[NEQ];
-    fk::cons2prim<NEQ>(md, Uc, t);
-    if constexpr (NEQ == 5 && sizeof(T) == 4) t[4] -= md.pr;
-#pragma unroll
-    for (int v = 0; v < NEQ; ++v) Wc1[v] = (T)t[v];
-  }
   double rhs[NEQ], rv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int v = 0; v < NEQ; ++v) rhs[v] = 0.0;
   T sig = (T)-1e9;
+  // states of the RK stage; U again, not kept across the faces (20 registers)
+  double u0[NEQ], Vc;
+  auto stage_states = [&] {
+    const double *U2 = U;
+    asm volatile("" : "+s"(U2));
+    fk::load_rec<NEQ>(U2 + c * NEQ, Uc);
+    if (P.rkSteps != 1) fk::load_rec<NEQ>(U0 + c * NEQ, u0);
+    Vc = vol[c];
+  };
 #pragma unroll 1
   for (int r = 0; r < R; ++r) {
     const bool in = NS == 4 || 4 * r + q < NS;
@@ -1159,8 +1160,9 @@ __global__ void __launch_bounds__(64, 2) pass_f_q(fk_params P, int64_t nc, const
       if (nb < 0) fk::ghost<NEQ, T>(mt, -nb, n, Rt);
       face_terms<NEQ, T, VISC, HEAT, MODE == 1>(P, mt, cs, nb, own, n, ga.w, L, Rt, VISC ? gvel + c * NG : nullptr,
                                                 VISC && nb >= 0 ? gvel + (int64_t)nb * NG : nullptr,
-                                                VISC ? wls + s : nullptr, Wc1, fr, fv, sig);
+                                                VISC ? wls + s : nullptr, md, U + c * NEQ, fr, fv, sig);
     }
+    if constexpr (MODE == 0 && R == 1) stage_states();  // on their way while the quad adds
 #pragma unroll
     for (int j = 0; j < 4; ++j) {  // lanes without a slot add 0
 #pragma unroll
@@ -1200,7 +1202,8 @@ __global__ void __launch_bounds__(64, 2) pass_f_q(fk_params P, int64_t nc, const
     const double dt = dt_ptr ? *dt_ptr : dt_val;
     if (clock && c == 0 && q == 0 && live) clock[1] += clock[0];
     double un[NEQ];
-    rk_stage<NEQ>(P, irk, dt, vol[c], Uc, U0 + c * NEQ, rhs, un);
+    if constexpr (R > 1) stage_states();
+    rk_stage<NEQ>(P, irk, dt, Vc, Uc, u0, rhs, un);
     int chem = 0, push = 0, it = 0, ts = 0;
     if constexpr (RLX == 1) push = fk::screen_cell(P, un, &chem, &it);
     if constexpr (RLX == 2) push = chem = fk::plain_cell4(P, un, &it, &ts);
@@ -1314,7 +1317,9 @@ __global__ void __launch_bounds__(kBlock) rk_update_w(fk_params P, int64_t nc, c
     for (int v = 0; v < NEQ; ++v) r[v] = (double)rhs[c * NEQ + v];
   }
   if (P.rkSteps == 1 || irk != 0) fk::load_rec<NEQ>(U + c * NEQ, uc);
-  rk_stage<NEQ>(P, irk, dt, Vc, uc, U0 + c * NEQ, r, un);
+  double u0[NEQ];
+  if (P.rkSteps != 1) fk::load_rec<NEQ>(U0 + c * NEQ, u0);
+  rk_stage<NEQ>(P, irk, dt, Vc, uc, u0, r, un);
 #pragma unroll
   for (int v = 0; v < NEQ; ++v) sU[threadIdx.x * SU + v] = un[v];
   fk::store_prims<NEQ>(fk::make_mat<double>(P), un, sWr + threadIdx.x * SWR);
