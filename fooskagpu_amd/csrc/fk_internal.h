@@ -89,8 +89,10 @@ struct fk_ctx {
   // state health found by pass G: (step << 32) | cell, the smallest of the
   // cells with a non-positive density or a non-finite primitive; ~0 if none
   unsigned long long *health = nullptr;
-  double *dtw = nullptr;     // minima of Vcfl / signal by wave (pass F on quads), dt_parts of them
-  int dt_parts = 0;
+  // two sets of minima of Vcfl / signal: the last dt stage's, and which are reset
+  unsigned long long *dtw = nullptr;
+  int dt_set = 0;
+  bool dt_clean[2] = {false, false};
   double *hres = nullptr;    // page-locked results that kernels write for the host, 64 doubles
   unsigned long long hseq = 0;  // number of the last result asked for
   double *dgrad = nullptr, *dtheta = nullptr;

@@ -451,6 +451,39 @@ __global__ void __launch_bounds__(kBlock, (sizeof(T) == 8 ? 2 : 1))
   }
 }
 
+// Smallest Vcfl / signal of a dt stage, kept in kDtSlots words on cache lines
+// of their own as keys whose unsigned order is the order of the doubles: each
+// wave of pass F lowers one of them (64 words: an atomic on one address
+// retires in about 12 ns), the update or dt_final folds the 64.  The order of
+// the waves does not matter to a minimum.  Two sets in turn: who folds one
+// resets the other.  Before, pass F's array was read by two more kernels, 13
+// us a step at 1M cells, or its quads' minima folded by one of 8.5 us.
+constexpr int kDtSlots = 64, kDtStride = 16;
+constexpr double kDtNone = 1e15;
+__device__ __forceinline__ unsigned long long dt_key(double d) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(d);
+  return u >> 63 ? ~u : u | 1ull << 63;
+}
+__device__ __forceinline__ double dt_unkey(unsigned long long k) {
+  return __longlong_as_double((long long)(k >> 63 ? k & ~(1ull << 63) : ~k));
+}
+__device__ __forceinline__ void dt_lower(unsigned long long *__restrict__ slots, double d) {
+  __hip_atomic_fetch_min(slots + (blockIdx.x % kDtSlots) * kDtStride, dt_key(fmin(kDtNone, d)), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+}
+// by the 64 lanes of a wave: the smallest of a set, and the other set reset
+__device__ __forceinline__ double dt_fold(const unsigned long long *__restrict__ slots,
+                                          unsigned long long *__restrict__ reset) {
+  const int l = threadIdx.x & 63;
+  double m = dt_unkey(slots[l * kDtStride]);
+  for (int off = 1; off < 64; off <<= 1) m = fmin(m, __shfl_xor(m, off, 64));
+  if (reset) reset[l * kDtStride] = dt_key(kDtNone);
+  return m;
+}
+__global__ void __launch_bounds__(64) dt_reset(unsigned long long *__restrict__ slots) {
+  slots[threadIdx.x * kDtStride] = dt_key(kDtNone);
+}
+
 // Side terms of a cell (fluxSource / computeCenterPress, two-phase).
 template <typename T>
 struct CellSide {
@@ -646,6 +679,7 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
                                                  double *__restrict__ rhs_out, double *__restrict__ dtc, int irk,
                                                  double dt_val, const double *__restrict__ dt_ptr,
                                                  float *__restrict__ Wout, double *__restrict__ clock,
+                                                 unsigned long long *__restrict__ dtmin,
                                                  uint32_t *__restrict__ rlist,
                                                  unsigned long long *__restrict__ rcnt,
                                                  unsigned long long *__restrict__ rpart) {
@@ -803,7 +837,17 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
       if constexpr (MODE == 1 && sizeof(T) == 4) reinterpret_cast<float *>(rhs_out)[c * NEQ + v] = (float)rhs[v];
       else rhs_out[c * NEQ + v] = rhs[v];
     }
-    if constexpr (MODE == 1) dtc[c] = volcfl[c] / (double)sig;
+    if constexpr (MODE == 1) {
+      double d = volcfl[c] / (double)sig;
+      dtc[c] = d;
+      const int l = threadIdx.x & 63;
+      const int64_t cw = c - l;  // lanes past the last cell are gone
+      for (int off = 1; off < 64; off <<= 1) {
+        const double o = __shfl_xor(d, off, 64);
+        if (cw + (l ^ off) < nc) d = fmin(d, o);
+      }
+      if (l == 0) dt_lower(dtmin, d);
+    }
   } else {
     const double dt = dt_ptr ? *dt_ptr : dt_val;
     if (clock && c == 0) clock[1] += clock[0];  // last stage of a step: the physical time
@@ -1095,18 +1139,18 @@ __global__ void __launch_bounds__(64, (NS == 4 || sizeof(T) == 4 ? 3 : 2)) pass_
                                                const T *__restrict__ gvel, double *__restrict__ rhs_out,
                                                double *__restrict__ dtc, int irk, double dt_val,
                                                const double *__restrict__ dt_ptr, float *__restrict__ Wout,
-                                               double *__restrict__ clock, double *__restrict__ dtmin,
+                                               double *__restrict__ clock,
+                                               unsigned long long *__restrict__ dtmin,
                                                uint32_t *__restrict__ rlist, unsigned long long *__restrict__ rcnt,
                                                unsigned long long *__restrict__ rpart) {
   static_assert(!RLX || (MODE == 0 && NEQ == 10), "fused relaxation: two-phase RK stage only");
   constexpr int R = (NS + 3) / 4, NG = ngrad<NEQ, HEAT>(), iu = Model<NEQ>::iu;
   const int64_t blk = xcd_block();
   const int q = threadIdx.x & 3;
-  if (blk * 16 >= nc) {  // a wave without cells still stores its counts and minimum
+  if (blk * 16 >= nc) {  // a wave without cells still stores its counts
     if (threadIdx.x == 0) {
       if constexpr (RLX != 0)
         for (int k = 0; k < RLX + 1; ++k) rpart[blk * (RLX + 1) + k] = 0;
-      if (MODE == 1 && dtmin) dtmin[blk] = 1e15;
     }
     return;
   }
@@ -1193,10 +1237,8 @@ __global__ void __launch_bounds__(64, (NS == 4 || sizeof(T) == 4 ? 3 : 2)) pass_
     if constexpr (MODE == 1) {
       double d = volcfl[c] / (double)sig;
       if (q == 0) dtc[c] = d;
-      if (dtmin) {  // minimum of the wave's cells for the RK update (dt_of)
-        for (int off = 4; off < 64; off <<= 1) d = fmin(d, __shfl_xor(d, off, 64));
-        if (threadIdx.x == 0) dtmin[blk] = fmin(1e15, d);
-      }
+      for (int off = 4; off < 64; off <<= 1) d = fmin(d, __shfl_xor(d, off, 64));
+      if (threadIdx.x == 0) dt_lower(dtmin, d);
     }
   } else {
     const double dt = dt_ptr ? *dt_ptr : dt_val;
@@ -1229,37 +1271,35 @@ __global__ void __launch_bounds__(64, (NS == 4 || sizeof(T) == 4 ? 3 : 2)) pass_
   }
 }
 
-// dt of the update kernels.  nmin > 0: from the minima that pass F's waves left,
-// which every block folds for itself; block 0 stores it.  Up to kDtFold of
-// them: two kernels and their gaps fewer than min_blocks + dt_final (with the
-// time's own kernel gone too a 12k-cell Sod step takes 34 instead of 39 us);
-// 5184 minima, folded by 3240 blocks, made the update 20 us long instead of 7,
-// so up to kDtParts dt_final folds them.  clock: the update ends a step, the
-// physical time advances.
-constexpr int kDtParts = 8192, kDtFold = 1024;
+// dt of the update kernels, slots: each block folds the set for itself; block
+// 0 stores dt and resets the other set.  Up to kDtFold blocks: 83k cells (3240
+// blocks) 155.2 us a step against 156.2 with dt_final ahead, mixed 3.07M cells
+// (12,000) 2275 against 2278; FP64 1.05M cells (41,160 short blocks) 1502
+// against 1498.
+// clock: the update ends a step, the physical time advances.
+constexpr int64_t kDtFold = 16384;
 struct DtSource {
-  double val;             // the dt, unless ptr or nmin says otherwise
+  double val;             // the dt, unless ptr or slots says otherwise
   const double *ptr;
-  const double *minima;
-  int nmin;
+  const unsigned long long *slots;
+  unsigned long long *reset;
   double cfl, maxDt;
   double *scal;           // [dt, time]
   int clock;
 };
 __device__ __forceinline__ double dt_of(const DtSource &s) {
   double dt = s.ptr ? *s.ptr : s.val;
-  if (s.nmin > 0) {
-    __shared__ double sh[kBlock / 64];
-    double m = 1e15;
-    for (int i = threadIdx.x; i < s.nmin; i += kBlock) m = fmin(m, s.minima[i]);
-    for (int off = 1; off < 64; off <<= 1) m = fmin(m, __shfl_xor(m, off, 64));
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
+  if (s.slots) {
+    __shared__ double sh;
+    if (threadIdx.x < 64) {
+      const double m = dt_fold(s.slots, blockIdx.x == 0 ? s.reset : nullptr);
+      if (threadIdx.x == 0) sh = fmin(s.cfl * m, s.maxDt);
+    }
     __syncthreads();
-    for (int k = 0; k < kBlock / 64; ++k) m = fmin(m, sh[k]);
-    dt = fmin(s.cfl * m, s.maxDt);
+    dt = sh;
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    if (s.nmin > 0) s.scal[0] = dt;
+    if (s.slots) s.scal[0] = dt;
     if (s.clock) s.scal[1] += dt;
   }
   return dt;
@@ -1271,20 +1311,22 @@ __global__ void __launch_bounds__(kBlock) rk_update(fk_params P, int64_t nc, con
                                                     const double *__restrict__ U0, double *__restrict__ Unew,
                                                     const RT *__restrict__ rhs_s, const double *__restrict__ vol,
                                                     int irk, DtSource ds) {
-  const double dt = dt_of(ds);
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= nc * NEQ) return;
+  const int64_t it = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const int64_t i = it < nc * NEQ ? it : 0;
   const double ri = (double)rhs_s[i];
   const int64_t c = i / NEQ;
   const int v = (int)(i - c * NEQ);
   const double Vc = vol[c];
+  const double ui = P.rkSteps == 1 || irk != 0 ? U[i] : 0.0, u0 = P.rkSteps != 1 ? U0[i] : 0.0;
+  const double dt = dt_of(ds);
+  if (it != i) return;
   constexpr int iz = NEQ == 5 ? 3 : 5;
   const int neglect = (v == iz && P.neglectZ == 1);
   double u;
-  if (P.rkSteps == 1) u = (1 - neglect) * (U[i] + dt * (1.0 / Vc) * ri);
-  else if (irk == 0) u = (1 - neglect) * (U0[i] + dt * (1.0 / Vc) * ri);
-  else if (irk == 1) u = (1 - neglect) * ((3.0 / 4.0) * U0[i] + (1.0 / 4.0) * U[i] + (1.0 / 4.0) * dt * (1.0 / Vc) * ri);
-  else u = (1 - neglect) * ((1.0 / 3.0) * U0[i] + (2.0 / 3.0) * U[i] + (2.0 / 3.0) * dt * (1.0 / Vc) * ri);
+  if (P.rkSteps == 1) u = (1 - neglect) * (ui + dt * (1.0 / Vc) * ri);
+  else if (irk == 0) u = (1 - neglect) * (u0 + dt * (1.0 / Vc) * ri);
+  else if (irk == 1) u = (1 - neglect) * ((3.0 / 4.0) * u0 + (1.0 / 4.0) * ui + (1.0 / 4.0) * dt * (1.0 / Vc) * ri);
+  else u = (1 - neglect) * ((1.0 / 3.0) * u0 + (2.0 / 3.0) * ui + (2.0 / 3.0) * dt * (1.0 / Vc) * ri);
   Unew[i] = u;
 }
 
@@ -1307,7 +1349,6 @@ __global__ void __launch_bounds__(kBlock) rk_update_w(fk_params P, int64_t nc, c
   __shared__ __attribute__((aligned(16))) float sWr[kBlock * SWR];
   const int64_t c0 = (int64_t)blockIdx.x * kBlock;
   const int64_t c = c0 + threadIdx.x < nc ? c0 + threadIdx.x : nc - 1;
-  const double dt = dt_of(ds);
   const double Vc = vol[c];
   double r[NEQ], uc[NEQ], un[NEQ];
   if constexpr (sizeof(RT) == 8) {
@@ -1319,6 +1360,7 @@ __global__ void __launch_bounds__(kBlock) rk_update_w(fk_params P, int64_t nc, c
   if (P.rkSteps == 1 || irk != 0) fk::load_rec<NEQ>(U + c * NEQ, uc);
   double u0[NEQ];
   if (P.rkSteps != 1) fk::load_rec<NEQ>(U0 + c * NEQ, u0);
+  const double dt = dt_of(ds);
   rk_stage<NEQ>(P, irk, dt, Vc, uc, u0, r, un);
 #pragma unroll
   for (int v = 0; v < NEQ; ++v) sU[threadIdx.x * SU + v] = un[v];
@@ -1347,38 +1389,17 @@ __device__ __forceinline__ void publish(double *host, unsigned long long seq) {
   if (threadIdx.x == 0) reinterpret_cast<volatile unsigned long long *>(host)[kHostSeq] = seq;
 }
 
-// min over cells of Vcfl/signal: per-block minima, then one block folds them
-// and forms dt = min(cfl * min, maxDt) on the device.
-__global__ void __launch_bounds__(kBlock) min_blocks(int64_t n, const double *__restrict__ x, double *__restrict__ out) {
-  __shared__ double sh[kBlock];
-  double m = 1e15;
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) m = fmin(m, x[i]);
-  sh[threadIdx.x] = m;
-  __syncthreads();
-  for (int s = kBlock / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) sh[threadIdx.x] = fmin(sh[threadIdx.x], sh[threadIdx.x + s]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[blockIdx.x] = sh[0];
-}
-
-__global__ void __launch_bounds__(kBlock) dt_final(int nb, const double *__restrict__ part, double cfl, double maxDt,
-                                                   double *__restrict__ scal, double *__restrict__ host,
-                                                   unsigned long long seq) {
-  __shared__ double sh[kBlock];
-  double m = 1e15;
-  for (int i = threadIdx.x; i < nb; i += kBlock) m = fmin(m, part[i]);
-  sh[threadIdx.x] = m;
-  __syncthreads();
-  for (int s = kBlock / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) sh[threadIdx.x] = fmin(sh[threadIdx.x], sh[threadIdx.x + s]);
-    __syncthreads();
-  }
+// dt = min(cfl * min, maxDt) from a set of pass F's minima, by one wave.
+__global__ void __launch_bounds__(64) dt_final(const unsigned long long *__restrict__ slots,
+                                               unsigned long long *__restrict__ reset, double cfl, double maxDt,
+                                               double *__restrict__ scal, double *__restrict__ host,
+                                               unsigned long long seq) {
+  const double dt = fmin(cfl * dt_fold(slots, reset), maxDt);
   if (threadIdx.x == 0) {
-    scal[0] = fmin(cfl * sh[0], maxDt);
-    if (host) host[0] = scal[0];  // fk_compute_time_step
+    scal[0] = dt;
+    if (host) host[0] = dt;  // fk_compute_time_step
   }
-  if (host && threadIdx.x < 64) publish(host, seq);
+  if (host) publish(host, seq);
 }
 
 // relaxation (relaxation.cu:77-114), reference Newton solves, in two passes:
@@ -1607,9 +1628,12 @@ void free_all(fk_ctx *c) {
   c->vol = c->volcfl = nullptr;
   c->U[0] = c->U[1] = c->U[2] = nullptr;
   c->face = c->gvel = nullptr;
-  c->rhs = c->dtc = c->red = c->dtw = c->dscal = c->dgrad = c->dtheta = nullptr;
+  c->dtw = nullptr;
+  c->rhs = c->dtc = c->red = c->dscal = c->dgrad = c->dtheta = nullptr;
   c->lcount = nullptr;
 }
+
+inline unsigned long long *dt_slots(const fk_ctx *c, int set) { return c->dtw + set * kDtSlots * kDtStride; }
 
 // Cells up to which pass G and pass F run four lanes per cell (pass_g_q,
 // pass_f_q) rather than one with the LDS paths.  What the quads win is waves
@@ -1747,17 +1771,21 @@ int launch_pass_f_t(fk_ctx *c, int irk, double dt, const double *dtp, double *Un
   c->pf_waves = (int64_t)(stage ? (int64_t)gs * (bs / 64) : (int64_t)gr * (kBlock / 64));
   const bool quad = quad_f(c, relax);
   if (quad) c->pf_waves = grid_quad(c->nc);
-  double *dtmin = nullptr;
-  if (MODE == 1) {
-    c->dt_parts = quad && grid_quad(c->nc) <= kDtParts ? (int)grid_quad(c->nc) : 0;
-    if (c->dt_parts) dtmin = c->dtw;
+  unsigned long long *dtmin = nullptr;
+  if (MODE == 1) {  // the other of the two sets of minima; a fold of this one resets it again
+    c->dt_set ^= 1;
+    dtmin = dt_slots(c, c->dt_set);
+    if (!c->dt_clean[c->dt_set])
+      LAUNCH_TIMED(c, "zero", hipLaunchKernelGGL(dt_reset, dim3(1), dim3(kDtSlots), 0, c->stream, dtmin));
+    c->dt_clean[c->dt_set] = false;
   }
 #define PF_ARGS(W) \
-  c->p, c->nc, U, U0, Unew, c->link, c->geo, wl, c->vol, c->volcfl, face, gv, c->rhs, c->dtc, irk, dt, dtp, W, clock
+  c->p, c->nc, U, U0, Unew, c->link, c->geo, wl, c->vol, c->volcfl, face, gv, c->rhs, c->dtc, irk, dt, dtp, W, clock,       \
+      dtmin
 #define PFQ(NEQ, VISC, HEAT, WO, RX, NAME, W, LIST, CNT, PART)                                                         \
   LAUNCH_TIMED(c, NAME,                                                                                                \
                hipLaunchKernelGGL((pass_f_q<NEQ, T, VISC, HEAT, MODE, NS, WO, RX>), dim3(grid_quad(c->nc)), dim3(64), 0, \
-                                  c->stream, PF_ARGS(W), dtmin, LIST, CNT, PART))
+                                  c->stream, PF_ARGS(W), LIST, CNT, PART))
 #define PF(NEQ, VISC, HEAT)                                                                                            \
   do {                                                                                                                 \
     if (quad) {                                                                                                        \
@@ -1906,7 +1934,7 @@ int do_pass_f_update(fk_ctx *c, int irk, double dt, const double *dtp, bool want
 
 // dt as given (val), or from the device (ptr)
 DtSource dt_source(const fk_ctx *c, double val, const double *ptr, double *clock) {
-  return DtSource{val, ptr, nullptr, 0, c->p.cfl, c->p.maxDt, c->dscal, clock != nullptr};
+  return DtSource{val, ptr, nullptr, nullptr, c->p.cfl, c->p.maxDt, c->dscal, clock != nullptr};
 }
 
 // RK stage from the stored residual (FP32 after the mixed dt stage, c->rhs_f32)
@@ -1956,30 +1984,27 @@ int wait_result(fk_ctx *c) {
 
 // dt of the last pass F MODE 1 into dscal[0] (and host[0])
 int do_dt_device(fk_ctx *c, double *host) {
-  const double *part = c->dtw;
-  int nb = c->dt_parts;
-  if (!nb) {
-    part = c->red;
-    nb = 1024;
-    LAUNCH_TIMED(c, "dt_reduce",
-                 hipLaunchKernelGGL(min_blocks, dim3(nb), dim3(kBlock), 0, c->stream, c->nc, c->dtc, c->red));
-  }
-  LAUNCH_TIMED(c, "dt_final", hipLaunchKernelGGL(dt_final, dim3(1), dim3(kBlock), 0, c->stream, nb, part, c->p.cfl,
-                                                 c->p.maxDt, c->dscal, host, host ? ++c->hseq : 0ull));
+  LAUNCH_TIMED(c, "dt_final", hipLaunchKernelGGL(dt_final, dim3(1), dim3(64), 0, c->stream, dt_slots(c, c->dt_set),
+                                                 dt_slots(c, c->dt_set ^ 1), c->p.cfl, c->p.maxDt, c->dscal, host,
+                                                 host ? ++c->hseq : 0ull));
+  c->dt_clean[c->dt_set ^ 1] = true;
   return FK_OK;
 }
 
 // The dt stage of fk_run_steps after pass F MODE 1: dt and the RK update.
 int do_dt_update(fk_ctx *c, int irk, bool want_w, double *clock) {
   DtSource ds = dt_source(c, 0.0, c->dscal, clock);
-  if (c->dt_parts && c->dt_parts <= kDtFold) {
+  const bool w = want_w && c->p.precision == FK_MIXED && c->prims_w;
+  if ((int64_t)grid_for(w ? c->nc : c->nc * c->neq) <= kDtFold) {
     ds.ptr = nullptr;
-    ds.minima = c->dtw;
-    ds.nmin = c->dt_parts;
-  } else {
-    int rc = do_dt_device(c, nullptr);
-    if (rc) return rc;
+    ds.slots = dt_slots(c, c->dt_set);
+    ds.reset = dt_slots(c, c->dt_set ^ 1);
+    int rc = do_update(c, irk, ds, want_w);
+    if (!rc) c->dt_clean[c->dt_set ^ 1] = true;
+    return rc;
   }
+  int rc = do_dt_device(c, nullptr);
+  if (rc) return rc;
   return do_update(c, irk, ds, want_w);
 }
 
@@ -2355,7 +2380,8 @@ int fk_upload_mesh(fk_ctx *c, int64_t nElem, int64_t nFcs, const int32_t *fc2el,
   HIPCHK(hipMalloc(&c->rhs, cs * neq * 8));
   HIPCHK(hipMalloc(&c->dtc, cs * 8));
   HIPCHK(hipMalloc(&c->red, 4096 * 8));
-  HIPCHK(hipMalloc(&c->dtw, kDtParts * 8));
+  HIPCHK(hipMalloc(&c->dtw, 2 * kDtSlots * kDtStride * 8));
+  c->dt_clean[0] = c->dt_clean[1] = false;
   HIPCHK(hipMalloc(&c->dscal, 16 * 8));
   HIPCHK(hipMalloc(&c->lcount, 16 * 8));
   HIPCHK(hipMalloc(&c->wprim, cs * neq * sizeof(float)));

@@ -193,3 +193,42 @@ def test_workgroups_of_one_lane_per_cell_with_a_remainder(gpu, name, precision):
             g.run_steps(2)
             out.append(g.download_state())
     assert all(np.array_equal(o, out[0]) for o in out[1:])
+
+
+@pytest.mark.parametrize("stage", [1, 2, 0])
+@pytest.mark.parametrize("n", [(1, 1, 1), (3, 3, 1), (8, 4, 4), (17, 13, 11)])
+def test_time_step_is_that_of_the_last_state(gpu, n, stage):
+    """The step's minimum of the cells of the state at hand, whatever stages
+    ran before it: a fast state, then a slow one, residuals without a time
+    step in between; from a part of a wave to more waves than the words that
+    hold the minima.  Against the oracle (1e-14, as for the step of one
+    state), and run_steps' first dt the same."""
+    m = Mesh.box(*n)
+    p = dict(cases.tgv(n=4).params, cfl=0.3)
+    slow = rough_state(5, m.n_cells, "random", 3)
+    fast = slow * [1, 5, 5, 5, 25]
+    want = []
+    for U in (slow, fast):
+        o = Oracle(p, m, U)
+        o.compute_face_values()
+        o.compute_rhs()
+        want.append(o.compute_time_step())
+    assert want[1] < want[0]
+    with GpuSolver(p, m, fast) as g:
+        g.set_tuning("stage_f", stage)
+
+        def dt_of(U, passes=1):
+            g.upload_state(U)
+            g.compute_face_values()
+            for _ in range(passes):
+                g.compute_rhs()
+            return g.compute_time_step()
+
+        got = [dt_of(slow), dt_of(fast), dt_of(slow), dt_of(fast, 3), dt_of(slow, 2)]
+        got.append(g.compute_time_step())
+        print(f"[dt] {m.n_cells} cells, stage_f {stage}: {got} oracle {want}", flush=True)
+        assert np.allclose(got, [want[0], want[1], want[0], want[1], want[0], want[0]], rtol=1e-14, atol=0)
+        for U, dt in ((slow, got[0]), (fast, got[1]), (slow, got[0])):
+            g.upload_state(U)
+            g.set_clock(0.0, 0.0, 0)
+            assert g.run_steps(1)[0] == dt
