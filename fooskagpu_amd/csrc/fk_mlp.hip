@@ -39,6 +39,7 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int HID = 64;
 constexpr int kParams = 8771;
@@ -52,10 +53,10 @@ struct Norm {
 };
 
 __device__ __forceinline__ uint16_t f2bf(float f) {  // round to nearest even
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);  // NaN stays NaN
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
+  const uint32_t u = __float_as_uint(f);
+  uint32_t r = (u + (0x7fffu + ((u >> 16) & 1u))) >> 16, n = (u >> 16) | 0x40;  // NaN stays NaN
+  asm("" : "+v"(r), "+v"(n));  // a select, not a branch around either
+  return (uint16_t)((u & 0x7fffffffu) > 0x7f800000u ? n : r);
 }
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float(((uint32_t)b) << 16); }
 
@@ -165,24 +166,54 @@ __device__ __forceinline__ void mlp_fwd16(const SmallW &sw, const uint16_t *wb, 
   __builtin_amdgcn_wave_barrier();
 }
 
-// Copy the FP32 forward parameters into LDS (block-wide; the caller's
-// barrier, that of load_wb, publishes them).
-__device__ __forceinline__ void load_small(const float *__restrict__ w, SmallW &s) {
-  for (int i = threadIdx.x; i < HID; i += blockDim.x) {
-    s.w1b[i] = make_float4(w[oW1 + 3 * i], w[oW1 + 3 * i + 1], w[oW1 + 3 * i + 2], w[oB1 + i]);
-    s.b2[i] = w[oB2 + i];
-    s.b3[i] = w[oB3 + i];
+// Copies of the weights into LDS by blocks of NT threads: the FP32 forward
+// parameters (SmallW, as one array) and the first ROWS rows of the BF16
+// weights, padded.  Neither part has a branch, so that all loads go out before
+// the first is stored: a block begins with one memory latency, not one for
+// each.
+template <int ROWS, int NT>
+struct WeightCopy {
+  static constexpr int K = ROWS * (HID / 8) / NT, S = 9 * HID + 3, KS = (S + NT - 1) / NT;
+  static_assert(K * NT == ROWS * (HID / 8), "whole words per thread");
+  uint4 v[K];
+  float c[KS];
+  // parameter behind float j of SmallW
+  static __device__ __forceinline__ int param(int j) {
+    const int r = j >> 2, k = j & 3;
+    int p = k < 3 ? oW1 + 3 * r + k : oB1 + r;
+    if (j >= 4 * HID) p = oB2 + j - 4 * HID;
+    if (j >= 5 * HID) p = oB3 + j - 5 * HID;
+    if (j >= 6 * HID) p = oW4 + j - 6 * HID;
+    if (j >= 9 * HID) p = oB4 + (j < S ? j - 9 * HID : 0);
+    return p;
   }
-  for (int i = threadIdx.x; i < 3 * HID; i += blockDim.x) s.w4[i] = w[oW4 + i];
-  if (threadIdx.x < 3) s.b4[threadIdx.x] = w[oB4 + threadIdx.x];
-}
-
-// Copy the first `rows` rows of the BF16 weights into LDS, padded (block-wide).
-__device__ __forceinline__ void load_wb(const uint16_t *__restrict__ g, uint16_t *s, int rows) {
-  for (int i = threadIdx.x; i < rows * (HID / 8); i += blockDim.x) {
-    const int row = i / (HID / 8), col = i % (HID / 8) * 8;
-    *reinterpret_cast<uint4 *>(s + row * kRow + col) = reinterpret_cast<const uint4 *>(g)[i];
+  __device__ __forceinline__ void load(const float *__restrict__ w, const uint16_t *__restrict__ g) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = reinterpret_cast<const uint4 *>(g)[k * NT + threadIdx.x];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) c[k] = w[param(k * NT + threadIdx.x)];
   }
+  __device__ __forceinline__ void store(SmallW &s, uint16_t *wb) const {
+    static_assert(offsetof(SmallW, b2) == 16 * HID && offsetof(SmallW, b3) == 20 * HID &&
+                  offsetof(SmallW, w4) == 24 * HID && offsetof(SmallW, b4) == 36 * HID, "SmallW as one array");
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      const int j = k * NT + threadIdx.x;
+      reinterpret_cast<float *>(&s)[j < S ? j : S] = c[k];  // the rest on the spare word b4[3]
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int j = k * NT + threadIdx.x, row = j / (HID / 8), col = j % (HID / 8) * 8;
+      *reinterpret_cast<uint4 *>(wb + row * kRow + col) = v[k];
+    }
+  }
+};
+template <int ROWS>
+__device__ __forceinline__ void load_weights(const float *__restrict__ w, const uint16_t *__restrict__ g, SmallW &s,
+                                             uint16_t *wb) {
+  WeightCopy<ROWS, 256> wc;
+  wc.load(w, g);
+  wc.store(s, wb);
   __syncthreads();
 }
 
@@ -194,8 +225,7 @@ __global__ void __launch_bounds__(256) mlp_infer_k(int64_t n, const float *__res
   __shared__ __attribute__((aligned(16))) uint16_t wb[2 * HID * kRow];
   __shared__ FwdLds lds[4];
   __shared__ SmallW sw;
-  load_small(w, sw);
-  load_wb(wbg, wb, 2 * HID);
+  load_weights<2 * HID>(w, wbg, sw, wb);
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int64_t nchunk = (n + 63) / 64;
   for (int64_t ch = (int64_t)blockIdx.x * 4 + wv; ch < (nchunk + 3) / 4 * 4; ch += (int64_t)gridDim.x * 4) {
@@ -228,8 +258,8 @@ struct TrainLds {
   uint16_t hT[HID * kRowT];                              // [k][m] of the layer input
   uint16_t dzT[HID * kRowT];                             // [n][m]
   float dzf[32 * HID];                                   // dz of layer 3 before rounding
-  float x[32 * 3], dy[32 * 3];
-  int64_t idx[32];
+  float x[32 * 3], y[32 * 3];                            // normalised inputs and targets
+  float err[32 * 3], dy[32 * 3];                         // error of each output, its share of the gradient
 };
 
 // Sample i of a training run: splitmix64 of (seed, i) modulo n.
@@ -246,75 +276,76 @@ __device__ __forceinline__ int64_t sample_index(uint64_t seed, uint64_t i, uint6
 // part[blockIdx.x] (each weight-gradient tile as soon as it is formed).
 //
 // A batch of 8192 is 256 blocks, one per CU, so the time is that of one
-// block's chain of layers: four waves share it.  In the forward pass a pair of
-// waves takes each 16-sample tile and splits its neurons, in the backward pass
-// the waves split weight-gradient rows, neurons or samples; each sum keeps its
-// terms and their order, so the gradient is that of one wave, bit for bit
-// (44 us with one wave per block; 20 us).
-__global__ void __launch_bounds__(256) mlp_train_k(int64_t B, const int64_t *__restrict__ idx, uint64_t seed,
+// block's chain of layers: eight waves share it.  In the forward pass a wave
+// takes a tile of 16 samples and 16 neurons (4 of the 64 tanh a lane would take
+// alone), in the backward pass four waves form the weight gradients, the other
+// four the sums over the samples beside them, and all eight the errors of the
+// layer below.  Weights, inputs and targets are asked for together at the
+// start.  Each sum keeps its terms and their order, so the gradient is that of
+// one wave, bit for bit (44 us with one wave per block, 20 with four and the
+// targets fetched where they are used; 13 us).
+constexpr int kTrainThreads = 512;
+__global__ void __launch_bounds__(kTrainThreads) mlp_train_k(int64_t B, const int64_t *__restrict__ idx, uint64_t seed,
                                                    uint64_t first, uint64_t n, const float *__restrict__ X,
                                                    const float *__restrict__ Y, const float *__restrict__ w,
                                                    const uint16_t *__restrict__ wbg, Norm nm,
                                                    float *__restrict__ part, float *__restrict__ loss_part) {
   __shared__ __attribute__((aligned(16))) TrainLds L;
   __shared__ SmallW sw;
-  load_small(w, sw);
-  load_wb(wbg, L.wb, 4 * HID);
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, m16 = l & 15, q = l >> 4;
-  const int t = wv & 1, half = wv >> 1;  // forward: tile of 16 samples, half of the neurons
+  const int t = wv & 1, nt = wv >> 1;  // tile of 16 samples, tile of 16 neurons
   float *g = part + (int64_t)blockIdx.x * kParams;
   const int64_t s0 = (int64_t)blockIdx.x * 32;
   const int ns = (int)(s0 + 32 < B ? 32 : B - s0);
   const float inv = 2.0f / (3.0f * (float)B);
-  if (threadIdx.x < 32)
-    L.idx[threadIdx.x] = (int)threadIdx.x >= ns ? 0
-                         : idx                  ? idx[s0 + threadIdx.x]
-                                                : sample_index(seed, first + s0 + threadIdx.x, n);
-  __syncthreads();
-  // inputs (normalised); padding samples get x = 0 and dy = 0
-  if (threadIdx.x < 96) {
-    const int mm = threadIdx.x / 3, j = threadIdx.x % 3;
-    L.x[threadIdx.x] = mm < ns ? (X[L.idx[mm] * 3 + j] - nm.xm[j]) / nm.xs[j] : 0.f;
+  // weights, and normalised by waves 6 and 7 the targets, by the others the
+  // inputs (each pair of waves the same ones: no branch); padding samples get
+  // x = 0 and, below, dy = 0
+  {
+    const int e = (threadIdx.x & 127) < 96 ? threadIdx.x & 127 : 95, mm = e / 3, j = e % 3;
+    const bool in = wv < 6;
+    int64_t k = s0 + (mm < ns ? mm : ns - 1);
+    k = idx ? idx[k] : sample_index(seed, first + k, n);
+    WeightCopy<4 * HID, kTrainThreads> wc;
+    wc.load(w, wbg);
+    const float raw = (in ? X : Y)[k * 3 + j];
+    const float v = fk::quot(raw - (in ? nm.xm[j] : nm.ym[j]), in ? nm.xs[j] : nm.ys[j]);
+    wc.store(sw, L.wb);
+    (in ? L.x : L.y)[e] = mm < ns ? v : 0.f;
   }
   __syncthreads();
-  // layer 1 (FP32): neurons k = 32 half + 8 q + i of sample 16 t + m16
+  // layer 1 (FP32): neurons k = 16 nt + 4 q + i of sample 16 t + m16
   {
     const int m = 16 * t + m16;
     const float x0 = L.x[m * 3 + 0], x1 = L.x[m * 3 + 1], x2 = L.x[m * 3 + 2];
-    u16x8 hv;
+    u16x4 hv;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float4 c = sw.w1b[32 * half + 8 * q + i];
+    for (int i = 0; i < 4; ++i) {
+      const float4 c = sw.w1b[16 * nt + 4 * q + i];
       hv[i] = f2bf(tanhf(c.w + c.x * x0 + c.y * x1 + c.z * x2));
     }
-    *reinterpret_cast<u16x8 *>(L.h1 + m * kRow + 32 * half + 8 * q) = hv;
+    *reinterpret_cast<u16x4 *>(L.h1 + m * kRow + 16 * nt + 4 * q) = hv;
   }
   __syncthreads();
-  // layers 2 and 3 (BF16 MFMA): this wave's two tiles of 16 neurons
+  // layers 2 and 3 (BF16 MFMA)
+  const int nn = 16 * nt + m16;
 #pragma unroll
   for (int layer = 0; layer < 2; ++layer) {
     const uint16_t *hin = layer == 0 ? L.h1 : L.h2, *W = L.wb + (layer == 0 ? 0 : HID * kRow);
     uint16_t *hout = layer == 0 ? L.h2 : L.h3;
-    const float *bias = layer == 0 ? sw.b2 : sw.b3;
-    bf16x8 a[2];
+    const float bias = (layer == 0 ? sw.b2 : sw.b3)[nn];
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) a[ks] = ld_bf8(hin + (16 * t + m16) * kRow + 32 * ks + 8 * q);
+    for (int ks = 0; ks < 2; ++ks)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ld_bf8(hin + (16 * t + m16) * kRow + 32 * ks + 8 * q),
+                                                    ld_bf8(W + nn * kRow + 32 * ks + 8 * q), acc, 0, 0, 0);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int nn = 16 * (2 * half + u) + m16;
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks], ld_bf8(W + nn * kRow + 32 * ks + 8 * q), acc, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) hout[(16 * t + 4 * q + i) * kRow + nn] = f2bf(tanhf(acc[i] + bias[nn]));
-    }
+    for (int i = 0; i < 4; ++i) hout[(16 * t + 4 * q + i) * kRow + nn] = f2bf(tanhf(acc[i] + bias));
     __syncthreads();
   }
   // layer 4 (FP32), waves 0 and 1: 16 neurons a lane, then the sample's four
   // lanes; the error of each output
-  float lsum = 0;
-  if (half == 0) {
+  if (nt == 0) {
     const int m = 16 * t + m16;
     float p[3] = {0.f, 0.f, 0.f};
 #pragma unroll
@@ -335,34 +366,20 @@ __global__ void __launch_bounds__(256) mlp_train_k(int64_t B, const int64_t *__r
     }
     if (q < 3) {
       const float pj = q == 0 ? p[0] : (q == 1 ? p[1] : p[2]);
-      L.dy[m * 3 + q] = sw.b4[q] + pj;
+      const float d = m < ns ? (sw.b4[q] + pj) - L.y[m * 3 + q] : 0.f;
+      L.err[m * 3 + q] = d;
+      L.dy[m * 3 + q] = d * inv;
     }
   }
   __syncthreads();
-  if (wv == 0) {
-    // wave 0: lanes l < 48 the outputs of tile 0, then of tile 1 (the order of
-    // the loss sum)
-    for (int tt = 0; tt < 2; ++tt)
-      if (l < 48) {
-        const int mm = tt * 16 + l / 3, j = l % 3;
-        float d = 0.f;
-        if (mm < ns) {
-          const float tgt = (Y[L.idx[mm] * 3 + j] - nm.ym[j]) / nm.ys[j];
-          d = L.dy[mm * 3 + j] - tgt;
-          lsum += d * d;
-        }
-        L.dy[mm * 3 + j] = d * inv;
-      }
-  }
-  __syncthreads();
   // layer 4 backward: dz3[m][k] = (sum_j dy W4[j][k]) (1 - h3^2), lane k = l,
-  // 8 samples a wave; then gW4[j][k] (waves 1 to 3), gb3 and gb4 (wave 0)
+  // 4 samples a wave
   {
     const int k = l;
     const float w4[3] = {sw.w4[k], sw.w4[HID + k], sw.w4[2 * HID + k]};
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int mm = 8 * wv + u;
+    for (int u = 0; u < 4; ++u) {
+      const int mm = 4 * wv + u;
       const float h = bf2f(L.h3[mm * kRow + k]);
       float dh = 0;
 #pragma unroll
@@ -374,91 +391,93 @@ __global__ void __launch_bounds__(256) mlp_train_k(int64_t B, const int64_t *__r
       L.dzT[k * kRowT + mm] = db;
       L.hT[k * kRowT + mm] = L.h2[mm * kRow + k];
     }
-    __syncthreads();
-    if (wv == 0) {
+  }
+  __syncthreads();
+  // layers 3 then 2.  Waves 4 to 7: gW = dz^T h (K = 32 samples), 16 rows each.
+  // Waves 0 to 3, lane k = l: sums over the samples, at layer 3 gb3 and gb4
+  // (wave 0) and gW4[j][k], at layer 2 gb2 (wave 0).  Then all: dh = dz W, a
+  // tile each; dz_below = dh (1 - h^2)
+#pragma unroll
+  for (int layer = 3; layer >= 2; --layer) {
+    if (wv >= 4) {
+      const int oW = layer == 3 ? oW3 : oW2, r = 16 * (wv - 4);
+      const bf16x8 a = ld_bf8(L.dzT + (r + m16) * kRowT + 8 * q);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const bf16x8 b = ld_bf8(L.hT + (16 * c + m16) * kRowT + 8 * q);
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) g[oW + (r + 4 * q + i) * HID + 16 * c + m16] = acc[i];
+      }
+    } else if (layer == 3 && wv == 0) {
       float gb3 = 0;
 #pragma unroll 8
-      for (int mm = 0; mm < 32; ++mm) gb3 += L.dzf[mm * HID + k];
-      g[oB3 + k] = gb3;
+      for (int mm = 0; mm < 32; ++mm) gb3 += L.dzf[mm * HID + l];
+      g[oB3 + l] = gb3;
       if (l < 3) {
         float sb = 0;
 #pragma unroll 8
         for (int mm = 0; mm < 32; ++mm) sb += L.dy[mm * 3 + l];
         g[oB4 + l] = sb;
       }
-    } else {
+    } else if (layer == 3) {
       const int j = wv - 1;
       float gw4 = 0;
 #pragma unroll 8
-      for (int mm = 0; mm < 32; ++mm) gw4 += L.dy[mm * 3 + j] * bf2f(L.h3[mm * kRow + k]);
-      g[oW4 + j * HID + k] = gw4;
-    }
-  }
-  // layers 3 then 2: gW = dz^T h (K = 32 samples), rows 16 wv .. of a wave;
-  // dh = dz W, a tile of samples and half the neurons a wave; dz_below = dh (1 - h^2)
-#pragma unroll
-  for (int layer = 3; layer >= 2; --layer) {
-    const int oW = layer == 3 ? oW3 : oW2;
-    {
-      const bf16x8 a = ld_bf8(L.dzT + (16 * wv + m16) * kRowT + 8 * q);
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        const bf16x8 b = ld_bf8(L.hT + (16 * nt + m16) * kRowT + 8 * q);
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) g[oW + (16 * wv + 4 * q + i) * HID + 16 * nt + m16] = acc[i];
-      }
-    }
-    const uint16_t *WT = L.wb + (layer == 3 ? 3 : 2) * HID * kRow;
-    const uint16_t *hin = layer == 3 ? L.h2 : L.h1;  // activations feeding this layer
-    uint16_t db[2][4];
-    {
-      bf16x8 a2[2];
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) a2[ks] = ld_bf8(L.dz + (16 * t + m16) * kRow + 32 * ks + 8 * q);
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int col = 16 * (2 * half + u) + m16;
-        f32x4 d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-          d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[ks], ld_bf8(WT + col * kRow + 32 * ks + 8 * q), d, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float h = bf2f(hin[(16 * t + 4 * q + i) * kRow + col]);
-          db[u][i] = f2bf(d[i] * (1.f - h * h));
-        }
-      }
-    }
-    __syncthreads();  // every wave has read dz, dzT and hT
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = 16 * t + 4 * q + i, col = 16 * (2 * half + u) + m16;
-        L.dz[row * kRow + col] = db[u][i];
-        L.dzT[col * kRowT + row] = db[u][i];
-      }
-    if (layer == 3)
-#pragma unroll
-      for (int u = 0; u < 8; ++u) L.hT[l * kRowT + 8 * wv + u] = L.h1[(8 * wv + u) * kRow + l];
-    __syncthreads();
-    // sums over the samples, lane k = l: the bias (wave 0), W1 (waves 1 to 3)
-    if (wv == 0) {
+      for (int mm = 0; mm < 32; ++mm) gw4 += L.dy[mm * 3 + j] * bf2f(L.h3[mm * kRow + l]);
+      g[oW4 + j * HID + l] = gw4;
+    } else if (wv == 0) {
       float sb = 0;
 #pragma unroll 8
       for (int mm = 0; mm < 32; ++mm) sb += bf2f(L.dz[mm * kRow + l]);
-      g[(layer == 3 ? oB2 : oB1) + l] = sb;
-    } else if (layer == 2) {
-      const int j = wv - 1;
-      float gw1 = 0;
-#pragma unroll 8
-      for (int mm = 0; mm < 32; ++mm) gw1 += bf2f(L.dz[mm * kRow + l]) * L.x[mm * 3 + j];
-      g[oW1 + 3 * l + j] = gw1;
+      g[oB2 + l] = sb;
     }
+    const uint16_t *WT = L.wb + (layer == 3 ? 3 : 2) * HID * kRow;
+    const uint16_t *hin = layer == 3 ? L.h2 : L.h1;  // activations feeding this layer
+    f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ld_bf8(L.dz + (16 * t + m16) * kRow + 32 * ks + 8 * q),
+                                                  ld_bf8(WT + nn * kRow + 32 * ks + 8 * q), d, 0, 0, 0);
+    uint16_t db[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float h = bf2f(hin[(16 * t + 4 * q + i) * kRow + nn]);
+      db[i] = f2bf(d[i] * (1.f - h * h));
+    }
+    __syncthreads();  // every wave has read dz, dzT and hT
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 16 * t + 4 * q + i;
+      L.dz[row * kRow + nn] = db[i];
+      L.dzT[nn * kRowT + row] = db[i];
+    }
+    if (layer == 3)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) L.hT[l * kRowT + 4 * wv + u] = L.h1[(4 * wv + u) * kRow + l];
+    __syncthreads();
   }
+  // gb1 (wave 0), gW1 (waves 1 to 3), the loss (wave 4: outputs l < 48 of tile
+  // 0, then of tile 1)
   if (wv == 0) {
+    float sb = 0;
+#pragma unroll 8
+    for (int mm = 0; mm < 32; ++mm) sb += bf2f(L.dz[mm * kRow + l]);
+    g[oB1 + l] = sb;
+  } else if (wv < 4) {
+    const int j = wv - 1;
+    float gw1 = 0;
+#pragma unroll 8
+    for (int mm = 0; mm < 32; ++mm) gw1 += bf2f(L.dz[mm * kRow + l]) * L.x[mm * 3 + j];
+    g[oW1 + 3 * l + j] = gw1;
+  } else if (wv == 4) {
+    float lsum = 0;
+    if (l < 48)
+      for (int tt = 0; tt < 2; ++tt) {
+        const float d = L.err[tt * 48 + l];
+        lsum += d * d;
+      }
     for (int off = 32; off > 0; off >>= 1) lsum += __shfl_down(lsum, off, 64);
     if (l == 0) loss_part[blockIdx.x] = lsum;
   }
@@ -475,37 +494,64 @@ __device__ __forceinline__ void pack_param(int i, float v, uint16_t *__restrict_
 }
 
 // Fixed-order sum of the per-block partials (deterministic), and with ADAM the
-// update of the FP32 master weights and their BF16 copies.  One wave a block
-// and 32 partials loaded ahead of the adds: the sum waits for memory, not for
-// its 35 blocks (58 us for 256 partials with one load at a time and 256
-// threads a block, and 9 us for the update and the copies as kernels of their
-// own; 8 us).
+// update of the FP32 master weights and their BF16 copies.  A block takes 64
+// parameters; the kernel waits for memory, not for its 138 blocks, so four
+// waves hold 64 partials each in flight (a wave counts no more than 63 loads),
+// add them one wave after the other, and the moments and weights are there by
+// then (58 us for 256 partials with one load at a time and 256 threads a
+// block, and 9 us for the update and the copies as kernels of their own; 8 us
+// in one wave with 32 ahead; 4 us).
 template <bool ADAM>
-__global__ void __launch_bounds__(64) mlp_update_k(int nb, const float *__restrict__ part, float *__restrict__ g,
-                                                   float *__restrict__ w, float *__restrict__ m,
-                                                   float *__restrict__ v, uint16_t *__restrict__ wb, float lr,
-                                                   float b1t, float b2t) {
-  const int i = blockIdx.x * 64 + threadIdx.x;
-  if (i >= kParams) return;
-  float s = 0;
-  int b = 0;
-  for (; b + 32 <= nb; b += 32) {
-    float p[32];
-#pragma unroll
-    for (int k = 0; k < 32; ++k) p[k] = part[(int64_t)(b + k) * kParams + i];
-#pragma unroll
-    for (int k = 0; k < 32; ++k) s += p[k];
+__global__ void __launch_bounds__(256) mlp_update_k(int nb, const float *__restrict__ part, float *__restrict__ g,
+                                                    float *__restrict__ w, float *__restrict__ m,
+                                                    float *__restrict__ v, uint16_t *__restrict__ wb, float lr,
+                                                    float b1t, float b2t) {
+  __shared__ float sum[64];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+  const int it = blockIdx.x * 64 + l, i = it < kParams ? it : kParams - 1;
+  float m0 = 0, v0 = 0, w0 = 0;
+  if constexpr (ADAM) {
+    m0 = m[i];
+    v0 = v[i];
+    w0 = w[i];
   }
-  for (; b < nb; ++b) s += part[(int64_t)b * kParams + i];
+  float s = 0;
+  for (int b0 = 0; b0 < nb; b0 += 256) {
+    const int b = b0 + 64 * wv, n = nb - b;
+    const float *p0 = part + (int64_t)b * kParams + i;
+    float p[64];
+    if (n >= 64) {
+#pragma unroll
+      for (int k = 0; k < 64; ++k) p[k] = p0[(int64_t)k * kParams];
+    } else {
+#pragma unroll
+      for (int k = 0; k < 64; ++k) {
+        const float x = part[(int64_t)(b + k < nb ? b + k : nb - 1) * kParams + i];
+        p[k] = k < n ? x : 0.f;
+      }
+    }
+#pragma unroll 1
+    for (int o = 0; o < 4; ++o) {
+      if (wv == o) {
+        if (b > 0) s = sum[l];
+#pragma unroll
+        for (int k = 0; k < 64; ++k) s += p[k];
+        sum[l] = s;
+      }
+      __syncthreads();
+    }
+  }
+  if (wv != 3 || it != i) return;
+  s = sum[l];
   if constexpr (!ADAM) {
     g[i] = s;
   } else {
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float mi = b1 * m[i] + (1 - b1) * s;
-    const float vi = b2 * v[i] + (1 - b2) * s * s;
+    const float mi = b1 * m0 + (1 - b1) * s;
+    const float vi = b2 * v0 + (1 - b2) * s * s;
     m[i] = mi;
     v[i] = vi;
-    const float wi = w[i] - lr * (mi / (1 - b1t)) / (sqrtf(vi / (1 - b2t)) + eps);
+    const float wi = w0 - lr * (mi / (1 - b1t)) / (sqrtf(vi / (1 - b2t)) + eps);
     w[i] = wi;
     pack_param(i, wi, wb);
   }
@@ -605,8 +651,7 @@ __global__ void __launch_bounds__(256) relax_infer_k(fk_params P, const double *
   const int64_t nfr = fk::list_front(counts[5]);
   const int64_t cf = (nfr + 63) / 64;
   if ((int64_t)blockIdx.x * 4 >= cf) return;  // whole block idle: skip the weight load
-  load_small(w, sw);
-  load_wb(wbg, wb, 2 * HID);
+  load_weights<2 * HID>(w, wbg, sw, wb);
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int64_t per = (cf + 3) / 4 * 4;
   for (int64_t ch = (int64_t)blockIdx.x * 4 + wv; ch < per; ch += (int64_t)gridDim.x * 4) {
@@ -1053,7 +1098,7 @@ static int grad_on(fk_ctx *c, const int64_t *didx, uint64_t seed, uint64_t first
     HIPCHK(hipMalloc(&m.part, (size_t)(nb + 1) * kParams * 4));
     m.part_cap = nb;
   }
-  hipLaunchKernelGGL(mlp_train_k, dim3(nb), dim3(256), 0, c->stream, B, didx, seed, first, (uint64_t)m.n_data, m.dx,
+  hipLaunchKernelGGL(mlp_train_k, dim3(nb), dim3(kTrainThreads), 0, c->stream, B, didx, seed, first, (uint64_t)m.n_data, m.dx,
                      m.dy, m.w, m.wb, norm_of(m), m.part, m.part + (size_t)nb * kParams);
   HIPCHK(hipGetLastError());
   *nblocks = nb;
@@ -1084,7 +1129,7 @@ int fk_mlp_grad(fk_ctx *c, const int64_t *idx, int64_t B, float *grad, float *lo
   int nb = 0;
   int rc = grad_on(c, didx, 0, 0, B, &nb);
   if (!rc) {
-    hipLaunchKernelGGL(mlp_update_k<false>, dim3((kParams + 63) / 64), dim3(64), 0, c->stream, nb, m.part, m.grad,
+    hipLaunchKernelGGL(mlp_update_k<false>, dim3((kParams + 63) / 64), dim3(256), 0, c->stream, nb, m.part, m.grad,
                        nullptr, nullptr, nullptr, nullptr, 0.f, 0.f, 0.f);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) rc = fail(FK_EDEVICE, std::string("mlp_update: ") + hipGetErrorString(e));
@@ -1105,7 +1150,7 @@ int fk_mlp_train(fk_ctx *c, int steps, int batch, float lr, uint64_t seed, float
   HIPCHK(hipSetDevice(c->device));
   // batch indices come from the step and the seed on the device: two kernels
   // a step, no copies, no waits (139 us a step of 8192 samples with indices
-  // drawn and uploaded by the host; 29 us)
+  // drawn and uploaded by the host; 19 us)
   int rc = FK_OK;
   for (int st = 0; st < steps && rc == FK_OK; ++st) {
     int nb = 0;
@@ -1117,7 +1162,7 @@ int fk_mlp_train(fk_ctx *c, int steps, int batch, float lr, uint64_t seed, float
     }
     ++m.adam_t;
     const float b1t = std::pow(0.9f, (float)m.adam_t), b2t = std::pow(0.999f, (float)m.adam_t);
-    hipLaunchKernelGGL(mlp_update_k<true>, dim3((kParams + 63) / 64), dim3(64), 0, c->stream, nb, m.part, nullptr, m.w,
+    hipLaunchKernelGGL(mlp_update_k<true>, dim3((kParams + 63) / 64), dim3(256), 0, c->stream, nb, m.part, nullptr, m.w,
                        m.m, m.v, m.wb, lr, b1t, b2t);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) rc = fail(FK_EDEVICE, hipGetErrorString(e));
