@@ -628,8 +628,8 @@ __device__ __forceinline__ void face_terms(const fk_params &P, const fk::Mat<T> 
 // (computeRHS.cu:78-146, computeViscousStresses.cu:66-174, update.cu:3-103,
 // computeTimeStep.cu:97-159)
 //
-// STAGE: the workgroup first copies the face states of its own cells (4 slots
-// each) and their velocity gradients into LDS; the mirror states and
+// STAGE: the workgroup first copies the face states of its own cells and, with
+// 4 slots, their velocity gradients into LDS; the mirror states and
 // neighbour gradients of faces inside the workgroup are then read from LDS,
 // only those of faces to other workgroups from global memory.
 //
@@ -649,8 +649,10 @@ __device__ __forceinline__ void face_terms(const fk_params &P, const fk::Mat<T> 
 //
 // Workgroup size (pass_f_block): 256 cells; with staging, FP64 128 cells,
 // whose face records and gradients take 52 KB of LDS per 128 cells (104 KB
-// at 256 would leave one workgroup per CU), and 128 cells (37 KB) with 6
-// slots.
+// at 256 would leave one workgroup per CU), and 128 cells with 6 slots.  These
+// stage the face states only (31 KB, five workgroups per CU; with the
+// gradients 37 KB and four: hexahedra 72^3 RK stage 93 against 89.7 us, dt
+// stage 89 against 84).
 template <typename T, bool STAGE, int NS = 4>
 constexpr int pass_f_block() {
   if (!STAGE) return kBlock;
@@ -659,7 +661,7 @@ constexpr int pass_f_block() {
 }
 
 // Layouts that pass F stages: 4 slots; 6 slots for two-phase FP32 records
-// (whole 16-byte words per workgroup row, 37 KB per 128 cells).  On 200^3
+// (whole 16-byte words per workgroup row).  On 200^3
 // hexahedra (8M cells) the fused stage went from 2.61 to 1.80 ms and the dt
 // stage from 2.46 to 1.75 ms; the last stage with the per-cell relaxation
 // slowed down there (2.74 to 3.01 ms, its registers at the lower occupancy
@@ -713,7 +715,7 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
         if (i < nw) __builtin_amdgcn_global_load_lds((const void *)(src + i), (lds_ptr)(dst + k * BS + wbase), 16, 0, 0);
       }
     }
-    if constexpr (VISC) {
+    if constexpr (VISC && NS == 4) {
       constexpr int WPC = NGS * (int)sizeof(T) / 4;  // 4-byte words per cell
       const int nw = (int)(ncell * WPC);
       const float *src = reinterpret_cast<const float *>(gvel + c0 * NGS);
@@ -744,7 +746,7 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
     return face + sl * NEQ;
   };
   auto grad_ptr = [&](int64_t cell) -> const T * {
-    if (STAGE && cell >= c0 && cell < c0 + BS) return sG + (cell - c0) * NGS;
+    if (STAGE && NS == 4 && cell >= c0 && cell < c0 + BS) return sG + (cell - c0) * NGS;
     return gvel + cell * NGS;
   };
   const fk::Mat<double> md = fk::make_mat<double>(P);
@@ -1766,7 +1768,7 @@ int launch_pass_f_t(fk_ctx *c, int irk, double dt, const double *dtp, double *Un
                      (c->neq == 10 ? pass_f_stage_ok<T, NS, 10>() : pass_f_stage_ok<T, NS, 5>());
   constexpr int bs = pass_f_block<T, true, NS>();
   const unsigned gs = (unsigned)(((c->nc + bs - 1) / bs + kXcd - 1) / kXcd * kXcd);
-  const size_t lds = stage ? (size_t)bs * (NS * c->neq + 12) * sizeof(T) : 0;
+  const size_t lds = stage ? (size_t)bs * (NS * c->neq + (NS == 4 ? 12 : 0)) * sizeof(T) : 0;
   // waves of this launch (per-wave relaxation counts of the fused last stage)
   c->pf_waves = (int64_t)(stage ? (int64_t)gs * (bs / 64) : (int64_t)gr * (kBlock / 64));
   const bool quad = quad_f(c, relax);
