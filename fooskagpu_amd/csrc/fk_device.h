@@ -61,6 +61,26 @@ __device__ __forceinline__ float quot(float a, float b) {
 }
 __device__ __forceinline__ double quot(double a, double b) { return a / b; }
 
+// Correctly rounded FP64 quotients x / d for several x: the reciprocal of d
+// to full precision once (hardware estimate, two Newton steps), then each
+// quotient by Markstein's correction of x (1 / d) with the exact residual
+// x - d q: four instructions instead of the twelve of a division.  The bits
+// of x / d while d, x and the quotient stay clear of the ends of the exponent
+// range (|x| > 2^-960; no operand here comes near); div_fixup gives IEEE's
+// results for zeros, infinities and NaN.
+struct Divisor {
+  double d, y;
+  __device__ __forceinline__ explicit Divisor(double v) : d(v) {
+    y = __builtin_amdgcn_rcp(v);
+    y = fma(fma(-v, y, 1.0), y, y);
+    y = fma(fma(-v, y, 1.0), y, y);
+  }
+  __device__ __forceinline__ double operator()(double x) const {
+    const double q = x * y;
+    return __builtin_amdgcn_div_fixup(fma(fma(-d, q, x), y, q), d, x);
+  }
+};
+
 // Quotient and square root of the face terms.  FP32: one reciprocal (or root)
 // and a product, with the bits of the forms above where divisor, reciprocal
 // and result are normal numbers, as densities, wave speeds and moduli are
@@ -68,11 +88,36 @@ __device__ __forceinline__ double quot(double a, double b) { return a / b; }
 // differences can lie below that and take quot.  Two instructions for eight
 // and one for six: pass F at size is bound by its instructions (mixed, 3.07M
 // cells: VALU busy 75 to 95 %; the dt stage, which also took the sound speeds
-// of both states twice, 390 -> 355 us, the RK stage 454 -> 442).
+// of both states twice, 390 -> 355 us, the RK stage 454 -> 442).  FP64: the
+// quotient by Divisor, and the root by Goldschmidt's iteration from the
+// hardware's estimate (two steps, correctly rounded by the last residual)
+// without the range scaling for operands below 2^-767 (four-lane pass F, 1.05M
+// cells: RK stage 258 -> 254 us, dt stage 250 -> 241).
 __device__ __forceinline__ float face_quot(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
-__device__ __forceinline__ double face_quot(double a, double b) { return a / b; }
+__device__ __forceinline__ double face_quot(double a, double b) { return Divisor(b)(a); }
+template <typename T>
+struct FaceDivisor;  // the same for several quotients by one divisor
+template <>
+struct FaceDivisor<float> {
+  float r;
+  __device__ __forceinline__ explicit FaceDivisor(float d) : r(__builtin_amdgcn_rcpf(d)) {}
+  __device__ __forceinline__ float operator()(float x) const { return x * r; }
+};
+template <>
+struct FaceDivisor<double> : Divisor {
+  using Divisor::Divisor;
+};
 __device__ __forceinline__ float face_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
-__device__ __forceinline__ double face_sqrt(double x) { return sqrt(x); }
+__device__ __forceinline__ double face_sqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  g = fma(fma(-g, g, x), h, g);
+  g = fma(fma(-g, g, x), h, g);
+  return x == 0 || x == __builtin_inf() ? x : g;
+}
 
 // ---------------- EOS (DP eqos.h:1-23, SP eqos.h:2-23) ----------------
 // two-phase stiffened gas with energy offset eta, phase k
@@ -111,26 +156,6 @@ template <typename T>
 __device__ __forceinline__ T clamp_avf(const Mat<T> &m, T a) {
   return fmin(fmax(m.avfMin / 100, a), (T)1.0 - m.avfMin / 100);
 }
-
-// Correctly rounded FP64 quotients x / d for several x: the reciprocal of d
-// to full precision once (hardware estimate, two Newton steps), then each
-// quotient by Markstein's correction of x (1 / d) with the exact residual
-// x - d q: four instructions instead of the twelve of a division.  The bits
-// of x / d while d, x and the quotient stay clear of the ends of the exponent
-// range (|x| > 2^-960; no operand here comes near); div_fixup gives IEEE's
-// results for zeros, infinities and NaN.
-struct Divisor {
-  double d, y;
-  __device__ __forceinline__ explicit Divisor(double v) : d(v) {
-    y = __builtin_amdgcn_rcp(v);
-    y = fma(fma(-v, y, 1.0), y, y);
-    y = fma(fma(-v, y, 1.0), y, y);
-  }
-  __device__ __forceinline__ double operator()(double x) const {
-    const double q = x * y;
-    return __builtin_amdgcn_div_fixup(fma(fma(-d, q, x), y, q), d, x);
-  }
-};
 
 // ---------------- conserved -> primitive (double) ----------------
 // Copies the N doubles of one AoS record into registers with 16-byte loads
@@ -287,8 +312,11 @@ struct Sound {
   T cL, cG, YL, YG;
   __device__ __forceinline__ Sound() {}
   __device__ __forceinline__ Sound(const Mat<T> &m, const T *W, T rho)
-      : cL(c_of(m, 0, W[1], W[6])), cG(c_of(m, 1, W[2], W[7])), YL(face_quot(W[0] * W[1], rho)),
-        YG(face_quot((1 - W[0]) * W[2], rho)) {}
+      : cL(c_of(m, 0, W[1], W[6])), cG(c_of(m, 1, W[2], W[7])) {
+    const FaceDivisor<T> d(rho);
+    YL = d(W[0] * W[1]);
+    YG = d((1 - W[0]) * W[2]);
+  }
   __device__ __forceinline__ T wood(const T *W, T rho) const {
     return face_quot((T)1, face_sqrt(rho * (face_quot(W[0], W[1] * cL * cL) + face_quot(1 - W[0], W[2] * cG * cG))));
   }
@@ -392,7 +420,7 @@ __device__ __forceinline__ void riemann(const Mat<T> &m, const T *L, const T *R,
     if constexpr (SIG) {  // formed here, before the star region: the sound speeds end here
       out.sigL = signal(m, L, uL, sl, rL);
       out.sigR = signal(m, R, uR, sr, rR);
-      asm volatile("" : "+v"(out.sigL), "+v"(out.sigR));
+      if constexpr (sizeof(T) == 8) asm volatile("" : "+v"(out.sigL), "+v"(out.sigR));
     }
     T S0 = fmin(uL - cL, uR - cR);
     T S2 = fmax(uL + cL, uR + cR);
@@ -419,8 +447,9 @@ __device__ __forceinline__ void riemann(const Mat<T> &m, const T *L, const T *R,
       unc0 = s[3] + (S1 - un) * n[0];
       unc1 = s[4] + (S1 - un) * n[1];
       unc2 = s[5] + (S1 - un) * n[2];
-      T rSL = face_quot(s[1] * (SK - un), SK - S1);
-      T rSG = face_quot(s[2] * (SK - un), SK - S1);
+      const FaceDivisor<T> dk(SK - S1);
+      T rSL = dk(s[1] * (SK - un));
+      T rSG = dk(s[2] * (SK - un));
       T V1 = a * rSL, V2 = a1 * rSG;
       T rS = V1 + V2;
       T pSL = face_quot((s[6] + m.pi[0]) * ((m.g[0] - 1) * s[1] - (m.g[0] + 1) * rSL), (m.g[0] - 1) * rSL - (m.g[0] + 1) * s[1]) - m.pi[0];
@@ -430,9 +459,9 @@ __device__ __forceinline__ void riemann(const Mat<T> &m, const T *L, const T *R,
       T press = s[0] * s[6] + (1 - s[0]) * s[7];
       T rhoK = s[0] * s[1] + (1 - s[0]) * s[2];
       T V8;
-      if (m.hllcToro == 1) V8 = face_quot(SK - un, SK - S1) * (C8 + (S1 - un) * (rhoK * S1 + face_quot(press, SK - un)));
-      else V8 = face_quot(SK - un, SK - S1) * (C8 + (S1 - un) * (S1 + face_quot(press, rhoK * (SK - un))));
-      T V9 = face_quot(s[8] * (SK - un), SK - S1);
+      if (m.hllcToro == 1) V8 = dk(SK - un) * (C8 + (S1 - un) * (rhoK * S1 + face_quot(press, SK - un)));
+      else V8 = dk(SK - un) * (C8 + (S1 - un) * (S1 + face_quot(press, rhoK * (SK - un))));
+      T V9 = dk(s[8] * (SK - un));
       H1 = SK * (V1 - C1);
       H2 = SK * (V2 - C2);
       H3 = SK * (rS * unc0 - rho * s[3]);

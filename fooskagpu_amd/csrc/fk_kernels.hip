@@ -471,6 +471,26 @@ __device__ __forceinline__ void dt_lower(unsigned long long *__restrict__ slots,
   __hip_atomic_fetch_min(slots + (blockIdx.x % kDtSlots) * kDtStride, dt_key(fmin(kDtNone, d)), __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
 }
+// Minimum over a full wave (G = 4: the quads' lanes hold the same value), in
+// lane 63, by DPP moves: three instructions a step (by __shfl_xor the dt stage
+// of 3.07M cells took 8 us longer).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_min(double v) {
+  const int hi = __double2hiint(v), lo = __double2loint(v);
+  return fmin(v, __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xf, false),
+                                  __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xf, false)));
+}
+template <int G>
+__device__ __forceinline__ double wave_min63(double v) {
+  if constexpr (G == 1) {
+    v = dpp_min<0xb1, 0xf>(v);  // quad_perm: lane ^ 1, then lane ^ 2
+    v = dpp_min<0x4e, 0xf>(v);
+  }
+  v = dpp_min<0x141, 0xf>(v);  // row_half_mirror, row_mirror: rows of 16
+  v = dpp_min<0x140, 0xf>(v);
+  v = dpp_min<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3, 31 into 2 and 3
+  return dpp_min<0x143, 0xc>(v);
+}
 // by the 64 lanes of a wave: the smallest of a set, and the other set reset
 __device__ __forceinline__ double dt_fold(const unsigned long long *__restrict__ slots,
                                           unsigned long long *__restrict__ reset) {
@@ -506,18 +526,27 @@ __device__ __forceinline__ CellSide<T> cell_side(const fk::Mat<double> &md, cons
   return cs;
 }
 
+// First-order state of a cell as the viscous terms of boundary faces take it.
+template <int NEQ, typename T>
+__device__ __forceinline__ void wall_state(const fk::Mat<double> &md, const double *U, T (&W)[NEQ]) {
+  double w[NEQ];
+  fk::cons2prim<NEQ>(md, U, w);
+  if constexpr (NEQ == 5 && sizeof(T) == 4) w[4] -= md.pr;  // FP32 path: pressure as deviation from pRef
+#pragma unroll
+  for (int v = 0; v < NEQ; ++v) W[v] = (T)w[v];
+}
+
 // Terms of one face for one of its cells: adds the inviscid and
 // non-conservative terms to rhs, the viscous ones to rv, and (SIG) raises sig
 // to the face's signal speed.  L, R: face states (owner, neighbour or ghost);
 // Gc, Gn: velocity gradients of this cell and the neighbour; wls: WALE width
-// of the slot; Uc: this cell's conserved state in memory, read for the
-// first-order viscous ghost of a boundary face (formed there only: kept across
-// the faces it takes 20 registers of the FP64 kernels).
-template <int NEQ, typename T, bool VISC, bool HEAT, bool SIG>
+// of the slot; state1(W): this cell's first-order state, for the viscous ghost
+// of a boundary face.
+template <int NEQ, typename T, bool VISC, bool HEAT, bool SIG, typename F>
 __device__ __forceinline__ void face_terms(const fk_params &P, const fk::Mat<T> &mt, const CellSide<T> &cs, int nb,
                                            bool own, const T (&n)[3], T A, const T (&L)[NEQ], const T (&R)[NEQ],
-                                           const T *Gc, const T *Gn, const T *wls, const fk::Mat<double> &md,
-                                           const double *Uc, double (&rhs)[NEQ], double (&rv)[5], T &sig) {
+                                           const T *Gc, const T *Gn, const T *wls, const F &state1,
+                                           double (&rhs)[NEQ], double (&rv)[5], T &sig) {
   constexpr int iu = Model<NEQ>::iu;
   fk::FaceRes<T, NEQ> fr;
   fk::riemann<NEQ, SIG, T>(mt, L, R, n, nb == -5, fr);
@@ -574,12 +603,7 @@ __device__ __forceinline__ void face_terms(const fk_params &P, const fk::Mat<T> 
 #pragma unroll
       for (int v = 0; v < NEQ; ++v) R1[v] = R[v];
     } else {
-      double u[NEQ], w[NEQ];
-      fk::load_rec<NEQ>(Uc, u);
-      fk::cons2prim<NEQ>(md, u, w);
-      if constexpr (NEQ == 5 && sizeof(T) == 4) w[4] -= md.pr;  // FP32 path: pressure as deviation from pRef
-#pragma unroll
-      for (int v = 0; v < NEQ; ++v) R1[v] = (T)w[v];
+      state1(R1);
       fk::ghost<NEQ, T>(mt, -nb, n, R1);
     }
     T mu;
@@ -783,6 +807,22 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
   // viscous contributions are summed apart (rv) and added to the inviscid sums
   // after the face loop: the canonical order shared with the oracle
   double rv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  // The first-order state is held across the faces where the registers are
+  // there (two-phase FP32: dt stage of 3.07M cells 364 -> 359 us), else formed
+  // at the boundary face that needs it (FP32 single-phase 135 -> 125 us).
+  constexpr bool kHold = VISC && NEQ == 10 && sizeof(T) == 4;
+  T Wc1[kHold ? NEQ : 1];
+  if constexpr (kHold) wall_state<NEQ, T>(md, Uc, Wc1);
+  auto state1 = [&](T(&W)[NEQ]) {
+    if constexpr (kHold) {
+#pragma unroll
+      for (int v = 0; v < NEQ; ++v) W[v] = Wc1[v];
+    } else {
+      double u[NEQ];
+      fk::load_rec<NEQ>(U + c * NEQ, u);
+      wall_state<NEQ, T>(md, u, W);
+    }
+  };
   // slot links loaded up front and rotated, as in pass G (mixed 6.85 against
   // 7.12 ms for the fused pass, FP64 14.4 against 14.8 ms)
   int mq[NS];
@@ -822,7 +862,7 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
       fk::ghost<NEQ, T>(mt, -nb, n, R);
     }
     face_terms<NEQ, T, VISC, HEAT, MODE == 1>(P, mt, cs, nb, own, n, A, L, R, VISC ? grad_ptr(c) : nullptr,
-                                              VISC && nb >= 0 ? grad_ptr(nb) : nullptr, VISC ? wls + s : nullptr, md, U + c * NEQ, rhs, rv, sig);
+                                              VISC && nb >= 0 ? grad_ptr(nb) : nullptr, VISC ? wls + s : nullptr, state1, rhs, rv, sig);
   }
   if constexpr (VISC) {
 #pragma unroll
@@ -842,13 +882,12 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
     if constexpr (MODE == 1) {
       double d = volcfl[c] / (double)sig;
       dtc[c] = d;
-      const int l = threadIdx.x & 63;
-      const int64_t cw = c - l;  // lanes past the last cell are gone
-      for (int off = 1; off < 64; off <<= 1) {
-        const double o = __shfl_xor(d, off, 64);
-        if (cw + (l ^ off) < nc) d = fmin(d, o);
+      if ((c | 63) < nc) {
+        d = wave_min63<1>(d);
+        if ((threadIdx.x & 63) == 63) dt_lower(dtmin, d);
+      } else {
+        dt_lower(dtmin, d);  // the last wave, in part
       }
-      if (l == 0) dt_lower(dtmin, d);
     }
   } else {
     const double dt = dt_ptr ? *dt_ptr : dt_val;
@@ -1169,6 +1208,11 @@ __global__ void __launch_bounds__(64, (NS == 4 || sizeof(T) == 4 ? 3 : 2)) pass_
 #pragma unroll
   for (int v = 0; v < NEQ; ++v) rhs[v] = 0.0;
   T sig = (T)-1e9;
+  auto state1 = [&](T(&W)[NEQ]) {
+    double u[NEQ];
+    fk::load_rec<NEQ>(U + c * NEQ, u);
+    wall_state<NEQ, T>(md, u, W);
+  };
   // states of the RK stage; U again, not kept across the faces (20 registers)
   double u0[NEQ], Vc;
   auto stage_states = [&] {
@@ -1206,7 +1250,7 @@ __global__ void __launch_bounds__(64, (NS == 4 || sizeof(T) == 4 ? 3 : 2)) pass_
       if (nb < 0) fk::ghost<NEQ, T>(mt, -nb, n, Rt);
       face_terms<NEQ, T, VISC, HEAT, MODE == 1>(P, mt, cs, nb, own, n, ga.w, L, Rt, VISC ? gvel + c * NG : nullptr,
                                                 VISC && nb >= 0 ? gvel + (int64_t)nb * NG : nullptr,
-                                                VISC ? wls + s : nullptr, md, U + c * NEQ, fr, fv, sig);
+                                                VISC ? wls + s : nullptr, state1, fr, fv, sig);
     }
     if constexpr (MODE == 0 && R == 1) stage_states();  // on their way while the quad adds
 #pragma unroll
@@ -1239,8 +1283,8 @@ __global__ void __launch_bounds__(64, (NS == 4 || sizeof(T) == 4 ? 3 : 2)) pass_
     if constexpr (MODE == 1) {
       double d = volcfl[c] / (double)sig;
       if (q == 0) dtc[c] = d;
-      for (int off = 4; off < 64; off <<= 1) d = fmin(d, __shfl_xor(d, off, 64));
-      if (threadIdx.x == 0) dt_lower(dtmin, d);
+      d = wave_min63<4>(d);
+      if (threadIdx.x == 63) dt_lower(dtmin, d);
     }
   } else {
     const double dt = dt_ptr ? *dt_ptr : dt_val;
