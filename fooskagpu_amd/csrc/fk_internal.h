@@ -89,10 +89,11 @@ struct fk_ctx {
   // state health found by pass G: (step << 32) | cell, the smallest of the
   // cells with a non-positive density or a non-finite primitive; ~0 if none
   unsigned long long *health = nullptr;
-  // two sets of minima of Vcfl / signal: the last dt stage's, and which are reset
+  // two sets of minima of Vcfl / signal: the last dt stage's (dt_set) and the
+  // next one's, which that stage has reset (dt_ready: there was one)
   unsigned long long *dtw = nullptr;
   int dt_set = 0;
-  bool dt_clean[2] = {false, false};
+  bool dt_ready = false;
   double *hres = nullptr;    // page-locked results that kernels write for the host, 64 doubles
   unsigned long long hseq = 0;  // number of the last result asked for
   double *dgrad = nullptr, *dtheta = nullptr;

@@ -455,8 +455,8 @@ __global__ void __launch_bounds__(kBlock, (sizeof(T) == 8 ? 2 : 1))
 // of their own as keys whose unsigned order is the order of the doubles: each
 // wave of pass F lowers one of them (64 words: an atomic on one address
 // retires in about 12 ns), the update or dt_final folds the 64.  The order of
-// the waves does not matter to a minimum.  Two sets in turn: who folds one
-// resets the other.  Before, pass F's array was read by two more kernels, 13
+// the waves does not matter to a minimum.  Two sets in turn: a dt stage resets
+// the one that it does not use, which the next one takes.  Before, pass F's array was read by two more kernels, 13
 // us a step at 1M cells, or its quads' minima folded by one of 8.5 us.
 constexpr int kDtSlots = 64, kDtStride = 16;
 constexpr double kDtNone = 1e15;
@@ -491,18 +491,16 @@ __device__ __forceinline__ double wave_min63(double v) {
   v = dpp_min<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3, 31 into 2 and 3
   return dpp_min<0x143, 0xc>(v);
 }
-// by the 64 lanes of a wave: the smallest of a set, and the other set reset
-__device__ __forceinline__ double dt_fold(const unsigned long long *__restrict__ slots,
-                                          unsigned long long *__restrict__ reset) {
-  const int l = threadIdx.x & 63;
-  double m = dt_unkey(slots[l * kDtStride]);
+// by the 64 lanes of a wave: the smallest of a set
+__device__ __forceinline__ double dt_fold(const unsigned long long *__restrict__ slots) {
+  double m = dt_unkey(slots[(threadIdx.x & 63) * kDtStride]);
   for (int off = 1; off < 64; off <<= 1) m = fmin(m, __shfl_xor(m, off, 64));
-  if (reset) reset[l * kDtStride] = dt_key(kDtNone);
   return m;
 }
-__global__ void __launch_bounds__(64) dt_reset(unsigned long long *__restrict__ slots) {
-  slots[threadIdx.x * kDtStride] = dt_key(kDtNone);
+__device__ __forceinline__ void dt_reset(unsigned long long *__restrict__ slots) {
+  if (blockIdx.x == 0 && threadIdx.x < kDtSlots) slots[threadIdx.x * kDtStride] = dt_key(kDtNone);
 }
+__global__ void __launch_bounds__(64) dt_reset_k(unsigned long long *__restrict__ slots) { dt_reset(slots); }
 
 // Side terms of a cell (fluxSource / computeCenterPress, two-phase).
 template <typename T>
@@ -706,6 +704,7 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
                                                  double dt_val, const double *__restrict__ dt_ptr,
                                                  float *__restrict__ Wout, double *__restrict__ clock,
                                                  unsigned long long *__restrict__ dtmin,
+                                                 unsigned long long *__restrict__ dtnext,
                                                  uint32_t *__restrict__ rlist,
                                                  unsigned long long *__restrict__ rcnt,
                                                  unsigned long long *__restrict__ rpart) {
@@ -713,6 +712,7 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
   constexpr int KR = RLX == 2 ? 3 : 2;  // counts per wave in rpart
   constexpr int NGS = ngrad<NEQ, HEAT>();
   constexpr int BS = pass_f_block<T, STAGE, NS>();
+  if constexpr (MODE == 1) dt_reset(dtnext);
   const int64_t c0 = xcd_block() * BS;
   const int64_t c = c0 + threadIdx.x;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
@@ -1182,10 +1182,12 @@ __global__ void __launch_bounds__(64, (NS == 4 || sizeof(T) == 4 ? 3 : 2)) pass_
                                                const double *__restrict__ dt_ptr, float *__restrict__ Wout,
                                                double *__restrict__ clock,
                                                unsigned long long *__restrict__ dtmin,
+                                               unsigned long long *__restrict__ dtnext,
                                                uint32_t *__restrict__ rlist, unsigned long long *__restrict__ rcnt,
                                                unsigned long long *__restrict__ rpart) {
   static_assert(!RLX || (MODE == 0 && NEQ == 10), "fused relaxation: two-phase RK stage only");
   constexpr int R = (NS + 3) / 4, NG = ngrad<NEQ, HEAT>(), iu = Model<NEQ>::iu;
+  if constexpr (MODE == 1) dt_reset(dtnext);
   const int64_t blk = xcd_block();
   const int q = threadIdx.x & 3;
   if (blk * 16 >= nc) {  // a wave without cells still stores its counts
@@ -1318,7 +1320,7 @@ __global__ void __launch_bounds__(64, (NS == 4 || sizeof(T) == 4 ? 3 : 2)) pass_
 }
 
 // dt of the update kernels, slots: each block folds the set for itself; block
-// 0 stores dt and resets the other set.  Up to kDtFold blocks: 83k cells (3240
+// 0 stores dt.  Up to kDtFold blocks: 83k cells (3240
 // blocks) 155.2 us a step against 156.2 with dt_final ahead, mixed 3.07M cells
 // (12,000) 2275 against 2278; FP64 1.05M cells (41,160 short blocks) 1502
 // against 1498.
@@ -1328,7 +1330,6 @@ struct DtSource {
   double val;             // the dt, unless ptr or slots says otherwise
   const double *ptr;
   const unsigned long long *slots;
-  unsigned long long *reset;
   double cfl, maxDt;
   double *scal;           // [dt, time]
   int clock;
@@ -1338,7 +1339,7 @@ __device__ __forceinline__ double dt_of(const DtSource &s) {
   if (s.slots) {
     __shared__ double sh;
     if (threadIdx.x < 64) {
-      const double m = dt_fold(s.slots, blockIdx.x == 0 ? s.reset : nullptr);
+      const double m = dt_fold(s.slots);
       if (threadIdx.x == 0) sh = fmin(s.cfl * m, s.maxDt);
     }
     __syncthreads();
@@ -1436,11 +1437,10 @@ __device__ __forceinline__ void publish(double *host, unsigned long long seq) {
 }
 
 // dt = min(cfl * min, maxDt) from a set of pass F's minima, by one wave.
-__global__ void __launch_bounds__(64) dt_final(const unsigned long long *__restrict__ slots,
-                                               unsigned long long *__restrict__ reset, double cfl, double maxDt,
+__global__ void __launch_bounds__(64) dt_final(const unsigned long long *__restrict__ slots, double cfl, double maxDt,
                                                double *__restrict__ scal, double *__restrict__ host,
                                                unsigned long long seq) {
-  const double dt = fmin(cfl * dt_fold(slots, reset), maxDt);
+  const double dt = fmin(cfl * dt_fold(slots), maxDt);
   if (threadIdx.x == 0) {
     scal[0] = dt;
     if (host) host[0] = dt;  // fk_compute_time_step
@@ -1817,17 +1817,18 @@ int launch_pass_f_t(fk_ctx *c, int irk, double dt, const double *dtp, double *Un
   c->pf_waves = (int64_t)(stage ? (int64_t)gs * (bs / 64) : (int64_t)gr * (kBlock / 64));
   const bool quad = quad_f(c, relax);
   if (quad) c->pf_waves = grid_quad(c->nc);
-  unsigned long long *dtmin = nullptr;
-  if (MODE == 1) {  // the other of the two sets of minima; a fold of this one resets it again
+  unsigned long long *dtmin = nullptr, *dtnext = nullptr;
+  if (MODE == 1) {  // the set of minima that the last dt stage reset
     c->dt_set ^= 1;
     dtmin = dt_slots(c, c->dt_set);
-    if (!c->dt_clean[c->dt_set])
-      LAUNCH_TIMED(c, "zero", hipLaunchKernelGGL(dt_reset, dim3(1), dim3(kDtSlots), 0, c->stream, dtmin));
-    c->dt_clean[c->dt_set] = false;
+    dtnext = dt_slots(c, c->dt_set ^ 1);
+    if (!c->dt_ready)
+      LAUNCH_TIMED(c, "zero", hipLaunchKernelGGL(dt_reset_k, dim3(1), dim3(kDtSlots), 0, c->stream, dtmin));
+    c->dt_ready = true;
   }
 #define PF_ARGS(W) \
   c->p, c->nc, U, U0, Unew, c->link, c->geo, wl, c->vol, c->volcfl, face, gv, c->rhs, c->dtc, irk, dt, dtp, W, clock,       \
-      dtmin
+      dtmin, dtnext
 #define PFQ(NEQ, VISC, HEAT, WO, RX, NAME, W, LIST, CNT, PART)                                                         \
   LAUNCH_TIMED(c, NAME,                                                                                                \
                hipLaunchKernelGGL((pass_f_q<NEQ, T, VISC, HEAT, MODE, NS, WO, RX>), dim3(grid_quad(c->nc)), dim3(64), 0, \
@@ -1980,7 +1981,7 @@ int do_pass_f_update(fk_ctx *c, int irk, double dt, const double *dtp, bool want
 
 // dt as given (val), or from the device (ptr)
 DtSource dt_source(const fk_ctx *c, double val, const double *ptr, double *clock) {
-  return DtSource{val, ptr, nullptr, nullptr, c->p.cfl, c->p.maxDt, c->dscal, clock != nullptr};
+  return DtSource{val, ptr, nullptr, c->p.cfl, c->p.maxDt, c->dscal, clock != nullptr};
 }
 
 // RK stage from the stored residual (FP32 after the mixed dt stage, c->rhs_f32)
@@ -2031,9 +2032,7 @@ int wait_result(fk_ctx *c) {
 // dt of the last pass F MODE 1 into dscal[0] (and host[0])
 int do_dt_device(fk_ctx *c, double *host) {
   LAUNCH_TIMED(c, "dt_final", hipLaunchKernelGGL(dt_final, dim3(1), dim3(64), 0, c->stream, dt_slots(c, c->dt_set),
-                                                 dt_slots(c, c->dt_set ^ 1), c->p.cfl, c->p.maxDt, c->dscal, host,
-                                                 host ? ++c->hseq : 0ull));
-  c->dt_clean[c->dt_set ^ 1] = true;
+                                                 c->p.cfl, c->p.maxDt, c->dscal, host, host ? ++c->hseq : 0ull));
   return FK_OK;
 }
 
@@ -2044,10 +2043,7 @@ int do_dt_update(fk_ctx *c, int irk, bool want_w, double *clock) {
   if ((int64_t)grid_for(w ? c->nc : c->nc * c->neq) <= kDtFold) {
     ds.ptr = nullptr;
     ds.slots = dt_slots(c, c->dt_set);
-    ds.reset = dt_slots(c, c->dt_set ^ 1);
-    int rc = do_update(c, irk, ds, want_w);
-    if (!rc) c->dt_clean[c->dt_set ^ 1] = true;
-    return rc;
+    return do_update(c, irk, ds, want_w);
   }
   int rc = do_dt_device(c, nullptr);
   if (rc) return rc;
@@ -2427,7 +2423,7 @@ int fk_upload_mesh(fk_ctx *c, int64_t nElem, int64_t nFcs, const int32_t *fc2el,
   HIPCHK(hipMalloc(&c->dtc, cs * 8));
   HIPCHK(hipMalloc(&c->red, 4096 * 8));
   HIPCHK(hipMalloc(&c->dtw, 2 * kDtSlots * kDtStride * 8));
-  c->dt_clean[0] = c->dt_clean[1] = false;
+  c->dt_ready = false;
   HIPCHK(hipMalloc(&c->dscal, 16 * 8));
   HIPCHK(hipMalloc(&c->lcount, 16 * 8));
   HIPCHK(hipMalloc(&c->wprim, cs * neq * sizeof(float)));
