@@ -75,12 +75,12 @@ def kernel_bytes(name, B, neq, mixed=True):
 
 # Entries of the counter summary for the kernels a timed run launches: the
 # mixed fused stage writes primitive records (pass_f_w); the FP64 entries
-# carry the fp64_ prefix and its last stage runs the plain relaxation.
+# carry the fp64_ prefix, the plain relaxation a kernel of its own there.
 TRAFFIC_NAMES = {
     "mixed_mlp": {"pass_g": "pass_g", "pass_f_rhs": "pass_f_rhs", "pass_f": "pass_f_w",
                   "pass_f_relax": "pass_f_relax", "rk_update": "rk_update"},
     "fp64": {"pass_g": "fp64_pass_g", "pass_f_rhs": "fp64_pass_f_rhs", "pass_f": "fp64_pass_f",
-             "pass_f_relax": "fp64_pass_f_relax_plain", "rk_update": "fp64_rk_update"},
+             "rk_update": "fp64_rk_update", "relax": "fp64_relax"},
 }
 
 

@@ -976,7 +976,8 @@ __global__ void __launch_bounds__((pass_f_block<T, STAGE, NS>()), ((MODE == 1 ||
 // then the quad adds the faces' terms in slot order.  Every term is formed by
 // the operations of pass_g / pass_f and added in the same order, so the
 // results are the same bits.  Own-cell work is repeated on the four lanes, so
-// that the kernels lose once the chip is full (quad_cells_g, quad_cells_f).
+// that pass G and the FP32 pass F lose once the chip is full (quad_cells_g,
+// quad_cells_f).
 // Sod 12k cells: pass G 10 -> 7 us, pass F 10 -> 6; bubble 83k: pass F 29 -> 21,
 // with the plain relaxation 64 -> 53.
 
@@ -1689,9 +1690,11 @@ inline unsigned long long *dt_slots(const fk_ctx *c, int set) { return c->dtw + 
 //   pass G  FP64 12 / 13 at 55k cells (single-phase), 16 / 19 at 48k and 23 / 21 at
 //           83k (two-phase); FP32 10 / 11 at 48k, 16 / 13 at 94k; 6 slots FP64
 //           21 / 23 at 27k, 33 / 26 at 55k; FP32 9 / 12 at 8k, 13 / 12 at 27k
-//   pass F  FP64 20 / 29 at 83k, 48 / 72 at 280k, 297 / 306 (residual 292 / 325)
-//           at 1.05M, 857 / 846 (832 / 905) at 3.1M: its one-lane kernel runs
-//           2 waves per SIMD; FP32 53 / 56 at 280k, 100 / 90 at 511k (two-phase),
+//   pass F  FP64 at every size (three waves per SIMD against two): two-phase 20 /
+//           29 at 83k, 733 / 773 (dt stage 689 / 772) at 3.1M, 1874 / 1997
+//           (1747 / 1987) at 8M, 3816 / 4146 (3599 / 4109) at 16M; single-phase
+//           1133 / 1190 (1054 / 1157) at 6.9M; 6 slots 583 / 653 at 1.3M, 2458 /
+//           2760 at 5.8M; FP32 53 / 56 at 280k, 100 / 90 at 511k (two-phase),
 //           51 / 59 at 511k, 178 / 160 at 1.6M (single-phase); 6 slots FP32
 //           28 / 29 at 55k, 63 / 60 at 176k
 //   with the relaxation (on the quad only the plain solve's residuals go in
@@ -1708,7 +1711,7 @@ inline int64_t quad_cells_f(const fk_ctx *c, int relax) {
     if (c->ns == 6) return 35000;
     return f64 ? 220000 : (relax == 2 ? 160000 : 50000);
   }
-  if (f64) return 4000000;
+  if (f64) return INT64_MAX;
   return c->ns == 6 ? 120000 : (c->neq == 5 ? 600000 : 350000);
 }
 inline bool quad_g(const fk_ctx *c) { return c->stage_g == 1 && c->nc <= quad_cells_g(c); }

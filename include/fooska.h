@@ -212,7 +212,8 @@ int fk_set_debug(fk_ctx *ctx, int on);
  *     mixed: 7.5 ms against 6.7 + 2.5 ms.  0 = always residual + update
  *     kernel.
  *  "stage_f" (default 1): pass F by the size of the mesh: four lanes per cell
- *     on small meshes (FP64 up to 4M cells), else one lane per cell with the
+ *     on small meshes and in FP64 (but for the last stage with the
+ *     relaxation), else one lane per cell with the
  *     face states and velocity gradients of its workgroup's cells in LDS, in-
  *     workgroup mirror states read from there (4 slots per cell: 256 cells,
  *     FP64 128; 6 slots: two-phase FP32, 128 cells, not in the last stage's
