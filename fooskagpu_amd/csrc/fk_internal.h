@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../include/fooska.h"
+#include "fk_plan.h"
 
 namespace fkx {
 
@@ -16,8 +17,6 @@ inline int fail(int code, const std::string &m) {
   g_err = m;
   return code;
 }
-
-constexpr int kBlock = 256;
 
 template <typename T>
 struct V4 {
@@ -109,7 +108,7 @@ struct fk_ctx {
   uint32_t *rfall = nullptr;   // surrogate relaxation: cells whose polish failed
   void *rstart = nullptr;      // surrogate relaxation: network starts (float2) of the chemical entries
   int64_t rstart_cap = 0;
-  unsigned long long *rpart = nullptr;  // per-workgroup relaxation counts [blocks][4]
+  unsigned long long *rpart = nullptr;  // per-workgroup or per-wave relaxation counts (relax_words)
   int64_t rlist_cap = 0;
   double dt = 0, time = 0;
   int64_t step = 0;

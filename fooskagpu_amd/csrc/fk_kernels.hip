@@ -102,7 +102,6 @@ constexpr int ngrad() {
 // L2).  Remap so that XCD x processes the contiguous block range
 // [x G/8, (x+1) G/8): neighbouring cells (close in the mesh order) then share
 // an L2.  G is a multiple of 8 (padded by grid_xcd).
-constexpr int kXcd = 8;
 __device__ __forceinline__ int64_t xcd_block() {
   const int64_t b = blockIdx.x, per = gridDim.x / kXcd;
   return (b % kXcd) * per + b / kXcd;
@@ -1610,9 +1609,6 @@ __global__ void __launch_bounds__(kBlock) accum_counts(const unsigned long long 
 // host helpers
 // ------------------------------------------------------------------------
 
-inline unsigned grid_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
-// grid of the XCD-remapped kernels: a multiple of 8 blocks
-inline unsigned grid_xcd(int64_t n) { return (grid_for(n) + kXcd - 1) / kXcd * kXcd; }
 inline size_t tsz(const fk_ctx *c) { return c->p.precision == FK_MIXED ? 4 : 8; }
 inline int ng_of(const fk_ctx *c) { return 9 + ((c->p.model == FK_MODEL_SINGLE && c->p.heatFlux == 1) ? 3 : 0); }
 
@@ -1682,41 +1678,12 @@ void free_all(fk_ctx *c) {
 
 inline unsigned long long *dt_slots(const fk_ctx *c, int set) { return c->dtw + set * kDtSlots * kDtStride; }
 
-// Cells up to which pass G and pass F run four lanes per cell (pass_g_q,
-// pass_f_q) rather than one with the LDS paths.  What the quads win is waves
-// in flight and shorter chains; what they lose is the own-cell work on four
-// lanes and, with records of half the size (FP32), pass F's LDS reuse.  us,
-// quads / one lane, on either side of the lines:
-//   pass G  FP64 12 / 13 at 55k cells (single-phase), 16 / 19 at 48k and 23 / 21 at
-//           83k (two-phase); FP32 10 / 11 at 48k, 16 / 13 at 94k; 6 slots FP64
-//           21 / 23 at 27k, 33 / 26 at 55k; FP32 9 / 12 at 8k, 13 / 12 at 27k
-//   pass F  FP64 at every size (three waves per SIMD against two): two-phase 20 /
-//           29 at 83k, 733 / 773 (dt stage 689 / 772) at 3.1M, 1874 / 1997
-//           (1747 / 1987) at 8M, 3816 / 4146 (3599 / 4109) at 16M; single-phase
-//           1133 / 1190 (1054 / 1157) at 6.9M; 6 slots 583 / 653 at 1.3M, 2458 /
-//           2760 at 5.8M; FP32 53 / 56 at 280k, 100 / 90 at 511k (two-phase),
-//           51 / 59 at 511k, 178 / 160 at 1.6M (single-phase); 6 slots FP32
-//           28 / 29 at 55k, 63 / 60 at 176k
-//   with the relaxation (on the quad only the plain solve's residuals go in
-//           parallel) FP64 64 / 70 at 162k, 106 / 103 at 280k; FP32 22 / 22 at 48k,
-//           34 / 31 at 94k, plain 81 / 85 at 162k; 6 slots FP64 26 / 31 at 27k,
-//           65 / 53 at 55k; FP32 22 / 26 at 27k, 48 / 40 at 85k
-inline int64_t quad_cells_g(const fk_ctx *c) {
-  if (c->ns == 6) return c->p.precision == FK_FP64 ? 40000 : 20000;
-  return 60000;
+inline bool quad_g(const fk_ctx *c) {
+  return c->stage_g == 1 && c->nc <= quad_cells_g(c->p.precision == FK_FP64, c->ns);
 }
-inline int64_t quad_cells_f(const fk_ctx *c, int relax) {
-  const bool f64 = c->p.precision == FK_FP64;
-  if (relax) {
-    if (c->ns == 6) return 35000;
-    return f64 ? 220000 : (relax == 2 ? 160000 : 50000);
-  }
-  if (f64) return INT64_MAX;
-  return c->ns == 6 ? 120000 : (c->neq == 5 ? 600000 : 350000);
+inline bool quad_f(const fk_ctx *c, int relax) {
+  return c->stage_f == 1 && c->nc <= quad_cells_f(c->p.precision == FK_FP64, c->ns, c->neq, relax);
 }
-inline bool quad_g(const fk_ctx *c) { return c->stage_g == 1 && c->nc <= quad_cells_g(c); }
-inline bool quad_f(const fk_ctx *c, int relax) { return c->stage_f == 1 && c->nc <= quad_cells_f(c, relax); }
-inline unsigned grid_quad(int64_t nc) { return (unsigned)((nc + 16 * kXcd - 1) / (16 * kXcd) * kXcd); }
 
 // Whether the last pass F also runs the relaxation's per-cell pass (kind 1
 // surrogate, 2 plain).  It saves reading the state back, but runs the solve at
@@ -1744,7 +1711,7 @@ int launch_pass_g_t(fk_ctx *c) {
   // face records through LDS (workgroup sizes: pass_g_block)
   const bool sout = c->stage_g;
   constexpr int gbs = pass_g_block<T, NS, true>();
-  const unsigned grs = (unsigned)(((c->nc + gbs - 1) / gbs + kXcd - 1) / kXcd * kXcd);
+  const unsigned grs = grid_blocks(c->nc, gbs);
 #define PG3(NEQ, VISC, HEAT, FW, SO)                                                                                  \
   LAUNCH_TIMED(c, "pass_g",                                                                                          \
                hipLaunchKernelGGL((pass_g<NEQ, T, VISC, HEAT, FW, NS, SO>), dim3(SO ? grs : gr),                      \
@@ -1814,12 +1781,11 @@ int launch_pass_f_t(fk_ctx *c, int irk, double dt, const double *dtp, double *Un
   const bool stage = c->stage_f && (NS == 4 || relax == 0) &&
                      (c->neq == 10 ? pass_f_stage_ok<T, NS, 10>() : pass_f_stage_ok<T, NS, 5>());
   constexpr int bs = pass_f_block<T, true, NS>();
-  const unsigned gs = (unsigned)(((c->nc + bs - 1) / bs + kXcd - 1) / kXcd * kXcd);
+  const unsigned gs = grid_blocks(c->nc, bs);
   const size_t lds = stage ? (size_t)bs * (NS * c->neq + (NS == 4 ? 12 : 0)) * sizeof(T) : 0;
   // waves of this launch (per-wave relaxation counts of the fused last stage)
-  c->pf_waves = (int64_t)(stage ? (int64_t)gs * (bs / 64) : (int64_t)gr * (kBlock / 64));
   const bool quad = quad_f(c, relax);
-  if (quad) c->pf_waves = grid_quad(c->nc);
+  c->pf_waves = quad ? grid_quad(c->nc) : pass_f_waves(c->nc, stage ? bs : kBlock);
   unsigned long long *dtmin = nullptr, *dtnext = nullptr;
   if (MODE == 1) {  // the set of minima that the last dt stage reset
     c->dt_set ^= 1;
@@ -2102,11 +2068,7 @@ int ensure_rlist(fk_ctx *c) {
   c->rlist_cap = 0;
   HIPCHK(hipMalloc(&c->rlist, (size_t)c->nc * sizeof(uint32_t)));
   HIPCHK(hipMalloc(&c->rfall, (size_t)c->nc * sizeof(uint32_t)));
-  // [blocks][4] partials of the relaxation kernels, or [waves][2 or 3] of the
-  // fused pass F (grid_xcd blocks of 4 waves, or one wave for 16 cells)
-  size_t parts = (size_t)grid_xcd(c->nc) * 12;
-  if (c->nc <= std::max(quad_cells_f(c, 1), quad_cells_f(c, 2))) parts = std::max(parts, (size_t)grid_quad(c->nc) * 3);
-  HIPCHK(hipMalloc(&c->rpart, parts * sizeof(unsigned long long)));
+  HIPCHK(hipMalloc(&c->rpart, (size_t)relax_words(c->nc, c->ns) * sizeof(unsigned long long)));
   c->rlist_cap = c->nc;
   return FK_OK;
 }
