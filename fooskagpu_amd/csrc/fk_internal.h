@@ -23,6 +23,9 @@ struct V4 {
   T x, y, z, w;
 };
 
+// Page-locked memory that a running kernel and the host both use.
+constexpr unsigned kHostCoherent = hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent;
+
 struct Timer {
   std::vector<std::string> names;
   std::vector<int64_t> counts;

@@ -1433,7 +1433,9 @@ __global__ void __launch_bounds__(kBlock) rk_update_w(fk_params P, int64_t nc, c
 constexpr int kHostSeq = 63;
 __device__ __forceinline__ void publish(double *host, unsigned long long seq) {
   __threadfence_system();
-  if (threadIdx.x == 0) reinterpret_cast<volatile unsigned long long *>(host)[kHostSeq] = seq;
+  if (threadIdx.x == 0)
+    __hip_atomic_store(reinterpret_cast<unsigned long long *>(host) + kHostSeq, seq, __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // dt = min(cfl * min, maxDt) from a set of pass F's minima, by one wave.
@@ -1986,15 +1988,14 @@ int do_update(fk_ctx *c, int irk, const DtSource &ds, bool want_w) {
 // about 20 us on top of the kernels; the result is polled for instead, up to
 // 2 ms, and then left to the synchronisation (which also reports errors).
 int wait_result(fk_ctx *c) {
-  const volatile unsigned long long *seq = reinterpret_cast<const volatile unsigned long long *>(c->hres) + kHostSeq;
+  const unsigned long long *seq = reinterpret_cast<const unsigned long long *>(c->hres) + kHostSeq;
   const auto t0 = std::chrono::steady_clock::now();
-  while (*seq != c->hseq) {
+  while (__atomic_load_n(seq, __ATOMIC_ACQUIRE) != c->hseq) {
     if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
       HIPCHK(hipStreamSynchronize(c->stream));
       return FK_OK;
     }
   }
-  std::atomic_thread_fence(std::memory_order_acquire);
   return FK_OK;
 }
 
@@ -2237,7 +2238,7 @@ int fk_create(int device, const fk_params *p, fk_ctx **out) {
     delete c;
     return fail(FK_EDEVICE, std::string("hipStreamCreate: ") + hipGetErrorString(e));
   }
-  e = hipHostMalloc(reinterpret_cast<void **>(&c->hres), 64 * sizeof(double), hipHostMallocDefault);
+  e = hipHostMalloc(reinterpret_cast<void **>(&c->hres), 64 * sizeof(double), kHostCoherent);
   if (e != hipSuccess) {
     (void)hipStreamDestroy(c->stream);
     delete c;

@@ -32,6 +32,8 @@ constexpr size_t kXferMinDown = (size_t)5 << 20, kXferMinUp = (size_t)16 << 20;
 // costs about 2 ms, which each new context would otherwise pay in its first
 // copy): allocated by the first large copy, freed with the last context, and
 // lent to one copy at a time.  A copy that finds them lent is one hipMemcpy.
+// Coherent memory, asked for: the host takes a slot while later kernels of the
+// stream run, and refills one for a later kernel without a synchronisation.
 constexpr size_t kXferSlot = (size_t)4 << 20;
 constexpr int kXferSlots = 2 * kXferThreads;
 struct XferPool {
@@ -41,8 +43,8 @@ struct XferPool {
   bool lent = false;
   std::atomic<unsigned long long> seq{0};
 
-  volatile unsigned long long *report(int slot) {
-    return reinterpret_cast<volatile unsigned long long *>(pin + kXferSlots * kXferSlot) + 8 * slot;
+  unsigned long long *report(int slot) {
+    return reinterpret_cast<unsigned long long *>(pin + kXferSlots * kXferSlot) + 8 * slot;
   }
   void attach() {
     std::lock_guard<std::mutex> lk(mu);
@@ -59,7 +61,7 @@ struct XferPool {
     if (lent) return nullptr;
     if (!pin) {
       void *p = nullptr;
-      if (hipHostMalloc(&p, kXferSlots * (kXferSlot + 64), hipHostMallocPortable) != hipSuccess) {
+      if (hipHostMalloc(&p, kXferSlots * (kXferSlot + 64), kHostCoherent) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
       }
@@ -77,13 +79,13 @@ struct XferPool {
 inline XferPool g_xfer;
 
 // n16 16-byte words and `tail` bytes after them from a to b, one of them a
-// slot.  The block that ends last writes seq to *report, host memory, behind a
-// system-wide fence of every block, and leaves *count at zero.
+// slot.  The block that ends last releases seq to *report, host memory, behind
+// a system-wide fence of every block, and leaves *count at zero.
 typedef unsigned int xfer_u4 __attribute__((ext_vector_type(4)));
 constexpr unsigned kXferBlocks = 64;
 static __global__ void __launch_bounds__(256) xfer_copy(const char *__restrict__ a, char *__restrict__ b, size_t n16,
                                                         int tail, unsigned *__restrict__ count,
-                                                        volatile unsigned long long *__restrict__ report,
+                                                        unsigned long long *__restrict__ report,
                                                         unsigned long long seq) {
   const xfer_u4 *src = reinterpret_cast<const xfer_u4 *>(a);
   xfer_u4 *dst = reinterpret_cast<xfer_u4 *>(b);
@@ -95,7 +97,7 @@ static __global__ void __launch_bounds__(256) xfer_copy(const char *__restrict__
   if (atomicAdd(count, 1u) == kXferBlocks - 1) {
     *count = 0;
     __threadfence_system();
-    *report = seq;
+    __hip_atomic_store(report, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -148,10 +150,9 @@ struct XferJob {
   // waits for a report; after 2 s (or an error elsewhere) for the stream
   bool wait(int s, unsigned long long seq) {
     const auto t0 = std::chrono::steady_clock::now();
-    for (int k = 0; *g_xfer.report(s) != seq; ++k)
+    for (int k = 0; __atomic_load_n(g_xfer.report(s), __ATOMIC_ACQUIRE) != seq; ++k)
       if ((k & 1023) == 1023 && (err.load() || std::chrono::steady_clock::now() - t0 > std::chrono::seconds(2)))
         return !bad(hipStreamSynchronize(c->stream));
-    std::atomic_thread_fence(std::memory_order_acquire);
     return true;
   }
   void work(int t) {
