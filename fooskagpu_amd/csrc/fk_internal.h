@@ -43,6 +43,7 @@ struct Timer {
 constexpr int kXferThreads = 8;
 struct Xfer {
   unsigned *count = nullptr;
+  bool clear = false;  // count is zero but for a copy under way
 };
 
 // Surrogate (MLP 3-64-64-64-3) state of a context.

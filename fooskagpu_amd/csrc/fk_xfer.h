@@ -101,19 +101,33 @@ static __global__ void __launch_bounds__(256) xfer_copy(const char *__restrict__
   }
 }
 
+static __global__ void __launch_bounds__(64) xfer_clear(unsigned *__restrict__ count) {
+  if ((int)threadIdx.x < kXferSlots) count[threadIdx.x] = 0;
+}
+
 // The slots for a copy of context c, or null: then the copy is one hipMemcpy.
+// The counts are cleared on the context's stream, which is not ordered with the
+// null stream, and again after a copy that failed.
 inline char *xfer_begin(fk_ctx *c) {
   if (!c->xfer.count) {
     unsigned *p = nullptr;
-    if (hipMalloc(&p, kXferSlots * sizeof(unsigned)) != hipSuccess ||
-        hipMemset(p, 0, kXferSlots * sizeof(unsigned)) != hipSuccess) {
+    if (hipMalloc(&p, kXferSlots * sizeof(unsigned)) != hipSuccess) {
       (void)hipGetLastError();
-      if (p) (void)hipFree(p);
       return nullptr;
     }
     c->xfer.count = p;
+    c->xfer.clear = false;
   }
-  return g_xfer.borrow();
+  char *pin = g_xfer.borrow();
+  if (pin && !c->xfer.clear) {
+    hipLaunchKernelGGL(xfer_clear, dim3(1), dim3(64), 0, c->stream, c->xfer.count);
+    if (hipGetLastError() != hipSuccess) {
+      g_xfer.give_back();
+      return nullptr;
+    }
+    c->xfer.clear = true;
+  }
+  return pin;
 }
 
 inline void xfer_free(fk_ctx *c) {
@@ -201,6 +215,7 @@ inline int xfer_staged(fk_ctx *c, char *pin, void *dev, void *host, size_t bytes
     if (t.joinable()) t.join();
   const hipError_t e = hipStreamSynchronize(c->stream);  // also after an error: nothing uses the slots any more
   g_xfer.give_back();
+  c->xfer.clear = !job.err.load() && e == hipSuccess;
   if (job.err.load()) return fail(FK_EDEVICE, std::string("copy: ") + hipGetErrorString((hipError_t)job.err.load()));
   if (e != hipSuccess) return fail(FK_EDEVICE, std::string("copy: ") + hipGetErrorString(e));
   return FK_OK;

@@ -85,7 +85,9 @@ inline hipError_t hipMemset(void *p, int v, size_t n) {
 }
 inline hipError_t hipMemcpy(void *d, const void *s, size_t n, int) { ++g_memcpys; memcpy(d, s, n); return hipSuccess; }
 inline hipError_t hipStreamSynchronize(hipStream_t s) { s->wait(); return hipSuccess; }
-inline hipError_t hipGetLastError() { return hipSuccess; }
+inline std::atomic<int> g_fail_launches{0};  // that many launches fail from now on
+inline thread_local hipError_t g_last = hipSuccess;
+inline hipError_t hipGetLastError() { hipError_t e = g_last; g_last = hipSuccess; return e; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline const char *hipGetErrorString(hipError_t) { return ""; }
 inline hipError_t hipEventCreate(hipEvent_t *) { return hipSuccess; }
@@ -101,6 +103,10 @@ inline unsigned atomicAdd(unsigned *p, unsigned v) { return __atomic_fetch_add(p
 // barrier when the others have reached it
 template <typename K, typename... A>
 inline void mock_launch(K k, unsigned grid, unsigned block, hipStream_t s, A... a) {
+  if (g_fail_launches.load() > 0 && g_fail_launches.fetch_sub(1) > 0) {
+    g_last = 1;
+    return;
+  }
   s->push([=] {
     for (unsigned b = 0; b < grid; ++b) {
       for (unsigned t = block; t-- > 0;) {
@@ -180,4 +186,43 @@ def test_slots_are_coherent_memory(run):
   say(copy_down(c, out.data(), dev, n) == FK_OK && out == in, "download");
   say(g_memcpys == 0, "through the slots");
   say((g_pin_flags & hipHostMallocCoherent) && (g_pin_flags & hipHostMallocPortable), "coherent slots");
+""")
+
+
+@pytest.mark.parametrize("stale", [1, 40, 0xabababab])
+def test_block_counts_are_cleared_before_the_first_piece(run, stale):
+    """The counters of a context's copies start in memory that held something
+    else; a count that starts above zero reports a piece before all of its
+    blocks have run, garbage never reports it."""
+    run(f"""
+  g_stale = {stale}u;
+  const size_t n = (size_t)40 << 20;
+  char *dev = device(n);
+  std::vector<char> in = pattern(n, 2), out(n);
+  const auto t0 = std::chrono::steady_clock::now();
+  for (unsigned k = 0; k < 3; ++k) {{
+    in = pattern(n, k);
+    say(copy_up(c, dev, in.data(), n) == FK_OK && std::memcmp(dev, in.data(), n) == 0, "upload");
+    say(copy_down(c, out.data(), dev, n) == FK_OK && out == in, "download");
+  }}
+  say(g_memcpys == 0, "through the slots");
+  say(std::chrono::steady_clock::now() - t0 < std::chrono::seconds(20), "no piece waits for its time-out");
+  say(!g_late, "nothing left to the null stream");
+""")
+
+
+def test_counts_are_cleared_again_after_a_failed_copy(run):
+    """A copy that fails leaves its counters to be cleared before the next."""
+    run("""
+  const size_t n = (size_t)40 << 20;
+  char *dev = device(n);
+  std::vector<char> in = pattern(n, 3), out(n);
+  say(copy_up(c, dev, in.data(), n) == FK_OK, "upload");
+  g_fail_launches = 3;
+  say(copy_up(c, dev, in.data(), n) != FK_OK, "failed upload");
+  g_fail_launches = 0;
+  for (int s = 0; s < kXferSlots; ++s) c->xfer.count[s] = 50;
+  in = pattern(n, 4);
+  say(copy_up(c, dev, in.data(), n) == FK_OK && std::memcmp(dev, in.data(), n) == 0, "next upload");
+  say(copy_down(c, out.data(), dev, n) == FK_OK && out == in, "next download");
 """)
