@@ -866,8 +866,9 @@ int pack(fk_ctx *c) {
   return FK_OK;
 }
 
-// Device scratch of one label or inference call (m.work); work_done gives a
-// large one back.
+// Device scratch of one label or inference call (m.work), its parts on 16-byte
+// words as the copies take them; work_done gives a large one back.
+size_t pad16(size_t bytes) { return (bytes + 15) / 16 * 16; }
 int work_take(fk_ctx *c, size_t bytes) {
   Mlp &m = c->mlp;
   if (bytes <= m.work_cap) return FK_OK;
@@ -1023,10 +1024,11 @@ int fk_mlp_label(fk_ctx *c, const double *U, int64_t n, float *x, float *y) {
   if (c->p.model != FK_MODEL_TWO_PHASE) return fail(FK_EINVAL, "labels need the two-phase model");
   if (n == 0) return FK_OK;
   HIPCHK(hipSetDevice(c->device));
-  int rc = work_take(c, (size_t)n * 104);
+  const size_t nx = pad16((size_t)n * 12);
+  int rc = work_take(c, (size_t)n * 80 + 2 * nx);
   if (rc) return rc;
   double *dU = reinterpret_cast<double *>(c->mlp.work);
-  float *dx = reinterpret_cast<float *>(dU + n * 10), *dy = dx + n * 3;
+  float *dx = reinterpret_cast<float *>(dU + n * 10), *dy = dx + nx / 4;
   rc = copy_up(c, dU, U, (size_t)n * 80);
   if (!rc) {
     hipLaunchKernelGGL(mlp_label_k, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, c->p, n, dU, dx, dy);
@@ -1178,9 +1180,10 @@ int fk_mlp_infer(fk_ctx *c, const float *x, int64_t n, float *y) {
   if (!c->mlp.w) return fail(FK_ESTATE, "no MLP weights");
   if (n == 0) return FK_OK;
   HIPCHK(hipSetDevice(c->device));
-  int rc = work_take(c, (size_t)n * 24);
+  const size_t nx = pad16((size_t)n * 12);
+  int rc = work_take(c, 2 * nx);
   if (rc) return rc;
-  float *dx = reinterpret_cast<float *>(c->mlp.work), *dy = dx + n * 3;
+  float *dx = reinterpret_cast<float *>(c->mlp.work), *dy = dx + nx / 4;
   rc = copy_up(c, dx, x, (size_t)n * 12);
   if (!rc) {
     const int64_t nchunk = (n + 63) / 64;

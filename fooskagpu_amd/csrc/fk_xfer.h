@@ -221,16 +221,18 @@ inline int xfer_staged(fk_ctx *c, char *pin, void *dev, void *host, size_t bytes
   return FK_OK;
 }
 
-// Synchronous copies, ordered after the work on the context's stream.
+// Synchronous copies, ordered after the work on the context's stream.  Device
+// memory between 16-byte words is not for xfer_copy.
+inline bool xfer_aligned(const void *dev) { return reinterpret_cast<uintptr_t>(dev) % 16 == 0; }
 inline int copy_down(fk_ctx *c, void *host, const void *dev, size_t bytes) {
-  if (bytes >= kXferMinDown)
+  if (bytes >= kXferMinDown && xfer_aligned(dev))
     if (char *pin = xfer_begin(c)) return xfer_staged(c, pin, const_cast<void *>(dev), host, bytes, true);
   HIPCHK(hipStreamSynchronize(c->stream));
   HIPCHK(hipMemcpy(host, dev, bytes, hipMemcpyDeviceToHost));
   return FK_OK;
 }
 inline int copy_up(fk_ctx *c, void *dev, const void *host, size_t bytes) {
-  if (bytes >= kXferMinUp)
+  if (bytes >= kXferMinUp && xfer_aligned(dev))
     if (char *pin = xfer_begin(c)) return xfer_staged(c, pin, dev, const_cast<void *>(host), bytes, false);
   HIPCHK(hipStreamSynchronize(c->stream));
   HIPCHK(hipMemcpy(dev, host, bytes, hipMemcpyHostToDevice));

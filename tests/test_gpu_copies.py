@@ -46,3 +46,26 @@ def test_uploads_of_several_threads(gpu):
     for t in th:
         t.join()
     assert not wrong
+
+
+@pytest.mark.parametrize("n", [450001, 450002, 450003])
+def test_labels_and_predictions_of_odd_counts(gpu, n):
+    """Features, targets and predictions large enough for the slots (5.4 MB)
+    that lie behind each other on the device and end between 16-byte words:
+    the same rows as in calls of a third."""
+    from fooskagpu_amd import surrogate
+    p = cases._two_phase_params()
+    U = surrogate.uniform_states(n, p, seed=n)
+    with GpuSolver(p) as g:
+        sg = surrogate.Surrogate(g)
+        print(f"[copies] {n} states", flush=True)
+        x, y = sg.label(U)
+        ok = surrogate.finite(x, y)
+        sg.set_weights(surrogate.init_weights(1), surrogate.fit_norm(*ok))
+        x = np.nan_to_num(x, posinf=0, neginf=0)
+        pred = sg.infer(x)
+        part = [slice(0, n // 3), slice(n // 3, 2 * n // 3), slice(2 * n // 3, n)]
+        xs, ys = zip(*[sg.label(U[s]) for s in part])
+        assert np.array_equal(np.nan_to_num(np.concatenate(xs), posinf=0, neginf=0), x)
+        assert np.array_equal(np.concatenate(ys), y, equal_nan=True)
+        assert np.array_equal(np.concatenate([sg.infer(x[s]) for s in part]), pred)

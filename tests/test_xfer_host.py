@@ -226,3 +226,22 @@ def test_counts_are_cleared_again_after_a_failed_copy(run):
   say(copy_up(c, dev, in.data(), n) == FK_OK && std::memcmp(dev, in.data(), n) == 0, "next upload");
   say(copy_down(c, out.data(), dev, n) == FK_OK && out == in, "next download");
 """)
+
+
+def test_only_aligned_device_memory_is_copied_in_wide_words(run):
+    """The copy kernel moves 16-byte words: a device address between them goes
+    to hipMemcpy; any number of bytes, at any host address, through the slots
+    (the tail of 1 to 15 bytes by itself)."""
+    run("""
+  for (int tail : {0, 1, 4, 12, 15}) {
+    const size_t n = ((size_t)18 << 20) + tail;
+    std::vector<char> in = pattern(n + 3, tail), out(n + 5);
+    for (int off : {0, 4, 8, 16}) {
+      char *dev = device(n) + off;
+      g_memcpys = 0;
+      say(copy_up(c, dev, in.data() + 3, n) == FK_OK && std::memcmp(dev, in.data() + 3, n) == 0, "upload");
+      say(copy_down(c, out.data() + 5, dev, n) == FK_OK && std::memcmp(out.data() + 5, in.data() + 3, n) == 0, "download");
+      say(g_memcpys == (off % 16 ? 2 : 0), off % 16 ? "by hipMemcpy" : "through the slots");
+    }
+  }
+""")
