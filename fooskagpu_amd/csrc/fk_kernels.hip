@@ -2133,7 +2133,7 @@ int do_relax(fk_ctx *c, fk_relax_stats *st, int mode = FK_RELAX_PLAIN) {
     if (st || nb > kCountParts)
       LAUNCH_TIMED(c, "relax_count", hipLaunchKernelGGL(fk::reduce_partials<3>, dim3(fk::reduce_grid(nb)), dim3(256), 0,
                                                         c->stream, c->rpart, nb, cnt));
-    const unsigned gch = (unsigned)std::max<int64_t>(1, std::min<int64_t>(grid_for(c->nc), 1024));
+    const unsigned gch = list_blocks(c->nc, 8);
     LAUNCH_TIMED(c, "relax_chem", hipLaunchKernelGGL(relax_chem, dim3(gch), dim3(kBlock), 0, c->stream, c->p,
                                                      c->U[c->ia], c->rlist, cnt, W));
     c->w_valid = W != nullptr;
@@ -2173,7 +2173,7 @@ int relax_plain_fused_finish(fk_ctx *c) {
     LAUNCH_TIMED(c, "relax_count", hipLaunchKernelGGL(fk::reduce_partials<3>, dim3(fk::reduce_grid(nw)), dim3(256), 0,
                                                       c->stream, c->rpart, nw, cnt));
   float *W = (c->p.precision == FK_MIXED && c->prims_w) ? c->wprim : nullptr;
-  const unsigned gch = (unsigned)std::max<int64_t>(1, std::min<int64_t>(grid_for(c->nc), 1024));
+  const unsigned gch = list_blocks(c->nc, 8);
   LAUNCH_TIMED(c, "relax_chem", hipLaunchKernelGGL(relax_chem, dim3(gch), dim3(kBlock), 0, c->stream, c->p,
                                                    c->U[c->ia], c->rlist, cnt, W));
   c->w_valid = W != nullptr;

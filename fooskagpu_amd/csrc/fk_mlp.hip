@@ -765,7 +765,7 @@ __global__ void __launch_bounds__(256) relax_fallback_k(fk_params P, double *__r
   const int64_t n = (int64_t)counts[7];
   unsigned long long nit = 0, nfb = 0;
   // 8 lanes per cell (fk::chem_dev8, thermal cells on each of them alike) up
-  // to kChemGroup cells, then one lane
+  // to kChemGroup cells, then one lane (blocks: list_blocks)
   const int per = n <= fk::kChemGroup ? 8 : 1;
   const int64_t nt = (int64_t)gridDim.x * 256 / per;
   const bool lead = per == 1 || (threadIdx.x & 7) == 0;
@@ -944,21 +944,20 @@ int fk_relax_mlp_finish(fk_ctx *c, bool warm) {
   Mlp &m = c->mlp;
   unsigned long long *cnt = (unsigned long long *)c->lcount;
   float *W = (c->p.precision == FK_MIXED && c->prims_w) ? c->wprim : nullptr;
-  const int64_t nchunk = (c->nc + 63) / 64;
-  const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>((nchunk + 3) / 4, 1024));
+  const unsigned grid = list_blocks(c->nc, 1), glist = list_blocks(c->nc, 4);
   if (warm) {
     int rc = ensure_rstart(c);  // fk_run_steps has allocated it before its first stage
     if (rc) return rc;
     float2 *st = static_cast<float2 *>(c->rstart);
     LAUNCH_TIMED(c, "relax_infer", hipLaunchKernelGGL(relax_infer_k, dim3(grid), dim3(256), 0, c->stream, c->p,
                                                       c->U[c->ia], c->rlist, m.w, m.wb, norm_of(m), cnt, st));
-    LAUNCH_TIMED(c, "relax_list", hipLaunchKernelGGL(relax_list_k<true>, dim3(grid), dim3(256), 0, c->stream, c->p,
+    LAUNCH_TIMED(c, "relax_list", hipLaunchKernelGGL(relax_list_k<true>, dim3(glist), dim3(256), 0, c->stream, c->p,
                                                      c->U[c->ia], c->rlist, st, cnt, W, c->nc, c->rfall));
   } else {
-    LAUNCH_TIMED(c, "relax_list", hipLaunchKernelGGL(relax_list_k<false>, dim3(grid), dim3(256), 0, c->stream, c->p,
+    LAUNCH_TIMED(c, "relax_list", hipLaunchKernelGGL(relax_list_k<false>, dim3(glist), dim3(256), 0, c->stream, c->p,
                                                      c->U[c->ia], c->rlist, nullptr, cnt, W, c->nc, c->rfall));
   }
-  const unsigned gfb = (unsigned)std::max<int64_t>(1, std::min<int64_t>((c->nc + 255) / 256, 256));
+  const unsigned gfb = list_blocks(c->nc, 8);
   LAUNCH_TIMED(c, "relax_fallback", hipLaunchKernelGGL(relax_fallback_k, dim3(gfb), dim3(256), 0, c->stream, c->p,
                                                        c->U[c->ia], c->rfall, cnt, W));
   c->w_valid = W != nullptr;

@@ -65,4 +65,25 @@ inline int64_t relax_words(int64_t nc, int ns) {
   return w;
 }
 
+// Up to this many listed cells a relaxation gives a cell to a group of lanes
+// (8 a reference chemical solve, 4 a polish): below, the chip has idle SIMDs and
+// the chain of one cell sets the time; above, the redundant work of a group's
+// lanes does.  Reference chemical solve, every cell of the mesh listed (us, one
+// lane / 8 lanes): 2k cells 387 / 84, 16k 395 / 157, 35k 399 / 251, 48k 400 /
+// 307, 64k 409 / 389, of 119k 533 / 611; as fallback of as many polishes 378 /
+// 87, 392 / 158, 399 / 254, 400 / 305, 402 / 395, of thermal cells, which every
+// lane of a group solves alike, 55 / 27, 396 / 112, 428 / 127, 541 / 189, 476 /
+// 221.  Polish from the cell state (one lane / 4 lanes): 2k 55 / 39, 16k 60 /
+// 37, 35k 74 / 59, 48k 76 / 68, 119k 88 / 129; from the network's start 510
+// cells 34 / 22, 25k 57 / 48, 50k 63 / 53, 119k 73 / 80.
+constexpr int64_t kChemGroup = 65536, kPolishGroup = 49152;
+
+// Blocks of a kernel over a list of up to nc cells, `lanes` lanes to a cell: all
+// of the mesh at once, up to 1024 blocks (two rounds of kChemGroup cells).  With
+// blocks for one lane a cell, groups of 8 took eight rounds and lost to one lane
+// (16k chemical cells 475 us, the polish of 4 lanes 94).
+inline unsigned list_blocks(int64_t nc, int lanes) {
+  return (unsigned)std::max<int64_t>(1, std::min<int64_t>(grid_for(nc * lanes), 1024));
+}
+
 }  // namespace fkx

@@ -7,8 +7,11 @@
 #include "../../include/fooska.h"
 #include "fk_device.h"
 #include "fk_math.h"
+#include "fk_plan.h"
 
 namespace fk {
+
+using fkx::kChemGroup, fkx::kPolishGroup;
 
 // ---------------- phase relaxation (relaxation.cu, thermRlx.cu, chemRlx.cu) ----------------
 
@@ -717,16 +720,6 @@ FK_HD inline void chem_cold(const fk_params &P, const double *U, double &T0, dou
 // that evaluate different residuals (or logarithms) at the same time; every
 // lane of a group holds the same iterate, and each quantity is formed by the
 // same operations as in the one-lane form, so the results are the same bits.
-
-// Up to this many listed cells the groups are used: below, the chip has idle
-// SIMDs and the chain sets the time; above, the redundant work of a group's
-// lanes does.  Reference chemical solve (us, one lane / 8 lanes): 510 cells
-// 370 / 124, 25k 390 / 205, 50k 400 / 283, 119k 533 / 611; its use as fallback
-// of 530 polishes 327 / 84.  Polish (one lane / 4 lanes): network start 510
-// cells 34 / 22, 25k 57 / 48, 50k 63 / 53, 119k 73 / 80; cell state 510 cells
-// 45 / 35, 25k 76 / 60, 50k 72 / 69, 119k 88 / 129.
-constexpr int64_t kChemGroup = 65536, kPolishGroup = 49152;
-
 
 // value of lane L of the quad on every lane of it
 template <int L>

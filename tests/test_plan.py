@@ -51,3 +51,21 @@ def test_relaxation_counts_fit_their_buffer_at_either_precision(probe):
     }
   std::printf("tried %ld\\n", tried);""")
     assert lines[:-1] == [] and int(lines[-1].split()[1]) > 10000, lines[:5]
+
+
+def test_a_list_of_every_cell_takes_at_most_two_rounds_on_groups(probe):
+    """Listed cells on groups of lanes (8 a chemical solve, 4 a polish) where
+    every cell of the mesh is listed: the grid holds the groups of all of them
+    at once, or half of the longest list that takes groups; and one lane a
+    cell as before, one round up to 262,144 cells."""
+    lines = probe("""
+  for (int64_t n = 1; n <= 1 << 20; n += 1 + n / 50) {
+    const int64_t chem = std::min(n, kChemGroup), polish = std::min(n, kPolishGroup);
+    auto rounds = [](int64_t lanes, unsigned blocks) { return (lanes + (int64_t)blocks * kBlock - 1) / ((int64_t)blocks * kBlock); };
+    const int64_t rc = rounds(chem * 8, list_blocks(n, 8)), rp = rounds(polish * 4, list_blocks(n, 4));
+    const int64_t r1 = rounds(std::min<int64_t>(n, 262144), list_blocks(n, 1));
+    if (rc > (chem <= 32768 ? 1 : 2) || rp > 1 || r1 > 1 || list_blocks(n, 8) > 1024)
+      std::printf("%ld cells: %ld %ld %ld\\n", (long)n, (long)rc, (long)rp, (long)r1);
+  }
+  std::printf("%u %u\\n", list_blocks(1, 8), list_blocks((int64_t)1 << 30, 1));""")
+    assert lines == ["1 1024"], lines[:5]
