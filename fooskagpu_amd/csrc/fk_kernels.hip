@@ -1493,8 +1493,8 @@ __global__ void __launch_bounds__(kBlock) relax_chem(fk_params P, double *__rest
                                                      unsigned long long *__restrict__ counts, float *__restrict__ W) {
   const int64_t n = fk::list_front(counts[5]);
   unsigned long long nit = 0;
-  // 8 lanes per cell (fk::chem_dev8) up to kChemGroup cells, then one lane
-  const int per = n <= fk::kChemGroup ? 8 : 1;
+  // short lists 8 lanes per cell (fk::chem_dev8)
+  const int per = chem_lanes(n, (int64_t)gridDim.x * kBlock);
   const int64_t nt = (int64_t)gridDim.x * kBlock / per;
   const bool lead = per == 1 || (threadIdx.x & 7) == 0;
   for (int64_t e = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / per; e < n; e += nt) {

@@ -691,9 +691,9 @@ __global__ void __launch_bounds__(256) relax_list_k(fk_params P, double *__restr
                                                     int64_t cap, uint32_t *__restrict__ fall) {
   // chunks of 64 entries: the chemical ones from the list's front, then the
   // thermal ones from its back
-  // (up to kPolishGroup of them 4 lanes to an entry, fk::chem_polish4)
+  // (short lists 4 lanes to an entry, fk::chem_polish4)
   const int64_t nfr = fk::list_front(counts[5]), nbk = fk::list_back(counts[5]);
-  const int per = nfr <= fk::kPolishGroup ? 4 : 1, epw = 64 / per;
+  const int per = polish_lanes(nfr, (int64_t)gridDim.x * 256), epw = 64 / per;
   const int64_t cf = (nfr + epw - 1) / epw, nchunk = cf + (nbk + 63) / 64;
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
   unsigned long long nit = 0, nwarm = 0;
@@ -764,9 +764,9 @@ __global__ void __launch_bounds__(256) relax_fallback_k(fk_params P, double *__r
                                                         float *__restrict__ W) {
   const int64_t n = (int64_t)counts[7];
   unsigned long long nit = 0, nfb = 0;
-  // 8 lanes per cell (fk::chem_dev8, thermal cells on each of them alike) up
-  // to kChemGroup cells, then one lane (blocks: list_blocks)
-  const int per = n <= fk::kChemGroup ? 8 : 1;
+  // short lists 8 lanes per cell (fk::chem_dev8, thermal cells on each of them
+  // alike)
+  const int per = chem_lanes(n, (int64_t)gridDim.x * 256);
   const int64_t nt = (int64_t)gridDim.x * 256 / per;
   const bool lead = per == 1 || (threadIdx.x & 7) == 0;
   for (int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) / per; e < n; e += nt) {
@@ -957,7 +957,7 @@ int fk_relax_mlp_finish(fk_ctx *c, bool warm) {
     LAUNCH_TIMED(c, "relax_list", hipLaunchKernelGGL(relax_list_k<false>, dim3(glist), dim3(256), 0, c->stream, c->p,
                                                      c->U[c->ia], c->rlist, nullptr, cnt, W, c->nc, c->rfall));
   }
-  const unsigned gfb = list_blocks(c->nc, 8);
+  const unsigned gfb = std::min(list_blocks(c->nc, 8), 512u);
   LAUNCH_TIMED(c, "relax_fallback", hipLaunchKernelGGL(relax_fallback_k, dim3(gfb), dim3(256), 0, c->stream, c->p,
                                                        c->U[c->ia], c->rfall, cnt, W));
   c->w_valid = W != nullptr;

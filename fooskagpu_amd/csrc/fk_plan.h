@@ -65,25 +65,33 @@ inline int64_t relax_words(int64_t nc, int ns) {
   return w;
 }
 
-// Up to this many listed cells a relaxation gives a cell to a group of lanes
-// (8 a reference chemical solve, 4 a polish): below, the chip has idle SIMDs and
-// the chain of one cell sets the time; above, the redundant work of a group's
-// lanes does.  Reference chemical solve, every cell of the mesh listed (us, one
-// lane / 8 lanes): 2k cells 387 / 84, 16k 395 / 157, 35k 399 / 251, 48k 400 /
-// 307, 64k 409 / 389, of 119k 533 / 611; as fallback of as many polishes 378 /
-// 87, 392 / 158, 399 / 254, 400 / 305, 402 / 395, of thermal cells, which every
-// lane of a group solves alike, 55 / 27, 396 / 112, 428 / 127, 541 / 189, 476 /
-// 221.  Polish from the cell state (one lane / 4 lanes): 2k 55 / 39, 16k 60 /
-// 37, 35k 74 / 59, 48k 76 / 68, 119k 88 / 129; from the network's start 510
-// cells 34 / 22, 25k 57 / 48, 50k 63 / 53, 119k 73 / 80.
+// A relaxation gives a listed cell to a group of lanes (8 a reference chemical
+// solve, 4 a polish) on short lists: there the chip has idle SIMDs and the chain
+// of one cell sets the time; on longer ones the redundant work of a group's
+// lanes does.  Every cell of the mesh listed, us, one lane / group: reference
+// chemical solve 2k cells 387 / 84, 16k 395 / 147, 35k 399 / 249, 48k 400 / 316,
+// 64k 409 / 404, 119k 533 / 611; as fallback of as many polishes 378 / 87, 392 /
+// 147, 399 / 256, 400 / 318, 402 / 412, of thermal cells, which every lane of a
+// group solves alike, 55 / 25, 396 / 120, 428 / 138, 541 / 177, 476 / 203.
+// Polish from the cell state 2k 55 / 39, 16k 60 / 38, 35k 74 / 62, 48k 76 / 68,
+// 119k 88 / 129; from the network's start 510 cells 34 / 22, 25k 57 / 48, 50k
+// 63 / 53, 119k 73 / 80.
 constexpr int64_t kChemGroup = 65536, kPolishGroup = 49152;
 
-// Blocks of a kernel over a list of up to nc cells, `lanes` lanes to a cell: all
-// of the mesh at once, up to 1024 blocks (two rounds of kChemGroup cells).  With
-// blocks for one lane a cell, groups of 8 took eight rounds and lost to one lane
-// (16k chemical cells 475 us, the polish of 4 lanes 94).
+// Blocks of a kernel over a list of up to nc cells: one lane a cell, up to 1024
+// blocks, but `lanes` lanes a cell as long as that makes no more than 512.  With
+// blocks for one lane alone, groups of 8 took eight rounds of a full list and
+// lost to one lane (16k chemical cells 475 us, their polish 94); more than 512
+// gain nothing on full lists and cost each step with short ones (fallback of
+// 373k hexahedra with 1024 blocks 1 us more than with 256, with 512 0.5).
 inline unsigned list_blocks(int64_t nc, int lanes) {
-  return (unsigned)std::max<int64_t>(1, std::min<int64_t>(grid_for(nc * lanes), 1024));
+  const int64_t most = std::max<int64_t>(std::min<int64_t>(grid_for(nc * lanes), 512), std::min<int64_t>(grid_for(nc), 1024));
+  return (unsigned)std::max<int64_t>(1, most);
 }
+
+// Lanes to a cell of a list of n on a grid of nt lanes: a group while the list
+// takes up to four rounds of the chemical solve, two of the polish.
+constexpr int chem_lanes(int64_t n, int64_t nt) { return n <= kChemGroup && n * 8 <= 4 * nt ? 8 : 1; }
+constexpr int polish_lanes(int64_t n, int64_t nt) { return n <= kPolishGroup && n * 4 <= 2 * nt ? 4 : 1; }
 
 }  // namespace fkx

@@ -7,11 +7,8 @@
 #include "../../include/fooska.h"
 #include "fk_device.h"
 #include "fk_math.h"
-#include "fk_plan.h"
 
 namespace fk {
-
-using fkx::kChemGroup, fkx::kPolishGroup;
 
 // ---------------- phase relaxation (relaxation.cu, thermRlx.cu, chemRlx.cu) ----------------
 
