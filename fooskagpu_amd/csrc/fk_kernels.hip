@@ -1690,12 +1690,15 @@ inline bool quad_f(const fk_ctx *c, int relax) {
 // Whether the last pass F also runs the relaxation's per-cell pass (kind 1
 // surrogate, 2 plain).  It saves reading the state back, but runs the solve at
 // pass F's registers, and with 6 FP32 slots without LDS staging.  us a step,
-// fused / apart: FP64 plain 115 / 128 at 7k cells, 181 / 172 at 83k, 881 / 856
-// at 511k, 4732 / 4639 at 3.1M; 6 slots FP32 surrogate 103 / 106 at 27k, 526 /
-// 508 at 373k, 1696 / 1599 at 1.3M; the others 0 to 3 % better fused.
+// fused / apart: FP64 plain 58 / 67 and 66 / 72 at 10k cells, 80 / 81 and 91 /
+// 89 at 25k (two flows), 110 / 101 at 48k, 881 / 856 at 511k, 4732 / 4639 at
+// 3.1M; 6 slots FP32 surrogate 103 / 106 at 27k, 526 / 508 at 373k, 1696 / 1599
+// at 1.3M.  FP32 plain 76 / 78 at 35k; 6 slots FP64 plain 161 / 162 at 36k, 198
+// / 198 at 64k.  The FP64 surrogate, 115 / 111 at 48k and 261 / 252 at 162k, is
+// left fused: where it begins to lose is not measured.
 inline bool fuse_pays(const fk_ctx *c, int kind) {
   if (c->ns == 6) return c->p.precision == FK_FP64 || c->nc <= 200000;
-  return !(kind == 2 && c->p.precision == FK_FP64) || c->nc <= 60000;
+  return !(kind == 2 && c->p.precision == FK_FP64) || c->nc <= 25000;
 }
 
 template <typename T, int NS>

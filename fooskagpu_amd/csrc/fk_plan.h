@@ -34,9 +34,14 @@ inline unsigned grid_quad(int64_t nc) { return grid_blocks(nc, 16); }  // one wa
 //           51 / 59 at 511k, 178 / 160 at 1.6M (single-phase); 6 slots FP32
 //           28 / 29 at 55k, 63 / 60 at 176k
 //   with the relaxation (on the quad only the plain solve's residuals go in
-//           parallel) FP64 64 / 70 at 162k, 106 / 103 at 280k; FP32 22 / 22 at 48k,
-//           34 / 31 at 94k, plain 81 / 85 at 162k; 6 slots FP64 26 / 31 at 27k,
-//           65 / 53 at 55k; FP32 22 / 26 at 27k, 48 / 40 at 85k
+//           parallel, without the shared divisors of one lane's) us a step:
+//           surrogate FP64 115 / 120 at 48k, 261 / 263 at 162k, 345 / 352 at
+//           236k, 492 / 487 at 329k; FP32 (the kernel) 21 / 21 at 48k, 28 / 23 at
+//           64k; plain FP64 80 / 83 at 25k (apart above, fuse_pays); FP32 63 / 67
+//           at 16k, 69 / 70 at 25k, 74 / 73 at 29k, 93 / 82 at 48k; 6 slots
+//           surrogate (the kernel) FP64 24 / 31 at 27k, 34 / 33 at 47k; FP32 24 /
+//           25 at 27k, 25 / 25 at 36k, 42 / 38 at 85k; plain FP64 130 / 133 at
+//           27k, 170 / 161 at 36k; FP32 101 / 103 at 27k, 143 / 135 at 36k
 inline int64_t quad_cells_g(bool f64, int ns) {
   if (ns == 6) return f64 ? 40000 : 20000;
   return 60000;
@@ -44,8 +49,8 @@ inline int64_t quad_cells_g(bool f64, int ns) {
 // relax: 0 none, 1 the surrogate's stage 1, 2 the plain relaxation in the kernel
 inline int64_t quad_cells_f(bool f64, int ns, int neq, int relax) {
   if (relax) {
-    if (ns == 6) return 35000;
-    return f64 ? 220000 : (relax == 2 ? 160000 : 50000);
+    if (ns == 6) return !f64 && relax == 2 ? 30000 : 35000;
+    return f64 ? 220000 : (relax == 2 ? 25000 : 50000);
   }
   if (f64) return INT64_MAX;
   return ns == 6 ? 120000 : (neq == 5 ? 600000 : 350000);

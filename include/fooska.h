@@ -235,7 +235,7 @@ int fk_set_debug(fk_ctx *ctx, int on);
  *     relaxation (FK_RELAX_MLP, FK_RELAX_COLD) or the plain Tsat
  *     classification and thermal solve (FK_RELAX_PLAIN, except while it emits
  *     training pairs); the chemical / listed cells follow in their own kernel.
- *     Apart where that is faster: FP64 plain on 4-slot meshes over 60,000
+ *     Apart where that is faster: FP64 plain on 4-slot meshes over 25,000
  *     cells, FP32 on 6-slot meshes over 200,000.
  * Unknown names return FK_EINVAL. */
 int fk_set_tuning(fk_ctx *ctx, const char *name, int64_t value);

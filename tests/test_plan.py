@@ -33,7 +33,7 @@ def test_relaxation_counts_fit_their_buffer_at_either_precision(probe):
     lines = probe("""
   std::vector<int64_t> sizes;
   for (int64_t n = 1; n < 2000; ++n) sizes.push_back(n);
-  for (int64_t at : {22000, 25000, 35000, 50000, 60000, 120000, 160000, 220000, 350000, 600000})
+  for (int64_t at : {22000, 25000, 30000, 35000, 50000, 60000, 120000, 160000, 220000, 350000, 600000})
     for (int64_t d = -300; d <= 300; ++d) sizes.push_back(at + d);
   for (int64_t n = 2000; n < (int64_t)1 << 28; n += n / 7) sizes.push_back(n);
   long tried = 0;
