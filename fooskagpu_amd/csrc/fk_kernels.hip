@@ -1231,6 +1231,7 @@ __global__ void __launch_bounds__(64, (NS == 4 || sizeof(T) == 4 ? 3 : 2)) pass_
     const V4<T> ga = ld4<T>(geo, s);
     const int lk = in ? link[s] : kNoFace;
     double fr[NEQ], fv[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    T sf = (T)-1e9;  // the face's signal speed (never negative), or no face
 #pragma unroll
     for (int v = 0; v < NEQ; ++v) fr[v] = 0.0;
     if (lk != kNoFace) {
@@ -1252,7 +1253,14 @@ __global__ void __launch_bounds__(64, (NS == 4 || sizeof(T) == 4 ? 3 : 2)) pass_
       if (nb < 0) fk::ghost<NEQ, T>(mt, -nb, n, Rt);
       face_terms<NEQ, T, VISC, HEAT, MODE == 1>(P, mt, cs, nb, own, n, ga.w, L, Rt, VISC ? gvel + c * NG : nullptr,
                                                 VISC && nb >= 0 ? gvel + (int64_t)nb * NG : nullptr,
-                                                VISC ? wls + s : nullptr, state1, fr, fv, sig);
+                                                VISC ? wls + s : nullptr, state1, fr, fv, sf);
+    }
+    if constexpr (MODE == 1) {  // in slot order: of NaNs only the last face's stays, as on one lane
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const T s1 = quad_bcast(sf, j);
+        if ((NS == 4 || s1 != (T)-1e9) && !(sig >= s1)) sig = s1;
+      }
     }
     if constexpr (MODE == 0 && R == 1) stage_states();  // on their way while the quad adds
 #pragma unroll
@@ -1275,7 +1283,6 @@ __global__ void __launch_bounds__(64, (NS == 4 || sizeof(T) == 4 ? 3 : 2)) pass_
     if constexpr (HEAT) rhs[4] += rv[4];
   }
   if constexpr (MODE != 0) {
-    sig = quad_max(sig);
 #pragma unroll
     for (int v = 0; v < NEQ; ++v)
       if (q == (v & 3)) {
