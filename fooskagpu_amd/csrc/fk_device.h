@@ -85,7 +85,8 @@ struct Divisor {
 // and a product, with the bits of the forms above where divisor, reciprocal
 // and result are normal numbers, as densities, wave speeds and moduli are
 // (the reciprocal's mantissa does not depend on the exponent); a limiter's
-// differences can lie below that and take quot.  Two instructions for eight
+// differences can lie below that and take quot, the divisor of the eddy
+// viscosity above, and is scaled.  Two instructions for eight
 // and one for six: pass F at size is bound by its instructions (mixed, 3.07M
 // cells: VALU busy 75 to 95 %; the dt stage, which also took the sound speeds
 // of both states twice, 390 -> 355 us, the RK stage 454 -> 442).  FP64: the
@@ -532,7 +533,10 @@ __device__ __forceinline__ T wale(const T g[3][3], T Ls) {
   T num = sum1 * face_sqrt(sum1);
   T den = sum1 * face_sqrt(face_sqrt(sum1)) + sum2 * sum2 * face_sqrt(sum2) + (T)1e-12;
   if (den < (T)1e-10) num = 0;
-  return face_quot(Ls * Ls * num, den);
+  // FP32: den, a fifth power of the strain rate and at least 1e-12, may lie
+  // above 2^126, where its reciprocal is no normal number: scaled by 2^-32
+  if constexpr (sizeof(T) == 4) return face_quot(Ls * Ls * num, den * (T)0x1p-32) * (T)0x1p-32;
+  else return face_quot(Ls * Ls * num, den);
 }
 
 }  // namespace fk
