@@ -350,12 +350,15 @@ __global__ void __launch_bounds__(kBlock, (sizeof(T) == 8 ? 2 : 1))
   }
   // Limiter, theta = min over faces of clamp(phi_f, 0, 1), and MUSCL face
   // states, variable by variable.  phi_f = (mx - W) / (2 d_f) where
-  // d_f = wu_f - W > 0, (mn - W) / (2 d_f) where d_f < 0, 1 where d_f = 0.  A
-  // rounded quotient is monotonic in its divisor, so the smallest clamped
-  // phi_f of either sign is that of the largest |d_f| of that sign: two
-  // divisions per variable instead of one per face, the same bits (a negative
-  // numerator clamps to 0 at every face; a NaN d_f counts as phi = 1, as
-  // before).  Slots past the last face have r = 0, so d = 0 there.  With the
+  // d_f = wu_f - W > 0, (mn - W) / (2 d_f) where d_f < 0, 1 where d_f = 0.  The
+  // quotient is monotonic in its divisor, so the smallest clamped phi_f of
+  // either sign is that of the largest |d_f| of that sign: two divisions per
+  // variable instead of one per face, the same bits (a negative numerator
+  // clamps to 0 at every face; a NaN d_f counts as phi = 1).  Monotonic: in FP64
+  // as a rounded quotient; in FP32 (fk::quot, not correctly rounded) because
+  // the hardware reciprocal does not rise anywhere over the mantissas of
+  // [0.5, 1] (all 2^23 + 1 compared) and meets its ends exactly (2 and 1), and
+  // the product and the scaling are rounded once each.  Slots past the last face have r = 0, so d = 0 there.  With the
   // products r g shared by wu and the extrapolation, mixed pass G executes
   // 1467 instead of 2136 VALU instructions per cell, FP64 (with the gradient's
   // shared divisor) 2796 instead of 4869: FP64 237 -> 187 us at 1.05M

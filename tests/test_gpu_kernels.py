@@ -232,3 +232,24 @@ def test_time_step_is_that_of_the_last_state(gpu, n, stage):
             g.upload_state(U)
             g.set_clock(0.0, 0.0, 0)
             assert g.run_steps(1)[0] == dt
+
+
+@pytest.mark.parametrize("kind", ["random", "uniform", "spike"])
+@pytest.mark.parametrize("elements", ["tets", "mixed"])
+@pytest.mark.parametrize("model", [_lib.MODEL_SINGLE, _lib.MODEL_TWO_PHASE])
+def test_limiter_of_the_variants_in_mixed_precision(gpu, model, elements, kind):
+    """FP32 quotients at the steepest slope of either sign (one lane per cell)
+    against the smallest of a quotient at every face (four lanes): limiter and
+    face states of rough states, bit for bit."""
+    p = dict(cases.BASE) if model == _lib.MODEL_SINGLE else cases._two_phase_params()
+    m = Mesh.box(14, 14, 14, jitter=0.1, seed=5) if elements == "tets" else Mesh.mixed_box(21, 14, 14, jitter=0.1, seed=5)
+    out = []
+    for stage in (1, 2, 0):
+        with GpuSolver(dict(p, precision=_lib.MIXED), m, rough_state(5 if model == _lib.MODEL_SINGLE else 10, m.n_cells, kind)) as g:
+            g.set_tuning("stage_g", stage)
+            g.set_debug(True)
+            g.compute_face_values()
+            out.append((g.download("theta"), g.download("face")[g.download("slots") >= 0]))
+    assert kind == "uniform" or (out[0][0] < 1).any()
+    for o in out[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(o, out[0]))
