@@ -458,8 +458,9 @@ __global__ void __launch_bounds__(kBlock, (sizeof(T) == 8 ? 2 : 1))
 // wave of pass F lowers one of them (64 words: an atomic on one address
 // retires in about 12 ns), the update or dt_final folds the 64.  The order of
 // the waves does not matter to a minimum.  Two sets in turn: a dt stage resets
-// the one that it does not use, which the next one takes.  Before, pass F's array was read by two more kernels, 13
-// us a step at 1M cells, or its quads' minima folded by one of 8.5 us.
+// the one that it does not use, which the next one takes.  Reading pass F's
+// array in two kernels of its own took 13 us a step at 1M cells, folding its
+// quads' minima in one 8.5 us.
 constexpr int kDtSlots = 64, kDtStride = 16;
 constexpr double kDtNone = 1e15;
 __device__ __forceinline__ unsigned long long dt_key(double d) {
