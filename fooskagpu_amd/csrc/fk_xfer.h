@@ -28,23 +28,26 @@ namespace fkx {
 // are there already, 10 MB 314 and 19 MB 540.
 constexpr size_t kXferMinDown = (size_t)5 << 20, kXferMinUp = (size_t)16 << 20;
 
-// The slots, 64 MB for the process with a report word each (page-locking
-// costs about 2 ms, which each new context would otherwise pay in its first
-// copy): allocated by the first large copy, freed with the last context, and
-// lent to one copy at a time.  A copy that finds them lent is one hipMemcpy.
+// The slots, up to 64 MB for the process with a report word each (page-locking
+// 64 MB costs about 2 ms, 16 MB 0.1 to 0.2, which each new context would
+// otherwise pay in its first copy): allocated by the first large copy at the
+// size that it uses, anew by one that uses more, freed with the last context,
+// and lent to one copy at a time.  A copy that finds them lent is one hipMemcpy.
 // Coherent memory, asked for: the host takes a slot while later kernels of the
 // stream run, and refills one for a later kernel without a synchronisation.
 constexpr size_t kXferSlot = (size_t)4 << 20;
 constexpr int kXferSlots = 2 * kXferThreads;
+constexpr size_t kXferReports = 4096;  // at the start of the block, 64 bytes a slot
 struct XferPool {
   std::mutex mu;
   char *pin = nullptr;
+  size_t cap = 0;
   int contexts = 0;
   bool lent = false;
   std::atomic<unsigned long long> seq{0};
 
   unsigned long long *report(int slot) {
-    return reinterpret_cast<unsigned long long *>(pin + kXferSlots * kXferSlot) + 8 * slot;
+    return reinterpret_cast<unsigned long long *>(pin) + 8 * slot;
   }
   void attach() {
     std::lock_guard<std::mutex> lk(mu);
@@ -52,24 +55,31 @@ struct XferPool {
   }
   void detach() {
     std::lock_guard<std::mutex> lk(mu);
-    if (--contexts > 0 || !pin) return;
-    (void)hipHostFree(pin);
-    pin = nullptr;
+    if (--contexts > 0) return;
+    drop();
   }
-  char *borrow() {
+  void drop() {
+    if (pin) (void)hipHostFree(pin);
+    pin = nullptr;
+    cap = 0;
+  }
+  // the slots' memory, at least `bytes`
+  char *borrow(size_t bytes) {
     std::lock_guard<std::mutex> lk(mu);
     if (lent) return nullptr;
-    if (!pin) {
+    if (cap < bytes) {
+      drop();
       void *p = nullptr;
-      if (hipHostMalloc(&p, kXferSlots * (kXferSlot + 64), kHostCoherent) != hipSuccess) {
+      if (hipHostMalloc(&p, kXferReports + bytes, kHostCoherent) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
       }
       pin = static_cast<char *>(p);
-      std::memset(pin + kXferSlots * kXferSlot, 0, kXferSlots * 64);
+      cap = bytes;
+      std::memset(pin, 0, kXferReports);
     }
     lent = true;
-    return pin;
+    return pin + kXferReports;
   }
   void give_back() {
     std::lock_guard<std::mutex> lk(mu);
@@ -105,10 +115,23 @@ static __global__ void __launch_bounds__(64) xfer_clear(unsigned *__restrict__ c
   if ((int)threadIdx.x < kXferSlots) count[threadIdx.x] = 0;
 }
 
+// Pieces and threads of a copy: mid sizes in smaller pieces, so that a few
+// threads share them; a thread, with two slots, for every two pieces.
+struct XferPlan {
+  size_t piece;
+  int threads;
+  explicit XferPlan(size_t bytes)
+      : piece(bytes >= 16 * kXferSlot ? kXferSlot : (bytes >= 4 * kXferSlot ? kXferSlot / 2 : kXferSlot / 4)) {
+    const size_t half = (bytes + piece - 1) / piece / 2;
+    threads = (int)(half < (size_t)kXferThreads ? half : kXferThreads);
+  }
+};
+static_assert(kXferSlots * 64 <= kXferReports, "a report word per slot");
+
 // The slots for a copy of context c, or null: then the copy is one hipMemcpy.
 // The counts are cleared on the context's stream, which is not ordered with the
 // null stream, and again after a copy that failed.
-inline char *xfer_begin(fk_ctx *c) {
+inline char *xfer_begin(fk_ctx *c, size_t bytes) {
   if (!c->xfer.count) {
     unsigned *p = nullptr;
     if (hipMalloc(&p, kXferSlots * sizeof(unsigned)) != hipSuccess) {
@@ -118,7 +141,8 @@ inline char *xfer_begin(fk_ctx *c) {
     c->xfer.count = p;
     c->xfer.clear = false;
   }
-  char *pin = g_xfer.borrow();
+  const XferPlan plan(bytes);
+  char *pin = g_xfer.borrow(2 * plan.threads * plan.piece);
   if (pin && !c->xfer.clear) {
     hipLaunchKernelGGL(xfer_clear, dim3(1), dim3(64), 0, c->stream, c->xfer.count);
     if (hipGetLastError() != hipSuccess) {
@@ -139,8 +163,9 @@ inline void xfer_free(fk_ctx *c) {
 struct XferJob {
   fk_ctx *c;
   char *pin, *dev, *host;
-  size_t bytes, piece;
+  size_t bytes;
   bool down;
+  size_t piece;
   std::atomic<size_t> next{0};
   std::atomic<int> err{0};
 
@@ -150,7 +175,7 @@ struct XferJob {
     if (e != hipSuccess) err.store((int)e);
     return err.load() != 0;
   }
-  char *slot(int s) { return pin + (size_t)s * kXferSlot; }
+  char *slot(int s) { return pin + (size_t)s * piece; }
   // starts the transfer of the piece at `at` through slot s; its report in *seq
   bool start(size_t at, int s, unsigned long long *seq) {
     const size_t n = len(at);
@@ -196,12 +221,9 @@ struct XferJob {
 };
 
 inline int xfer_staged(fk_ctx *c, char *pin, void *dev, void *host, size_t bytes, bool down) {
-  XferJob job{c, pin, static_cast<char *>(dev), static_cast<char *>(host), bytes, 0, down};
-  // mid sizes in smaller pieces, so that a few threads share them; a thread
-  // for every two
-  job.piece = bytes >= 16 * kXferSlot ? kXferSlot : (bytes >= 4 * kXferSlot ? kXferSlot / 2 : kXferSlot / 4);
-  const size_t pieces = (bytes + job.piece - 1) / job.piece;
-  const int nt = (int)(pieces / 2 < (size_t)kXferThreads ? pieces / 2 : kXferThreads);
+  const XferPlan plan(bytes);
+  XferJob job{c, pin, static_cast<char *>(dev), static_cast<char *>(host), bytes, down, plan.piece};
+  const int nt = plan.threads;
   std::thread th[kXferThreads];
   for (int t = 1; t < nt; ++t) {
     try {
@@ -226,14 +248,14 @@ inline int xfer_staged(fk_ctx *c, char *pin, void *dev, void *host, size_t bytes
 inline bool xfer_aligned(const void *dev) { return reinterpret_cast<uintptr_t>(dev) % 16 == 0; }
 inline int copy_down(fk_ctx *c, void *host, const void *dev, size_t bytes) {
   if (bytes >= kXferMinDown && xfer_aligned(dev))
-    if (char *pin = xfer_begin(c)) return xfer_staged(c, pin, const_cast<void *>(dev), host, bytes, true);
+    if (char *pin = xfer_begin(c, bytes)) return xfer_staged(c, pin, const_cast<void *>(dev), host, bytes, true);
   HIPCHK(hipStreamSynchronize(c->stream));
   HIPCHK(hipMemcpy(host, dev, bytes, hipMemcpyDeviceToHost));
   return FK_OK;
 }
 inline int copy_up(fk_ctx *c, void *dev, const void *host, size_t bytes) {
   if (bytes >= kXferMinUp && xfer_aligned(dev))
-    if (char *pin = xfer_begin(c)) return xfer_staged(c, pin, dev, const_cast<void *>(host), bytes, false);
+    if (char *pin = xfer_begin(c, bytes)) return xfer_staged(c, pin, dev, const_cast<void *>(host), bytes, false);
   HIPCHK(hipStreamSynchronize(c->stream));
   HIPCHK(hipMemcpy(dev, host, bytes, hipMemcpyHostToDevice));
   return FK_OK;

@@ -64,14 +64,17 @@ struct Stream {
 };
 typedef Stream *hipStream_t;
 inline thread_local struct { unsigned x; } blockIdx, threadIdx;
+inline size_t g_pin_bytes = 0, g_pins = 0;                   // page-locked now, and how often
 inline unsigned g_pin_flags = 0, g_memcpys = 0, g_stale = 0;  // g_stale: what new device memory holds
 inline std::function<void()> g_late;                         // the null stream's clearing, not done yet
 inline hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) {
   g_pin_flags = flags;
+  g_pin_bytes = n;
+  ++g_pins;
   *p = aligned_alloc(4096, (n + 4095) / 4096 * 4096);
   return hipSuccess;
 }
-inline hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
+inline hipError_t hipHostFree(void *p) { free(p); g_pin_bytes = 0; return hipSuccess; }
 template <typename T>
 inline hipError_t hipMalloc(T **p, size_t n) {
   *p = static_cast<T *>(aligned_alloc(4096, (n + 4095) / 4096 * 4096));
@@ -244,4 +247,27 @@ def test_only_aligned_device_memory_is_copied_in_wide_words(run):
       say(g_memcpys == (off % 16 ? 2 : 0), off % 16 ? "by hipMemcpy" : "through the slots");
     }
   }
+""")
+
+
+def test_no_more_is_page_locked_than_the_copy_uses(run):
+    """Page-locking takes up to 2 ms for 64 MB, which a program's first copy
+    pays: it locks what its own pieces go through, a larger copy later what it
+    needs, and a smaller one nothing."""
+    run("""
+  const size_t mb = (size_t)1 << 20;
+  std::vector<char> in = pattern(100 * mb + 7, 5), out(100 * mb + 7);
+  char *dev = device(100 * mb + 7);
+  size_t pins = 0, locked = 0;
+  for (size_t n : {6 * mb + 3, 18 * mb, 40 * mb, 7 * mb, 100 * mb + 7, 20 * mb}) {
+    say(copy_up(c, dev, in.data(), n) == FK_OK && copy_down(c, out.data(), dev, n) == FK_OK &&
+        std::memcmp(out.data(), in.data(), n) == 0, "copied");
+    say(g_pin_bytes <= 2 * n && g_pin_bytes <= 65 * mb || g_pins == pins, "locked by need");
+    say(g_pin_bytes >= locked, "kept");
+    pins = g_pins;
+    locked = g_pin_bytes;
+  }
+  say(pins <= 4, "locked anew for larger copies alone");
+  g_xfer.detach();
+  say(g_pin_bytes == 0, "given back");
 """)
