@@ -88,7 +88,7 @@ constexpr int64_t kChemGroup = 65536, kPolishGroup = 49152;
 // blocks for one lane alone, groups of 8 took eight rounds of a full list and
 // lost to one lane (16k chemical cells 475 us, their polish 94); more than 512
 // gain nothing on full lists and cost each step with short ones (fallback of
-// 373k hexahedra with 1024 blocks 1 us more than with 256, with 512 0.5).
+// 373k hexahedra with 1024 blocks 1 us more than with 256, with 512 0.7).
 inline unsigned list_blocks(int64_t nc, int lanes) {
   const int64_t most = std::max<int64_t>(std::min<int64_t>(grid_for(nc * lanes), 512), std::min<int64_t>(grid_for(nc), 1024));
   return (unsigned)std::max<int64_t>(1, most);
